@@ -111,44 +111,47 @@ struct TileCfg {
     const char *name;
     int bm, bn;
     int resident;  // workgroups that fit a CU at once (registers / LDS)
-    // Fraction of the MFMA rate the inner loop sustains with a full CU, by operand layout (measured
-    // on the AlexNet layer shapes): [0] A along r, B along j (forward); [1] both along their free
-    // index (gradInput); [2] both along r (gradWeight); [3] A along i, B along r; [4] A along r, B gathered
-    // (the 64-row tiles: narrow gathered products run faster on the small tile, products on columns do not).  The figures are fitted to
-    // measured launch times together with the occupancy factors of model_cycles.
+    // Fraction of the MFMA rate (kFlopsPerCycle) the inner loop sustains with a full CU, by operand layout: [0] A along r, B along j (forward); [1] both along their free
+    // index (gradInput); [2] both along r (gradWeight); [3] A along i, B along r; [4] A along r, B gathered.
+    // Measured like the occupancy tables below.  None is near 1: on uniform random operands these kernels are held by the
+    // card's power, not by its issue slots (the clock falls to about 1.6 GHz; the same launches on zeros run a fifth
+    // faster), as is the library's bf16 product (1.13 PFLOP/s at 8192^3, which is 189 TFLOP/s at six products each).
     double eff[5];
     int (*launch)(const GemmArgs &, int, int, bool, hipStream_t);
-    // Fraction of that rate kept with k = 1..4 workgroups resident per CU (nullptr: the tables of model_cycles), and
-    // the row count from which the tile is no longer considered (0: no limit).
+    // Fraction of that rate kept with k = 1..4 workgroups resident per CU, and the row count from which the tile is no longer considered (0: no limit).
     const double *occ;
     int below_rows;
-    // Short-row variant: the rows of the tile its wavefronts multiply (0: all of them).  It takes scattered products
-    // of exactly one tile of rows, of which no more than this many are in use.
+    // Scattered products of exactly one tile of rows, of which no more than this many are in use (0: any product).  The
+    // kernel is that of the 64-row tile of the same width.
     int rows_used;
     // The tile has no loader for a first operand contiguous along its rows.
     bool a_rc_only;
 };
 
-// The 64 x 128 tile's wavefronts own 64 x 32 outputs, half the MFMAs per reduction step of the large tiles: it needs all
-// four workgroups on a CU to keep the matrix pipe busy (measured on the 64-row products of the AlexNet-style stack: the
-// 64 x 4800 gathered gradInput runs 10 % faster in seven splits that fill every round than unsplit with three
-// workgroups per CU).  Taller tiles re-read the second operand less often, so it only stands in where they do not fit.
-const double kOccNarrow[5] = {0.0, 0.50, 0.75, 0.88, 1.0};
+// Rate kept with k workgroups on a CU, by tile: measured on 3x3 forward products of 2304 reduction indices and exactly
+// k workgroups per CU (128 x 128: 111, 168, 186 TFLOP/s with one, two, three).
+const double kOcc2[5] = {0.0, 0.74, 1.0};
+const double kOcc3[5] = {0.0, 0.60, 0.90, 1.0};
+const double kOcc4[5] = {0.0, 0.52, 0.83, 0.94, 1.0};
+const double kOccSmall[5] = {0.0, 0.40, 0.76, 0.93, 1.0};
 
 const TileCfg kCfgs[] = {
-    {"128x128", 128, 128, 4, {0.90, 0.90, 0.88, 0.86, 0.90}, gemm_fast_128x128, nullptr, 0, 0, false},
-    {"192x128", 192, 128, 3, {0.90, 0.90, 0.90, 0.86, 0.90}, gemm_fast_192x128, nullptr, 0, 0, false},
-    {"64x256", 64, 256, 3, {0.76, 0.74, 0.90, 0.74, 0.70}, gemm_fast_64x256, nullptr, 0, 0, false},
-    {"128x256", 128, 256, 2, {0.85, 0.87, 0.95, 0.85, 0.85}, gemm_fast_128x256, nullptr, 0, 0, false},
-    {"256x128", 256, 128, 2, {0.90, 0.75, 0.95, 0.75, 0.90}, gemm_fast_256x128, nullptr, 0, 0, false},
-    {"64x64", 64, 64, 4, {0.68, 0.60, 0.74, 0.60, 0.72}, gemm_fast_64x64, nullptr, 0, 0, false},
-    {"64x128", 64, 128, 4, {0.84, 0.78, 0.84, 0.78, 0.86}, gemm_fast_64x128, kOccNarrow, 128, 0, false},
-    {"48x128", 64, 128, 4, {0, 0, 0, 0, 0.84}, gemm_fast_48x128, kOccNarrow, 128, 48, false},
-    {"48x256", 64, 256, 3, {0, 0, 0, 0, 0.70}, gemm_fast_48x256, nullptr, 0, 48, false},
-    {"96x128", 96, 128, 4, {0.84, 0, 0.84, 0, 0.86}, gemm_fast_96x128, kOccNarrow, 128, 0, true},
+    {"128x128", 128, 128, 3, {0.44, 0.44, 0.44, 0.44, 0.45}, gemm_fast_128x128, kOcc3, 0, 0, false},
+    {"192x128", 192, 128, 2, {0.43, 0.43, 0.43, 0.43, 0.44}, gemm_fast_192x128, kOcc2, 0, 0, false},
+    {"64x256", 64, 256, 2, {0.38, 0.38, 0.38, 0.38, 0.40}, gemm_fast_64x256, kOcc2, 0, 0, false},
+    {"128x256", 128, 256, 2, {0.46, 0.46, 0.46, 0.46, 0.47}, gemm_fast_128x256, kOcc2, 0, 0, false},
+    {"256x128", 256, 128, 2, {0.46, 0.46, 0.46, 0.46, 0.47}, gemm_fast_256x128, kOcc2, 0, 0, false},
+    {"64x64", 64, 64, 4, {0.32, 0.32, 0.32, 0.32, 0.33}, gemm_fast_64x64, kOccSmall, 0, 0, false},
+    {"64x128", 64, 128, 4, {0.38, 0.38, 0.38, 0.38, 0.39}, gemm_fast_64x128, kOcc4, 128, 0, false},
+    {"48x128", 64, 128, 4, {0, 0, 0, 0, 0.38}, gemm_fast_64x128, kOcc4, 128, 48, false},
+    {"48x256", 64, 256, 2, {0, 0, 0, 0, 0.38}, gemm_fast_64x256, kOcc2, 0, 48, false},
+    {"96x128", 96, 128, 3, {0.40, 0, 0.40, 0, 0.42}, gemm_fast_96x128, kOcc3, 128, 0, true},
 };
 
 inline long cdiv(long a, long b) { return (a + b - 1) / b; }
+
+// Flops a CU retires per cycle with six bf16 products for one fp32 product: 4096 / 6.
+constexpr double kFlopsPerCycle = 4096.0 / 6.0;
 
 // Rough time model (in CU-cycles) used only to rank (tile, split) candidates.
 // A CU retires 256 flops per cycle at best; with fewer workgroups resident it
@@ -156,15 +159,11 @@ inline long cdiv(long a, long b) { return (a + b - 1) / b; }
 // run in further rounds; every round pays a prologue/epilogue; a split adds
 // the traffic of writing and re-reading the partial sums.
 double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_total, int nsplit, int cus) {
-    // With both operands along r (layout 2) two resident workgroups already keep the MFMA pipe as
-    // busy as three: measured on the 192 x 1600 gradWeight product, 39 splits (two per CU) beat 59.
-    static const double kOccDefault[5] = {0.0, 0.70, 0.88, 0.96, 1.0};
-    static const double kOccBothR[5] = {0.0, 0.70, 0.98, 0.96, 1.0};
-    const double *kOcc = c.occ ? c.occ : layout == 2 ? kOccBothR : kOccDefault;
+    const double *kOcc = c.occ;
     const long tiles = cdiv(M, c.bm) * cdiv(J, c.bn);
     const long wgs = tiles * nsplit;
     const long steps = cdiv(steps_total, nsplit);
-    const double per_step = 2.0 * (c.rows_used ? c.rows_used : c.bm) * c.bn * GEMM_BK / 256.0 / c.eff[layout];
+    const double per_step = 2.0 * c.bm * c.bn * GEMM_BK / kFlopsPerCycle / c.eff[layout];
     const double ovh = 3000.0 + 6.0 * c.bm * c.bn / 64.0;
     const long slots = (long)cus * c.resident;
     const long full = wgs / slots, rest = wgs - full * slots;
@@ -174,7 +173,7 @@ double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_tot
         const int k = (int)(on_busiest < c.resident ? on_busiest : c.resident);
         t += on_busiest * steps * per_step / kOcc[k] + ovh * (k > 1 ? 1.0 : 1.5);
     }
-    if (nsplit > 1) t += (double)(nsplit + 2) * M * J * 4.0 / (4.5e12 / 2.4e9);  // bytes / (bytes per cycle)
+    if (nsplit > 1) t += 5000.0 + (double)(nsplit + 2) * M * J * 4.0 / (4.5e12 / 2.4e9);  // launch, bytes / (bytes per cycle)
     return t;
 }
 
@@ -231,10 +230,15 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
             const int sps = (int)cdiv(steps_total, ns);
             if ((int)cdiv(steps_total, sps) != ns) continue;  // would leave an empty split
             const double t = model_cycles(c, layout, p.M, p.J, steps_total, ns, cus);
-            if (!plan.cfg || t < best_t) {
+            // A product with tiles for less than half the chip is split anyway: there, of plans that the model puts
+            // within 2 % of each other, the one split further is the more exact (every addition to an accumulator is
+            // rounded; a 128 x 9216 product over 4096: relative error 3.7e-7 in seven parts, 2.7e-7 in fourteen, 63 us either
+            // way).  Larger products take the fastest: preferring more parts everywhere cost the AlexNet-style step 6 %.
+            const bool few = p.nb <= 1 && 2 * tiles <= cus;
+            if (!plan.cfg || t < best_t * (!few || ns == plan.nsplit ? 1.0 : ns > plan.nsplit ? 1.02 : 0.98)) {
+                if (!plan.cfg || t < best_t) best_t = t;
                 plan.cfg = &c;
                 plan.nsplit = ns;
-                best_t = t;
             }
         }
     }

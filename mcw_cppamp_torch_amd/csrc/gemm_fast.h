@@ -1,40 +1,46 @@
-// The fast fp32 MFMA GEMM kernel (see gemm_mfma.h for the problem statement).
-// Included by one small translation unit per tile configuration.
+// The tiled fp32 GEMM kernel (see gemm_mfma.h for the problem statement): fp32 operands, fp32 sums and results, with the
+// products formed on the bf16 matrix instructions.
+//
+// Every operand element is split without loss into three bf16 parts, x = h + m + l: h is x rounded to nearest, m the
+// remainder rounded, l what is left (8 + 8 + 8 significant bits hold the 24 of an fp32 number).  A product a*b is the sum
+// of the part products that matter in fp32, h*h + (h*m + m*h) + (h*l + m*m + l*h), each exact in the fp32 accumulator's
+// input; the three dropped ones are below 2^-24 of the product together, and of either sign.  That is six
+// v_mfma_f32_32x32x16_bf16 where eight v_mfma_f32_32x32x2_f32 of twice the cycles each stood: 2.7 times the matrix
+// rate (dense bf16 runs at 16 times the fp32 rate).  An accumulator also takes 6 rounded additions per 16 reduction
+// indices instead of 16.
+//
+// Measured against the fp32-instruction kernel that stood here (uniform random operands): forward of 64 -> 128 planes, 9x9,
+// 128 images of 64x64: 4.2 -> 2.5 ms (128 -> 213 TFLOP/s); AlexNet-style step at batch 128: 4.51 -> 3.23 ms; error against
+// 64 bits over 3x3 to 11x11 layers and Linear products: 0.6 to 1.0 of the former (uniform operands).  What bounds it now is
+// power: see the efficiency figures in gemm_dispatch.hip.
+//
+// What the split cannot hold is multiplied in fp32 instead: an operand that is infinite, NaN or so large that h
+// rounds to infinity leaves an infinity or NaN in every accumulator it reaches, and a product sum that falls
+// below the normal numbers leaves a denormal.  A wavefront that finds one of these in a 32x32 block at the end computes
+// the block again from the operands with v_mfma_f32_32x32x2_f32 (recompute_block).  Operands below 2^-109 in
+// magnitude keep an absolute error of 2^-134 (the smallest bf16 step), which only such a sum can notice.
 //
 // Structure
 //   * A workgroup of WGM x WGN wavefronts owns a BM x BN tile of C, each
-//     wavefront TM x TN blocks of 32x32 outputs, one v_mfma_f32_32x32x2_f32
-//     accumulator (16 registers per lane) per block.
+//     wavefront TM x TN blocks of 32x32 outputs, one accumulator (16 registers per lane) per block.
 //   * No bounds checks and no branches around loads.  A tile at the lower/right
 //     edge is shifted back so that it lies inside the matrix and stores only the
 //     rows/columns no other tile owns; a reduction step that would run past R is
 //     shifted back to end at R and the part the previous step already covered
 //     is zeroed on its way to LDS.  Needs M >= BM, J >= BN, R >= 16; smaller
 //     problems take the bounds-checked generic kernel.
-//   * LDS holds both operand tiles as [x][r] (x the free index, r the
-//     reduction index).  Each lane fetches its MFMA operands with 128-bit LDS
-//     reads: lane (x, h) reads r = 8h .. 8h+7, and MFMA step s takes r = s from
-//     the lower half-wave and r = 8 + s from the upper one.  A and B use the
-//     same permutation of r, so the sum over r is unchanged.  The row layout
-//     follows the operand's loader, so that its 128-bit LDS writes and the
-//     operand reads are both free of bank conflicts (the LDS conflict counter
-//     reads zero for either): a tile written a column at a time (consecutive
-//     lanes = consecutive rows) has rows of 16 + 4 floats; a tile written a row
-//     at a time (four lanes per row) has rows of 16 floats whose four 16-byte
-//     quarters are stored at quarter (r/4) xor ((x/4) mod 4).
-//   * LDS is double buffered; the next tile's global loads are issued between
-//     the current tile's MFMAs and written to the other buffer afterwards: one
-//     barrier per reduction step.
-//   * Two variants for row counts the 32-row blocks fit badly: ROWS16 (16x16 blocks over the first 48 rows of a
-//     64-row tile, scattered products only) and the 96-row tile, whose first-operand loads the threads do not divide.
-//   * Between the MFMAs of a step there are memory and scalar instructions only.
-//     fp32 MFMAs and ordinary vector instructions share the SIMD's ALU (a v_add
-//     between two MFMAs costs 6 to 13 cycles of matrix time, measured), and a
-//     wavefront with MFMAs to issue keeps the other wavefronts of its SIMD from
-//     issuing anything, so nothing the loop does is hidden by another wavefront:
-//     operands are fetched with buffer loads (descriptor and offsets in scalar
-//     registers, a constant lane offset), and the loop is unrolled by two so
-//     that the LDS buffer folds into the offset field of the LDS instructions.
+//   * The split is made once per element and workgroup, on the way from registers to LDS.  LDS holds the parts of both
+//     operand tiles as [part][octet][x] units of eight bf16 (x the free index, octet = r/8): lane (x, h) of a wavefront
+//     fetches its MFMA operand, r = 8h .. 8h+7 of row x, with one 128-bit read, consecutive lanes from
+//     consecutive units.  The octet planes are 128 bytes longer than their rows need, so that the 64-bit writes of a
+//     tile loaded four lanes to a row fall on different banks too.
+//   * LDS is double buffered and the global loads run one step further ahead: while step s is multiplied, the
+//     registers hold step s+1, which is split and written to the other buffer in slices between the MFMAs, and every
+//     register is refilled for step s+2 as soon as it has been split: one barrier per reduction step, and a load has a
+//     whole step to arrive.
+//   * Operands are fetched with buffer loads (descriptor and offsets in scalar registers, a constant lane offset), and
+//     the loop is unrolled by two so that the LDS buffer folds into the offset field of the LDS instructions: the only
+//     vector instructions of the loop are the split's (11 per two elements).
 #pragma once
 
 #include <type_traits>
@@ -48,37 +54,32 @@ namespace thgpu {
 // 64 consecutive rows; lanes run along the rows.
 constexpr int LD_XC_BLOCK = 3;
 
-// LDS row layout by loader kind: pitch in floats, and the column at which element r of row x is stored.
-//
-// Measured on this hardware with eight wavefronts issuing nothing else: a conflict-free ds_read_b128 takes 4 cycles
-// per wavefront and is served sixteen lanes at a time, where the sixteen are lanes 0-3, 12-15, 20-23, 24-27, then
-// 4-7, 8-11, 16-19, 28-31 (likewise in the upper half-wave), over 64 banks; a ds_write_b128 is served eight
-// consecutive lanes at a time, whose 16-byte units must differ modulo 128 bytes.  Hence:
-//   * 32x32 blocks (lane l reads row l%32, quarter pair l/32): rows written a column at a time (consecutive lanes =
-//     consecutive rows) are padded to 20 floats; rows written four lanes to a row keep 16 floats, quarter q of row x
-//     stored at q xor (x/4)%4.  Reads and writes of both are conflict-free (the conflict counter reads zero).
-//   * 16x16 blocks (SMALL16: lane l reads row l%16, quarter l/16): the row-written tile stores quarter q of row x
-//     at p(q) xor (x/4)%4 with p = (0, 3, 1, 2), conflict-free both ways (the plain xor puts rows 0-3 and rows 4-7
-//     of two lane quarters on the same banks).  The column-written tile keeps its 20-float rows: its writes need
-//     an odd pitch in 16-byte units, and no placement of four quarters in such a row also frees these reads of
-//     conflicts; they take 8 cycles instead of 4, two of a step's five operand reads.
-template <int KIND, bool SMALL16 = false>
-struct LdsRow {
-    static constexpr bool kSwizzled = KIND == LD_RC_VEC;
-    static constexpr int kPitch = kSwizzled ? GEMM_BK : GEMM_BK + 4;
-    __device__ static __forceinline__ int col(int x, int r) {
-        if (!kSwizzled) return r;
-        const int q = SMALL16 ? (0x9C >> (2 * (r >> 2))) & 3 : r >> 2;
-        return (r & 3) | (((q ^ (x >> 2)) & 3) << 2);
-    }
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+// Bytes of one octet plane of an X-row operand tile, of one part of it, and of the whole tile.
+template <int X>
+struct PartTile {
+    static constexpr int kOctet = X * 16 + 128;
+    static constexpr int kPart = 2 * kOctet;
+    static constexpr int kBytes = 3 * kPart;
 };
 
-// Four floats at a 4-byte aligned address: the hardware handles the
-// misalignment of a 128-bit global load; the type only keeps the compiler from
-// assuming 16-byte alignment.
-struct __attribute__((packed, aligned(4))) float4u {
-    float x, y, z, w;
-};
+// The three parts of two elements, two bf16 to a word.
+__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
+    auto round2 = [](float a, float b) {
+        return __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){a, b}, bf16x2));
+    };
+    auto low = [](unsigned p) { return __builtin_bit_cast(float, p << 16); };
+    auto high = [](unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); };
+    h = round2(x0, x1);
+    const float r0 = x0 - low(h), r1 = x1 - high(h);
+    m = round2(r0, r1);
+    l = round2(r0 - low(m), r1 - high(m));
+}
 
 // Wavefronts per SIMD the register allocation must leave room for: the
 // accumulators take (BM/WGM)*(BN/WGN)/64 registers of the 512 a lane has.
@@ -87,24 +88,18 @@ constexpr int gemm_min_waves() {
     return (BM / WGM) * (BN / WGN) / 64 >= 96 ? 2 : 3;
 }
 
-// ROWS16 > 0 selects the short-row variant: the workgroup still loads BM = 64 rows of the first operand, but its
-// wavefronts multiply only the first 16*ROWS16 of them, in 16x16 blocks (v_mfma_f32_16x16x4_f32, four registers per
-// lane and block).  It exists for scattered products whose row count is 48 (three planes at stride 4 x 4), which
-// would otherwise spend a quarter of their MFMAs on padding; it has the scattered store only.
-template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int ROWS16 = 0>
+template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED>
 __global__ __launch_bounds__(WGM *WGN * 64)
     __attribute__((amdgpu_waves_per_eu(gemm_min_waves<BM, BN, WGM, WGN>()))) void gemm_fast_kernel(const GemmArgs g) {
     constexpr int NT = WGM * WGN * 64;
     constexpr int BK = GEMM_BK;
-    constexpr bool SMALL = ROWS16 > 0;
-    constexpr int TM = SMALL ? ROWS16 : BM / WGM / 32, TN = SMALL ? BN / WGN / 16 : BN / WGN / 32;
-    static_assert(!SMALL || (WGM == 1 && BM == 64 && ROWS16 <= 4 && LB == LD_XC_GATHER && !RED && TN % 2 == 0),
-                  "the short-row variant: one row of wavefronts over a 64-row tile, gathered B, scattered store");
+    constexpr int TM = BM / WGM / 32, TN = BN / WGN / 32;
     // A first operand along r whose 128-bit loads the threads do not divide (96 rows: 384 loads, 256 threads): the
     // last round of loads is made by the leading wavefronts only (a uniform branch; wavefront w loads rows
     // 16w .. 16w+15 of every 64).
     constexpr bool PART_A = LA == LD_RC_VEC && (BM * BK) % (NT * 4) != 0;
     constexpr int NA = PART_A ? (BM * BK + NT * 4 - 1) / (NT * 4) * 4 : BM * BK / NT, NB = BN * BK / NT;
+    static_assert(BK == 16, "two octets of reduction indices per step");
     static_assert(!PART_A || (NT == 256 && BM % 16 == 0), "partial loader shape");
     static_assert(BM % (WGM * 32) == 0 && BN % (WGN * 32) == 0, "wave tile must be whole 32x32 blocks");
     static_assert(NT % 16 == 0 && NA >= 4 && NB >= 4 && NA % 4 == 0 && NB % 4 == 0, "loader shape");
@@ -118,10 +113,10 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     static_assert(!RED || (LA != LD_XC_SCALAR && LB != LD_XC_SCALAR),
                   "reduction batching needs r-contiguous or gathered operands");
 
-    using RowA = LdsRow<KA, SMALL>;
-    using RowB = LdsRow<LB, SMALL>;
-    __shared__ __attribute__((aligned(16))) float As[2][BM][RowA::kPitch];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BN][RowB::kPitch];
+    using TileA = PartTile<BM>;
+    using TileB = PartTile<BN>;
+    __shared__ __attribute__((aligned(16))) char As[2][TileA::kBytes];
+    __shared__ __attribute__((aligned(16))) char Bs[2][TileB::kBytes];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: row bases stay uniform
@@ -152,7 +147,6 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     // ---- loader set-up -------------------------------------------------------------
     // Thread -> (x, r) of its first element inside an operand tile:
     //   LD_RC_VEC     x = tid/4 (+64 per load), r = 4*(tid%4) .. +3   (one 128-bit load each)
-    //   LD_RC_SCALAR  x = tid/16 (+16 per load), r = tid%16
     //   LD_XC_SCALAR  x = tid % X, r = (tid / X) * CNT .. + CNT-1     (CNT loads down the column)
     //   LD_XC_BLOCK   x = lane (+64 per block of rows), r = 4*wave .. +3
     // A load address is a wave-uniform base (tile, image, step, load number: all
@@ -172,8 +166,8 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         voffA = (unsigned)(((long)a_r * g.sA + a_x) * 4);
         tileA = reinterpret_cast<const char *>(g.A + i0);
     } else {
-        a_x = LA == LD_RC_VEC ? tid >> 2 : tid >> 4;
-        a_r = LA == LD_RC_VEC ? (tid & 3) * 4 : tid & 15;
+        a_x = tid >> 2;
+        a_r = (tid & 3) * 4;
         voffA = (unsigned)(((long)a_x * g.sA + a_r) * 4);
         tileA = reinterpret_cast<const char *>(g.A + (long)i0 * g.sA);
     }
@@ -194,40 +188,37 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         voffB = (unsigned)(((long)b_r * g.sB + (long)(img - img0) * g.bsB + n) * 4);
         tileB = reinterpret_cast<const char *>(g.B + (long)img0 * g.bsB);
     } else {
-        b_x = LB == LD_RC_VEC ? tid >> 2 : tid >> 4;
-        b_r = LB == LD_RC_VEC ? (tid & 3) * 4 : tid & 15;
+        b_x = tid >> 2;
+        b_r = (tid & 3) * 4;
         voffB = (unsigned)(((long)b_x * g.sB + b_r) * 4);
         tileB = reinterpret_cast<const char *>(g.B + (long)j0 * g.sB);
     }
     constexpr int UA = LA == LD_RC_VEC ? NA / 4 : NA;  // load instructions per step and operand
     constexpr int UB = LB == LD_RC_VEC ? NB / 4 : NB;
 
-    // One accumulator per block: 16 registers (32x32 blocks) or 4 (16x16 blocks of the short-row variant).
-    using Acc = std::conditional_t<SMALL, floatx4, floatx16>;
-    constexpr int ACCV = SMALL ? 4 : 16;
-    Acc acc[TM][TN];
+    floatx16 acc[TM][TN];
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
         for (int b = 0; b < TN; ++b)
 #pragma unroll
-            for (int v = 0; v < ACCV; ++v) acc[a][b][v] = 0.0f;
+            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
 
     // Row sums of the first operand (GemmProblem::rowsum), reduction batching only.  The column tiles of a row of
     // tiles all load the same first-operand tiles, so they share the work: the workgroup of column tile tj sums the
-    // steps whose index is tj modulo the number of column tiles, from the MFMA operands its first column of
-    // wavefronts holds in registers anyway (lane (x, h) holds r = 8h .. 8h+7 of row x).  A handful of vector adds
-    // every tilesJ-th step; the partial sums go to rowsum_ws[row][split * tilesJ + tj].
-    float bsum[TM];
+    // steps whose index is tj modulo the number of column tiles, from the registers the loads arrive in (fp32, before the
+    // split; thread t holds four elements of row t/4 of every 64).  A handful of vector adds every tilesJ-th step; the
+    // partial sums go to rowsum_ws[row][split * tilesJ + tj].
+    constexpr int RS = RED ? NA / 4 : 1;
+    float bsum[RS];
 #pragma unroll
-    for (int a = 0; a < TM; ++a) bsum[a] = 0.0f;
-    const bool rs_on = RED && !SMALL && g.rowsum_ws != nullptr && wn == 0;
+    for (int q = 0; q < RS; ++q) bsum[q] = 0.0f;
+    const bool rs_on = RED && g.rowsum_ws != nullptr;
     int rs_next = 0;
     if (rs_on) rs_next = (int)(((unsigned)tj + g.tilesJ - (unsigned)step % g.tilesJ) % g.tilesJ);
 
     float ra[NA], rb[NB];
     auto a_unit_live = [&](int u) { return !PART_A || u * (NT / 4) + 16 * wave < BM; };
-    auto always_live = [](int) { return true; };
     if (PART_A) {
 #pragma unroll
         for (int q = 0; q < NA; ++q) ra[q] = 0.0f;
@@ -239,10 +230,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
 
     // Load number u of an operand for the step whose uniform base is `base`.  Buffer loads: the address is a
     // descriptor in scalar registers (the step's base) plus a scalar offset (which load) plus the lane's constant
-    // 32-bit offset, so the loop spends no vector ALU instruction on addressing.  That matters more than its
-    // instruction count suggests: fp32 MFMAs and ordinary vector instructions share the SIMD's ALU (a v_add
-    // between two MFMAs costs 6 to 13 cycles of matrix-pipe time, measured), while scalar instructions and the
-    // issue of memory instructions run beside the matrix pipe.
+    // 32-bit offset, so the loop spends no vector ALU instruction on addressing.
     typedef float float4v __attribute__((ext_vector_type(4)));
     auto descriptor = [](const char *base) {
         // raw buffer, no bounds (every offset below 2^32 passes), dword format
@@ -260,8 +248,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
             dst[u * 4 + 2] = v.z;
             dst[u * 4 + 3] = v.w;
         } else {
-            const int so = KIND == LD_RC_SCALAR  ? u * (NT / 16) * st
-                           : KIND == LD_XC_BLOCK ? (u & 3) * st + (u >> 2) * 256
+            const int so = KIND == LD_XC_BLOCK    ? (u & 3) * st + (u >> 2) * 256
                            : KIND == LD_XC_GATHER ? roff[u] * 4
                                                   : u * st;
             dst[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)voff, so, 0));
@@ -318,186 +305,231 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         constexpr int CNT = decltype(count_tag)::value;
 #pragma unroll
         for (int q = 0; q < CNT; ++q) {
-            const int rel = (KIND == LD_RC_VEC || KIND == LD_XC_BLOCK) ? t_r + (q & 3)
-                            : KIND == LD_RC_SCALAR                          ? t_r
-                                                                            : t_r + q;
+            const int rel = (KIND == LD_RC_VEC || KIND == LD_XC_BLOCK) ? t_r + (q & 3) : t_r + q;
             v[q] = rel < shift ? 0.0f : v[q];
         }
     };
-
-    auto stash_one = [&](auto kind_tag, auto tile, int t_x, int t_r, const float *src, auto count_tag, auto live) {
-        constexpr int KIND = decltype(kind_tag)::value;
-        using Row = LdsRow<KIND, SMALL>;
-        constexpr int CNT = decltype(count_tag)::value;
-        if (KIND == LD_RC_VEC) {
-#pragma unroll
-            for (int q = 0; q < CNT / 4; ++q)
-                if (live(q))
-                    *reinterpret_cast<float4 *>(&tile[t_x + q * (NT / 4)][Row::col(t_x + q * (NT / 4), t_r)]) =
-                        make_float4(src[q * 4], src[q * 4 + 1], src[q * 4 + 2], src[q * 4 + 3]);
-        } else if (KIND == LD_RC_SCALAR) {
-#pragma unroll
-            for (int q = 0; q < CNT; ++q) tile[t_x + q * (NT / 16)][Row::col(t_x + q * (NT / 16), t_r)] = src[q];
-        } else if (KIND == LD_XC_BLOCK) {
-#pragma unroll
-            for (int w = 0; w < CNT / 4; ++w)
-                *reinterpret_cast<float4 *>(&tile[t_x + 64 * w][Row::col(t_x + 64 * w, t_r)]) =
-                    make_float4(src[w * 4], src[w * 4 + 1], src[w * 4 + 2], src[w * 4 + 3]);
-        } else {
-#pragma unroll
-            for (int w = 0; w < CNT / 4; ++w)
-                *reinterpret_cast<float4 *>(&tile[t_x][Row::col(t_x, t_r + 4 * w)]) =
-                    make_float4(src[w * 4], src[w * 4 + 1], src[w * 4 + 2], src[w * 4 + 3]);
-        }
-    };
-    auto stash = [&](int buf, int shift) {
+    auto mask_step = [&](int shift) {
         if (shift > 0) {  // uniform: only the last step of an image can be partial
             mask_one(std::integral_constant<int, KA>{}, a_r, ra, std::integral_constant<int, NA>{}, shift);
             mask_one(std::integral_constant<int, LB>{}, b_r, rb, std::integral_constant<int, NB>{}, shift);
         }
-        stash_one(std::integral_constant<int, KA>{}, As[buf], a_x, a_r, ra, std::integral_constant<int, NA>{}, a_unit_live);
-        stash_one(std::integral_constant<int, LB>{}, Bs[buf], b_x, b_r, rb, std::integral_constant<int, NB>{}, always_live);
     };
 
-    // ---- prologue: first step ---------------------------------------------------------
+    // Splits group number q of a thread's elements and writes the parts to LDS.  A group is eight elements of a row
+    // where the loader gives a thread whole octets, otherwise four.
+    constexpr int GA = (KA == LD_XC_SCALAR && NA % 8 == 0) ? 8 : 4;
+    constexpr int GB = (LB != LD_RC_VEC && NB % 8 == 0) ? 8 : 4;
+    char *const a_dst = &As[0][0] + (a_r >> 3) * TileA::kOctet + a_x * 16 + (a_r & 7) * 2;
+    char *const b_dst = &Bs[0][0] + (b_r >> 3) * TileB::kOctet + b_x * 16 + (b_r & 7) * 2;
+    auto stash_group = [&](auto kind_tag, auto group_tag, auto tile_tag, char *dst, const float *src, int q) {
+        constexpr int KIND = decltype(kind_tag)::value;
+        constexpr int G = decltype(group_tag)::value;
+        using Tile = decltype(tile_tag);
+        // four-element groups lie in rows apart (LD_RC_VEC: 64 rows a load, LD_XC_BLOCK: the next 64 rows)
+        const int off = G == 8 ? q * Tile::kOctet : (KIND == LD_RC_VEC ? q * (NT / 4) : q * 64) * 16;
+        static_assert(G == 8 || KIND == LD_RC_VEC || KIND == LD_XC_BLOCK || decltype(group_tag)::value == 4, "group");
+        unsigned p[3][G / 2];
+#pragma unroll
+        for (int e = 0; e < G / 2; ++e) split_pair(src[q * G + 2 * e], src[q * G + 2 * e + 1], p[0][e], p[1][e], p[2][e]);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            if constexpr (G == 8)
+                *reinterpret_cast<uintx4 *>(dst + off + t * Tile::kPart) = (uintx4){p[t][0], p[t][1], p[t][2], p[t][3]};
+            else
+                *reinterpret_cast<uintx2 *>(dst + off + t * Tile::kPart) = (uintx2){p[t][0], p[t][1]};
+        }
+    };
+    static_assert(GA == 8 || KA != LD_XC_SCALAR || NA == 4, "an x-contiguous loader of four elements has one group");
+    static_assert(GB == 8 || LB == LD_RC_VEC || NB == 4, "an x-contiguous loader of four elements has one group");
+    auto stash_a = [&](int buf, int q) {
+        if (GA == 8 || a_unit_live(q))
+            stash_group(std::integral_constant<int, KA>{}, std::integral_constant<int, GA>{}, TileA{},
+                        a_dst + buf * TileA::kBytes, ra, q);
+    };
+    auto stash_b = [&](int buf, int q) {
+        stash_group(std::integral_constant<int, LB>{}, std::integral_constant<int, GB>{}, TileB{},
+                    b_dst + buf * TileB::kBytes, rb, q);
+    };
+    constexpr int QA = NA / GA, QB = NB / GB;
+    // The loads that refill group q.
+    auto refill_a = [&](const char *base, int q) {
+        constexpr int PER = UA / QA;
+#pragma unroll
+        for (int u = q * PER; u < (q + 1) * PER; ++u)
+            if (a_unit_live(u)) load_unit(std::integral_constant<int, KA>{}, base, g.sA, voffA, ra, u);
+    };
+    auto refill_b = [&](const char *base, int q) {
+        constexpr int PER = UB / QB;
+#pragma unroll
+        for (int u = q * PER; u < (q + 1) * PER; ++u) load_unit(std::integral_constant<int, LB>{}, base, g.sB, voffB, rb, u);
+    };
+    auto add_row_sums = [&]() {
+        if constexpr (RED) {
+#pragma unroll
+            for (int q = 0; q < RS; ++q) bsum[q] += (ra[4 * q] + ra[4 * q + 1]) + (ra[4 * q + 2] + ra[4 * q + 3]);
+        }
+    };
+
+    // ---- prologue: the first step to LDS, the second to registers ---------------------
     const char *ga = tileA, *gb = tileB;
     int shift = 0;
     if (nsteps > 0) {
         fetch_rows(ld_r0);
         step_bases(ga, gb, shift);
 #pragma unroll
-        for (int u = 0; u < UA; ++u)
-            if (a_unit_live(u)) load_unit(std::integral_constant<int, KA>{}, ga, g.sA, voffA, ra, u);
+        for (int q = 0; q < QA; ++q) refill_a(ga, q);
 #pragma unroll
-        for (int u = 0; u < UB; ++u) load_unit(std::integral_constant<int, LB>{}, gb, g.sB, voffB, rb, u);
-        stash(0, shift);
+        for (int q = 0; q < QB; ++q) refill_b(gb, q);
         advance();
         fetch_rows(ld_r0);
+        mask_step(shift);
+        if (rs_on && rs_next == 0) {
+            add_row_sums();
+            rs_next = (int)g.tilesJ;
+        }
+#pragma unroll
+        for (int q = 0; q < QA; ++q) stash_a(0, q);
+#pragma unroll
+        for (int q = 0; q < QB; ++q) stash_b(0, q);
+        if (nsteps > 1) {
+            step_bases(ga, gb, shift);
+#pragma unroll
+            for (int q = 0; q < QA; ++q) refill_a(ga, q);
+#pragma unroll
+            for (int q = 0; q < QB; ++q) refill_b(gb, q);
+            advance();
+            fetch_rows(ld_r0);
+        }
     }
     __syncthreads();
 
     // ---- main loop ----------------------------------------------------------------------
-    // Step s computes from LDS buffer s&1 while the loads of step s+1 are issued
-    // in slices between its MFMAs (a steady trickle of requests; a burst at the
-    // head of the step would hold the wavefront, and with it its MFMAs, in the
-    // memory pipeline's queue) and written to the other buffer afterwards.
-    // Two steps per trip, one per LDS buffer, so that the buffer is a compile-time constant and folds into the
-    // offset field of every LDS instruction instead of costing vector adds per step.
+    // Step s multiplies from LDS buffer s&1.  Its six part products are six slices of MFMAs; between them the groups of
+    // step s+1 are split and written to the other buffer and their registers refilled for step s+2.
+    const char *const a_src = &As[0][0] + half * TileA::kOctet + (wm * (TM * 32) + l32) * 16;
+    const char *const b_src = &Bs[0][0] + half * TileB::kOctet + (wn * (TN * 32) + l32) * 16;
     auto one_step = [&](auto buf_tag, int s) {
         constexpr int buf = decltype(buf_tag)::value;
-        const bool more = s + 1 < nsteps;
-        const bool rs_hit = rs_on && s == rs_next;  // uniform
-        if (rs_hit) rs_next += (int)g.tilesJ;
-        // The last step has nothing to fetch; it re-reads the previous addresses
-        // (valid, cached) rather than branching around the loads.
+        // The last step splits registers that nobody will read and the last two load from the previous addresses
+        // (valid, cached) rather than branching around either.
+        const bool more = s + 2 < nsteps;
+        mask_step(shift);
+        if (rs_on && s + 1 == rs_next && s + 1 < nsteps) {  // uniform
+            add_row_sums();
+            rs_next += (int)g.tilesJ;
+        }
         if (more) step_bases(ga, gb, shift);
 
-        // What every slice of a step does besides its MFMAs: its share of the next step's loads, and the row
-        // offsets of the step after that (requested once every LDS operand of this step has arrived, so that the
-        // scalar loads share the wait counter with no outstanding LDS read; taken delivery of two slices later,
-        // still under this step's MFMAs).
-        constexpr int SLICES = 8;
-        auto slice_tail = [&](auto slice_tag) {
+        bf16x8 av[TM][3], bv[TN][3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {  // in the order of their first use
+            const int ta = u == 0 ? 2 : u - 1, tb = u == 0 ? 0 : 3 - u;
+#pragma unroll
+            for (int a = 0; a < TM; ++a)
+                av[a][ta] = *reinterpret_cast<const bf16x8 *>(a_src + buf * TileA::kBytes + ta * TileA::kPart + a * 512);
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+                bv[b][tb] = *reinterpret_cast<const bf16x8 *>(b_src + buf * TileB::kBytes + tb * TileB::kPart + b * 512);
+        }
+        constexpr int SLICES = 6;
+        auto slice_of = [&](auto slice_tag) {
             constexpr int slice = decltype(slice_tag)::value;
+            // lh hl mm mh hm hh: the small ones first, while a short sum is still small, so that a reduction of one step
+            // is rounded once at its full magnitude
+            constexpr int pa = slice == 0 ? 2 : slice == 2 || slice == 3 ? 1 : 0;
+            constexpr int pb = slice == 1 ? 2 : slice == 2 || slice == 4 ? 1 : 0;
 #pragma unroll
-            for (int u = 0; u < UA; ++u)
-                if (u * SLICES / UA == slice && a_unit_live(u))
-                    load_unit(std::integral_constant<int, KA>{}, ga, g.sA, voffA, ra, u);
+            for (int a = 0; a < TM; ++a)
 #pragma unroll
-            for (int u = 0; u < UB; ++u)
-                if (u * SLICES / UB == slice) load_unit(std::integral_constant<int, LB>{}, gb, g.sB, voffB, rb, u);
-            if (slice == 5) {
+                for (int b = 0; b < TN; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[a][pa], bv[b][pb], acc[a][b], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < QA; ++q)
+                if (q * SLICES / (QA + QB) == slice) {
+                    stash_a(buf ^ 1, q);
+                    refill_a(ga, q);
+                }
+#pragma unroll
+            for (int q = 0; q < QB; ++q)
+                if ((QA + q) * SLICES / (QA + QB) == slice) {
+                    stash_b(buf ^ 1, q);
+                    refill_b(gb, q);
+                }
+            if (slice == 3) {
                 int pos = ld_r0 + BK;
                 if (RED && pos >= g.R) pos = 0;
                 fetch_rows(pos);
             }
-            if (!RED && slice == 7) pin_rows();
+            if (!RED && slice == 5) pin_rows();
+            // One MFMA, then a few of the split's vector instructions under it (a 32x32x16 MFMA holds the matrix unit for 32
+            // cycles, a vector instruction issues in 4): 2 to 5 % over leaving them in clusters, with the 128 x 256 tile
+            // most (a 64-plane 9x9 layer's forward: 213 -> 219 TFLOP/s).  Nothing gained with reduction batching.
+            if constexpr (!RED && slice < 5) {
+#pragma unroll
+                for (int q = 0; q < TM * TN; ++q) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+                }
+            }
             __builtin_amdgcn_sched_barrier(0);
         };
-        auto component = [](const float4 &v, int e) { return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; };
-
-        if constexpr (SMALL) {
-            // 16x16 blocks: lane (x, q) reads r = 4q .. 4q+3 of its row and column with one 128-bit read each, and
-            // MFMA e takes r = 4q + e from quarter-wave q.
-            const int q4 = lane >> 4, l16 = lane & 15;
-            float4 av[TM], bv[TN];
-#pragma unroll
-            for (int a = 0; a < TM; ++a)
-                av[a] = *reinterpret_cast<const float4 *>(&As[buf][a * 16 + l16][RowA::col(l16, 4 * q4)]);
-#pragma unroll
-            for (int b = 0; b < TN; ++b)
-                bv[b] = *reinterpret_cast<const float4 *>(&Bs[buf][wn * (TN * 16) + b * 16 + l16][RowB::col(l16, 4 * q4)]);
-            auto half_slice = [&](auto e_tag, auto bh_tag) {
-                constexpr int e = decltype(e_tag)::value, bh = decltype(bh_tag)::value;
-#pragma unroll
-                for (int a = 0; a < TM; ++a)
-#pragma unroll
-                    for (int b = bh * (TN / 2); b < (bh + 1) * (TN / 2); ++b)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(component(av[a], e), component(bv[b], e),
-                                                                         acc[a][b], 0, 0, 0);
-                slice_tail(std::integral_constant<int, e * 2 + bh>{});
-            };
-            using std::integral_constant;
-            half_slice(integral_constant<int, 0>{}, integral_constant<int, 0>{});
-            half_slice(integral_constant<int, 0>{}, integral_constant<int, 1>{});
-            half_slice(integral_constant<int, 1>{}, integral_constant<int, 0>{});
-            half_slice(integral_constant<int, 1>{}, integral_constant<int, 1>{});
-            half_slice(integral_constant<int, 2>{}, integral_constant<int, 0>{});
-            half_slice(integral_constant<int, 2>{}, integral_constant<int, 1>{});
-            half_slice(integral_constant<int, 3>{}, integral_constant<int, 0>{});
-            half_slice(integral_constant<int, 3>{}, integral_constant<int, 1>{});
-        } else {
-            // MFMA operands: 8 reduction indices per lane and block, two 128-bit reads.
-            float4 av[TM][2], bv[TN][2];
-#pragma unroll
-            for (int h2 = 0; h2 < 2; ++h2) {
-#pragma unroll
-                for (int a = 0; a < TM; ++a)
-                    av[a][h2] = *reinterpret_cast<const float4 *>(
-                        &As[buf][wm * (TM * 32) + a * 32 + l32][RowA::col(l32, 8 * half + 4 * h2)]);
-#pragma unroll
-                for (int b = 0; b < TN; ++b)
-                    bv[b][h2] = *reinterpret_cast<const float4 *>(
-                        &Bs[buf][wn * (TN * 32) + b * 32 + l32][RowB::col(l32, 8 * half + 4 * h2)]);
-            }
-            auto slice_of = [&](auto slice_tag) {
-                constexpr int slice = decltype(slice_tag)::value;
-                constexpr int h2 = slice / 4, e = slice % 4;
-#pragma unroll
-                for (int a = 0; a < TM; ++a)
-#pragma unroll
-                    for (int b = 0; b < TN; ++b)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(component(av[a][h2], e), component(bv[b][h2], e),
-                                                                         acc[a][b], 0, 0, 0);
-                if constexpr (RED && (slice == 3 || slice == 7)) {
-                    if (rs_hit) {
-#pragma unroll
-                        for (int a = 0; a < TM; ++a)
-                            bsum[a] += (av[a][h2].x + av[a][h2].y) + (av[a][h2].z + av[a][h2].w);
-                    }
-                }
-                slice_tail(slice_tag);
-            };
-            using std::integral_constant;
-            slice_of(integral_constant<int, 0>{});
-            slice_of(integral_constant<int, 1>{});
-            slice_of(integral_constant<int, 2>{});
-            slice_of(integral_constant<int, 3>{});
-            slice_of(integral_constant<int, 4>{});
-            slice_of(integral_constant<int, 5>{});
-            slice_of(integral_constant<int, 6>{});
-            slice_of(integral_constant<int, 7>{});
-        }
-        if (more) {
-            stash(buf ^ 1, shift);
-            advance();
-        }
+        using std::integral_constant;
+        slice_of(integral_constant<int, 0>{});
+        slice_of(integral_constant<int, 1>{});
+        slice_of(integral_constant<int, 2>{});
+        slice_of(integral_constant<int, 3>{});
+        slice_of(integral_constant<int, 4>{});
+        slice_of(integral_constant<int, 5>{});
+        if (more) advance();
+        else shift = 0;
         __syncthreads();
     };
     for (int s = 0; s < nsteps; s += 2) {
         one_step(std::integral_constant<int, 0>{}, s);
         if (s + 1 < nsteps) one_step(std::integral_constant<int, 1>{}, s + 1);
     }
+
+    // ---- blocks the split could not hold --------------------------------------------------
+    // The sum of one 32x32 block in fp32, straight from the operands: lane (x, h) takes r = 2t + h of step t.
+    auto recompute_block = [&](int a, int b) {
+        floatx16 sum;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
+        const int i = i0 + wm * (TM * 32) + a * 32 + l32, j = j0 + wn * (TN * 32) + b * 32 + l32;
+        unsigned im = 0, n = (unsigned)j;
+        if (!RED && LB != LD_RC_VEC) g.divN.divmod((unsigned)j, im, n);
+        const float *const arow = g.A + (LA == LD_XC_SCALAR ? (long)i : (long)i * g.sA);
+        const float *const bcol = g.B + (LB == LD_XC_GATHER   ? (long)im * g.bsB + g.coltab[n]
+                                         : LB == LD_XC_SCALAR ? (long)im * g.bsB + n
+                                                              : (long)j * g.sB);
+        for (int st = step; st < step_end; ++st) {
+            unsigned img = 0, w = (unsigned)st;
+            if (RED) g.divSpi.divmod((unsigned)st, img, w);
+            const int r_end = ((int)w + 1) * BK < g.R ? ((int)w + 1) * BK : g.R;
+            for (int r = (int)w * BK; r < r_end; r += 2) {
+                const int rl = r + half;
+                float av = 0.0f, bv = 0.0f;
+                if (rl < r_end) {
+                    av = arow[(RED ? (long)img * g.rbA : 0L) + (LA == LD_XC_SCALAR ? (long)rl * g.sA : (long)rl)];
+                    bv = bcol[(RED ? (long)img * g.rbB : 0L) + (LB == LD_XC_GATHER   ? (long)g.rowtab[rl]
+                                                                : LB == LD_XC_SCALAR ? (long)rl * g.sB
+                                                                                     : (long)rl)];
+                }
+                sum = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, sum, 0, 0, 0);
+            }
+        }
+        return sum;
+    };
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) {
+            bool odd = false;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) odd |= __builtin_amdgcn_classf(acc[a][b][v], 0x297);  // NaN, infinite, denormal
+            if (__builtin_amdgcn_ballot_w64(odd)) acc[a][b] = recompute_block(a, b);
+        }
 
     // ---- epilogue ----------------------------------------------------------------------
     // Accumulator register v of lane l holds D[8*(v/4) + 4*(l/32) + v%4][l%32].
@@ -585,18 +617,14 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     };
     // The scattered store (see GemmProblem::scatter): rows are (plane, row phase, column phase) triples, columns
     // cells of a per-image grid; an element lands at a strided position of the image or is dropped.
-    // Block geometry of the accumulators: 32x32 blocks keep D[8*(v/4) + 4*(l/32) + v%4][l%32] in register v of lane
-    // l, 16x16 blocks D[4*(l/16) + v][l%16].
-    constexpr int BLK = SMALL ? 16 : 32;
     auto write_scatter = [&]() {
         const bool masked = g.mask != nullptr;
-        const int lcol = lane & (BLK - 1);
         long cbase[TN];  // float offset of the cell's phase-(0,0) pixel; may lie before the image (pH, pW)
         int hy[TN], wx[TN];
         bool own[TN];
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
-            const int jg = j0 + wn * (TN * BLK) + b * BLK + lcol;
+            const int jg = j0 + wn * (TN * 32) + b * 32 + l32;
             own[b] = jg >= own_j0;
             unsigned im, n, y, x;
             g.divN.divmod((unsigned)jg, im, n);
@@ -608,10 +636,10 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         const long plane = (long)g.scat_H * g.scat_W;
 #pragma unroll
         for (int a = 0; a < TM; ++a) {
-            const int iu = i0 + wm * (TM * BLK) + a * BLK;
+            const int iu = i0 + wm * (TM * 32) + a * 32;
 #pragma unroll
-            for (int v = 0; v < ACCV; ++v) {
-                const int row = SMALL ? iu + 4 * (lane >> 4) + v : iu + 8 * (v / 4) + (v % 4) + 4 * half;
+            for (int v = 0; v < 16; ++v) {
+                const int row = iu + 8 * (v / 4) + (v % 4) + 4 * half;
                 if (row < own_i0 || row >= g.scat_rows) continue;
                 unsigned c, rem, ph, pw;
                 g.divScatS.divmod((unsigned)row, c, rem);
@@ -629,47 +657,35 @@ __global__ __launch_bounds__(WGM *WGN * 64)
             }
         }
     };
-    if constexpr (RED && !SMALL) {
-        if (rs_on) {  // all of a wavefront or none
+    if constexpr (RED) {
+        if (rs_on) {
             const long slots = (long)g.nsplit * g.tilesJ;
             float *dst = g.rowsum_ws + ((long)split * g.tilesJ + tj);
 #pragma unroll
-            for (int a = 0; a < TM; ++a) {
-                const float total = bsum[a] + __shfl_xor(bsum[a], 32);  // the two halves hold different r
-                const int row = i0 + wm * (TM * 32) + a * 32 + l32;
-                if (half == 0 && row >= own_i0) dst[row * slots] = total;
+            for (int q = 0; q < RS; ++q) {
+                float total = bsum[q] + __shfl_xor(bsum[q], 1);  // four lanes hold the quarters of a row
+                total += __shfl_xor(total, 2);
+                const int row = i0 + a_x + q * (NT / 4);
+                if (a_r == 0 && a_x + q * (NT / 4) < BM && row >= own_i0) dst[row * slots] = total;
             }
         }
     }
     using std::integral_constant;
     if constexpr (LB == LD_XC_GATHER && !RED) {
-        if (SMALL || g.scatter) {
+        if (g.scatter) {
             write_scatter();
             return;
         }
     }
-    if constexpr (!SMALL) {
-        if (g.nsplit > 1) {
-            if (edge_tile) write_out(integral_constant<int, 0>{}, integral_constant<bool, true>{});
-            else write_out(integral_constant<int, 0>{}, integral_constant<bool, false>{});
-        } else if (g.beta == 0.0f) {
-            if (edge_tile) write_out(integral_constant<int, 1>{}, integral_constant<bool, true>{});
-            else write_out(integral_constant<int, 1>{}, integral_constant<bool, false>{});
-        } else {
-            write_out(integral_constant<int, 2>{}, integral_constant<bool, true>{});
-        }
+    if (g.nsplit > 1) {
+        if (edge_tile) write_out(integral_constant<int, 0>{}, integral_constant<bool, true>{});
+        else write_out(integral_constant<int, 0>{}, integral_constant<bool, false>{});
+    } else if (g.beta == 0.0f) {
+        if (edge_tile) write_out(integral_constant<int, 1>{}, integral_constant<bool, true>{});
+        else write_out(integral_constant<int, 1>{}, integral_constant<bool, false>{});
+    } else {
+        write_out(integral_constant<int, 2>{}, integral_constant<bool, true>{});
     }
-}
-
-// The short-row variant (see the kernel's ROWS16): first operand along r, gathered B, scattered store, unsplit.
-template <int BN, int WGN, int ROWS16>
-int gemm_fast_short_rows_go(const GemmArgs &g, hipStream_t s) {
-    if (!g.scatter || g.nsplit != 1 || g.M != 64 || g.scat_rows > 16 * ROWS16)
-        return fail("gemm: the short-row kernel takes an unsplit scattered product of 64 padded rows, at most %d used",
-                    16 * ROWS16);
-    hipLaunchKernelGGL((gemm_fast_kernel<64, BN, 1, WGN, LD_RC_VEC, LD_XC_GATHER, false, ROWS16>), dim3(g.total),
-                       dim3(WGN * 64), 0, s, g);
-    return 0;
 }
 
 template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED>
@@ -698,14 +714,9 @@ int gemm_fast_dispatch(const GemmArgs &g, int la, int lb, bool red, hipStream_t 
         }                                                                              \
     }
     THGPU_CASE(LD_RC_VEC, LD_RC_VEC)
-    THGPU_CASE(LD_RC_VEC, LD_RC_SCALAR)
     THGPU_CASE(LD_RC_VEC, LD_XC_SCALAR)
     THGPU_CASE(LD_RC_VEC, LD_XC_GATHER)
-    THGPU_CASE(LD_RC_SCALAR, LD_RC_VEC)
-    THGPU_CASE(LD_RC_SCALAR, LD_RC_SCALAR)
-    THGPU_CASE(LD_RC_SCALAR, LD_XC_SCALAR)
     THGPU_CASE(LD_XC_SCALAR, LD_RC_VEC)
-    THGPU_CASE(LD_XC_SCALAR, LD_RC_SCALAR)
     THGPU_CASE(LD_XC_SCALAR, LD_XC_SCALAR)
 #undef THGPU_CASE
     return fail("gemm: unknown loader combination (%d, %d)", la, lb);

@@ -157,7 +157,6 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // How an operand tile travels from global memory to LDS.
 enum Loader {
     LD_RC_VEC = 0,     // contiguous along r: 128-bit loads along r (rows need 4-byte alignment only)
-    LD_RC_SCALAR = 1,  // contiguous along r: 16 lanes read 16 consecutive r, one float each
     LD_XC_SCALAR = 2,  // contiguous along the free index: lanes read consecutive rows/columns
     // 3 is used inside the kernel (block-wise x-contiguous loads of a 192-row first operand)
     LD_XC_GATHER = 4,  // second operand only: element (r, x) at rowtab[r] + coltab[x]; lanes run along x
@@ -173,9 +172,6 @@ int gemm_fast_64x64(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x256(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_96x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);  // first operand along r only
-// Short-row variants: 48 of the tile's 64 rows multiplied (scattered products of a gathered B only).
-int gemm_fast_48x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
-int gemm_fast_48x256(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 // The bounds-checked kernel for shapes smaller than a tile (gemm_generic.hip).
 int gemm_generic_64x64(const GemmArgs &g, bool a_rc, bool b_rc, bool red, hipStream_t s);
 
