@@ -341,8 +341,10 @@ int gemm_launch(const GemmProblem &p) {
 
     g.nsplit = best ? best_split : 1;
     const int bm = best ? best->bm : 64, bn = best ? best->bn : 64;
-    if (!best && red) {
-        // The generic kernel splits too: enough workgroups to fill the chip.
+    if (!best && !p.scatter && g.steps_total > 0) {
+        // The generic kernel splits too: enough workgroups to fill the chip, eight steps each at least.  One workgroup per
+        // 64 x 64 tile would walk the whole reduction of a small product alone (50 x 128 over 4096, a Linear layer
+        // behind a small net: 144 us unsplit, 14 us in 32 parts).
         const long tiles = cdiv(p.M, 64) * cdiv(p.J, 64);
         long want = cdiv(2L * cus, tiles);
         const long cap = g.steps_total / 8 > 0 ? g.steps_total / 8 : 1;
