@@ -603,7 +603,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                     float *c = reinterpret_cast<float *>(out + (long)ir * row_bytes + voff[b]);
                     float val = acc[a][b][v];
                     if (MODE != 0) val = val * g.alpha + bias_v[v];
-                    if (MODE == 2) val += g.beta * *c;
+                    if constexpr (MODE == 2) val += g.beta * held[v][b];
                     if (act) val = val > g.act_threshold ? val : g.act_value;
                     if (masked) {
                         const float mv = *reinterpret_cast<const float *>(msk + (long)ir * mask_row_bytes + mvoff[b]);
@@ -622,6 +622,18 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         long cbase[TN];  // float offset of the cell's phase-(0,0) pixel; may lie before the image (pH, pW)
         int hy[TN], wx[TN];
         bool own[TN];
+            // What C held, requested as one batch before the first store (a load per store, each waited for, ran a
+            // 4096 x 9216 accumulation over 128 indices at 1.7 TB/s).
+            float held[MODE == 2 ? 16 : 1][MODE == 2 ? TN : 1];
+            if constexpr (MODE == 2) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int ir = iu + 8 * (v / 4) + (v % 4);
+#pragma unroll
+                    for (int b = 0; b < TN; ++b)
+                        held[v][b] = *reinterpret_cast<const float *>(out + (long)ir * row_bytes + voff[b]);
+                }
+            }
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
             const int jg = j0 + wn * (TN * 32) + b * 32 + l32;
@@ -684,7 +696,8 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         if (edge_tile) write_out(integral_constant<int, 1>{}, integral_constant<bool, true>{});
         else write_out(integral_constant<int, 1>{}, integral_constant<bool, false>{});
     } else {
-        write_out(integral_constant<int, 2>{}, integral_constant<bool, true>{});
+        if (edge_tile) write_out(integral_constant<int, 2>{}, integral_constant<bool, true>{});
+        else write_out(integral_constant<int, 2>{}, integral_constant<bool, false>{});
     }
 }
 
