@@ -225,6 +225,7 @@ GemmProblem gradweight_problem(long B, int C, int H, int W, int M, int kH, int k
     }
     p.R = (int)N;
     p.nb = (int)B;
+    p.row_quads = sW == 1 && Wo % 4 == 0;
     p.beta = 1.0f;
     p.flops = 2.0 * M * (double)N * K * B;
     p.tag = "gemm_conv_gradweight";

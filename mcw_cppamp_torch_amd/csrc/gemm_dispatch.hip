@@ -112,11 +112,12 @@ struct TileCfg {
     int bm, bn;
     int resident;  // workgroups that fit a CU at once (registers / LDS)
     // Fraction of the MFMA rate (kFlopsPerCycle) the inner loop sustains with a full CU, by operand layout: [0] A along r, B along j (forward); [1] both along their free
-    // index (gradInput); [2] both along r (gradWeight); [3] A along i, B along r; [4] A along r, B gathered.
+    // index (gradInput); [2] both along r (gradWeight); [3] A along i, B along r; [4] A along r, B gathered;
+    // [5] the same with reduction batching.
     // Measured like the occupancy tables below.  None is near 1: on uniform random operands these kernels are held by the
     // card's power, not by its issue slots (the clock falls to about 1.6 GHz; the same launches on zeros run a fifth
     // faster), as is the library's bf16 product (1.13 PFLOP/s at 8192^3, which is 189 TFLOP/s at six products each).
-    double eff[5];
+    double eff[6];
     int (*launch)(const GemmArgs &, int, int, bool, hipStream_t);
     // Fraction of that rate kept with k = 1..4 workgroups resident per CU, and the row count from which the tile is no longer considered (0: no limit).
     const double *occ;
@@ -136,16 +137,16 @@ const double kOcc4[5] = {0.0, 0.52, 0.83, 0.94, 1.0};
 const double kOccSmall[5] = {0.0, 0.40, 0.76, 0.93, 1.0};
 
 const TileCfg kCfgs[] = {
-    {"128x128", 128, 128, 3, {0.44, 0.44, 0.44, 0.44, 0.45}, gemm_fast_128x128, kOcc3, 0, 0, false},
-    {"192x128", 192, 128, 2, {0.43, 0.43, 0.43, 0.43, 0.44}, gemm_fast_192x128, kOcc2, 0, 0, false},
-    {"64x256", 64, 256, 2, {0.38, 0.38, 0.38, 0.38, 0.40}, gemm_fast_64x256, kOcc2, 0, 0, false},
-    {"128x256", 128, 256, 2, {0.46, 0.46, 0.46, 0.46, 0.47}, gemm_fast_128x256, kOcc2, 0, 0, false},
-    {"256x128", 256, 128, 2, {0.46, 0.46, 0.46, 0.46, 0.47}, gemm_fast_256x128, kOcc2, 0, 0, false},
-    {"64x64", 64, 64, 4, {0.32, 0.32, 0.32, 0.32, 0.33}, gemm_fast_64x64, kOccSmall, 0, 0, false},
-    {"64x128", 64, 128, 4, {0.38, 0.38, 0.38, 0.38, 0.39}, gemm_fast_64x128, kOcc4, 128, 0, false},
-    {"48x128", 64, 128, 4, {0, 0, 0, 0, 0.38}, gemm_fast_64x128, kOcc4, 128, 48, false},
-    {"48x256", 64, 256, 2, {0, 0, 0, 0, 0.38}, gemm_fast_64x256, kOcc2, 0, 48, false},
-    {"96x128", 96, 128, 3, {0.40, 0, 0.40, 0, 0.42}, gemm_fast_96x128, kOcc3, 128, 0, true},
+    {"128x128", 128, 128, 3, {0.44, 0.44, 0.44, 0.44, 0.45, 0.42}, gemm_fast_128x128, kOcc3, 0, 0, false},
+    {"192x128", 192, 128, 2, {0.43, 0.43, 0.43, 0.43, 0.44, 0.43}, gemm_fast_192x128, kOcc2, 0, 0, false},
+    {"64x256", 64, 256, 2, {0.38, 0.38, 0.38, 0.38, 0.40, 0.33}, gemm_fast_64x256, kOcc2, 0, 0, false},
+    {"128x256", 128, 256, 2, {0.46, 0.46, 0.46, 0.46, 0.47, 0.42}, gemm_fast_128x256, kOcc2, 0, 0, false},
+    {"256x128", 256, 128, 2, {0.46, 0.46, 0.46, 0.46, 0.47, 0.48}, gemm_fast_256x128, kOcc2, 0, 0, false},
+    {"64x64", 64, 64, 4, {0.32, 0.32, 0.32, 0.32, 0.33, 0.28}, gemm_fast_64x64, kOccSmall, 0, 0, false},
+    {"64x128", 64, 128, 4, {0.38, 0.38, 0.38, 0.38, 0.39, 0.37}, gemm_fast_64x128, kOcc4, 128, 0, false},
+    {"48x128", 64, 128, 4, {0, 0, 0, 0, 0.38, 0}, gemm_fast_64x128, kOcc4, 128, 48, false},
+    {"48x256", 64, 256, 2, {0, 0, 0, 0, 0.38, 0}, gemm_fast_64x256, kOcc2, 0, 48, false},
+    {"96x128", 96, 128, 3, {0.40, 0, 0.40, 0, 0.42, 0.40}, gemm_fast_96x128, kOcc3, 128, 0, true},
 };
 
 inline long cdiv(long a, long b) { return (a + b - 1) / b; }
@@ -208,7 +209,7 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
         return offA < (1L << 30) && offB < (1L << 30) && offC < (1L << 30) && offC2 < (1L << 30);
     };
     const bool fast_ok = p.R == 0 || p.R >= GEMM_BK;
-    const int layout = gather ? 4 : p.a_rc ? (p.b_rc ? 2 : 0) : (p.b_rc ? 3 : 1);
+    const int layout = gather ? (p.nb > 1 || p.rowsum ? 5 : 4) : p.a_rc ? (p.b_rc ? 2 : 0) : (p.b_rc ? 3 : 1);
     for (const TileCfg &c : kCfgs) {
         if (!fast_ok || p.M < c.bm || p.J < c.bn || !offsets_fit(c.bm, c.bn)) continue;
         if (force && std::strcmp(force, c.name) != 0) continue;
@@ -262,7 +263,8 @@ int gemm_launch(const GemmProblem &p) {
     if (p.M <= 0 || p.J <= 0) return 0;
     if ((long)p.M * p.J >= (1L << 31)) return fail("gemm: output of %d x %d exceeds 32-bit tile indexing", p.M, p.J);
 
-    const bool red = p.nb > 1;
+    // (one image's gradWeight runs as a reduction batch of one where it wants the row sums of A)
+    const bool red = p.nb > 1 || (p.rowsum && p.a_rc && (p.b_rc || p.rowtab));
     const bool gather = p.rowtab != nullptr;
     if (gather && (!p.coltab || p.b_rc || !p.a_rc)) return fail("gemm: a gathered B needs both tables and an r-contiguous A");
     if (red && !(p.a_rc && (p.b_rc || gather))) return fail("gemm: reduction batching needs r-contiguous operands");
@@ -383,7 +385,11 @@ int gemm_launch(const GemmProblem &p) {
 
     // ---- loaders: r-contiguous operands use 128-bit loads (4-byte alignment suffices) --------
     const int la = p.a_rc ? LD_RC_VEC : LD_XC_SCALAR;
-    const int lb = p.b_rc ? LD_RC_VEC : gather ? LD_XC_GATHER : LD_XC_SCALAR;
+    const int lb = p.b_rc ? LD_RC_VEC
+                   : !gather ? LD_XC_SCALAR
+                   : !red ? LD_XC_GATHER
+                   : p.row_quads ? LD_RC_GATHER_VEC
+                                 : LD_RC_GATHER;
     if (gather && !best) return fail("gemm: a gathered B needs a shape the tiled kernel takes (M, J >= 64, R >= 16)");
     if (p.C2 && !best) return fail("gemm: a second copy of the result needs a shape the tiled kernel takes");
     if (p.j_store > 0 && (!best || g.nsplit < 2))

@@ -109,9 +109,12 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     static_assert((LB != LD_XC_SCALAR && LB != LD_XC_GATHER) || NT % BN == 0,
                   "x-contiguous loaders give every thread one row/column");
     static_assert(LB != LD_XC_GATHER || BN % 64 == 0, "a wavefront of the gathering loader shares its reduction indices");
-    static_assert(LA != LD_XC_GATHER, "only the second operand is gathered");
-    static_assert(!RED || (LA != LD_XC_SCALAR && LB != LD_XC_SCALAR),
-                  "reduction batching needs r-contiguous or gathered operands");
+    static_assert(LA == LD_RC_VEC || LA == LD_XC_SCALAR, "only the second operand is gathered");
+    // The second operand gathered with four lanes to a column (element (r, x) at rowtab[r] + coltab[x] either way).
+    constexpr bool RG = LB == LD_RC_GATHER || LB == LD_RC_GATHER_VEC;
+    constexpr bool GATHER = LB == LD_XC_GATHER || RG;
+    static_assert(!RG || (RED && NT == 256), "lanes along the reduction: reduction batching only");
+    static_assert(!RED || (LA == LD_RC_VEC && (LB == LD_RC_VEC || RG)), "reduction batching needs operands loaded along r");
 
     using TileA = PartTile<BM>;
     using TileB = PartTile<BN>;
@@ -171,7 +174,16 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         voffA = (unsigned)(((long)a_x * g.sA + a_r) * 4);
         tileA = reinterpret_cast<const char *>(g.A + (long)i0 * g.sA);
     }
-    if (LB == LD_XC_GATHER) {
+    // Lanes along r: the column offsets in bytes of the thread's column of every 64.
+    unsigned coffB[RG ? NB / 4 : 1];
+    if (RG) {
+        b_x = tid >> 2;
+        b_r = (tid & 3) * 4;
+        voffB = 0;
+#pragma unroll
+        for (int q = 0; q < (RG ? NB / 4 : 1); ++q) coffB[q] = (unsigned)g.coltab[j0 + b_x + q * (NT / 4)] * 4u;
+        tileB = reinterpret_cast<const char *>(g.B);
+    } else if (LB == LD_XC_GATHER) {
         b_x = tid % BN;
         b_r = (wave * 64 / BN) * NB;  // = (tid / BN) * NB, kept uniform: the row offsets are scalar loads
         unsigned img0, n0, img, n;
@@ -194,7 +206,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         tileB = reinterpret_cast<const char *>(g.B + (long)j0 * g.sB);
     }
     constexpr int UA = LA == LD_RC_VEC ? NA / 4 : NA;  // load instructions per step and operand
-    constexpr int UB = LB == LD_RC_VEC ? NB / 4 : NB;
+    constexpr int UB = LB == LD_RC_VEC || LB == LD_RC_GATHER_VEC ? NB / 4 : NB;
 
     floatx16 acc[TM][TN];
 #pragma unroll
@@ -226,7 +238,9 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     // Gathered B: float offsets of the rows of the step being loaded (uniform), and of the step after it.  The
     // latter are fetched (scalar loads) in the middle of a step, a whole step before they turn into addresses,
     // so that no step starts by waiting for its row offsets.
-    int roff[LB == LD_XC_GATHER ? NB : 1], roff_nx[LB == LD_XC_GATHER ? NB : 1];
+    // (With lanes along r each lane holds the offsets of its own four r, or of the first of them.)
+    constexpr int NROW = LB == LD_XC_GATHER ? NB : LB == LD_RC_GATHER ? 4 : 1;
+    int roff[NROW], roff_nx[NROW];
 
     // Load number u of an operand for the step whose uniform base is `base`.  Buffer loads: the address is a
     // descriptor in scalar registers (the step's base) plus a scalar offset (which load) plus the lane's constant
@@ -247,9 +261,20 @@ __global__ __launch_bounds__(WGM *WGN * 64)
             dst[u * 4 + 1] = v.y;
             dst[u * 4 + 2] = v.z;
             dst[u * 4 + 3] = v.w;
+        } else if (KIND == LD_RC_GATHER_VEC) {
+            const float4v v = __builtin_bit_cast(
+                float4v, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(coffB[u % (RG ? NB / 4 : 1)] + (unsigned)roff[0] * 4u), 0, 0));
+            dst[u * 4 + 0] = v.x;
+            dst[u * 4 + 1] = v.y;
+            dst[u * 4 + 2] = v.z;
+            dst[u * 4 + 3] = v.w;
+        } else if (KIND == LD_RC_GATHER) {
+            dst[u] = __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(
+                           rsrc, (int)(coffB[u / 4 % (RG ? NB / 4 : 1)] + (unsigned)roff[u % 4 % NROW] * 4u), 0, 0));
         } else {
             const int so = KIND == LD_XC_BLOCK    ? (u & 3) * st + (u >> 2) * 256
-                           : KIND == LD_XC_GATHER ? roff[u] * 4
+                           : KIND == LD_XC_GATHER ? roff[u % NROW] * 4
                                                   : u * st;
             dst[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)voff, so, 0));
         }
@@ -263,21 +288,21 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         const int r0 = ld_r0 + BK <= g.R ? ld_r0 : g.R - BK;
         shift = ld_r0 - r0;
         ga = tileA + ((RED ? (long)ld_img * g.rbA : 0L) + (LA == LD_XC_SCALAR ? (long)r0 * g.sA : (long)r0)) * 4;
-        if (LB == LD_XC_GATHER) {
+        if (GATHER) {
             gb = tileB + (RED ? (long)ld_img * g.rbB : 0L) * 4;
 #pragma unroll
-            for (int u = 0; u < NB; ++u) roff[u] = roff_nx[u];
+            for (int u = 0; u < NROW; ++u) roff[u] = roff_nx[u];
         } else {
             gb = tileB + ((RED ? (long)ld_img * g.rbB : 0L) + (LB == LD_XC_SCALAR ? (long)r0 * g.sB : (long)r0)) * 4;
         }
     };
     // Row offsets of the step whose reduction window starts at `pos` (moved back like the step itself).
     auto fetch_rows = [&](int pos) {
-        if (LB == LD_XC_GATHER) {
+        if (GATHER) {
             const int r0 = pos + BK <= g.R ? pos : g.R - BK;
             const int *rt = g.rowtab + r0 + b_r;
 #pragma unroll
-            for (int u = 0; u < NB; ++u) roff_nx[u] = rt[u];
+            for (int u = 0; u < NROW; ++u) roff_nx[u] = rt[u];
         }
     };
     // Takes delivery of them (an empty statement that names the values keeps the compiler from postponing the
@@ -285,7 +310,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     auto pin_rows = [&]() {
         if (LB == LD_XC_GATHER) {
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
+            for (int u = 0; u < NROW; ++u) {
                 int t = __builtin_amdgcn_readfirstlane(roff_nx[u]);
                 asm("" : "+s"(t));
                 roff_nx[u] = t;
@@ -305,7 +330,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         constexpr int CNT = decltype(count_tag)::value;
 #pragma unroll
         for (int q = 0; q < CNT; ++q) {
-            const int rel = (KIND == LD_RC_VEC || KIND == LD_XC_BLOCK) ? t_r + (q & 3) : t_r + q;
+            const int rel = (KIND == LD_XC_SCALAR || KIND == LD_XC_GATHER) ? t_r + q : t_r + (q & 3);
             v[q] = rel < shift ? 0.0f : v[q];
         }
     };
@@ -319,16 +344,15 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     // Splits group number q of a thread's elements and writes the parts to LDS.  A group is eight elements of a row
     // where the loader gives a thread whole octets, otherwise four.
     constexpr int GA = (KA == LD_XC_SCALAR && NA % 8 == 0) ? 8 : 4;
-    constexpr int GB = (LB != LD_RC_VEC && NB % 8 == 0) ? 8 : 4;
+    constexpr int GB = ((LB == LD_XC_SCALAR || LB == LD_XC_GATHER) && NB % 8 == 0) ? 8 : 4;
     char *const a_dst = &As[0][0] + (a_r >> 3) * TileA::kOctet + a_x * 16 + (a_r & 7) * 2;
     char *const b_dst = &Bs[0][0] + (b_r >> 3) * TileB::kOctet + b_x * 16 + (b_r & 7) * 2;
     auto stash_group = [&](auto kind_tag, auto group_tag, auto tile_tag, char *dst, const float *src, int q) {
         constexpr int KIND = decltype(kind_tag)::value;
         constexpr int G = decltype(group_tag)::value;
         using Tile = decltype(tile_tag);
-        // four-element groups lie in rows apart (LD_RC_VEC: 64 rows a load, LD_XC_BLOCK: the next 64 rows)
-        const int off = G == 8 ? q * Tile::kOctet : (KIND == LD_RC_VEC ? q * (NT / 4) : q * 64) * 16;
-        static_assert(G == 8 || KIND == LD_RC_VEC || KIND == LD_XC_BLOCK || decltype(group_tag)::value == 4, "group");
+        // four-element groups lie in rows apart (four lanes to a row: NT/4 rows, LD_XC_BLOCK: the next 64 rows)
+        const int off = G == 8 ? q * Tile::kOctet : (KIND == LD_XC_BLOCK ? q * 64 : q * (NT / 4)) * 16;
         unsigned p[3][G / 2];
 #pragma unroll
         for (int e = 0; e < G / 2; ++e) split_pair(src[q * G + 2 * e], src[q * G + 2 * e + 1], p[0][e], p[1][e], p[2][e]);
@@ -341,7 +365,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         }
     };
     static_assert(GA == 8 || KA != LD_XC_SCALAR || NA == 4, "an x-contiguous loader of four elements has one group");
-    static_assert(GB == 8 || LB == LD_RC_VEC || NB == 4, "an x-contiguous loader of four elements has one group");
+    static_assert(GB == 8 || LB == LD_RC_VEC || RG || NB == 4, "an x-contiguous loader of four elements has one group");
     auto stash_a = [&](int buf, int q) {
         if (GA == 8 || a_unit_live(q))
             stash_group(std::integral_constant<int, KA>{}, std::integral_constant<int, GA>{}, TileA{},
@@ -421,6 +445,11 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         }
         if (more) step_bases(ga, gb, shift);
 
+        if (RG) {  // vector loads: ahead of this step's refills, whose arrival nobody should wait for on their account
+            int pos = ld_r0 + BK;
+            if (pos >= g.R) pos = 0;
+            fetch_rows(pos);
+        }
         bf16x8 av[TM][3], bv[TN][3];
 #pragma unroll
         for (int u = 0; u < 3; ++u) {  // in the order of their first use
@@ -456,7 +485,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                     stash_b(buf ^ 1, q);
                     refill_b(gb, q);
                 }
-            if (slice == 3) {
+            if (slice == 3 && !RG) {
                 int pos = ld_r0 + BK;
                 if (RED && pos >= g.R) pos = 0;
                 fetch_rows(pos);
@@ -500,7 +529,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         unsigned im = 0, n = (unsigned)j;
         if (!RED && LB != LD_RC_VEC) g.divN.divmod((unsigned)j, im, n);
         const float *const arow = g.A + (LA == LD_XC_SCALAR ? (long)i : (long)i * g.sA);
-        const float *const bcol = g.B + (LB == LD_XC_GATHER   ? (long)im * g.bsB + g.coltab[n]
+        const float *const bcol = g.B + (GATHER               ? (long)im * g.bsB + g.coltab[n]
                                          : LB == LD_XC_SCALAR ? (long)im * g.bsB + n
                                                               : (long)j * g.sB);
         for (int st = step; st < step_end; ++st) {
@@ -512,7 +541,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                 float av = 0.0f, bv = 0.0f;
                 if (rl < r_end) {
                     av = arow[(RED ? (long)img * g.rbA : 0L) + (LA == LD_XC_SCALAR ? (long)rl * g.sA : (long)rl)];
-                    bv = bcol[(RED ? (long)img * g.rbB : 0L) + (LB == LD_XC_GATHER   ? (long)g.rowtab[rl]
+                    bv = bcol[(RED ? (long)img * g.rbB : 0L) + (GATHER               ? (long)g.rowtab[rl]
                                                                 : LB == LD_XC_SCALAR ? (long)rl * g.sB
                                                                                      : (long)rl)];
                 }
@@ -593,6 +622,18 @@ __global__ __launch_bounds__(WGM *WGN * 64)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) bias_v[v] = 0.0f;
             }
+            // What C held, requested as one batch before the first store (a load per store, each waited for, ran a
+            // 4096 x 9216 accumulation over 128 indices at 1.7 TB/s).
+            float held[MODE == 2 ? 16 : 1][MODE == 2 ? TN : 1];
+            if constexpr (MODE == 2) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int ir = iu + 8 * (v / 4) + (v % 4);
+#pragma unroll
+                    for (int b = 0; b < TN; ++b)
+                        held[v][b] = *reinterpret_cast<const float *>(out + (long)ir * row_bytes + voff[b]);
+                }
+            }
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int ir = iu + 8 * (v / 4) + (v % 4);  // uniform; the lane's row is ir + 4*half
@@ -622,18 +663,6 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         long cbase[TN];  // float offset of the cell's phase-(0,0) pixel; may lie before the image (pH, pW)
         int hy[TN], wx[TN];
         bool own[TN];
-            // What C held, requested as one batch before the first store (a load per store, each waited for, ran a
-            // 4096 x 9216 accumulation over 128 indices at 1.7 TB/s).
-            float held[MODE == 2 ? 16 : 1][MODE == 2 ? TN : 1];
-            if constexpr (MODE == 2) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int ir = iu + 8 * (v / 4) + (v % 4);
-#pragma unroll
-                    for (int b = 0; b < TN; ++b)
-                        held[v][b] = *reinterpret_cast<const float *>(out + (long)ir * row_bytes + voff[b]);
-                }
-            }
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
             const int jg = j0 + wn * (TN * 32) + b * 32 + l32;
@@ -718,17 +747,22 @@ int gemm_fast_dispatch(const GemmArgs &g, int la, int lb, bool red, hipStream_t 
             return fail("gemm: this tile has no x-contiguous loader for that side");   \
         } else {                                                                       \
             if (red) {                                                                 \
-                if constexpr (LA_ != LD_XC_SCALAR && LB_ != LD_XC_SCALAR)              \
+                if constexpr (LA_ == LD_RC_VEC && LB_ != LD_XC_SCALAR && LB_ != LD_XC_GATHER) \
                     return gemm_fast_go<BM, BN, WGM, WGN, LA_, LB_, true>(g, s);       \
                 else                                                                   \
-                    return fail("gemm: reduction batching needs r-contiguous operands"); \
+                    return fail("gemm: reduction batching needs operands loaded along r"); \
             }                                                                          \
-            return gemm_fast_go<BM, BN, WGM, WGN, LA_, LB_, false>(g, s);              \
+            if constexpr (LB_ == LD_RC_GATHER || LB_ == LD_RC_GATHER_VEC)              \
+                return fail("gemm: a gather along r needs reduction batching");        \
+            else                                                                       \
+                return gemm_fast_go<BM, BN, WGM, WGN, LA_, LB_, false>(g, s);          \
         }                                                                              \
     }
     THGPU_CASE(LD_RC_VEC, LD_RC_VEC)
     THGPU_CASE(LD_RC_VEC, LD_XC_SCALAR)
     THGPU_CASE(LD_RC_VEC, LD_XC_GATHER)
+    THGPU_CASE(LD_RC_VEC, LD_RC_GATHER)
+    THGPU_CASE(LD_RC_VEC, LD_RC_GATHER_VEC)
     THGPU_CASE(LD_XC_SCALAR, LD_RC_VEC)
     THGPU_CASE(LD_XC_SCALAR, LD_XC_SCALAR)
 #undef THGPU_CASE

@@ -10,9 +10,9 @@ int gemm_fast_96x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s)
     if (lb == LD_RC_VEC)
         return red ? gemm_fast_go<96, 128, 1, 4, LD_RC_VEC, LD_RC_VEC, true>(g, s)
                    : gemm_fast_go<96, 128, 1, 4, LD_RC_VEC, LD_RC_VEC, false>(g, s);
-    if (lb == LD_XC_GATHER)
-        return red ? gemm_fast_go<96, 128, 1, 4, LD_RC_VEC, LD_XC_GATHER, true>(g, s)
-                   : gemm_fast_go<96, 128, 1, 4, LD_RC_VEC, LD_XC_GATHER, false>(g, s);
+    if (lb == LD_RC_GATHER && red) return gemm_fast_go<96, 128, 1, 4, LD_RC_VEC, LD_RC_GATHER, true>(g, s);
+    if (lb == LD_RC_GATHER_VEC && red) return gemm_fast_go<96, 128, 1, 4, LD_RC_VEC, LD_RC_GATHER_VEC, true>(g, s);
+    if (lb == LD_XC_GATHER && !red) return gemm_fast_go<96, 128, 1, 4, LD_RC_VEC, LD_XC_GATHER, false>(g, s);
     if (lb == LD_XC_SCALAR && !red) return gemm_fast_go<96, 128, 1, 4, LD_RC_VEC, LD_XC_SCALAR, false>(g, s);
     return fail("gemm: unknown loader combination (%d, %d)", la, lb);
 }

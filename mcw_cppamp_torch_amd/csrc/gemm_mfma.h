@@ -32,6 +32,9 @@ struct GemmProblem {
     // B[image*rbB + rowtab[r] + coltab[j]]).  Needs !b_rc, a_rc and a shape the tiled kernel takes; sB is unused.
     const int *rowtab = nullptr;  // R entries (floats)
     const int *coltab = nullptr;  // N entries (floats)
+    // Gathered B with reduction batching: the four row offsets from any r that is a multiple of 4 are consecutive, and R
+    // is such a multiple (unit stride, rows of whole quads).
+    bool row_quads = false;
     long b_extent = 0;            // floats addressable from B (gathered B only; checked against 32-bit offsets)
     long sA = 0;                  // the non-unit stride of A
     long sB = 0;                  // the non-unit stride of B
@@ -160,6 +163,13 @@ enum Loader {
     LD_XC_SCALAR = 2,  // contiguous along the free index: lanes read consecutive rows/columns
     // 3 is used inside the kernel (block-wise x-contiguous loads of a 192-row first operand)
     LD_XC_GATHER = 4,  // second operand only: element (r, x) at rowtab[r] + coltab[x]; lanes run along x
+    // The same with reduction batching (x a tap, r a pixel), four lanes to a column, each four consecutive r: one float
+    // at a time, or one 128-bit load where the four are consecutive in memory (GemmProblem::row_quads).  64 lanes along
+    // the taps would touch 64/kW cache lines per load, where 16 taps by 16 pixels touch a third of that: gradWeight of
+    // 64 -> 128 planes, 3x3, 112x112 (64 images), 64 x 128 tile: 96 TFLOP/s along the taps, 125 along r, 154 with
+    // 128-bit loads; 5x5 and 11x11 layers 6 to 10 % faster as well.
+    LD_RC_GATHER = 5,
+    LD_RC_GATHER_VEC = 6,
 };
 
 // Launch one tile configuration of the fast kernel (gemm_fast.h).  la/lb are
