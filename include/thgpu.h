@@ -298,6 +298,17 @@ void THGPUTensor_zero(THGPUTensor *self);
  * getParameters first): what nn.Sequential:zeroGradParameters amounts to on a stack of small layers.  Returns 0
  * or a status with thgpu_last_error() set; nothing is written when a tensor is rejected. */
 int thgpu_fill_many(THGPUTensor **tensors, int count, float value);
+/* y[i] += value * x[i] for `count` pairs of contiguous tensors of equal sizes in one kernel launch, element by element as
+ * THGPUTensor_cadd (what nn.Module:updateParameters does tensor by tensor, mcw_nn/Module.lua:75-82).  Pairs whose y
+ * shares memory with another pair's tensors are all updated one after the other, in the order given.  Returns 0 or a
+ * status; nothing is written when a pair is rejected. */
+int thgpu_axpy_many(THGPUTensor **y, THGPUTensor **x, int count, float value);
+
+/* nn.Linear on a batch of rows, every operand contiguous (mcw_nn/Linear.lua:34-57,81-97 as one product with the bias
+ * added where it is stored, and one sum over the rows): output = input * weight' + bias, resized to [rows, outputs], and
+ * gradBias += scale * column sums of gradOutput.  Return 0 or a status. */
+int thgpu_Linear_updateOutput(THGPUTensor *input, THGPUTensor *weight, THGPUTensor *bias, THGPUTensor *output);
+int thgpu_Linear_accGradBias(THGPUTensor *gradOutput, THGPUTensor *gradBias, float scale);
 
 /* gputorch/lib/THC/THCTensorCopy.h:7-23.  copy handles any strides
  * (THCTensorCopy.cpp:170-290); host<->device copies are blocking

@@ -168,6 +168,9 @@ _SIGNATURES = {
     "THGPUTensor_get4d": (c_float, [TensorP] + [c_long] * 4),
     "THGPUTensor_fill": (None, [TensorP, c_float]),
     "thgpu_fill_many": (c_int, [ctypes.POINTER(TensorP), c_int, c_float]),
+    "thgpu_Linear_updateOutput": (c_int, [TensorP, TensorP, TensorP, TensorP]),
+    "thgpu_Linear_accGradBias": (c_int, [TensorP, TensorP, c_float]),
+    "thgpu_axpy_many": (c_int, [ctypes.POINTER(TensorP), ctypes.POINTER(TensorP), c_int, c_float]),
     "THGPUTensor_zero": (None, [TensorP]),
     "THGPUTensor_copy": (None, [TensorP, TensorP]),
     "THGPUTensor_copyGPU": (None, [TensorP, TensorP]),

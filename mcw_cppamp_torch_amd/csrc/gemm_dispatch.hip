@@ -46,7 +46,8 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const RowSumJob rs, c
                                                            long mask_sC, long mask_bsC, FastDiv divCW,
                                                            float *__restrict__ C2, long c2_sC, long c2_bsC, int c2_pitch,
                                                            const unsigned side_first_block, const WeightJob side,
-                                                           const unsigned j_store) {
+                                                           const unsigned j_store,
+                                                           const float *__restrict__ bias_col) {
     // workgroups behind the reduction's carry a job of the next layer's (side_jobs.h)
     if (blockIdx.x >= side_first_block) {
         reorder_weight(side, (blockIdx.x - side_first_block) * 256u + threadIdx.x);
@@ -100,6 +101,7 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const RowSumJob rs, c
     float *c = C + (long)i * sC + coff;
     float val = alpha * sum;
     if (bias) val += bias[i];
+    if (bias_col) val += bias_col[j];
     if (beta != 0.0f) val += beta * *c;
     if (act) val = val > act_threshold ? val : act_value;
     if (mask) val = mask[(long)i * mask_sC + moff] > mask_threshold ? val : 0.0f;
@@ -275,6 +277,9 @@ int gemm_launch(const GemmProblem &p) {
     g.B = p.B;
     g.C = p.C;
     g.bias = p.bias;
+    g.bias_col = p.bias_col;
+    if (p.bias_col && (p.bias || red || gather || p.C2 || (p.N > 0 && p.N != p.J)))
+        return fail("gemm: a bias per column needs a plain product");
     g.rowtab = p.rowtab;
     g.coltab = p.coltab;
     g.M = p.M;
@@ -439,7 +444,7 @@ int gemm_launch(const GemmProblem &p) {
                                p.M, p.J, g.N, p.sC, p.bsC, FastDiv((uint32_t)p.J), g.divN, g.nsplit, p.alpha,
                                p.beta, g.act, g.act_threshold, g.act_value, g.mask, g.mask_threshold, g.c_pitch,
                                g.mask_pitch, g.mask_sC, g.mask_bsC, g.divCW, g.C2, g.c2_sC, g.c2_bsC, g.c2_pitch,
-                               side_first, side, (unsigned)(p.j_store > 0 ? p.j_store : p.J));
+                               side_first, side, (unsigned)(p.j_store > 0 ? p.j_store : p.J), p.bias_col);
         }
         if (check_launch("gemm_split_reduce")) return 1;
     }

@@ -589,10 +589,12 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         // owns the column.
         unsigned voff[TN], mvoff[TN], tvoff[TN];
         bool own[TN];
+        float col_bias[TN];
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
             const int jg = j0 + wn * (TN * 32) + b * 32 + l32;
             own[b] = jg >= own_j0;  // else the neighbouring tile stores it
+            col_bias[b] = MODE != 0 && g.bias_col ? g.bias_col[jg] : 0.0f;
             long col = jg - j0, mcol = jg - j0, tcol = 0;
             if (per_image) {
                 unsigned im, n, y, x;
@@ -643,7 +645,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                     if (CHECK && !own[b]) continue;
                     float *c = reinterpret_cast<float *>(out + (long)ir * row_bytes + voff[b]);
                     float val = acc[a][b][v];
-                    if (MODE != 0) val = val * g.alpha + bias_v[v];
+                    if (MODE != 0) val = val * g.alpha + (bias_v[v] + col_bias[b]);
                     if constexpr (MODE == 2) val += g.beta * held[v][b];
                     if (act) val = val > g.act_threshold ? val : g.act_value;
                     if (masked) {

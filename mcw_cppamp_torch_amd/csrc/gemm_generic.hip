@@ -212,6 +212,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_generic_kernel(const GemmA
                     float *c = g.C + (long)i * g.sC + coff;
                     val *= g.alpha;
                     if (g.bias) val += g.bias[i];
+                    if (g.bias_col) val += g.bias_col[jg];
                     if (g.beta != 0.0f) val += g.beta * *c;
                     if (g.act) val = val > g.act_threshold ? val : g.act_value;
                     if (g.mask) val = g.mask[(long)i * g.mask_sC + moff] > g.mask_threshold ? val : 0.0f;

@@ -23,6 +23,7 @@ struct GemmProblem {
     const float *B = nullptr;
     float *C = nullptr;
     const float *bias = nullptr;  // added per output row i when non-null
+    const float *bias_col = nullptr;  // added per output column j when non-null (N == J only)
     int M = 0;                    // rows of C
     int J = 0;                    // columns of C (all images together in column batching)
     int R = 0;                    // reduction length (per image in reduction batching)
@@ -114,7 +115,7 @@ struct GemmArgs {
     const float *A;
     const float *B;
     float *C;
-    const float *bias;
+    const float *bias, *bias_col;
     float *ws;  // partial sums [nsplit][M][J] when nsplit > 1
     const int *rowtab, *coltab;  // gathered B
     int M, J, R, N;

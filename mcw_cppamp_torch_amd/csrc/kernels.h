@@ -49,6 +49,8 @@ int maxpool_bwd_launch(const float *gout, const float *indices, long planes, int
 int threshold_fwd_launch(const float *in, float *out, long n, float th, float val);
 int threshold_bwd_launch(const float *in, const float *gout, float *gin, long n, float th);
 int gradbias_launch(const float *gout, float *gbias, long B, int M, long N, float scale);
+// out[j] += scale * sum over the rows of in[row][j]  (nn.Linear's bias gradient)
+int column_sums_launch(const float *in, float *out, long rows, long cols, float scale);
 
 // Convolution without the column buffer (conv_implicit.hip).  conv_mode: 0 = im2col / GEMM / col2im,
 // 1 = gathered GEMMs where the shape fits and the route pays, 2 = wherever the shape fits.  The two

@@ -727,6 +727,44 @@ int thgpu_Threshold_updateGradInput(THGPUTensor *input, THGPUTensor *gradOutput,
     return rc;
 }
 
+// nn.Linear on a batch, dense operands.  The bias is added where the product is stored, with the roundings of the
+// reference's zero / addr(ones, bias) / addmm sequence (mcw_nn/Linear.lua:34-57), which takes four launches.
+int thgpu_Linear_updateOutput(THGPUTensor *input, THGPUTensor *weight, THGPUTensor *bias, THGPUTensor *output) {
+    if (!input || !weight || !bias || !output) return fail("Linear: null tensor");
+    if (input->nDimension != 2 || weight->nDimension != 2 || bias->nDimension != 1 ||
+        input->size[1] != weight->size[1] || bias->size[0] != weight->size[0])
+        return fail("Linear: size mismatch");
+    const long B = input->size[0], I = input->size[1], O = weight->size[0];
+    if (B <= 0 || I <= 0 || O <= 0 || B >= (1L << 31) || I >= (1L << 31) || O >= (1L << 31))
+        return fail("Linear: dimension out of range");
+    if (!tensor_ready(input, B * I) || !tensor_ready(weight, O * I) || !tensor_ready(bias, O))
+        return fail("Linear: operands must be contiguous");
+    THGPUTensor_resize2d(output, B, O);
+    if (!tensor_ready(output, B * O)) return fail("Linear: could not size output");
+    GemmProblem p;
+    p.A = dptr(input);
+    p.B = dptr(weight);
+    p.C = dptr(output);
+    p.bias_col = dptr(bias);
+    p.M = (int)B;
+    p.J = p.N = (int)O;
+    p.R = (int)I;
+    p.a_rc = p.b_rc = true;
+    p.sA = p.sB = I;
+    p.sC = O;
+    p.tag = "gemm_linear_fwd";
+    return gemm_launch(p);
+}
+
+int thgpu_Linear_accGradBias(THGPUTensor *gradOutput, THGPUTensor *gradBias, float scale) {
+    if (!gradOutput || !gradBias) return fail("Linear: null tensor");
+    if (gradOutput->nDimension != 2 || gradBias->nDimension != 1 || gradOutput->size[1] != gradBias->size[0])
+        return fail("Linear: size mismatch");
+    const long B = gradOutput->size[0], O = gradOutput->size[1];
+    if (!tensor_ready(gradOutput, B * O) || !tensor_ready(gradBias, O)) return fail("Linear: operands must be contiguous");
+    return column_sums_launch(dptr(gradOutput), dptr(gradBias), B, O, scale);
+}
+
 int thgpu_conv_set_mode(int mode) {
     if (mode < 0 || mode > 2)
         return fail("conv mode must be 0 (columns), 1 (gathered where it pays) or 2 (gathered where it fits)");

@@ -906,7 +906,8 @@ struct __attribute__((packed, aligned(4))) gb_float4u {  // four floats at a 4-b
 
 __global__ __launch_bounds__(256) void gradbias_partial_kernel(const float *__restrict__ gout,
                                                                float *__restrict__ part, int B, int M, int N,
-                                                               int imgs_per_slice, int nslices, const FastDiv divQ) {
+                                                               int imgs_per_slice, int nslices, const FastDiv divQ,
+                                                               float *__restrict__ gbias, float scale) {
     const int m = blockIdx.x, slice = blockIdx.y;
     const int b0 = slice * imgs_per_slice;
     const int b1 = b0 + imgs_per_slice < B ? b0 + imgs_per_slice : B;
@@ -946,7 +947,10 @@ __global__ __launch_bounds__(256) void gradbias_partial_kernel(const float *__re
         if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) part[(long)m * nslices + slice] = red[0];
+    if (threadIdx.x == 0) {
+        if (gbias) gbias[m] += scale * red[0];  // the only slice
+        else part[(long)m * nslices + slice] = red[0];
+    }
 }
 
 __global__ __launch_bounds__(256) void gradbias_final_kernel(const float *__restrict__ part,
@@ -957,6 +961,33 @@ __global__ __launch_bounds__(256) void gradbias_final_kernel(const float *__rest
     float sum = 0.0f;
     for (int s = 0; s < nslices; ++s) sum += part[(long)m * nslices + s];
     gbias[m] += scale * sum;
+}
+
+// Column sums of a row-major matrix of few rows (a batch): sixteen wavefronts share 64 columns, wavefront w adds rows
+// w, w + 16, ... with four loads in flight, then the sixteen are added in a fixed tree.  Latency of one launch is what
+// bounds it: it stands for a fill of ones and a product with one row (11 us and 5 us at 128 x 4096; 6 us now).
+__global__ __launch_bounds__(1024) void column_sums_kernel(const float *__restrict__ in, float *__restrict__ out,
+                                                           int rows, int cols, float scale) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long col = (long)blockIdx.x * 64 + lane;
+    float sum = 0.0f;
+    if (col < cols) {
+        const float *src = in + col;
+        for (long r0 = wave; r0 < rows; r0 += 64) {
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = r0 + 16 * u < rows ? src[(r0 + 16 * u) * cols] : 0.0f;
+            sum += (v[0] + v[1]) + (v[2] + v[3]);
+        }
+    }
+    __shared__ float part[16][64];
+    part[wave][lane] = sum;
+    __syncthreads();
+    for (int h = 8; h > 0; h >>= 1) {
+        if (wave < h) part[wave][lane] += part[wave + h][lane];
+        __syncthreads();
+    }
+    if (wave == 0 && col < cols) out[col] += scale * part[0][lane];
 }
 
 }  // namespace
@@ -1232,6 +1263,19 @@ int threshold_bwd_launch(const float *in, const float *gout, float *gin, long n,
     return check_launch("threshold_bwd");
 }
 
+int column_sums_launch(const float *in, float *out, long rows, long cols, float scale) {
+    hipStream_t s = stream();
+    if (!s) return 1;
+    if (rows <= 0 || cols <= 0) return 0;
+    if (rows >= (1L << 31) || cols >= (1L << 31)) return fail("column sums: matrix too large");
+    {
+        LaunchScope scope("column_sums", 0.0, 4.0 * (rows * cols + 2.0 * cols));
+        hipLaunchKernelGGL(column_sums_kernel, dim3((unsigned)((cols + 63) / 64)), dim3(1024), 0, s, in, out, (int)rows,
+                           (int)cols, scale);
+    }
+    return check_launch("column_sums");
+}
+
 int gradbias_launch(const float *gout, float *gbias, long B, int M, long N, float scale) {
     hipStream_t s = stream();
     if (!s) return 1;
@@ -1241,7 +1285,9 @@ int gradbias_launch(const float *gout, float *gbias, long B, int M, long N, floa
     long nslices = (4L * num_cus() + M - 1) / M;
     if (nslices > B) nslices = B;
     if (nslices > 65535) nslices = 65535;
-    if (nslices < 1) nslices = 1;
+    // Planes of at most 16384 floats (64 a lane) in one launch, one workgroup each: behind it the second stage of a few
+    // sums cost as much as the first (37 planes of 4125: 2 x 5 us).
+    if (nslices < 1 || B * N <= 16384) nslices = 1;
     const int ips = (int)((B + nslices - 1) / nslices);
     nslices = (B + ips - 1) / ips;
     if (nslices < 1) nslices = 1;
@@ -1252,9 +1298,11 @@ int gradbias_launch(const float *gout, float *gbias, long B, int M, long N, floa
     {
         LaunchScope scope("gradbias", 0.0, 4.0 * B * M * N);
         hipLaunchKernelGGL(gradbias_partial_kernel, dim3((unsigned)M, (unsigned)nslices), dim3(256), 0, s, gout,
-                           part, (int)B, M, (int)N, ips, (int)nslices, FastDiv((uint32_t)((N + 3) / 4)));
+                           part, (int)B, M, (int)N, ips, (int)nslices, FastDiv((uint32_t)((N + 3) / 4)),
+                           nslices == 1 ? gbias : nullptr, scale);
     }
     if (check_launch("gradbias")) return 1;
+    if (nslices == 1) return 0;
     {
         LaunchScope scope("gradbias_final", 0.0, 4.0 * M * (nslices + 2));
         hipLaunchKernelGGL(gradbias_final_kernel, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, s, part, gbias,

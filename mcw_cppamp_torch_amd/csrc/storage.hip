@@ -43,23 +43,84 @@ int fill_device(float *p, long n, float v) {
     return check_launch("fill");
 }
 
-// One launch that fills several buffers (a network's gradient tensors): entry e owns the virtual index range
-// [start[e], start[e+1]) of the concatenation.
-constexpr int kFillManyMax = 32;
-struct FillMany {
-    float *p[kFillManyMax];
-    long start[kFillManyMax + 1];
+// One launch over several buffers (a network's gradients, its parameters and gradients): workgroup c takes chunk c of
+// the concatenation, entry e owning chunks first[e] .. first[e+1]-1.  The entry is found once per workgroup (uniform), not
+// per element, and whole 16-byte units are stored where the buffers are aligned.
+constexpr int kManyMax = 32;
+constexpr unsigned kManyChunk = 4096;  // floats: sixteen per lane
+struct Many {
+    float *p[kManyMax];
+    const float *x[kManyMax];  // axpy only
+    long n[kManyMax];
+    unsigned first[kManyMax + 1];
     int count;
 };
 
-__global__ __launch_bounds__(256) void fill_many_kernel(const FillMany f, float v) {
-    const long total = f.start[f.count];
-    const long stride = (long)gridDim.x * blockDim.x;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        int e = 0;
-        while (i >= f.start[e + 1]) ++e;  // at most 32 ranges
-        f.p[e][i - f.start[e]] = v;
+// AXPY: p += v * x, two roundings (TH/generic/THBlas.c:96-99); otherwise p = v.
+template <bool AXPY>
+__global__ __launch_bounds__(256) void many_kernel(const Many f, float v) {
+    int e = 0;
+    while (blockIdx.x >= f.first[e + 1]) ++e;
+    const long begin = (long)(blockIdx.x - f.first[e]) * kManyChunk;
+    const long left = f.n[e] - begin;
+    float *const p = f.p[e] + begin;
+    const float *const x = AXPY ? f.x[e] + begin : nullptr;
+    const unsigned n = left < (long)kManyChunk ? (unsigned)left : kManyChunk;
+    auto one = [&](float y, float xv) { return AXPY ? __fadd_rn(y, __fmul_rn(v, xv)) : v; };
+    const bool aligned = ((reinterpret_cast<uintptr_t>(p) | (AXPY ? reinterpret_cast<uintptr_t>(x) : 0)) & 15) == 0;
+    if (aligned && n == kManyChunk) {
+        float4 *const p4 = reinterpret_cast<float4 *>(p);
+        const float4 *const x4 = reinterpret_cast<const float4 *>(x);
+        float4 y[4], w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            y[q] = AXPY ? p4[threadIdx.x + 256 * q] : float4{};
+            w[q] = AXPY ? x4[threadIdx.x + 256 * q] : float4{};
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            p4[threadIdx.x + 256 * q] =
+                make_float4(one(y[q].x, w[q].x), one(y[q].y, w[q].y), one(y[q].z, w[q].z), one(y[q].w, w[q].w));
+        return;
     }
+    for (unsigned i = threadIdx.x; i < n; i += 256) p[i] = one(AXPY ? p[i] : 0.0f, AXPY ? x[i] : 0.0f);
+}
+
+// Launches for entries [0, count) of the caller's list, kManyMax at a time.
+template <bool AXPY, typename Entry>
+int many_launch(int count, float v, const char *tag, Entry entry) {
+    hipStream_t s = stream();
+    if (!s) return 1;
+    for (int i = 0; i < count;) {
+        Many f;
+        f.count = 0;
+        f.first[0] = 0;
+        double total = 0.0;
+        for (; i < count && f.count < kManyMax; ++i) {
+            float *p;
+            const float *x;
+            const long n = entry(i, p, x);
+            if (n == 0) continue;
+            const long chunks = (n + kManyChunk - 1) / kManyChunk;
+            if (chunks + (long)f.first[f.count] >= (1L << 31)) {
+                if (f.count == 0) return fail("%s: tensor too large", tag);
+                break;  // the next launch's
+            }
+            f.p[f.count] = p;
+            f.x[f.count] = x;
+            f.n[f.count] = n;
+            f.first[f.count + 1] = f.first[f.count] + (unsigned)chunks;
+            ++f.count;
+            total += (double)n;
+        }
+        if (f.count == 0) continue;
+        {
+            LaunchScope scope(tag, 0.0, (AXPY ? 12.0 : 4.0) * total);
+            hipLaunchKernelGGL(many_kernel<AXPY>, dim3(f.first[f.count]), dim3(256), 0, s, f, v);
+        }
+        if (check_launch(tag)) return 1;
+    }
+    return 0;
 }
 
 // Blocking host<->device copies: stage through the caller's pageable memory
@@ -377,26 +438,41 @@ extern "C" int thgpu_fill_many(THGPUTensor **tensors, int count, float value) {
         if (THGPUTensor_nElement(t) > 0 && (!THGPUTensor_isContiguous(t) || !tensor_backed(t)))
             return fail("thgpu_fill_many: tensor %d is not contiguous or exceeds its storage", i);
     }
-    for (int first = 0; first < count; first += kFillManyMax) {
-        FillMany f;
-        f.count = 0;
-        f.start[0] = 0;
-        for (int i = first; i < count && i < first + kFillManyMax; ++i) {
-            const long n = THGPUTensor_nElement(tensors[i]);
-            if (n == 0) continue;
-            f.p[f.count] = THGPUTensor_data(tensors[i]);
-            f.start[f.count + 1] = f.start[f.count] + n;
-            ++f.count;
-        }
-        const long total = f.start[f.count];
-        if (total == 0) continue;
-        long blocks = (total + 255) / 256;
-        if (blocks > 4096) blocks = 4096;
-        {
-            LaunchScope scope("fill", 0.0, 4.0 * total);
-            hipLaunchKernelGGL(fill_many_kernel, dim3((unsigned)blocks), dim3(256), 0, s, f, value);
-        }
-        if (check_launch("fill")) return 1;
+    return many_launch<false>(count, value, "fill", [&](int i, float *&p, const float *&x) {
+        p = THGPUTensor_data(tensors[i]);
+        x = nullptr;
+        return THGPUTensor_nElement(tensors[i]);
+    });
+}
+
+extern "C" int thgpu_axpy_many(THGPUTensor **y, THGPUTensor **x, int count, float value) {
+    if (count < 0 || (count > 0 && (!y || !x))) return fail("thgpu_axpy_many: invalid arguments");
+    if (!stream()) return 1;
+    for (int i = 0; i < count; ++i) {  // every pair is checked before anything is launched
+        if (!y[i] || !x[i]) return fail("thgpu_axpy_many: null tensor");
+        const long n = THGPUTensor_nElement(y[i]);
+        if (THGPUTensor_nElement(x[i]) != n) return fail("thgpu_axpy_many: sizes of pair %d do not match", i);
+        if (n > 0 && (!THGPUTensor_isContiguous(y[i]) || !tensor_backed(y[i]) || !THGPUTensor_isContiguous(x[i]) ||
+                      !tensor_backed(x[i])))
+            return fail("thgpu_axpy_many: pair %d is not contiguous or exceeds its storage", i);
     }
+    // Buffers that share memory (a weight used by two modules) are updated one after the other, in the order given.
+    auto overlap = [](THGPUTensor *a, THGPUTensor *b) {
+        const float *pa = THGPUTensor_data(a), *pb = THGPUTensor_data(b);
+        return pa < pb + THGPUTensor_nElement(b) && pb < pa + THGPUTensor_nElement(a);
+    };
+    bool shared = false;
+    for (int i = 0; i < count && !shared; ++i)
+        for (int j = 0; j < count && !shared; ++j) shared = (i != j && overlap(y[i], y[j])) || (i != j && overlap(y[i], x[j]));
+    auto launch = [&](int first, int n) {
+        return many_launch<true>(n, value, "axpy", [&](int i, float *&p, const float *&q) {
+            p = THGPUTensor_data(y[first + i]);
+            q = THGPUTensor_data(x[first + i]);
+            return THGPUTensor_nElement(y[first + i]);
+        });
+    };
+    if (!shared) return launch(0, count);
+    for (int i = 0; i < count; ++i)
+        if (launch(i, 1)) return 1;
     return 0;
 }

@@ -55,6 +55,38 @@ def _require_gpu(*tensors):
                              "move tensors and modules with :gpu())")
 
 
+def _zero_all(tensors):
+    """Zeroes every tensor (GPU tensors and host arrays); two or more dense GPU tensors in one launch."""
+    dense = [t for t in tensors if isinstance(t, GPUTensor) and t.isContiguous()]
+    if len(dense) < 2:
+        dense = []
+    else:
+        arr = (_lib.TensorP * len(dense))(*[t._p for t in dense])
+        _lib.check_status(lib.thgpu_fill_many(arr, len(dense), 0.0))
+    served = set(id(t) for t in dense)
+    for t in tensors:
+        if not isinstance(t, GPUTensor):
+            t[...] = 0
+        elif id(t) not in served:
+            t.zero()
+
+
+def _add_all(params, value, grads):
+    """p += value * g for every pair, in order; pairs of dense GPU tensors of one size in one launch where all are."""
+    pairs = list(zip(params, grads))
+    if len(pairs) > 1 and all(isinstance(p, GPUTensor) and isinstance(g, GPUTensor) and p.isContiguous() and
+                              g.isContiguous() and p.nElement() == g.nElement() for p, g in pairs):
+        ys = (_lib.TensorP * len(pairs))(*[p._p for p, _ in pairs])
+        xs = (_lib.TensorP * len(pairs))(*[g._p for _, g in pairs])
+        _lib.check_status(lib.thgpu_axpy_many(ys, xs, len(pairs), value))
+        return
+    for p, g in pairs:
+        if isinstance(p, GPUTensor):
+            p.add(value, g)
+        else:
+            p += np.float32(value) * g
+
+
 class Module(object):
     def __init__(self):
         self.gradInput = FloatTensor()
@@ -89,20 +121,12 @@ class Module(object):
 
     def zeroGradParameters(self):
         _, grads = self.parameters()
-        for g in grads or []:
-            if isinstance(g, GPUTensor):
-                g.zero()
-            else:
-                g[...] = 0
+        _zero_all(grads or [])
 
     def updateParameters(self, learningRate):
         # mcw_nn/Module.lua:75-82
         params, grads = self.parameters()
-        for p, g in zip(params or [], grads or []):
-            if isinstance(p, GPUTensor):
-                p.add(-learningRate, g)
-            else:
-                p += np.float32(-learningRate) * g
+        _add_all(params or [], -learningRate, grads or [])
 
     def accUpdateGradParameters(self, input, gradOutput, lr):
         # mcw_nn/Module.lua:49-57: accumulate straight into the parameters with scale -lr
@@ -219,18 +243,7 @@ class Sequential(Module):
         for m in plain:
             _, g = m.parameters()
             grads.extend(g or [])
-        gpu = [g for g in grads if isinstance(g, GPUTensor) and g.isContiguous()]
-        if len(gpu) > 1:
-            arr = (_lib.TensorP * len(gpu))(*[g._p for g in gpu])
-            _lib.check_status(lib.thgpu_fill_many(arr, len(gpu), 0.0))
-        else:
-            gpu = []
-        for g in grads:
-            if isinstance(g, GPUTensor):
-                if not any(g is h for h in gpu):
-                    g.zero()
-            else:
-                g[...] = 0
+        _zero_all(grads)
 
     def fuse(self):
         """Lets the neighbours of every nn.Threshold / nn.ReLU do its work while they store their own results: a
@@ -296,9 +309,23 @@ class Sequential(Module):
         return self
 
     def updateParameters(self, learningRate):
-        # mcw_nn/Sequential.lua:91-95
+        # mcw_nn/Sequential.lua:91-95 calls every module's updateParameters, in order.  Neighbours that keep Module's
+        # own implementation are served together (their dense GPU tensors in one launch).
+        params, grads = [], []
+
+        def flush():
+            _add_all(params, -learningRate, grads)
+            del params[:], grads[:]
+
         for m in self.modules:
-            m.updateParameters(learningRate)
+            if type(m).updateParameters is Module.updateParameters and type(m).parameters is Module.parameters:
+                p, g = m.parameters()
+                params.extend(p or [])
+                grads.extend(g or [])
+            else:
+                flush()
+                m.updateParameters(learningRate)
+        flush()
 
     def parameters(self):
         # mcw_nn/Sequential.lua:121-141: the modules' parameters and gradients, flattened in module order
@@ -521,12 +548,20 @@ class Linear(Module):
             if nunit == 1:
                 self.output.zero().add(self.bias[0])
                 self.output.select(1, 0).addmv(1, input, self.weight.select(0, 0))
+            elif self._dense(input, input.size(1)) and self.output.isContiguous():
+                _lib.check_status(lib.thgpu_Linear_updateOutput(input._p, self.weight._p, self.bias._p, self.output._p))
             else:
                 self.output.zero().addr(1, GPUTensor(nframe).fill(1), self.bias)
                 self.output.addmm(1, input, self.weight.t())
         else:
             raise ValueError("input must be vector or matrix")
         return self.output
+
+    def _dense(self, input, inputs):
+        """Whether a batch and the parameters are laid out for the library's own Linear entry points."""
+        return (input.isContiguous() and self.weight.isContiguous() and self.bias.isContiguous() and
+                self.weight.dim() == 2 and self.bias.dim() == 1 and input.size(0) > 0 and inputs > 0 and
+                self.weight.size(0) == self.bias.size(0) and self.weight.size(1) == inputs)
 
     def updateGradInput(self, input, gradOutput):
         if self.gradInput is None:
@@ -549,12 +584,16 @@ class Linear(Module):
             self.gradBias.add(scale, gradOutput)
         elif input.dim() == 2:
             nframe, nunit = input.size(0), self.bias.size(0)
-            ones = GPUTensor(nframe).fill(1)
             if nunit == 1:
                 self.gradWeight.select(0, 0).addmv(scale, input.t(), gradOutput.select(1, 0))
             else:
                 self.gradWeight.addmm(scale, gradOutput.t(), input)
-            self.gradBias.addmv(scale, gradOutput.t(), ones)
+            if (gradOutput.dim() == 2 and gradOutput.size(0) == nframe and gradOutput.isContiguous() and
+                    self.gradBias.isContiguous() and self.gradBias.dim() == 1 and
+                    gradOutput.size(1) == self.gradBias.size(0)):
+                _lib.check_status(lib.thgpu_Linear_accGradBias(gradOutput._p, self.gradBias._p, scale))
+            else:
+                self.gradBias.addmv(scale, gradOutput.t(), GPUTensor(nframe).fill(1))
 
 
 class SpatialMaxPooling(Module):

@@ -1,0 +1,78 @@
+"""Operators that stand for several launches: parameter updates of many tensors at once, nn.Linear's bias in the store of
+its product and its bias gradient as one sum, the one-launch bias gradient of small convolution layers."""
+import numpy as np
+import pytest
+
+from helpers import rng_for
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gt():
+    import mcw_cppamp_torch_amd as pkg
+    assert pkg._lib.lib.thgpu_init() == 0
+    return pkg
+
+
+def dev(gt, a):
+    return gt.FloatTensor(np.ascontiguousarray(a, np.float32)).gpu()
+
+
+def pointers(gt, tensors):
+    return (gt._lib.TensorP * len(tensors))(*[t._p for t in tensors])
+
+
+# ends of chunks, of 16-byte units and of a launch's 32 entries; offset 1 makes a pair unaligned
+@pytest.mark.parametrize("sizes,offset", [([1, 3, 4095, 4096, 4097, 12289], 0), ([4096, 8192, 5], 1), ([7] * 33 + [4096], 0)])
+def test_axpy_many_equals_add_bit_for_bit(gt, sizes, offset):
+    rng = rng_for(401)
+    hosts = [(rng.standard_normal(n).astype(np.float32), rng.standard_normal(n).astype(np.float32)) for n in sizes]
+    place = lambda a: dev(gt, np.concatenate([np.full(offset, 9, np.float32), a])).narrow(0, offset, a.size)
+    ys, xs = [place(y) for y, _ in hosts], [place(x) for _, x in hosts]
+    gt._lib.check_status(gt._lib.lib.thgpu_axpy_many(pointers(gt, ys), pointers(gt, xs), len(ys), -0.37))
+    for (y, x), got in zip(hosts, ys):
+        assert np.array_equal(got.float(), y + np.float32(-0.37) * x)
+
+
+def test_axpy_many_updates_a_shared_tensor_once_per_pair_and_rejects_bad_pairs(gt):
+    rng = rng_for(402)
+    y, a, b = (rng.integers(-8, 9, size=5000).astype(np.float32) for _ in range(3))
+    dy, da, db = dev(gt, y), dev(gt, a), dev(gt, b)
+    lib = gt._lib.lib
+    assert lib.thgpu_axpy_many(pointers(gt, [dy, dy]), pointers(gt, [da, db]), 2, 2.0) == 0
+    assert np.array_equal(dy.float(), y + 2 * a + 2 * b)
+    short = dev(gt, b[:4])
+    assert lib.thgpu_axpy_many(pointers(gt, [da, dy]), pointers(gt, [db, short]), 2, 1.0) != 0
+    assert b"sizes" in lib.thgpu_last_error() and np.array_equal(da.float(), a)
+
+
+# batch, inputs, outputs: below a tile (split and not), a tile and its edges, split tiles
+@pytest.mark.parametrize("batch,inputs,outputs", [(1, 5, 2), (3, 4096, 10), (50, 300, 128), (64, 64, 64), (65, 130, 200),
+                                                  (128, 2049, 333)])
+def test_linear_integer_exact(gt, batch, inputs, outputs):
+    rng = rng_for(403)
+    ints = lambda *s: rng.integers(-3, 4, size=s).astype(np.float32)
+    x, w, b, go = ints(batch, inputs), ints(outputs, inputs), ints(outputs), ints(batch, outputs)
+    m = gt.nn.Linear(inputs, outputs)
+    m._assign("weight", w)
+    m._assign("bias", b)
+    m.gradBias[...] = 1
+    m.gpu()
+    assert np.array_equal(m.forward(dev(gt, x)).float(), x @ w.T + b)
+    m.accGradParameters(dev(gt, x), dev(gt, go), 2.0)
+    assert np.array_equal(m.gradBias.float(), 1 + 2 * go.sum(0))
+    wide = dev(gt, np.concatenate([x, x], 1)).narrow(1, 0, inputs)  # rows apart: the tensor library's own sequence
+    assert np.array_equal(m.forward(wide).float(), x @ w.T + b)
+
+
+@pytest.mark.parametrize("batch,side", [(1, 1), (3, 7), (4, 64), (5, 64)])  # 5 * 64 * 64 > 16384: two stages
+def test_bias_gradient_of_a_small_layer(gt, batch, side):
+    rng = rng_for(404)
+    m = gt.nn.SpatialConvolutionMM(2, 5, 1, 1)
+    m.gradBias[...] = 3
+    m.gpu()
+    x, go = (rng.integers(-3, 4, size=(batch, c, side, side)).astype(np.float32) for c in (2, 5))
+    m.forward(dev(gt, x))
+    m.accGradParameters(dev(gt, x), dev(gt, go), 0.5)
+    assert np.array_equal(m.gradBias.float(), 3 + 0.5 * go.sum((0, 2, 3)))
