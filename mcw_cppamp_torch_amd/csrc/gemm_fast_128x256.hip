@@ -1,4 +1,4 @@
-// Fast fp32 MFMA GEMM, 128 x 256 workgroup tile (2 x 2 wavefronts).
+// Tiled fp32 GEMM, 128 x 256 workgroup tile (2 x 2 wavefronts).
 #include "gemm_fast.h"
 
 #include <type_traits>

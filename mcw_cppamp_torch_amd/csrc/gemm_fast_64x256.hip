@@ -1,4 +1,4 @@
-// Fast fp32 MFMA GEMM, 64 x 256 workgroup tile (1 x 4 wavefronts).
+// Tiled fp32 GEMM, 64 x 256 workgroup tile (1 x 4 wavefronts).
 #include "gemm_fast.h"
 
 #include <type_traits>

@@ -1,4 +1,4 @@
-// Fast fp32 MFMA GEMM, 96 x 128 workgroup tile (1 x 4 wavefronts, each 96 x 32): for products of 96 to 127 rows,
+// Tiled fp32 GEMM, 96 x 128 workgroup tile (1 x 4 wavefronts, each 96 x 32): for products of 96 to 127 rows,
 // which two 64-row tiles would cover with a third of their work repeated.  First operand along r only (its 384
 // 128-bit loads per step are made by 256 threads in two rounds, the second by the first two wavefronts).
 #include "gemm_fast.h"

@@ -1,4 +1,4 @@
-// fp32 GEMM on CDNA4 matrix cores (v_mfma_f32_32x32x2_f32), shared by
+// fp32 GEMM on CDNA4 matrix cores (six bf16 part products per product, gemm_fast.h; fp32 MFMA in gemm_generic.hip), shared by
 // THGPUBlas_gemm and the three GEMMs of nn.SpatialConvolutionMM.
 //
 // The kernels compute, in row-major terms with the output contiguous along j,
