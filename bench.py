@@ -57,6 +57,8 @@ sys.path.insert(0, ROOT)
 
 METRIC = "images/sec fwd+bwd, AlexNet-style conv stack b128 fp32; GEMM % fp32 MFMA peak"
 PEAK_MFMA_F32_TFLOPS = 157.3
+# The tiled GEMM kernel forms an fp32 product from six bf16 part products: dense bf16 peak / 6.
+PEAK_SPLIT_F32_TFLOPS = 2500.0 / 6.0
 PEAK_HBM_GBS = 8000.0
 ROUTES = {"columns": 0, "auto": 1, "gathered": 2}   # thgpu_conv_set_mode values
 # rocprofv3's FETCH_SIZE / WRITE_SIZE read these fractions of the bytes a plain float4 copy kernel of known size
@@ -699,7 +701,7 @@ def main():
                 ent["flops_per_step"] += fl
                 gemm_shapes.append({"gemm": kname, "launches_per_step": r["calls"] / steps,
                                     "ms_per_step": round(ms, 4), "tflops": round(fl / ms / 1e9, 2),
-                                    "frac": round(fl / ms / 1e9 / PEAK_MFMA_F32_TFLOPS, 4)})
+                                    "frac": round(fl / ms / 1e9 / PEAK_SPLIT_F32_TFLOPS, 4)})
                 g_ms += ms
                 g_fl += fl
                 g_calls += r["calls"]
@@ -721,7 +723,7 @@ def main():
             if ent.get("bound") == "mfma":
                 fl, ms = ent.pop("flops_per_step"), ent["ms_per_step"]
                 ent.update(ms_per_step=round(ms, 4), tflops=round(fl / ms / 1e9, 2),
-                           frac=round(fl / ms / 1e9 / PEAK_MFMA_F32_TFLOPS, 4))
+                           frac=round(fl / ms / 1e9 / PEAK_SPLIT_F32_TFLOPS, 4))
             else:
                 by, ms = ent.pop("bytes_per_step"), ent["ms_per_step"]
                 ent["ms_per_step"] = round(ms, 4)
@@ -739,8 +741,9 @@ def main():
                          % (g_fl + other_fl, algorithmic))
             res["roofline"] = {
                 "bound": "mfma", "kernel": "gemm_fast_kernel<...> (all conv GEMM launches of a step)",
-                "achieved": round(g_fl / g_ms / 1e9, 2), "peak": PEAK_MFMA_F32_TFLOPS, "unit": "TFLOP/s",
-                "frac": round(g_fl / g_ms / 1e9 / PEAK_MFMA_F32_TFLOPS, 4),
+                "achieved": round(g_fl / g_ms / 1e9, 2), "peak": round(PEAK_SPLIT_F32_TFLOPS, 1),
+                "unit": "TFLOP/s", "frac": round(g_fl / g_ms / 1e9 / PEAK_SPLIT_F32_TFLOPS, 4),
+                "frac_of_fp32_mfma_peak": round(g_fl / g_ms / 1e9 / PEAK_MFMA_F32_TFLOPS, 4),
                 "traffic": traffic, "traffic_note": why,
                 "launches_per_step": g_calls / steps, "ms_per_step": round(g_ms, 4),
                 "flops_per_step": g_fl,
