@@ -34,8 +34,9 @@
 //     fetches its MFMA operand, r = 8h .. 8h+7 of row x, with one 128-bit read, consecutive lanes from
 //     consecutive units.  The octet planes are 64 bytes longer than their rows need: LDS writes go to 32 banks (128 bytes),
 //     and of sixteen lanes that write 64 bits each, four to a row, half then fall on each 64 bytes of them.  (With 128 bytes
-//     both halves fell on the same banks: 95 % conflict cycles with both operands along r, 50 - 65 % with one; AlexNet-style
-//     step 3.18 -> 3.08 ms, VGG-A 16.1 -> 15.4 ms, 64 -> 128 planes 9x9 9.14 -> 8.54 ms for the three passes.)
+//     both halves fell on the same banks: 95 % conflict cycles with both operands along r, 50 - 65 % with one, none now.
+//     VGG-A step 15.8 -> 15.4 ms, 64 -> 128 planes 9x9 8.9 -> 8.5 ms for the three passes; within the 2 % by which
+//     cards differ on the AlexNet-style step.)
 //   * LDS is double buffered and the global loads run one step further ahead: while step s is multiplied, the
 //     registers hold step s+1, which is split and written to the other buffer in slices between the MFMAs, and every
 //     register is refilled for step s+2 as soon as it has been split: one barrier per reduction step, and a load has a
