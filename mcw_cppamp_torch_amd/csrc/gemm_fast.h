@@ -1,8 +1,9 @@
 // The tiled fp32 GEMM kernel (see gemm_mfma.h for the problem statement): fp32 operands, fp32 sums and results, with the
 // products formed on the bf16 matrix instructions.
 //
-// Every operand element is split without loss into three bf16 parts, x = h + m + l: h is x rounded to nearest, m the
-// remainder rounded, l what is left (8 + 8 + 8 significant bits hold the 24 of an fp32 number).  A product a*b is the sum
+// Every operand element is split into three bf16 parts, x = h + m + l: h is x rounded to nearest, m the
+// remainder rounded, l what is left (8 + 8 + 8 significant bits hold the 24 of an fp32 number; without loss for zero
+// and from 2^-110 up, see below).  A product a*b is the sum
 // of the part products that matter in fp32, h*h + (h*m + m*h) + (h*l + m*m + l*h), each exact in the fp32 accumulator's
 // input; the three dropped ones are below 2^-24 of the product together, and of either sign.  That is six
 // v_mfma_f32_32x32x16_bf16 where eight v_mfma_f32_32x32x2_f32 of twice the cycles each stood: 2.7 times the matrix
@@ -14,11 +15,16 @@
 // 64 bits over 3x3 to 11x11 layers and Linear products: 0.6 to 1.0 of the former (uniform operands).  What bounds it now is
 // power: see the efficiency figures in gemm_dispatch.hip.
 //
-// What the split cannot hold is multiplied in fp32 instead: an operand that is infinite, NaN or so large that h
-// rounds to infinity leaves an infinity or NaN in every accumulator it reaches, and a product sum that falls
-// below the normal numbers leaves a denormal.  A wavefront that finds one of these in a 32x32 block at the end computes
-// the block again from the operands with v_mfma_f32_32x32x2_f32 (recompute_block).  Operands below 2^-109 in
-// magnitude keep an absolute error of 2^-134 (the smallest bf16 step), which only such a sum can notice.
+// What the split cannot hold is multiplied in fp32 instead, with v_mfma_f32_32x32x2_f32 (recompute):
+//   * An operand below 2^-110 in magnitude can have bits under the smallest bf16 step, 2^-133, and then comes out short by
+//     up to 2^-134.  Against a large partner that reaches a result of ordinary size, so it is found at the operand: what
+//     l has to hold is a bf16 number exactly when the low half of its fp32 word is zero, and every thread collects these
+//     words (one v_or3_b32 per two elements: AlexNet-style step 3.20 -> 3.24 ms, 64 -> 128 planes 9x9 9.1 -> 9.4 ms for the
+//     three passes).  A workgroup that met a non-zero one multiplies its tile again.
+//     (Conversion, subtraction and the matrix instruction keep denormals on gfx950, so nothing else is lost.)
+//   * An operand that is infinite, NaN or so large that h rounds to infinity leaves an infinity or NaN in every
+//     accumulator it reaches, and a product sum that falls below the normal numbers leaves a denormal: a wavefront
+//     that finds one of these among its outputs computes them again.
 //
 // Structure
 //   * A workgroup of WGM x WGN wavefronts owns a BM x BN tile of C, each
@@ -43,7 +49,7 @@
 //     whole step to arrive.
 //   * Operands are fetched with buffer loads (descriptor and offsets in scalar registers, a constant lane offset), and
 //     the loop is unrolled by two so that the LDS buffer folds into the offset field of the LDS instructions: the only
-//     vector instructions of the loop are the split's (11 per two elements).
+//     vector instructions of the loop are the split's (12 per two elements).
 #pragma once
 
 #include <type_traits>
@@ -71,8 +77,9 @@ struct PartTile {
     static constexpr int kBytes = 3 * kPart;
 };
 
-// The three parts of two elements, two bf16 to a word.
-__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
+// The three parts of two elements, two bf16 to a word.  `lost` collects the remainders that l rounds: a set bit in its low
+// half says that some element was not held in full.
+__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l, unsigned &lost) {
     auto round2 = [](float a, float b) {
         return __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){a, b}, bf16x2));
     };
@@ -81,14 +88,19 @@ __device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsi
     h = round2(x0, x1);
     const float r0 = x0 - low(h), r1 = x1 - high(h);
     m = round2(r0, r1);
-    l = round2(r0 - low(m), r1 - high(m));
+    const float s0 = r0 - low(m), s1 = r1 - high(m);
+    l = round2(s0, s1);
+    // (written out: from the operators the compiler gathers the words of several pairs before it combines them, and spills)
+    asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(s0), "v"(s1));
 }
 
-// Wavefronts per SIMD the register allocation must leave room for: the
-// accumulators take (BM/WGM)*(BN/WGN)/64 registers of the 512 a lane has.
+// Wavefronts per SIMD the register allocation must leave room for: the accumulators take (BM/WGM)*(BN/WGN)/64 registers
+// of the 512 a lane has, and no more workgroups run on a CU than its 160 KB of LDS hold tile buffers for (four wavefronts
+// each, one to a SIMD).
 template <int BM, int BN, int WGM, int WGN>
 constexpr int gemm_min_waves() {
-    return (BM / WGM) * (BN / WGN) / 64 >= 96 ? 2 : 3;
+    constexpr int by_lds = 160 * 1024 / (2 * (PartTile<BM>::kBytes + PartTile<BN>::kBytes));
+    return (BM / WGM) * (BN / WGN) / 64 >= 96 || by_lds < 3 ? 2 : 3;
 }
 
 template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED>
@@ -350,6 +362,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     constexpr int GB = ((LB == LD_XC_SCALAR || LB == LD_XC_GATHER) && NB % 8 == 0) ? 8 : 4;
     char *const a_dst = &As[0][0] + (a_r >> 3) * TileA::kOctet + a_x * 16 + (a_r & 7) * 2;
     char *const b_dst = &Bs[0][0] + (b_r >> 3) * TileB::kOctet + b_x * 16 + (b_r & 7) * 2;
+    unsigned lost = 0;  // see split_pair
     auto stash_group = [&](auto kind_tag, auto group_tag, auto tile_tag, char *dst, const float *src, int q) {
         constexpr int KIND = decltype(kind_tag)::value;
         constexpr int G = decltype(group_tag)::value;
@@ -358,7 +371,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         const int off = G == 8 ? q * Tile::kOctet : (KIND == LD_XC_BLOCK ? q * 64 : q * (NT / 4)) * 16;
         unsigned p[3][G / 2];
 #pragma unroll
-        for (int e = 0; e < G / 2; ++e) split_pair(src[q * G + 2 * e], src[q * G + 2 * e + 1], p[0][e], p[1][e], p[2][e]);
+        for (int e = 0; e < G / 2; ++e) split_pair(src[q * G + 2 * e], src[q * G + 2 * e + 1], p[0][e], p[1][e], p[2][e], lost);
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             if constexpr (G == 8)
@@ -522,46 +535,101 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         if (s + 1 < nsteps) one_step(std::integral_constant<int, 1>{}, s + 1);
     }
 
-    // ---- blocks the split could not hold --------------------------------------------------
-    // The sum of one 32x32 block in fp32, straight from the operands: lane (x, h) takes r = 2t + h of step t.
-    auto recompute_block = [&](int a, int b) {
-        floatx16 sum;
+    // ---- what the split could not hold -----------------------------------------------------
+    // Did any thread's element lose bits?  (The operand tiles in LDS have been read: the loop ends with a barrier.)
+    unsigned *const lost_of = reinterpret_cast<unsigned *>(&As[0][0]);
+    const bool lost_here = __builtin_amdgcn_ballot_w64((lost & 0xffffu) != 0) != 0;
+    if (lane == 0) lost_of[wave] = lost_here ? 1u : 0u;
+    __syncthreads();
+    unsigned lost_any = 0;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
-        const int i = i0 + wm * (TM * 32) + a * 32 + l32, j = j0 + wn * (TN * 32) + b * 32 + l32;
-        unsigned im = 0, n = (unsigned)j;
-        if (!RED && LB != LD_RC_VEC) g.divN.divmod((unsigned)j, im, n);
-        const float *const arow = g.A + (LA == LD_XC_SCALAR ? (long)i : (long)i * g.sA);
-        const float *const bcol = g.B + (GATHER               ? (long)im * g.bsB + g.coltab[n]
-                                         : LB == LD_XC_SCALAR ? (long)im * g.bsB + n
-                                                              : (long)j * g.sB);
+    for (int w = 0; w < NT / 64; ++w) lost_any |= lost_of[w];
+    // The wavefront's outputs in fp32, straight from the operands: eight reduction indices at a time, four to a lane half,
+    // whose loads are in flight together.  (A step that would run past R is moved back as in the main loop.)
+    auto recompute = [&]() {
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+        struct __attribute__((packed, aligned(4))) Quad {
+            float v[4];
+        };
+        const float *arow[TM], *bcol[TN];
+#pragma unroll
+        for (int a = 0; a < TM; ++a) {
+            const long i = i0 + wm * (TM * 32) + a * 32 + l32;
+            arow[a] = g.A + (LA == LD_XC_SCALAR ? i : i * g.sA);
+        }
+#pragma unroll
+        for (int b = 0; b < TN; ++b) {
+            const unsigned j = (unsigned)(j0 + wn * (TN * 32) + b * 32 + l32);
+            unsigned im = 0, n = j;
+            if (!RED && LB != LD_RC_VEC) g.divN.divmod(j, im, n);
+            bcol[b] = g.B + (GATHER               ? (long)im * g.bsB + g.coltab[n]
+                             : LB == LD_XC_SCALAR ? (long)im * g.bsB + n
+                                                  : (long)j * g.sB);
+        }
+#pragma unroll 1
         for (int st = step; st < step_end; ++st) {
             unsigned img = 0, w = (unsigned)st;
             if (RED) g.divSpi.divmod((unsigned)st, img, w);
-            const int r_end = ((int)w + 1) * BK < g.R ? ((int)w + 1) * BK : g.R;
-            for (int r = (int)w * BK; r < r_end; r += 2) {
-                const int rl = r + half;
-                float av = 0.0f, bv = 0.0f;
-                if (rl < r_end) {
-                    av = arow[(RED ? (long)img * g.rbA : 0L) + (LA == LD_XC_SCALAR ? (long)rl * g.sA : (long)rl)];
-                    bv = bcol[(RED ? (long)img * g.rbB : 0L) + (GATHER               ? (long)g.rowtab[rl]
-                                                                : LB == LD_XC_SCALAR ? (long)rl * g.sB
-                                                                                     : (long)rl)];
+            const int first = (int)w * BK, r0 = first + BK <= g.R ? first : g.R - BK;
+            const long imA = RED ? (long)img * g.rbA : 0L, imB = RED ? (long)img * g.rbB : 0L;
+#pragma unroll 1
+            for (int c = 0; c < BK; c += 8) {
+                const int r = r0 + c + 4 * half;  // the lane's r .. r+3
+                float x[TM][4], y[TN][4];
+#pragma unroll
+                for (int a = 0; a < TM; ++a)
+                    if (LA == LD_XC_SCALAR) {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) x[a][t] = arow[a][(long)(r + t) * g.sA];
+                    } else {
+                        const Quad q = *reinterpret_cast<const Quad *>(arow[a] + imA + r);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) x[a][t] = q.v[t];
+                    }
+                int off[4];
+                if (GATHER) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) off[t] = g.rowtab[r + t];
                 }
-                sum = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, sum, 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < TN; ++b)
+                    if (LB == LD_RC_VEC) {
+                        const Quad q = *reinterpret_cast<const Quad *>(bcol[b] + imB + r);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) y[b][t] = q.v[t];
+                    } else {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) y[b][t] = bcol[b][imB + (GATHER ? (long)off[t] : (long)(r + t) * g.sB)];
+                    }
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const bool covered = r + t < first;  // by the step before
+#pragma unroll
+                    for (int a = 0; a < TM; ++a) x[a][t] = covered ? 0.0f : x[a][t];
+#pragma unroll
+                    for (int b = 0; b < TN; ++b) y[b][t] = covered ? 0.0f : y[b][t];
+#pragma unroll
+                    for (int a = 0; a < TM; ++a)
+#pragma unroll
+                        for (int b = 0; b < TN; ++b)
+                            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[a][t], y[b][t], acc[a][b], 0, 0, 0);
+                }
             }
         }
-        return sum;
     };
+    bool odd = lost_any != 0;
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
-        for (int b = 0; b < TN; ++b) {
-            bool odd = false;
+        for (int b = 0; b < TN; ++b)
 #pragma unroll
             for (int v = 0; v < 16; ++v) odd |= __builtin_amdgcn_classf(acc[a][b][v], 0x297);  // NaN, infinite, denormal
-            if (__builtin_amdgcn_ballot_w64(odd)) acc[a][b] = recompute_block(a, b);
-        }
+    if (__builtin_amdgcn_ballot_w64(odd)) recompute();
 
     // ---- epilogue ----------------------------------------------------------------------
     // Accumulator register v of lane l holds D[8*(v/4) + 4*(l/32) + v%4][l%32].

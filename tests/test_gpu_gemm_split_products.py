@@ -1,8 +1,12 @@
 """The tiled GEMM kernel forms its products from three bf16 parts of each operand: its error against 64 bits, and the
-values that the parts cannot hold (infinities, NaN, numbers that round to infinity in bf16, results below the normal
-range), which it multiplies in fp32 instead."""
+values that the parts cannot hold (operands with bits below the smallest bf16 step, infinities, NaN, numbers that round to
+infinity in bf16, results below the normal range), which it multiplies in fp32 instead.  Every tile and loader: the four
+operand layouts through the BLAS entry point, the gathering loaders and reduction batching through convolution layers."""
+import functools
+
 import numpy as np
 import pytest
+import torch
 
 from helpers import rng_for
 
@@ -69,3 +73,131 @@ def test_results_below_the_normal_range(gt):
     A[:, ::4] = np.float32(1.5 * 2.0 ** -65)
     B[::4, :] = np.float32(2.0 ** -65)
     assert np.array_equal(product(gt, A, B), np.full((m, n), np.float32(8 * 1.5 * 2.0 ** -130)))
+
+
+TILES = {"128x128": (128, 128), "192x128": (192, 128), "64x256": (64, 256), "128x256": (128, 256),
+         "256x128": (256, 128), "64x64": (64, 64), "64x128": (64, 128), "96x128": (96, 128)}
+LAYOUTS = [(tile, ta, tb) for tile in TILES for ta in "nt" for tb in "nt" if not (tile == "96x128" and ta == "t")]
+
+
+def blas(gt, ta, tb, A, B):
+    """C = A B (A m x k, B k x n) with either operand stored along k ('n' for A, 't' for B) or along its free index; the
+    per-kernel timing labels of the product come with it."""
+    (m, k), n = A.shape, B.shape[1]
+    da = gt.FloatTensor(np.ascontiguousarray(A if ta == "n" else A.T)).gpu()
+    db = gt.FloatTensor(np.ascontiguousarray(B if tb == "n" else B.T)).gpu()
+    dc = gt.FloatTensor(np.full((m, n), 7.0, np.float32)).gpu()
+    rec = gt.gputorch
+    rec.synchronize()
+    rec.prof_reset()
+    rec.prof_enable(True)
+    try:
+        rec.gemm(tb, ta, n, m, k, 1.0, db, n if tb == "n" else k, da, k if ta == "n" else m, 0.0, dc, n)
+        rec.synchronize()
+        labels = [key for key in rec.prof_report() if key.startswith("gemm_blas")]
+    finally:
+        rec.prof_enable(False)
+        rec.prof_reset()
+    return dc.float(), labels
+
+
+def columns64(x, geo):
+    """im2col in 64 bits: (B, C*kH*kW, N)."""
+    kH, kW, pH, pW, sH, sW = geo
+    return torch.nn.functional.unfold(torch.from_numpy(x).double(), (kH, kW), padding=(pH, pW), stride=(sH, sW)).numpy()
+
+
+def image64(cols, shape, geo):
+    kH, kW, pH, pW, sH, sW = geo
+    return torch.nn.functional.fold(torch.from_numpy(cols), shape[2:], (kH, kW), padding=(pH, pW), stride=(sH, sW)).numpy()
+
+
+def conv64(x, w, go, geo):
+    """Output, gradInput and gradWeight of a layer in 64 bits."""
+    cols, g = columns64(x, geo), go.reshape(go.shape[0], go.shape[1], -1).astype(np.float64)
+    W = w.astype(np.float64)
+    return (np.matmul(W, cols).reshape(go.shape), image64(np.matmul(W.T, g), x.shape, geo),
+            np.matmul(g, cols.transpose(0, 2, 1)).sum(0))
+
+
+def conv(gt, x, w, go, geo):
+    """The same of nn.SpatialConvolutionMM, bias zero; labels of its products."""
+    kH, kW, pH, pW, sH, sW = geo
+    m = gt.nn.SpatialConvolutionMM(x.shape[1], w.shape[0], kW, kH, sW, sH, 0, padW=pW, padH=pH)
+    m._assign("weight", w)
+    m.bias[...] = 0
+    m.gradWeight[...] = 0
+    m.gpu()
+    dx, dgo = gt.FloatTensor(x).gpu(), gt.FloatTensor(go).gpu()
+    rec = gt.gputorch
+    rec.synchronize()
+    rec.prof_reset()
+    rec.prof_enable(True)
+    try:
+        out = m.forward(dx)
+        gi = m.updateGradInput(dx, dgo)
+        m.accGradParameters(dx, dgo, 1.0)
+        rec.synchronize()
+        labels = [key for key in rec.prof_report() if key.startswith("gemm_conv")]
+    finally:
+        rec.prof_enable(False)
+        rec.prof_reset()
+    return out.float(), gi.float(), m.gradWeight.float(), labels
+
+
+def magnitudes(rng, shape, exponent):
+    """Numbers of full precision (as far as fp32 has it there), 1 to 2 times a power of two, either sign."""
+    return np.ldexp(rng.uniform(1, 2, shape), exponent).astype(np.float32) * rng.choice(np.float32([-1, 1]), shape)
+
+
+# exponents of the small operand and of its partner: results from just above the normal range to ordinary numbers
+SMALL = [(-112, 0), (-120, 0), (-126, 60), (-140, 120)]
+
+
+@pytest.mark.parametrize("split", [1, 2])
+@pytest.mark.parametrize("tile,ta,tb", LAYOUTS)
+def test_small_operands(gt, switches, tile, ta, tb, split):
+    """Operands with bits under the smallest bf16 step, either one, in every row (column) or in a single one, which few
+    threads load: the bound of fp32 sums (k products and additions, each rounded; one more per part)."""
+    switches("gemm_tile", tile)
+    switches("gemm_split", split)
+    (m, n), k = (d + 3 for d in TILES[tile]), 16 * 16 + 5
+    rng = rng_for(303)
+    for small, large in SMALL:
+        for swap in (False, True):
+            for everywhere in (False, True):
+                rows, other = (n, m) if swap else (m, n)
+                P, Q = magnitudes(rng, (rows, k), min(0, 100 - large)), magnitudes(rng, (k, other), large)
+                some = np.s_[:] if everywhere else np.s_[rng.integers(rows)]
+                P[some] = magnitudes(rng, P[some].shape, small)
+                A, B = (Q.T, P.T) if swap else (P, Q)
+                got, labels = blas(gt, ta, tb, A, B)
+                assert len(labels) == 1 and "tile=%s split=%d" % (tile, split) in labels[0], labels
+                ref = A.astype(np.float64) @ B.astype(np.float64)
+                S = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)
+                assert np.all(np.abs(got - ref) <= (k + split + 1) * 2.0 ** -24 * S), (small, large, swap, everywhere)
+
+
+@functools.lru_cache(maxsize=None)
+def small_layer(batch, width, small, large, which):
+    rng = rng_for(304)
+    C = M = 256
+    x, w, go = (magnitudes(rng, shape, small if which == name else large)
+                for name, shape in (("x", (batch, C, 32, width)), ("w", (M, C * 9)), ("go", (batch, M, 32, width))))
+    geo = (3, 3, 1, 1, 1, 1)
+    return x, w, go, geo, conv64(x, w, go, geo), conv64(np.abs(x), np.abs(w), np.abs(go), geo)
+
+
+# width 8: image rows of whole quads (128-bit gathers in gradWeight); 9: not.  Two images and one.
+@pytest.mark.parametrize("tile", list(TILES))
+@pytest.mark.parametrize("batch,width", [(2, 8), (2, 9), (1, 8), (1, 9)])
+def test_small_operands_in_convolution_layers(gt, gathered_route, switches, tile, batch, width):
+    switches("gemm_tile", tile)
+    for small, large in ((-120, 20), (-130, 50)):
+        for which in ("x", "w", "go"):
+            x, w, go, geo, ref, S = small_layer(batch, width, small, large, which)
+            *got, labels = conv(gt, x, w, go, geo)
+            assert len(labels) == 3 and all("tile=%s " % tile in l for l in labels), labels
+            # the longest sums: taps, gradients, pixels; at most 256 parts
+            for g, r, s, terms in zip(got, ref, S, (w.shape[1], w.shape[0] * 9, batch * 32 * width)):
+                assert np.all(np.abs(g.reshape(r.shape) - r) <= (terms + 258) * 2.0 ** -24 * s), (small, large, which, terms)
