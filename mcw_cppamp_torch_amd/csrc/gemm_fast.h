@@ -467,8 +467,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
             fetch_rows(pos);
         }
         bf16x8 av[TM][3], bv[TN][3];
-#pragma unroll
-        for (int u = 0; u < 3; ++u) {  // in the order of their first use
+        auto fetch_parts = [&](int u) {  // in the order of their first use
             const int ta = u == 0 ? 2 : u - 1, tb = u == 0 ? 0 : 3 - u;
 #pragma unroll
             for (int a = 0; a < TM; ++a)
@@ -476,7 +475,12 @@ __global__ __launch_bounds__(WGM *WGN * 64)
 #pragma unroll
             for (int b = 0; b < TN; ++b)
                 bv[b][tb] = *reinterpret_cast<const bf16x8 *>(b_src + buf * TileB::kBytes + tb * TileB::kPart + b * 512);
-        }
+        };
+        // (the widest tile's per-lane row offsets leave no registers for all of them: the last ones come a slice later)
+        constexpr bool LATE = LB == LD_RC_GATHER && TN == 4;
+        fetch_parts(0);
+        fetch_parts(1);
+        if (!LATE) fetch_parts(2);
         constexpr int SLICES = 6;
         auto slice_of = [&](auto slice_tag) {
             constexpr int slice = decltype(slice_tag)::value;
@@ -501,6 +505,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                     stash_b(buf ^ 1, q);
                     refill_b(gb, q);
                 }
+            if (LATE && slice == 0) fetch_parts(2);
             if (slice == 3 && !RG) {
                 int pos = ld_r0 + BK;
                 if (RED && pos >= g.R) pos = 0;
@@ -695,20 +700,23 @@ __global__ __launch_bounds__(WGM *WGN * 64)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) bias_v[v] = 0.0f;
             }
-            // What C held, requested as one batch before the first store (a load per store, each waited for, ran a
-            // 4096 x 9216 accumulation over 128 indices at 1.7 TB/s).
-            float held[MODE == 2 ? 16 : 1][MODE == 2 ? TN : 1];
-            if constexpr (MODE == 2) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int ir = iu + 8 * (v / 4) + (v % 4);
-#pragma unroll
-                    for (int b = 0; b < TN; ++b)
-                        held[v][b] = *reinterpret_cast<const float *>(out + (long)ir * row_bytes + voff[b]);
-                }
-            }
+            // What C held, requested in batches of sixteen loads before the stores that need them.  A load per store, each
+            // waited for, ran a 4096 x 9216 accumulation over 128 indices at 1.7 TB/s; one batch of all 16 * TN spilled
+            // 60 to 300 registers (118 us, 2.6 TB/s; 96 us and 3.2 now, 4096 x 4096 77 -> 49 us).
+            constexpr int ROWS = MODE == 2 && TN > 1 ? 16 / TN : 16;
+            float held[MODE == 2 ? ROWS : 1][MODE == 2 ? TN : 1];
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
+                if (MODE == 2 && v % ROWS == 0) {
+#pragma unroll
+                    for (int q = 0; q < ROWS; ++q) {
+                        const int ir = iu + 8 * ((v + q) / 4) + ((v + q) % 4);
+#pragma unroll
+                        for (int b = 0; b < TN; ++b)
+                            held[MODE == 2 ? q : 0][MODE == 2 ? b : 0] =
+                                *reinterpret_cast<const float *>(out + (long)ir * row_bytes + voff[b]);
+                    }
+                }
                 const int ir = iu + 8 * (v / 4) + (v % 4);  // uniform; the lane's row is ir + 4*half
                 if (CHECK && ir + 4 * half < own_i0) continue;
 #pragma unroll
@@ -717,7 +725,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                     float *c = reinterpret_cast<float *>(out + (long)ir * row_bytes + voff[b]);
                     float val = acc[a][b][v];
                     if (MODE != 0) val = val * g.alpha + (bias_v[v] + col_bias[b]);
-                    if constexpr (MODE == 2) val += g.beta * held[v][b];
+                    if constexpr (MODE == 2) val += g.beta * held[v % ROWS][b];
                     if (act) val = val > g.act_threshold ? val : g.act_value;
                     if (masked) {
                         const float mv = *reinterpret_cast<const float *>(msk + (long)ir * mask_row_bytes + mvoff[b]);
