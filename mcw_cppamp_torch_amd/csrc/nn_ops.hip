@@ -762,6 +762,7 @@ int thgpu_Linear_accGradBias(THGPUTensor *gradOutput, THGPUTensor *gradBias, flo
         return fail("Linear: size mismatch");
     const long B = gradOutput->size[0], O = gradOutput->size[1];
     if (!tensor_ready(gradOutput, B * O) || !tensor_ready(gradBias, O)) return fail("Linear: operands must be contiguous");
+    if (scale == 0.0f) return 0;  // BLAS: a zero factor leaves the result as it is, whatever the gradient holds
     return column_sums_launch(dptr(gradOutput), dptr(gradBias), B, O, scale);
 }
 

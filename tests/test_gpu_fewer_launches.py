@@ -66,6 +66,16 @@ def test_linear_integer_exact(gt, batch, inputs, outputs):
     assert np.array_equal(m.forward(wide).float(), x @ w.T + b)
 
 
+def test_linear_gradients_with_scale_zero_stay_as_they_are(gt):
+    m = gt.nn.Linear(7, 5)
+    m.gradBias[...] = 3
+    m.gradWeight[...] = 2
+    m.gpu()
+    go = np.full((4, 5), np.nan, np.float32)
+    m.accGradParameters(dev(gt, np.full((4, 7), np.inf, np.float32)), dev(gt, go), 0.0)
+    assert np.all(m.gradBias.float() == 3) and np.all(m.gradWeight.float() == 2)
+
+
 @pytest.mark.parametrize("batch,side", [(1, 1), (3, 7), (4, 64), (5, 64)])  # 5 * 64 * 64 > 16384: two stages
 def test_bias_gradient_of_a_small_layer(gt, batch, side):
     rng = rng_for(404)
