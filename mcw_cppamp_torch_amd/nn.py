@@ -87,6 +87,11 @@ def _add_all(params, value, grads):
             p += np.float32(value) * g
 
 
+def _plain(module, *methods):
+    """Whether the module keeps Module's own implementation of the methods: none overridden by its class or set on it."""
+    return all(getattr(getattr(module, m), "__func__", None) is getattr(Module, m) for m in methods)
+
+
 class Module(object):
     def __init__(self):
         self.gradInput = FloatTensor()
@@ -235,8 +240,7 @@ class Sequential(Module):
         # container) that overrides the method has its own called.
         plain, grads = [], []
         for m in self.modules:
-            if type(m).zeroGradParameters is Module.zeroGradParameters and type(m).parameters in (
-                    Module.parameters,):
+            if _plain(m, "zeroGradParameters", "parameters"):
                 plain.append(m)
             else:
                 m.zeroGradParameters()
@@ -318,7 +322,7 @@ class Sequential(Module):
             del params[:], grads[:]
 
         for m in self.modules:
-            if type(m).updateParameters is Module.updateParameters and type(m).parameters is Module.parameters:
+            if _plain(m, "updateParameters", "parameters"):
                 p, g = m.parameters()
                 params.extend(p or [])
                 grads.extend(g or [])

@@ -230,6 +230,23 @@ def test_more_module_defaults_follow_the_lua_constructors(pkg):
         seq.insert(nn.ReLU(), 9)
 
 
+def test_sequential_calls_a_method_set_on_a_module(pkg):
+    """mcw_nn/Sequential.lua:85-95 calls every module's own method, also one that a program put on the object."""
+    nn = pkg.nn
+    seq = nn.Sequential().add(nn.Linear(3, 2)).add(nn.Linear(2, 2))
+    for m in seq.modules:
+        m.gradWeight[...], m.gradBias[...] = 1, 1
+    frozen, moved = (np.array(m.weight) for m in seq.modules)
+    called = []
+    seq.get(0).updateParameters = lambda lr: called.append(("update", lr))
+    seq.get(0).zeroGradParameters = lambda: called.append(("zero",))
+    seq.updateParameters(0.5)
+    assert np.array_equal(seq.get(0).weight, frozen) and np.array_equal(seq.get(1).weight, moved - np.float32(0.5))
+    seq.zeroGradParameters()
+    assert called == [("update", 0.5), ("zero",)]
+    assert np.all(seq.get(0).gradWeight == 1) and np.all(seq.get(1).gradWeight == 0)
+
+
 def test_product_never_imports_the_oracle_and_bench_refuses_more_than_one_gpu():
     import glob
     import os
