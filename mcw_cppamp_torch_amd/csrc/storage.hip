@@ -5,8 +5,10 @@
 #include "common.h"
 #include "kernels.h"
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <unordered_map>
 #include <vector>
 
@@ -84,6 +86,34 @@ __global__ __launch_bounds__(256) void many_kernel(const Many f, float v) {
         return;
     }
     for (unsigned i = threadIdx.x; i < n; i += 256) p[i] = one(AXPY ? p[i] : 0.0f, AXPY ? x[i] : 0.0f);
+}
+
+// Whether some y[i] shares memory with a y[j] or x[j] of another pair.  The results are sorted by address: neighbours show
+// whether two of them meet, and where none do, a search finds the ones that an x[j] meets.
+inline bool results_shared(THGPUTensor **y, THGPUTensor **x, int count) {
+    struct Range {
+        const float *begin, *end;
+        int pair;
+    };
+    std::vector<Range> ys;
+    ys.reserve((size_t)count);
+    for (int i = 0; i < count; ++i)
+        if (const long n = THGPUTensor_nElement(y[i])) {
+            const float *p = THGPUTensor_data(y[i]);
+            ys.push_back({p, p + n, i});
+        }
+    std::sort(ys.begin(), ys.end(), [](const Range &a, const Range &b) { return a.begin < b.begin; });
+    for (size_t k = 1; k < ys.size(); ++k)
+        if (ys[k].begin < ys[k - 1].end) return true;
+    for (int j = 0; j < count; ++j) {
+        const long n = THGPUTensor_nElement(x[j]);
+        if (n == 0) continue;
+        const float *p = THGPUTensor_data(x[j]);
+        auto k = std::upper_bound(ys.begin(), ys.end(), p, [](const float *v, const Range &r) { return v < r.end; });
+        for (; k != ys.end() && k->begin < p + n; ++k)
+            if (k->pair != j) return true;
+    }
+    return false;
 }
 
 // Launches for entries [0, count) of the caller's list, kManyMax at a time.
@@ -457,13 +487,12 @@ extern "C" int thgpu_axpy_many(THGPUTensor **y, THGPUTensor **x, int count, floa
             return fail("thgpu_axpy_many: pair %d is not contiguous or exceeds its storage", i);
     }
     // Buffers that share memory (a weight used by two modules) are updated one after the other, in the order given.
-    auto overlap = [](THGPUTensor *a, THGPUTensor *b) {
-        const float *pa = THGPUTensor_data(a), *pb = THGPUTensor_data(b);
-        return pa < pb + THGPUTensor_nElement(b) && pb < pa + THGPUTensor_nElement(a);
-    };
-    bool shared = false;
-    for (int i = 0; i < count && !shared; ++i)
-        for (int j = 0; j < count && !shared; ++j) shared = (i != j && overlap(y[i], y[j])) || (i != j && overlap(y[i], x[j]));
+    bool shared;
+    try {
+        shared = results_shared(y, x, count);
+    } catch (const std::bad_alloc &) {
+        return fail("thgpu_axpy_many: out of host memory");
+    }
     auto launch = [&](int first, int n) {
         return many_launch<true>(n, value, "axpy", [&](int i, float *&p, const float *&q) {
             p = THGPUTensor_data(y[first + i]);

@@ -66,6 +66,50 @@ def test_linear_integer_exact(gt, batch, inputs, outputs):
     assert np.array_equal(m.forward(wide).float(), x @ w.T + b)
 
 
+@pytest.mark.parametrize("n", [2, 40, 300])
+def test_axpy_many_finds_shared_memory_among_many_pairs(gt, n):
+    """Results that meet one another or another pair's operand are updated in the order given: a pair's operand is another
+    pair's result, results overlap by one element, and (not shared) an operand is its own pair's result."""
+    rng = rng_for(405)
+    host = rng.integers(-8, 9, size=40 * n).astype(np.float32)
+    order = rng.permutation(n)
+    for kind in ("operand", "overlap", "own", "apart"):
+        whole, other = dev(gt, host), dev(gt, host[::-1])
+        y0, x0 = host.copy(), host[::-1].copy()
+        begin = [int(40 * i) for i in order]
+        ys, xs = [whole.narrow(0, b, 40) for b in begin], [other.narrow(0, b, 40) for b in begin]
+        hy, hx = [y0[b:b + 40] for b in begin], [x0[b:b + 40] for b in begin]
+        if kind == "operand":
+            xs[0], hx[0] = ys[n - 1], hy[n - 1]
+        elif kind == "overlap":
+            c = begin[n - 1] - 1 if begin[n - 1] > 0 else 1
+            ys[n - 1], hy[n - 1] = whole.narrow(0, c, 40), y0[c:c + 40]
+        elif kind == "own":
+            xs[n - 1], hx[n - 1] = ys[n - 1], hy[n - 1]
+        gt._lib.check_status(gt._lib.lib.thgpu_axpy_many(pointers(gt, ys), pointers(gt, xs), n, 2.0))
+        for y, x in zip(hy, hx):
+            y += 2 * x
+        assert np.array_equal(whole.float(), y0), kind
+
+
+def test_axpy_many_host_time_grows_with_the_number_of_pairs(gt):
+    """Ten times the pairs take about ten times as long on the host (all pairs against all: a hundred)."""
+    import time
+    took = {}
+    for n in (300, 3000):
+        whole, other = gt.GPUTensor(8 * n).fill(1), gt.GPUTensor(8 * n).fill(1)
+        pairs = [(whole.narrow(0, 8 * i, 8), other.narrow(0, 8 * i, 8)) for i in range(n)]
+        ys, xs = pointers(gt, [y for y, _ in pairs]), pointers(gt, [x for _, x in pairs])
+        times = []
+        for _ in range(7):
+            gt.gputorch.synchronize()
+            start = time.perf_counter()
+            assert gt._lib.lib.thgpu_axpy_many(ys, xs, n, 0.5) == 0
+            times.append(time.perf_counter() - start)
+        took[n] = min(times)
+    assert took[3000] < 40 * took[300], took
+
+
 def test_linear_gradients_with_scale_zero_stay_as_they_are(gt):
     m = gt.nn.Linear(7, 5)
     m.gradBias[...] = 3
