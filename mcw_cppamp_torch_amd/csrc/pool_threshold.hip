@@ -1291,10 +1291,10 @@ int gradbias_launch(const float *gout, float *gbias, long B, int M, long N, floa
     const int ips = (int)((B + nslices - 1) / nslices);
     nslices = (B + ips - 1) / ips;
     if (nslices < 1) nslices = 1;
-    // The partial sums live behind the GEMM's split workspace, which the
+    // The partial sums of several slices live behind the GEMM's split workspace, which the
     // gradWeight GEMM enqueued before has finished with (same stream).
-    float *part = workspace(sizeof(float) * (size_t)M * nslices);
-    if (!part) return 1;
+    float *part = nullptr;
+    if (nslices > 1 && !(part = workspace(sizeof(float) * (size_t)M * nslices))) return 1;
     {
         LaunchScope scope("gradbias", 0.0, 4.0 * B * M * N);
         hipLaunchKernelGGL(gradbias_partial_kernel, dim3((unsigned)M, (unsigned)nslices), dim3(256), 0, s, gout,

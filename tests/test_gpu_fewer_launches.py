@@ -130,3 +130,27 @@ def test_bias_gradient_of_a_small_layer(gt, batch, side):
     m.forward(dev(gt, x))
     m.accGradParameters(dev(gt, x), dev(gt, go), 0.5)
     assert np.array_equal(m.gradBias.float(), 3 + 0.5 * go.sum((0, 2, 3)))
+
+
+def test_bias_gradient_of_one_launch_allocates_nothing(gt):
+    """A layer whose gradients take one launch each must not set up scratch memory: counted in a fresh process, whose
+    library has none yet."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = """
+import numpy as np, mcw_cppamp_torch_amd as gt
+lib = gt._lib.lib
+m = gt.nn.SpatialConvolutionMM(2, 5, 1, 1).gpu()
+x, go = gt.GPUTensor(1, 2, 7, 7).fill(1), gt.GPUTensor(1, 5, 7, 7).fill(2)
+m.forward(x)
+gt.gputorch.synchronize()
+before = lib.thgpu_device_alloc_calls()
+m.accGradParameters(x, go, 1)
+gt.gputorch.synchronize()
+print("allocations", lib.thgpu_device_alloc_calls() - before)
+"""
+    out = subprocess.run([sys.executable, "-c", code], cwd=root, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
+                         timeout=100)
+    assert out.stdout.splitlines()[-1:] == ["allocations 0"], out.stdout
