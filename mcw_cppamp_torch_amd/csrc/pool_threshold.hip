@@ -969,25 +969,28 @@ __global__ __launch_bounds__(256) void gradbias_final_kernel(const float *__rest
 __global__ __launch_bounds__(1024) void column_sums_kernel(const float *__restrict__ in, float *__restrict__ out,
                                                            int rows, int cols, float scale) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long col = (long)blockIdx.x * 64 + lane;
-    float sum = 0.0f;
-    if (col < cols) {
-        const float *src = in + col;
-        for (long r0 = wave; r0 < rows; r0 += 64) {
-            float v[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = r0 + 16 * u < rows ? src[(r0 + 16 * u) * cols] : 0.0f;
-            sum += (v[0] + v[1]) + (v[2] + v[3]);
-        }
-    }
     __shared__ float part[16][64];
-    part[wave][lane] = sum;
-    __syncthreads();
-    for (int h = 8; h > 0; h >>= 1) {
-        if (wave < h) part[wave][lane] += part[wave + h][lane];
+    for (long first = (long)blockIdx.x * 64; first < cols; first += (long)gridDim.x * 64) {
+        const long col = first + lane;
+        float sum = 0.0f;
+        if (col < cols) {
+            const float *src = in + col;
+            for (long r0 = wave; r0 < rows; r0 += 64) {
+                float v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = r0 + 16 * u < rows ? src[(r0 + 16 * u) * cols] : 0.0f;
+                sum += (v[0] + v[1]) + (v[2] + v[3]);
+            }
+        }
+        part[wave][lane] = sum;
+        __syncthreads();
+        for (int h = 8; h > 0; h >>= 1) {
+            if (wave < h) part[wave][lane] += part[wave + h][lane];
+            __syncthreads();
+        }
+        if (wave == 0 && col < cols) out[col] += scale * part[0][lane];
         __syncthreads();
     }
-    if (wave == 0 && col < cols) out[col] += scale * part[0][lane];
 }
 
 }  // namespace
@@ -1270,8 +1273,9 @@ int column_sums_launch(const float *in, float *out, long rows, long cols, float 
     if (rows >= (1L << 31) || cols >= (1L << 31)) return fail("column sums: matrix too large");
     {
         LaunchScope scope("column_sums", 0.0, 4.0 * (rows * cols + 2.0 * cols));
-        hipLaunchKernelGGL(column_sums_kernel, dim3((unsigned)((cols + 63) / 64)), dim3(1024), 0, s, in, out, (int)rows,
-                           (int)cols, scale);
+        // (a launch has fewer than 2^32 threads)
+        const long blocks = (cols + 63) / 64 < (1L << 21) ? (cols + 63) / 64 : 1L << 21;
+        hipLaunchKernelGGL(column_sums_kernel, dim3((unsigned)blocks), dim3(1024), 0, s, in, out, (int)rows, (int)cols, scale);
     }
     return check_launch("column_sums");
 }

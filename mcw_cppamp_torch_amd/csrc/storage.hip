@@ -116,32 +116,38 @@ inline bool results_shared(THGPUTensor **y, THGPUTensor **x, int count) {
     return false;
 }
 
-// Launches for entries [0, count) of the caller's list, kManyMax at a time.
+// Launches for entries [0, count) of the caller's list, kManyMax at a time and fewer than 2^32 threads each: what is left
+// of a tensor that does not fit goes to the next launch.
 template <bool AXPY, typename Entry>
 int many_launch(int count, float v, const char *tag, Entry entry) {
     hipStream_t s = stream();
     if (!s) return 1;
+    constexpr long kMaxChunks = (1L << 24) - 1;  // of 256 threads
+    long done = 0;                               // elements of entry i that earlier launches took
     for (int i = 0; i < count;) {
         Many f;
         f.count = 0;
         f.first[0] = 0;
         double total = 0.0;
-        for (; i < count && f.count < kManyMax; ++i) {
+        while (i < count && f.count < kManyMax && (long)f.first[f.count] < kMaxChunks) {
             float *p;
             const float *x;
-            const long n = entry(i, p, x);
-            if (n == 0) continue;
-            const long chunks = (n + kManyChunk - 1) / kManyChunk;
-            if (chunks + (long)f.first[f.count] >= (1L << 31)) {
-                if (f.count == 0) return fail("%s: tensor too large", tag);
-                break;  // the next launch's
+            const long n = entry(i, p, x) - done;
+            const long room = (kMaxChunks - (long)f.first[f.count]) * kManyChunk;
+            const long part = n < room ? n : room;
+            if (part > 0) {
+                f.p[f.count] = p + done;
+                f.x[f.count] = x ? x + done : nullptr;
+                f.n[f.count] = part;
+                f.first[f.count + 1] = f.first[f.count] + (unsigned)((part + kManyChunk - 1) / kManyChunk);
+                ++f.count;
+                total += (double)part;
             }
-            f.p[f.count] = p;
-            f.x[f.count] = x;
-            f.n[f.count] = n;
-            f.first[f.count + 1] = f.first[f.count] + (unsigned)chunks;
-            ++f.count;
-            total += (double)n;
+            done += part;
+            if (part == n) {
+                ++i;
+                done = 0;
+            }
         }
         if (f.count == 0) continue;
         {

@@ -120,6 +120,14 @@ def test_linear_gradients_with_scale_zero_stay_as_they_are(gt):
     assert np.all(m.gradBias.float() == 3) and np.all(m.gradWeight.float() == 2)
 
 
+def test_linear_bias_gradient_of_more_columns_than_a_launch_has_threads_for(gt):
+    n = (1 << 28) + 70  # 64 columns to a workgroup of 1024: 2^32 threads and more
+    go, gb = gt.GPUTensor(1, n).fill(2), gt.GPUTensor(n).fill(1)
+    gt._lib.check_status(gt._lib.lib.thgpu_Linear_accGradBias(go._p, gb._p, 0.5))
+    for at in (0, 1 << 27, n - 200):
+        assert np.all(gb.narrow(0, at, 200).float() == 2), at
+
+
 @pytest.mark.parametrize("batch,side", [(1, 1), (3, 7), (4, 64), (5, 64)])  # 5 * 64 * 64 > 16384: two stages
 def test_bias_gradient_of_a_small_layer(gt, batch, side):
     rng = rng_for(404)
