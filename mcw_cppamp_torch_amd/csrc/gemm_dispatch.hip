@@ -113,20 +113,18 @@ struct TileCfg {
     const char *name;
     int bm, bn;
     int resident;  // workgroups that fit a CU at once (registers / LDS)
-    // Fraction of the MFMA rate (kFlopsPerCycle) the inner loop sustains with a full CU, by operand layout: [0] A along r, B along j (forward); [1] both along their free
-    // index (gradInput); [2] both along r (gradWeight); [3] A along i, B along r; [4] A along r, B gathered;
-    // [5] the same with reduction batching.
+    // Fraction of the MFMA rate (kFlopsPerCycle) the inner loop sustains with a full CU, by operand layout: [0] A along r,
+    // B along j (forward); [1] both along their free index (gradInput); [2] both along r (gradWeight); [3] A along i, B
+    // along r; [4] A along r, B gathered; [5] the same with reduction batching.
     // Measured like the occupancy tables below.  None is near 1: on uniform random operands these kernels are held by the
     // card's power, not by its issue slots (the clock falls to about 1.6 GHz; the same launches on zeros run a fifth
     // faster), as is the library's bf16 product (1.13 PFLOP/s at 8192^3, which is 189 TFLOP/s at six products each).
     double eff[6];
     int (*launch)(const GemmArgs &, int, int, bool, hipStream_t);
-    // Fraction of that rate kept with k = 1..4 workgroups resident per CU, and the row count from which the tile is no longer considered (0: no limit).
+    // Fraction of that rate kept with k = 1..4 workgroups resident per CU, and the row count from which the tile is no
+    // longer considered (0: no limit).
     const double *occ;
     int below_rows;
-    // Scattered products of exactly one tile of rows, of which no more than this many are in use (0: any product).  The
-    // kernel is that of the 64-row tile of the same width.
-    int rows_used;
     // The tile has no loader for a first operand contiguous along its rows.
     bool a_rc_only;
 };
@@ -139,16 +137,14 @@ const double kOcc4[5] = {0.0, 0.52, 0.83, 0.94, 1.0};
 const double kOccSmall[5] = {0.0, 0.40, 0.76, 0.93, 1.0};
 
 const TileCfg kCfgs[] = {
-    {"128x128", 128, 128, 3, {0.44, 0.44, 0.44, 0.44, 0.45, 0.42}, gemm_fast_128x128, kOcc3, 0, 0, false},
-    {"192x128", 192, 128, 2, {0.43, 0.43, 0.43, 0.43, 0.44, 0.43}, gemm_fast_192x128, kOcc2, 0, 0, false},
-    {"64x256", 64, 256, 2, {0.38, 0.38, 0.38, 0.38, 0.40, 0.33}, gemm_fast_64x256, kOcc2, 0, 0, false},
-    {"128x256", 128, 256, 2, {0.46, 0.46, 0.46, 0.46, 0.47, 0.42}, gemm_fast_128x256, kOcc2, 0, 0, false},
-    {"256x128", 256, 128, 2, {0.46, 0.46, 0.46, 0.46, 0.48, 0.48}, gemm_fast_256x128, kOcc2, 0, 0, false},
-    {"64x64", 64, 64, 4, {0.32, 0.32, 0.32, 0.32, 0.33, 0.28}, gemm_fast_64x64, kOccSmall, 0, 0, false},
-    {"64x128", 64, 128, 4, {0.38, 0.38, 0.38, 0.38, 0.39, 0.37}, gemm_fast_64x128, kOcc4, 128, 0, false},
-    {"48x128", 64, 128, 4, {0, 0, 0, 0, 0.38, 0}, gemm_fast_64x128, kOcc4, 128, 48, false},
-    {"48x256", 64, 256, 2, {0, 0, 0, 0, 0.38, 0}, gemm_fast_64x256, kOcc2, 0, 48, false},
-    {"96x128", 96, 128, 3, {0.40, 0, 0.40, 0, 0.42, 0.40}, gemm_fast_96x128, kOcc3, 128, 0, true},
+    {"128x128", 128, 128, 3, {0.44, 0.44, 0.44, 0.44, 0.45, 0.42}, gemm_fast_128x128, kOcc3, 0, false},
+    {"192x128", 192, 128, 2, {0.43, 0.43, 0.43, 0.43, 0.44, 0.43}, gemm_fast_192x128, kOcc2, 0, false},
+    {"64x256", 64, 256, 2, {0.38, 0.38, 0.38, 0.38, 0.40, 0.33}, gemm_fast_64x256, kOcc2, 0, false},
+    {"128x256", 128, 256, 2, {0.46, 0.46, 0.46, 0.46, 0.47, 0.42}, gemm_fast_128x256, kOcc2, 0, false},
+    {"256x128", 256, 128, 2, {0.46, 0.46, 0.46, 0.46, 0.48, 0.48}, gemm_fast_256x128, kOcc2, 0, false},
+    {"64x64", 64, 64, 4, {0.32, 0.32, 0.32, 0.32, 0.33, 0.28}, gemm_fast_64x64, kOccSmall, 0, false},
+    {"64x128", 64, 128, 4, {0.38, 0.38, 0.38, 0.38, 0.39, 0.37}, gemm_fast_64x128, kOcc4, 128, false},
+    {"96x128", 96, 128, 3, {0.40, 0, 0.40, 0, 0.42, 0.40}, gemm_fast_96x128, kOcc3, 128, true},
 };
 
 inline long cdiv(long a, long b) { return (a + b - 1) / b; }
@@ -224,7 +220,6 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
         if (force && std::strcmp(force, c.name) != 0) continue;
         if (!force && c.below_rows > 0 && p.M >= c.below_rows) continue;
         if (c.a_rc_only && !p.a_rc) continue;
-        if (c.rows_used > 0 && !(p.scatter && layout == 4 && p.M == c.bm && p.scat_rows <= c.rows_used)) continue;
         const long tiles = cdiv(p.M, c.bm) * cdiv(p.J, c.bn);
         // (a product run wider than its result has one narrow tile per row block: it may split further to fill the GPU)
         const int split_cap = p.j_store > 0 ? 1024 : 256;

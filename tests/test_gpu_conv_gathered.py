@@ -483,13 +483,13 @@ SHORT_ROWS = [
 ]
 
 
-@pytest.mark.parametrize("tile", ["48x128", "48x256"])
+@pytest.mark.parametrize("tile", ["64x128", "64x256"])
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("cfg", SHORT_ROWS)
 def test_strided_gradinput_short_row_kernel_integer_exact(gt, gathered_route, switches, cfg, masked, tile):
-    """The scattered product whose rows fit 48 of its 64-row tile runs on the kernel that multiplies 48 rows in
-    16x16 blocks.  Small integers make every sum exact, so the result must equal the oracle's bit for bit, with and
-    without the fused nn.Threshold mask, and nothing outside gradInput may be written."""
+    """A scattered product of fewer than 64 rows runs on a 64-row tile and drops the rows behind its own.  Small integers
+    make every sum exact, so the result must equal the oracle's bit for bit, with and without the fused nn.Threshold
+    mask, and nothing outside gradInput may be written."""
     B, C, H, W, kH, kW, pH, pW, sH, sW = cfg
     M = 24
     geo = (kH, kW, pH, pW, sH, sW)
