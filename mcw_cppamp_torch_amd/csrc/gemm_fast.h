@@ -3,17 +3,32 @@
 //
 // Every operand element is split into three bf16 parts, x = h + m + l: h is x rounded to nearest, m the
 // remainder rounded, l what is left (8 + 8 + 8 significant bits hold the 24 of an fp32 number; without loss for zero
-// and from 2^-110 up, see below).  A product a*b is the sum
-// of the part products that matter in fp32, h*h + (h*m + m*h) + (h*l + m*m + l*h), each exact in the fp32 accumulator's
+// and from 2^-110 up, see below).  A product a*b is the sum of the part products that matter in fp32,
+// h*h + (h*m + m*h) + (h*l + m*m + l*h), each exact in the fp32 accumulator's
 // input; the three dropped ones are below 2^-24 of the product together, and of either sign.  That is six
 // v_mfma_f32_32x32x16_bf16 where eight v_mfma_f32_32x32x2_f32 of twice the cycles each stood: 2.7 times the matrix
-// rate (dense bf16 runs at 16 times the fp32 rate).  An accumulator also takes 6 rounded additions per 16 reduction
-// indices instead of 16.
+// rate (dense bf16 runs at 16 times the fp32 rate).
 //
-// Measured against the fp32-instruction kernel that stood here (uniform random operands): forward of 64 -> 128 planes, 9x9,
-// 128 images of 64x64: 4.2 -> 2.5 ms (128 -> 213 TFLOP/s); AlexNet-style step at batch 128: 4.51 -> 3.23 ms; error against
-// 64 bits over 3x3 to 11x11 layers and Linear products: 0.6 to 1.0 of the former (uniform operands).  What bounds it now is
-// power: see the efficiency figures in gemm_dispatch.hip.
+// How the sums are rounded.  The bf16 instruction adds its sixteen products to the accumulator in two groups of eight, each
+// rounded to nearest, after what lies far below the larger addend (2^-26 to 2^-32 of it, by which side is the
+// smaller) has been cut towards minus infinity.  Left to run along the whole reduction, as in the fp32 kernel, that is
+// twelve roundings of the full sum per sixteen indices (a sixth more error than before where half of an operand is zero,
+// as behind a ReLU) and a mean error that grows with the reduction: -2.3e-7 of a result's standard deviation at 4608
+// indices.  Sums over many results keep such a mean and pass it on: bias gradients of the AlexNet-style stack were 10
+// times as far from 64 bits as with the fp32 instructions.  So
+//   * the six products of one step (16 indices) are summed from zero, the small ones first, and the sum is added to the
+//     accumulator by 16 vector additions: one rounding of the full sum per step;
+//   * the sign of the product alternates: the first operand is negated in odd steps (its sum is then subtracted; free), the
+//     second in odd columns (one v_xor_b32 per element), whose accumulators hold the negated result.  What the instruction
+//     cuts pushes one step up and the next one down, one column up and its neighbour down.
+// Error against 64 bits now: root mean square 0.25 to 0.6 of the fp32 instructions' from 64 indices up (uniform operands,
+// half of one zero, positive: 0.26, 0.36 and 0.6 at 4608, 1024 and 576 indices), no mean error to be seen (below 2e-10);
+// gradients of the AlexNet-style stack 2e-7 (fp32 instructions 3e-7 to 5e-7).  The additions cost 10 %: AlexNet-style step
+// 3.17 -> 3.53 ms, VGG-A step 15.8 -> 17.3 ms, 64 -> 128 planes 9x9 9.1 -> 10.4 ms for the three passes.
+//
+// Against the fp32-instruction kernel that stood here (uniform random operands): AlexNet-style step at batch 128
+// 4.51 -> 3.53 ms, 9x9 layer 13.2 -> 10.4 ms.  What bounds it is power and, with the additions, the vector unit: see the
+// efficiency figures in gemm_dispatch.hip.
 //
 // What the split cannot hold is multiplied in fp32 instead, with v_mfma_f32_32x32x2_f32 (recompute):
 //   * An operand below 2^-110 in magnitude can have bits under the smallest bf16 step, 2^-133, and then comes out short by
@@ -49,10 +64,13 @@
 //     whole step to arrive.
 //   * Operands are fetched with buffer loads (descriptor and offsets in scalar registers, a constant lane offset), and
 //     the loop is unrolled by two so that the LDS buffer folds into the offset field of the LDS instructions: the only
-//     vector instructions of the loop are the split's (12 per two elements).
+//     vector instructions of the loop are the split's (12 or, for the second operand, 14 per two elements) and the additions.
+//   * The MFMAs go block by block.  The parts of the tile's shorter side stay in registers for the step; those of the longer
+//     one are read from LDS a block row ahead, or just before their use where registers are short.
 #pragma once
 
 #include <type_traits>
+#include <utility>
 
 #include "gemm_mfma.h"
 
@@ -92,6 +110,12 @@ __device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsi
     l = round2(s0, s1);
     // (written out: from the operators the compiler gathers the words of several pairs before it combines them, and spills)
     asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(s0), "v"(s1));
+}
+
+// f(0), f(1), ... with the index as a compile-time constant.
+template <typename F, int... I>
+__device__ __forceinline__ void for_each_index(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
 }
 
 // Wavefronts per SIMD the register allocation must leave room for: the accumulators take (BM/WGM)*(BN/WGN)/64 registers
@@ -363,7 +387,8 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     char *const a_dst = &As[0][0] + (a_r >> 3) * TileA::kOctet + a_x * 16 + (a_r & 7) * 2;
     char *const b_dst = &Bs[0][0] + (b_r >> 3) * TileB::kOctet + b_x * 16 + (b_r & 7) * 2;
     unsigned lost = 0;  // see split_pair
-    auto stash_group = [&](auto kind_tag, auto group_tag, auto tile_tag, char *dst, const float *src, int q) {
+    const unsigned odd_column = (unsigned)(b_x & 1) << 31;  // the sign of a thread's elements of the second operand
+    auto stash_group = [&](auto kind_tag, auto group_tag, auto tile_tag, char *dst, const float *src, int q, auto sign) {
         constexpr int KIND = decltype(kind_tag)::value;
         constexpr int G = decltype(group_tag)::value;
         using Tile = decltype(tile_tag);
@@ -371,7 +396,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         const int off = G == 8 ? q * Tile::kOctet : (KIND == LD_XC_BLOCK ? q * 64 : q * (NT / 4)) * 16;
         unsigned p[3][G / 2];
 #pragma unroll
-        for (int e = 0; e < G / 2; ++e) split_pair(src[q * G + 2 * e], src[q * G + 2 * e + 1], p[0][e], p[1][e], p[2][e], lost);
+        for (int e = 0; e < G / 2; ++e) split_pair(sign(src[q * G + 2 * e]), sign(src[q * G + 2 * e + 1]), p[0][e], p[1][e], p[2][e], lost);
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             if constexpr (G == 8)
@@ -385,11 +410,12 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     auto stash_a = [&](int buf, int q) {
         if (GA == 8 || a_unit_live(q))
             stash_group(std::integral_constant<int, KA>{}, std::integral_constant<int, GA>{}, TileA{},
-                        a_dst + buf * TileA::kBytes, ra, q);
+                        a_dst + buf * TileA::kBytes, ra, q, [&](float x) { return buf ? -x : x; });
     };
     auto stash_b = [&](int buf, int q) {
         stash_group(std::integral_constant<int, LB>{}, std::integral_constant<int, GB>{}, TileB{},
-                    b_dst + buf * TileB::kBytes, rb, q);
+                    b_dst + buf * TileB::kBytes, rb, q,
+                    [&](float x) { return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) ^ odd_column); });
     };
     constexpr int QA = NA / GA, QB = NB / GB;
     // The loads that refill group q.
@@ -445,10 +471,14 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     __syncthreads();
 
     // ---- main loop ----------------------------------------------------------------------
-    // Step s multiplies from LDS buffer s&1.  Its six part products are six slices of MFMAs; between them the groups of
+    // Step s multiplies from LDS buffer s&1, block by block; between the MFMAs the groups of
     // step s+1 are split and written to the other buffer and their registers refilled for step s+2.
     const char *const a_src = &As[0][0] + half * TileA::kOctet + (wm * (TM * 32) + l32) * 16;
     const char *const b_src = &Bs[0][0] + half * TileB::kOctet + (wn * (TN * 32) + l32) * 16;
+    // Two sums in turn, so that the additions of one block run under the MFMAs of the next, where the registers hold both
+    // (1 to 2 % on the 8-block tiles), and the parts of the longer side one block row ahead likewise.
+    constexpr bool PING = !(TM == 2 && TN == 2 && WGN == 2) && !(TM * TN == 8 && LB == LD_RC_GATHER);
+    constexpr int AHEAD = TM * TN == 8 || LB == LD_RC_GATHER ? 0 : 1;
     auto one_step = [&](auto buf_tag, int s) {
         constexpr int buf = decltype(buf_tag)::value;
         // The last step splits registers that nobody will read and the last two load from the previous addresses
@@ -466,71 +496,79 @@ __global__ __launch_bounds__(WGM *WGN * 64)
             if (pos >= g.R) pos = 0;
             fetch_rows(pos);
         }
-        bf16x8 av[TM][3], bv[TN][3];
-        auto fetch_parts = [&](int u) {  // in the order of their first use
-            const int ta = u == 0 ? 2 : u - 1, tb = u == 0 ? 0 : 3 - u;
-#pragma unroll
-            for (int a = 0; a < TM; ++a)
-                av[a][ta] = *reinterpret_cast<const bf16x8 *>(a_src + buf * TileA::kBytes + ta * TileA::kPart + a * 512);
-#pragma unroll
-            for (int b = 0; b < TN; ++b)
-                bv[b][tb] = *reinterpret_cast<const bf16x8 *>(b_src + buf * TileB::kBytes + tb * TileB::kPart + b * 512);
+        // Block by block; the parts of the tile's shorter side stay, those of the longer one are read a block row ahead.
+        constexpr bool A_STAYS = TM <= TN;
+        constexpr int STAY = A_STAYS ? TM : TN, PASS = A_STAYS ? TN : TM, BLOCKS = TM * TN;
+        bf16x8 stay[STAY][3], pass[1 + AHEAD][3];
+        auto read_a = [&](int a, int t) {
+            return *reinterpret_cast<const bf16x8 *>(a_src + buf * TileA::kBytes + t * TileA::kPart + a * 512);
         };
-        // (the widest tile's per-lane row offsets leave no registers for all of them: the last ones come a slice later)
-        constexpr bool LATE = LB == LD_RC_GATHER && TN == 4;
-        fetch_parts(0);
-        fetch_parts(1);
-        if (!LATE) fetch_parts(2);
-        constexpr int SLICES = 6;
-        auto slice_of = [&](auto slice_tag) {
-            constexpr int slice = decltype(slice_tag)::value;
-            // lh hl mm mh hm hh: the small ones first, while a short sum is still small, so that a reduction of one step
-            // is rounded once at its full magnitude
-            constexpr int pa = slice == 0 ? 2 : slice == 2 || slice == 3 ? 1 : 0;
-            constexpr int pb = slice == 1 ? 2 : slice == 2 || slice == 4 ? 1 : 0;
+        auto read_b = [&](int b, int t) {
+            return *reinterpret_cast<const bf16x8 *>(b_src + buf * TileB::kBytes + t * TileB::kPart + b * 512);
+        };
+        auto read_pass = [&](int k) {
 #pragma unroll
-            for (int a = 0; a < TM; ++a)
+            for (int t = 2; t >= 0; --t) pass[k & AHEAD][t] = A_STAYS ? read_b(k, t) : read_a(k, t);
+        };
 #pragma unroll
-                for (int b = 0; b < TN; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[a][pa], bv[b][pb], acc[a][b], 0, 0, 0);
+        for (int t = 2; t >= 0; --t)
+#pragma unroll
+            for (int k = 0; k < STAY; ++k) stay[k][t] = A_STAYS ? read_a(k, t) : read_b(k, t);
+        if (AHEAD) read_pass(0);
+        floatx16 sum[PING ? 2 : 1];
+        auto add_sum = [&](int block) {
+            const int k = block / STAY, m = block % STAY;
+            floatx16 &to = A_STAYS ? acc[m][k] : acc[k][m];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) to[v] = buf ? to[v] - sum[PING ? block & 1 : 0][v] : to[v] + sum[PING ? block & 1 : 0][v];
+            asm volatile("" : "+v"(to));  // here: left to itself the compiler moves the additions behind the step, sums and all
+        };
+        auto block_of = [&](auto block_tag) {
+            constexpr int block = decltype(block_tag)::value;
+            constexpr int k = block / STAY, m = block % STAY;
+            if (m == 0 && k + AHEAD < PASS) read_pass(k + AHEAD);
+            floatx16 part;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) part[v] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < 6; ++u) {
+                // lh hl mm mh hm hh: the small ones first, while the sum is still small
+                const int pa = u == 0 ? 2 : u == 2 || u == 3 ? 1 : 0;
+                const int pb = u == 1 ? 2 : u == 2 || u == 4 ? 1 : 0;
+                part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A_STAYS ? stay[m][pa] : pass[k & AHEAD][pa],
+                                                               A_STAYS ? pass[k & AHEAD][pb] : stay[m][pb], part, 0, 0, 0);
+            }
+            sum[PING ? block & 1 : 0] = part;
+            if (PING && block > 0) add_sum(block - 1);
 #pragma unroll
             for (int q = 0; q < QA; ++q)
-                if (q * SLICES / (QA + QB) == slice) {
+                if (q * BLOCKS / (QA + QB) == block) {
                     stash_a(buf ^ 1, q);
                     refill_a(ga, q);
                 }
 #pragma unroll
             for (int q = 0; q < QB; ++q)
-                if ((QA + q) * SLICES / (QA + QB) == slice) {
+                if ((QA + q) * BLOCKS / (QA + QB) == block) {
                     stash_b(buf ^ 1, q);
                     refill_b(gb, q);
                 }
-            if (LATE && slice == 0) fetch_parts(2);
-            if (slice == 3 && !RG) {
+            if (block == BLOCKS / 2 && !RG) {
                 int pos = ld_r0 + BK;
                 if (RED && pos >= g.R) pos = 0;
                 fetch_rows(pos);
             }
-            if (!RED && slice == 5) pin_rows();
-            // One MFMA, then a few of the split's vector instructions under it (a 32x32x16 MFMA holds the matrix unit for 32
-            // cycles, a vector instruction issues in 4): 2 to 5 % over leaving them in clusters, with the 128 x 256 tile
-            // most (a 64-plane 9x9 layer's forward: 213 -> 219 TFLOP/s).  Nothing gained with reduction batching.
-            if constexpr (!RED && slice < 5) {
+            if (!RED && block == BLOCKS - 1) pin_rows();
+            // One MFMA, then a few vector instructions under it (a 32x32x16 MFMA holds the matrix unit for 32 cycles, a vector
+            // instruction issues in 4): 2 % over leaving them in clusters; 4, 6 and 8 measure alike.
 #pragma unroll
-                for (int q = 0; q < TM * TN; ++q) {
-                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
-                }
+            for (int q = 0; q < 6; ++q) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, 6, 0);
             }
+            if (!PING || block == BLOCKS - 1) add_sum(block);
             __builtin_amdgcn_sched_barrier(0);
         };
-        using std::integral_constant;
-        slice_of(integral_constant<int, 0>{});
-        slice_of(integral_constant<int, 1>{});
-        slice_of(integral_constant<int, 2>{});
-        slice_of(integral_constant<int, 3>{});
-        slice_of(integral_constant<int, 4>{});
-        slice_of(integral_constant<int, 5>{});
+        for_each_index(block_of, std::make_integer_sequence<int, BLOCKS>{});
         if (more) advance();
         else shift = 0;
         __syncthreads();
@@ -551,6 +589,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     for (int w = 0; w < NT / 64; ++w) lost_any |= lost_of[w];
     // The wavefront's outputs in fp32, straight from the operands: eight reduction indices at a time, four to a lane half,
     // whose loads are in flight together.  (A step that would run past R is moved back as in the main loop.)
+    const float column_sign = l32 & 1 ? -1.0f : 1.0f;  // of the accumulators
     auto recompute = [&]() {
 #pragma unroll
         for (int a = 0; a < TM; ++a)
@@ -617,7 +656,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
 #pragma unroll
                     for (int a = 0; a < TM; ++a) x[a][t] = covered ? 0.0f : x[a][t];
 #pragma unroll
-                    for (int b = 0; b < TN; ++b) y[b][t] = covered ? 0.0f : y[b][t];
+                    for (int b = 0; b < TN; ++b) y[b][t] = covered ? 0.0f : y[b][t] * column_sign;
 #pragma unroll
                     for (int a = 0; a < TM; ++a)
 #pragma unroll
@@ -649,6 +688,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         char *const out0 = MODE == 0 ? reinterpret_cast<char *>(g.ws + (long)split * g.M * g.J)
                                      : reinterpret_cast<char *>(g.C);
         // Fused threshold / mask of the final value (uniform conditions; both off for partial sums).
+        const float alpha = MODE != 0 ? column_sign * g.alpha : column_sign;  // (and + 0 makes a zero positive)
         const bool act = MODE != 0 && g.act != 0;
         const bool masked = MODE != 0 && g.mask != nullptr;
         const long mask_row_bytes = g.mask_sC * 4;
@@ -723,8 +763,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                 for (int b = 0; b < TN; ++b) {
                     if (CHECK && !own[b]) continue;
                     float *c = reinterpret_cast<float *>(out + (long)ir * row_bytes + voff[b]);
-                    float val = acc[a][b][v];
-                    if (MODE != 0) val = val * g.alpha + (bias_v[v] + col_bias[b]);
+                    float val = acc[a][b][v] * alpha + (MODE != 0 ? bias_v[v] + col_bias[b] : 0.0f);
                     if constexpr (MODE == 2) val += g.beta * held[v % ROWS][b];
                     if (act) val = val > g.act_threshold ? val : g.act_value;
                     if (masked) {
@@ -772,7 +811,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                     const int h = hy[b] + (int)ph, w = wx[b] + (int)pw;
                     if (!own[b] || h < 0 || h >= g.scat_H || w < 0 || w >= g.scat_W) continue;
                     const long off = cbase[b] + roff;
-                    float val = acc[a][b][v] * g.alpha;
+                    float val = acc[a][b][v] * (column_sign * g.alpha) + 0.0f;
                     if (masked) val = g.mask[off] > g.mask_threshold ? val : 0.0f;
                     g.C[off] = val;
                 }
