@@ -235,13 +235,8 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
             const int sps = (int)cdiv(steps_total, ns);
             if ((int)cdiv(steps_total, sps) != ns) continue;  // would leave an empty split
             const double t = model_cycles(c, layout, p.M, p.J, steps_total, ns, cus);
-            // A product with tiles for less than half the chip is split anyway: there, of plans that the model puts
-            // within 2 % of each other, the one split further is the more exact (every addition to an accumulator is
-            // rounded; a 128 x 9216 product over 4096: relative error 3.7e-7 in seven parts, 2.7e-7 in fourteen, 63 us either
-            // way).  Larger products take the fastest: preferring more parts everywhere cost the AlexNet-style step 6 %.
-            const bool few = p.nb <= 1 && 2 * tiles <= cus;
-            if (!plan.cfg || t < best_t * (!few || ns == plan.nsplit ? 1.0 : ns > plan.nsplit ? 1.02 : 0.98)) {
-                if (!plan.cfg || t < best_t) best_t = t;
+            if (!plan.cfg || t < best_t) {
+                best_t = t;
                 plan.cfg = &c;
                 plan.nsplit = ns;
             }
@@ -417,8 +412,9 @@ int gemm_launch(const GemmProblem &p) {
         const long n = g.nsplit > 1 ? (long)p.M * p.J : 0;  // an unsplit product has stored its own result
         RowSumJob rs;
         std::memset(&rs, 0, sizeof(rs));
-        // few outputs, many splits: four wavefronts per 64 outputs (from 12 splits on: 256 x 169 outputs in 27 parts and two
-        // more like it, 3x3 layers of one 13x13 image: 53.1 -> 50.8 us a pass against 32 splits as the line)
+        // few outputs, many splits: four wavefronts per 64 outputs.  From 4 K to 123 K outputs the launch alone takes the same
+        // either way up to 16 splits, 0.2 us less at 24, 0.5 at 32 and 2.4 at 64; behind its product (256 x 169 outputs in 27
+        // parts and two more like it, 3x3 layers of one 13x13 image) 12 as the line gave 53.1 -> 50.8 us a pass against 32.
         const int quarters = (n > 0 && n < 128 * 1024 && g.nsplit >= 12) ? 1 : 0;
         unsigned blocks = (unsigned)cdiv(n, quarters ? 64 : 256);
         if (rowsum) {

@@ -1289,8 +1289,9 @@ int gradbias_launch(const float *gout, float *gbias, long B, int M, long N, floa
     long nslices = (4L * num_cus() + M - 1) / M;
     if (nslices > B) nslices = B;
     if (nslices > 65535) nslices = 65535;
-    // Planes of at most 16384 floats (64 a lane) in one launch, one workgroup each: behind it the second stage of a few
-    // sums cost as much as the first (37 planes of 4125: 2 x 5 us).
+    // Planes of at most 16384 floats (64 a lane) in one launch, one workgroup each: the second stage of a few sums costs as
+    // much as the first.  A whole accGradParameters of 2 to 60 planes, two launches against one: 18 - 20 -> 15 - 17 us at
+    // 2048 floats, 18 - 19 -> 16 - 18 at 8192, 18 - 22 -> 18 - 20 at 16384, 20 - 24 -> 22 - 25 at 32768.
     if (nslices < 1 || B * N <= 16384) nslices = 1;
     const int ips = (int)((B + nslices - 1) / nslices);
     nslices = (B + ips - 1) / ips;
