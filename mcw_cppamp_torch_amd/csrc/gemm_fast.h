@@ -23,11 +23,11 @@
 //     cuts pushes one step up and the next one down, one column up and its neighbour down.
 // Error against 64 bits now: root mean square 0.25 to 0.6 of the fp32 instructions' from 64 indices up (uniform operands,
 // half of one zero, positive: 0.26, 0.36 and 0.6 at 4608, 1024 and 576 indices), no mean error to be seen (below 2e-10);
-// gradients of the AlexNet-style stack 2e-7 (fp32 instructions 3e-7 to 5e-7).  The additions cost 10 %: AlexNet-style step
-// 3.17 -> 3.53 ms, VGG-A step 15.8 -> 17.3 ms, 64 -> 128 planes 9x9 9.1 -> 10.4 ms for the three passes.
+// gradients of the AlexNet-style stack 2e-7 (fp32 instructions 3e-7 to 5e-7).  The additions cost a tenth: AlexNet-style step
+// 3.2 -> 3.5 ms, VGG-A step 15.8 -> 17.0 ms, 64 -> 128 planes 9x9 9.1 -> 10.0 ms for the three passes.
 //
 // Against the fp32-instruction kernel that stood here (uniform random operands): AlexNet-style step at batch 128
-// 4.51 -> 3.53 ms, 9x9 layer 13.2 -> 10.4 ms.  What bounds it is power and, with the additions, the vector unit: see the
+// 4.51 -> 3.5 ms, 9x9 layer 13.2 -> 10.0 ms.  What bounds it is power and, with the additions, the vector unit: see the
 // efficiency figures in gemm_dispatch.hip.
 //
 // What the split cannot hold is multiplied in fp32 instead, with v_mfma_f32_32x32x2_f32 (recompute):
@@ -56,7 +56,7 @@
 //     consecutive units.  The octet planes are 64 bytes longer than their rows need: LDS writes go to 32 banks (128 bytes),
 //     and of sixteen lanes that write 64 bits each, four to a row, half then fall on each 64 bytes of them.  (With 128 bytes
 //     both halves fell on the same banks: 95 % conflict cycles with both operands along r, 50 - 65 % with one, none now.
-//     VGG-A step 15.8 -> 15.4 ms, 64 -> 128 planes 9x9 8.9 -> 8.5 ms for the three passes; within the 2 % by which
+//     VGG-A step 2.5 % faster, 64 -> 128 planes 9x9 1 to 4 %; within the 2 % by which
 //     cards differ on the AlexNet-style step.)
 //   * LDS is double buffered and the global loads run one step further ahead: while step s is multiplied, the
 //     registers hold step s+1, which is split and written to the other buffer in slices between the MFMAs, and every

@@ -519,8 +519,10 @@ class SpatialConvolutionMM(Module):
 
 
 class Linear(Module):
-    """nn.Linear(inputSize, outputSize): the statement-for-statement mirror of mcw_nn/Linear.lua:3-101 on GPU tensors
-    (addmv / addr / addmm of the tensor library; 1-D and 2-D inputs, the nunit == 1 special case included)."""
+    """nn.Linear(inputSize, outputSize) with the results of mcw_nn/Linear.lua:3-101: 1-D and 2-D inputs, the nunit == 1
+    special case included.  A batch whose operands are dense takes its output from one product that adds the bias where it
+    stores (thgpu_Linear_updateOutput) and its bias gradient from one sum over the rows (thgpu_Linear_accGradBias);
+    everything else is the Lua module statement for statement (addmv / addr / addmm of the tensor library)."""
 
     _assign = SpatialConvolutionMM._assign
 
