@@ -233,7 +233,7 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
             if (tiles * ns > 8L * cus * c.resident && ns > 1 && fsplit <= 0) break;
             if (ns > 1 && p.ws_fixed && (long)ns * p.M * p.J > p.ws_fixed_floats) break;  // partial sums must fit
             const int sps = (int)cdiv(steps_total, ns);
-            if ((int)cdiv(steps_total, sps) != ns) continue;  // would leave an empty split
+            if (sps > 0 && (int)cdiv(steps_total, sps) != ns) continue;  // would leave an empty split
             const double t = model_cycles(c, layout, p.M, p.J, steps_total, ns, cus);
             if (!plan.cfg || t < best_t) {
                 best_t = t;
