@@ -6,6 +6,9 @@
 #include "side_jobs.h"
 
 #include <cstring>
+#include <map>
+#include <mutex>
+#include <new>
 
 namespace thgpu {
 
@@ -189,7 +192,8 @@ struct GemmPlan {
     int nsplit = 1;
 };
 
-GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
+// `any`: the first tile and split that can run the problem, without ranking them.
+GemmPlan rank_plans(const GemmProblem &p, int steps_total, bool any) {
     GemmPlan plan;
     const bool gather = p.rowtab != nullptr;
     const int cus = num_cus();
@@ -234,6 +238,11 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
             if (ns > 1 && p.ws_fixed && (long)ns * p.M * p.J > p.ws_fixed_floats) break;  // partial sums must fit
             const int sps = (int)cdiv(steps_total, ns);
             if (sps > 0 && (int)cdiv(steps_total, sps) != ns) continue;  // would leave an empty split
+            if (any) {
+                plan.cfg = &c;
+                plan.nsplit = ns;
+                return plan;
+            }
             const double t = model_cycles(c, layout, p.M, p.J, steps_total, ns, cus);
             if (!plan.cfg || t < best_t) {
                 best_t = t;
@@ -241,6 +250,40 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
                 plan.nsplit = ns;
             }
         }
+    }
+    return plan;
+}
+
+// What the planner's answer depends on.
+struct PlanKey {
+    long v[20];
+    bool operator<(const PlanKey &o) const { return std::memcmp(v, o.v, sizeof(v)) < 0; }
+};
+
+// Ranking walks up to a thousand splits of eight tiles, 3 to 20 us, more than a launch takes to enqueue, and a program asks
+// for the same few products in every pass: the answers are kept by shape (host time of an AlexNet-style step, together with
+// gemm_tiled_fits, which no longer ranks: 285 -> 189 us; first-layer shape, three passes: 43 -> 30 us).  At 4096 shapes the map
+// starts over.
+GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
+    const Tuning &tune = tuning();
+    if (tune.gemm_tile[0] || tune.gemm_split > 0) return rank_plans(p, steps_total, false);
+    static std::mutex mutex;
+    static std::map<PlanKey, GemmPlan> plans;
+    const PlanKey key = {{p.M, p.J, p.R, p.N, steps_total, p.nb > 1 || p.rowsum,
+                          (p.a_rc ? 1 : 0) + (p.b_rc ? 2 : 0) + (p.rowtab ? 4 : 0) + (p.scatter ? 8 : 0) + (p.C2 ? 16 : 0), p.j_store,
+                          p.sA, p.sB, p.sC, p.bsB, p.bsC, p.b_extent, p.C2 ? p.c2_sC : 0, p.C2 ? p.c2_bsC : 0,
+                          p.C2 ? p.c2_pitch : 0, p.C2 ? p.c_w : 0, p.ws_fixed ? 1 : 0, p.ws_fixed ? p.ws_fixed_floats : 0}};
+    {
+        std::lock_guard<std::mutex> lock(mutex);
+        const auto it = plans.find(key);
+        if (it != plans.end()) return it->second;
+    }
+    const GemmPlan plan = rank_plans(p, steps_total, false);
+    try {
+        std::lock_guard<std::mutex> lock(mutex);
+        if (plans.size() >= 4096) plans.clear();
+        plans[key] = plan;
+    } catch (const std::bad_alloc &) {  // not kept, then
     }
     return plan;
 }
@@ -253,7 +296,7 @@ inline int steps_of(const GemmProblem &p) {
 
 bool gemm_tiled_fits(const GemmProblem &p) {
     if (p.M <= 0 || p.J <= 0 || (long)p.M * p.J >= (1L << 31)) return false;
-    return plan_gemm(p, steps_of(p)).cfg != nullptr;
+    return rank_plans(p, steps_of(p), true).cfg != nullptr;
 }
 
 int gemm_launch(const GemmProblem &p) {
