@@ -258,7 +258,7 @@ struct PhaseGeom {
     int A, Bk;     // taps per residue class: ceil(kH/sH), ceil(kW/sW)
     int Yn, Xn;    // cells per image: y = (h + pH) / sH over the image rows, likewise x
     int Hq, Wq;    // gradOutput padded by (A-1, Bk-1) in front and up to Yn + A - 1, Xn + Bk - 1 behind
-    int rows, rows_pad;
+    int rows;
 };
 
 PhaseGeom phase_geom(int C, int H, int W, int kH, int kW, int pH, int pW, int sH, int sW) {
@@ -270,7 +270,6 @@ PhaseGeom phase_geom(int C, int H, int W, int kH, int kW, int pH, int pW, int sH
     q.Hq = q.Yn + q.A - 1;
     q.Wq = q.Xn + q.Bk - 1;
     q.rows = C * sH * sW;
-    q.rows_pad = q.rows < 64 ? 64 : q.rows;
     return q;
 }
 
@@ -285,7 +284,7 @@ GemmProblem gradinput_strided_problem(long B, int C, int H, int W, int M, int kH
     p.bsB = (long)M * q.Hq * q.Wq;
     p.b_extent = B * p.bsB;
     p.bsC = (long)C * H * W;
-    p.M = q.rows_pad;
+    p.M = q.rows;
     p.J = (int)(B * q.Yn * q.Xn);
     p.N = q.Yn * q.Xn;
     p.R = M * q.A * q.Bk;
@@ -319,10 +318,9 @@ WeightJob bank_job(const float *weight, float *wt, int C, int H, int W, int M, i
         wj.A = q.A;
         wj.Bk = q.Bk;
         wj.rows = q.rows;
-        wj.rows_pad = q.rows_pad;
-        wj.count = (unsigned)((long)q.rows_pad * M * q.A * q.Bk);
+        wj.count = (unsigned)((long)q.rows * M * q.A * q.Bk);
     } else {
-        wj.sH = wj.sW = wj.A = wj.Bk = wj.rows = wj.rows_pad = 0;
+        wj.sH = wj.sW = wj.A = wj.Bk = wj.rows = 0;
         wj.count = (unsigned)((long)M * C * kH * kW);
     }
     return wj;
@@ -364,7 +362,7 @@ void conv_implicit_offer_bank(const float *weight, float *scratch, long B, int C
     long nw = (long)M * C * kH * kW;
     if (sH != 1 || sW != 1) {
         const PhaseGeom q = phase_geom(C, H, W, kH, kW, pH, pW, sH, sW);
-        nw = (long)q.rows_pad * M * q.A * q.Bk;
+        nw = (long)q.rows * M * q.A * q.Bk;
     }
     if (nw >= (1L << 31)) return;  // the product itself will refuse
     offer_bank_job(bank_job(weight, scratch + B * M * (long)Hq * Wq, C, H, W, M, kH, kW, pH, pW, sH, sW));
@@ -381,7 +379,7 @@ int conv_mode() {
 void conv_set_mode(int mode) { g_mode = mode; }
 
 // Shapes the gathered GEMMs take: the padded batch must stay within 32-bit byte offsets and a tile of the fast
-// kernel must take both products that share finput (the GEMM's own planner answers that: M, J >= 64, R >= 16,
+// kernel must take both products that share finput (the GEMM's own planner answers that: R >= 16,
 // offsets of operands and output below 2^30 floats, a tile the tuning switches allow).
 // Forward and gradWeight share finput (the padded input), so a layer takes both or neither.  K >= 16 is the GEMM's
 // shortest reduction (forward); a gradWeight product with fewer than 64 taps runs 64 columns wide (gradweight_problem).
@@ -389,69 +387,93 @@ static bool forward_fits(long B, int C, int H, int W, int M, int kH, int kW, int
     const long Hp = H + 2L * pH, Wp = W + 2L * pW;
     const long Ho = (Hp - kH) / sH + 1, Wo = (Wp - kW) / sW + 1;
     const long K = (long)C * kH * kW, N = Ho * Wo;
-    if (!(M >= 64 && K >= 16 && N >= 16 && B * N >= 64 && B * N < (1L << 31) && B * C * Hp * Wp < kMaxExtent)) return false;
+    if (!(M >= 1 && K >= 16 && N >= 16 && B * N < (1L << 31) && B * C * Hp * Wp < kMaxExtent)) return false;
     return gemm_tiled_fits(forward_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW)) &&
            gemm_tiled_fits(gradweight_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW));
 }
 
 static bool gradinput_fits(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
     if (sH != 1 || sW != 1) {
-        // by residue class of the pixel coordinates: any padding, rows padded to a whole tile
+        // by residue class of the pixel coordinates: any padding
         const PhaseGeom q = phase_geom(C, H, W, kH, kW, pH, pW, sH, sW);
         const long cols = B * (long)q.Yn * q.Xn;
         if (!(cols >= 64 && cols < (1L << 31) && (long)M * q.A * q.Bk >= 16 && B * M * (long)q.Hq * q.Wq < kMaxExtent &&
-              (long)q.rows_pad * cols < (1L << 31)))
+              (long)q.rows * cols < (1L << 31)))
             return false;
         return gemm_tiled_fits(gradinput_strided_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW));
     }
     if (kH - 1 - pH < 0 || kW - 1 - pW < 0) return false;
     const long Hq = H + kH - 1, Wq = W + kW - 1;
-    if (!(C >= 64 && B * H * W >= 64 && (long)M * kH * kW >= 16 && B * M * Hq * Wq < kMaxExtent &&
+    if (!(C >= 1 && (long)M * kH * kW >= 16 && B * M * Hq * Wq < kMaxExtent &&
           B * (long)H * W < (1L << 31)))
         return false;
     return gemm_tiled_fits(gradinput_problem(B, C, H, W, M, kH, kW, pH, pW));
 }
 
-// Where the gathered route pays (measured on the AlexNet-, OverFeat- and VGG-style layers and the reference's
-// benchmark set).  Forward and gradWeight: wherever a tiled kernel takes the product -- the gathered products run at
-// the rate of those on columns (0.84 - 0.92 of the matrix peak on the 512- and 1024-plane layers, either way), and
-// the columns' trip through memory is saved.  gradInput: the gathered product has one row per input plane, so it
-// wants C to fill its 64-row tiles, and one column per input pixel, so it wants the layer padded (see below).
+// Forward and gradWeight gather wherever a tiled kernel takes the product: the gathered products run at the rate of those on
+// columns, and the columns' trip through memory is saved.
 bool conv_use_gathered(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
     const int mode = conv_mode();
     if (mode == 0 || !forward_fits(B, C, H, W, M, kH, kW, pH, pW, sH, sW)) return false;
-    return true;
+    // Fewer planes than a 64-row tile: the columns and the bias gradient's pass over gradOutput go all the same (450 -> 18 planes
+    // 11x11, 19 images: 1656 -> 900 us a pass).  Padded layers of fewer than 256 positions take as long either way (0.91 to
+    // 1.07 on ten layers of 64 and 128 positions; 1.5 without padding, where there is no copy to make).  Mode 2 keeps the
+    // columns of all of them, for callers that read them from finput.
+    const long Ho = (H + 2L * pH - kH) / sH + 1, Wo = (W + 2L * pW - kW) / sW + 1;
+    return M >= 64 || (mode == 1 && (B * Ho * Wo >= 256 || (pH == 0 && pW == 0)));
+}
+
+// What gradInput takes on either route, in microseconds: the planner's estimate of its product and the traffic around it, at
+// 4.5 TB/s and for the re-ordering of the kernel bank at 3.  The gathered product has one row per input plane (and residue
+// class) in tiles of 32 or 64 and one column per input pixel; the product on columns is often bound by writing them, of which
+// the estimate sees a part.  Over 329 layers (1 to 128 images, 3 to 1024 input planes, kernels of 3 to 11, strides of 1, 2 and 4),
+// both sides measured, the choice costs 0.6 % over the better one each time, at most 21 %; the rules before it (64-row
+// tiles, an excess of work below two) cost 10 times the time where a strided layer has few pixels and a long reduction,
+// which its unsplit product walks in a handful of workgroups (384 planes 7x7, 28x28 images: 21 us on columns, 192).
+static double gathered_gradinput_us(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
+    const long N = ((H + 2L * pH - kH) / sH + 1) * ((W + 2L * pW - kW) / sW + 1);
+    int top, left, Hq, Wq;
+    conv_implicit_q_layout(C, H, W, kH, kW, pH, pW, sH, sW, &top, &left, &Hq, &Wq);
+    const GemmProblem p = sH != 1 || sW != 1 ? gradinput_strided_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW)
+                                             : gradinput_problem(B, C, H, W, M, kH, kW, pH, pW);
+    return gemm_estimate_us(p) + 4.0 * B * M * (N + (double)Hq * Wq) / 4.5e6 + 4.0 * 2 * p.M * (double)p.R / 3e6;
+}
+
+static double column_gradinput_us(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
+    const long N = ((H + 2L * pH - kH) / sH + 1) * ((W + 2L * pW - kW) / sW + 1), K = (long)C * kH * kW;
+    GemmProblem p;
+    p.a_rc = false;
+    p.sA = K;
+    p.sB = N;
+    p.bsB = (long)M * N;
+    p.sC = N;
+    p.bsC = K * N;
+    p.M = (int)K;
+    p.J = (int)(B * N);
+    p.N = (int)N;
+    p.R = M;
+    return gemm_estimate_us(p) + 4.0 * B * (1.7 * K * N + (double)C * H * W) / 4.5e6;
 }
 
 bool conv_use_gathered_gradinput(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
     const int mode = conv_mode();
     if (mode == 0 || !gradinput_fits(B, C, H, W, M, kH, kW, pH, pW, sH, sW)) return false;
-    if (mode == 2) return true;
-    if (sH != 1 || sW != 1) {
-        // The product by residue class executes rows_pad*A*Bk*sH*sW / (C*kH*kW) times the layer's flops (rows
-        // padded to a tile, taps rounded up to whole strides) but saves the gradient columns, kH*kW/(sH*sW) times
-        // the input written and read back: it pays while that excess stays small.
-        const PhaseGeom q = phase_geom(C, H, W, kH, kW, pH, pW, sH, sW);
-        const double excess = (double)q.rows_pad * q.A * q.Bk / ((double)C * kH * kW);
-        return excess <= 2.0;
-    }
-    const long rows = (C + 63L) / 64 * 64;
-    // An unpadded (or lightly padded) layer has fewer output positions than input pixels, and the gathered
-    // product computes one column per input pixel: it executes H*W / (Ho*Wo) times the layer's flops, where the
-    // column route pays the algorithmic flops plus the gradient columns' trip through memory (8*K*N bytes per
-    // image).  At the measured rates (120 TFLOP/s, 4.5 TB/s) the columns win once (H*W/(Ho*Wo) - 1) * M exceeds
-    // about 100; measured on the reference benchmark's unpadded layers, the switch-over lies between 100 (gathered
-    // still 9 % ahead) and 150 (columns 19 % ahead).
+    const bool strided = sH != 1 || sW != 1;
+    if (mode == 2) return strided || C >= 64;
+    // Unit stride, planes that fill 64-row tiles, little work on pixels that no position covers: the one sum of the gathered
+    // product is also rounded less than the taps' sums that col2im adds up (2 x 64 planes 9x9: 1.39e-7 from 64 bits, columns
+    // 1.59e-7), so it stays for single images too, where the columns are up to 30 % faster.
     const long Ho = H + 2L * pH - kH + 1, Wo = W + 2L * pW - kW + 1;
-    const bool inflation_ok = ((long)H * W - Ho * Wo) * M <= 110 * Ho * Wo;
-    return rows * 8 <= C * 9L && inflation_ok;
+    if (!strided && (C + 63L) / 64 * 64 * 8 <= C * 9L && ((long)H * W - Ho * Wo) * M <= 110 * Ho * Wo) return true;
+    return gathered_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW) <=
+           column_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
 }
 
 long conv_implicit_gradinput_scratch(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH,
                                      int sW) {
     if (sH != 1 || sW != 1) {
         const PhaseGeom q = phase_geom(C, H, W, kH, kW, pH, pW, sH, sW);
-        return B * M * (long)q.Hq * q.Wq + (long)q.rows_pad * M * q.A * q.Bk;
+        return B * M * (long)q.Hq * q.Wq + (long)q.rows * M * q.A * q.Bk;
     }
     return B * M * (H + kH - 1L) * (W + kW - 1L) + (long)C * M * kH * kW;
 }
@@ -585,7 +607,7 @@ static int conv_implicit_gradinput_strided(const float *gradOutput, const float 
     const int Ho = (H + 2 * pH - kH) / sH + 1, Wo = (W + 2 * pW - kW) / sW + 1;
     float *Q = scratch;
     float *Wt = scratch + B * M * (long)q.Hq * q.Wq;
-    const long nw = (long)q.rows_pad * M * q.A * q.Bk;
+    const long nw = (long)q.rows * M * q.A * q.Bk;
     if (nw >= (1L << 31)) return fail("SpatialConvolutionMM: kernel bank too large for the strided gradInput product");
     const WeightJob wj = bank_job(weight, Wt, C, H, W, M, kH, kW, pH, pW, sH, sW);
     // With gradOutput already in place only the kernel bank is re-ordered (zero planes to pad), unless a launch before

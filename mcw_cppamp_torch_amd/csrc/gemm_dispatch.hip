@@ -148,6 +148,7 @@ const TileCfg kCfgs[] = {
     {"64x64", 64, 64, 4, {0.29, 0.29, 0.29, 0.29, 0.30, 0.25}, gemm_fast_64x64, kOccSmall, 0, false},
     {"64x128", 64, 128, 4, {0.33, 0.33, 0.33, 0.33, 0.34, 0.33}, gemm_fast_64x128, kOcc4, 128, false},
     {"96x128", 96, 128, 3, {0.35, 0, 0.35, 0, 0.37, 0.35}, gemm_fast_96x128, kOcc3, 128, true},
+    {"32x128", 32, 128, 4, {0.22, 0, 0.22, 0, 0.22, 0.25}, gemm_fast_32x128, kOcc4, 33, true},
 };
 
 inline long cdiv(long a, long b) { return (a + b - 1) / b; }
@@ -160,7 +161,7 @@ constexpr double kFlopsPerCycle = 4096.0 / 6.0;
 // hides less of their latencies (kOcc); workgroups beyond what fits at once
 // run in further rounds; every round pays a prologue/epilogue; a split adds
 // the traffic of writing and re-reading the partial sums.
-double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_total, int nsplit, int cus) {
+double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_total, int nsplit, int cus, bool accumulate) {
     const double *kOcc = c.occ;
     const long tiles = cdiv(M, c.bm) * cdiv(J, c.bn);
     const long wgs = tiles * nsplit;
@@ -169,12 +170,17 @@ double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_tot
     const double ovh = 3000.0 + 6.0 * c.bm * c.bn / 64.0;
     const long slots = (long)cus * c.resident;
     const long full = wgs / slots, rest = wgs - full * slots;
-    const double round = c.resident * steps * per_step / kOcc[c.resident] + ovh;
+    // A CU stores an output in half a cycle (4.8 TB/s over the chip); where a reduction is too short to hide that, a round
+    // takes what its tiles' stores take and, at its start, one tile's more (20 indices, 225 x 161772: 64 us with two 128 x 256
+    // tiles to a CU, 42 us with four of 64 x 128; an accumulating store also reads).
+    const double stores = 0.55 * c.bm * c.bn * (accumulate ? 2.0 : 1.0);
+    auto at_least = [](double a, double b) { return a > b ? a : b; };
+    const double round = at_least(c.resident * steps * per_step / kOcc[c.resident] + ovh, (c.resident + 1) * stores);
     double t = full * round;
     if (rest > 0) {
         const long on_busiest = cdiv(rest, cus);
         const int k = (int)(on_busiest < c.resident ? on_busiest : c.resident);
-        double last = on_busiest * steps * per_step / kOcc[k] + ovh * (k > 1 ? 1.0 : 1.5);
+        double last = at_least(on_busiest * steps * per_step / kOcc[k] + ovh * (k > 1 ? 1.0 : 1.5), (on_busiest + 1) * stores);
         // Behind full rounds a thin last one costs half of what it would alone: workgroups do not end in step, and the
         // last ones run at the clock that an idle chip allows (512 x 50176 over 2304, 128 x 128 tiles: 2.04 rounds,
         // 816 us with the last counted in full, measured 620; in three parts, 2.3 rounds of larger tiles, 561 us and
@@ -190,6 +196,7 @@ double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_tot
 struct GemmPlan {
     const TileCfg *cfg = nullptr;
     int nsplit = 1;
+    double cycles = 0;  // the model's estimate
 };
 
 // `any`: the first tile and split that can run the problem, without ranking them.
@@ -220,7 +227,8 @@ GemmPlan rank_plans(const GemmProblem &p, int steps_total, bool any) {
     const bool fast_ok = p.R == 0 || p.R >= GEMM_BK;
     const int layout = gather ? (p.nb > 1 || p.rowsum ? 5 : 4) : p.a_rc ? (p.b_rc ? 2 : 0) : (p.b_rc ? 3 : 1);
     for (const TileCfg &c : kCfgs) {
-        if (!fast_ok || p.M < c.bm || p.J < c.bn || !offsets_fit(c.bm, c.bn)) continue;
+        if (!fast_ok || !offsets_fit(c.bm, c.bn)) continue;
+        if ((p.M < c.bm && c.bm > GEMM_SHORT_TILE) || (p.J < c.bn && c.bn > GEMM_SHORT_TILE)) continue;
         if (force && std::strcmp(force, c.name) != 0) continue;
         if (!force && c.below_rows > 0 && p.M >= c.below_rows) continue;
         if (c.a_rc_only && !p.a_rc) continue;
@@ -243,11 +251,12 @@ GemmPlan rank_plans(const GemmProblem &p, int steps_total, bool any) {
                 plan.nsplit = ns;
                 return plan;
             }
-            const double t = model_cycles(c, layout, p.M, p.J, steps_total, ns, cus);
+            const double t = model_cycles(c, layout, p.M, p.J, steps_total, ns, cus, p.beta != 0.0f);
             if (!plan.cfg || t < best_t) {
                 best_t = t;
                 plan.cfg = &c;
                 plan.nsplit = ns;
+                plan.cycles = t;
             }
         }
     }
@@ -256,7 +265,7 @@ GemmPlan rank_plans(const GemmProblem &p, int steps_total, bool any) {
 
 // What the planner's answer depends on.
 struct PlanKey {
-    long v[20];
+    long v[21];
     bool operator<(const PlanKey &o) const { return std::memcmp(v, o.v, sizeof(v)) < 0; }
 };
 
@@ -272,7 +281,7 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
     const PlanKey key = {{p.M, p.J, p.R, p.N, steps_total, p.nb > 1 || p.rowsum,
                           (p.a_rc ? 1 : 0) + (p.b_rc ? 2 : 0) + (p.rowtab ? 4 : 0) + (p.scatter ? 8 : 0) + (p.C2 ? 16 : 0), p.j_store,
                           p.sA, p.sB, p.sC, p.bsB, p.bsC, p.b_extent, p.C2 ? p.c2_sC : 0, p.C2 ? p.c2_bsC : 0,
-                          p.C2 ? p.c2_pitch : 0, p.C2 ? p.c_w : 0, p.ws_fixed ? 1 : 0, p.ws_fixed ? p.ws_fixed_floats : 0}};
+                          p.C2 ? p.c2_pitch : 0, p.C2 ? p.c_w : 0, p.ws_fixed ? 1 : 0, p.ws_fixed ? p.ws_fixed_floats : 0, p.beta != 0.0f}};
     {
         std::lock_guard<std::mutex> lock(mutex);
         const auto it = plans.find(key);
@@ -297,6 +306,15 @@ inline int steps_of(const GemmProblem &p) {
 bool gemm_tiled_fits(const GemmProblem &p) {
     if (p.M <= 0 || p.J <= 0 || (long)p.M * p.J >= (1L << 31)) return false;
     return rank_plans(p, steps_of(p), true).cfg != nullptr;
+}
+
+double gemm_estimate_us(const GemmProblem &p) {
+    const GemmPlan plan = plan_gemm(p, steps_of(p));
+    if (plan.cfg) return plan.cycles / 2400.0;
+    // the generic kernel: 25 TFLOP/s over whole 64 x 64 tiles, or its stores
+    const double compute = 2.0 * 64 * 64 * cdiv(p.M, 64) * cdiv(p.J, 64) * (double)p.R / 25e6;
+    const double store = 4.0 * p.M * (double)p.J / 4.5e6;
+    return 4.0 + (compute > store ? compute : store);
 }
 
 int gemm_launch(const GemmProblem &p) {
@@ -412,7 +430,8 @@ int gemm_launch(const GemmProblem &p) {
     g.total = (unsigned)total;
     // Row sums of A ride along with a tiled reduction-batched product (never with the fixed workspace of the
     // entry point that may not allocate: nothing there asks for them).
-    const bool rowsum = p.rowsum && best && red && !p.ws_fixed;
+    // (An unsplit product of few rows leaves them to their own launch, which reads as little and needs no scratch.)
+    const bool rowsum = p.rowsum && best && red && !p.ws_fixed && (g.nsplit > 1 || p.M >= 64);
     if (p.rowsum_done) *p.rowsum_done = rowsum;
     const size_t rowsum_floats = rowsum ? (size_t)g.nsplit * g.tilesJ * p.M : 0;
     if (g.nsplit > 1 || rowsum) {
@@ -435,7 +454,7 @@ int gemm_launch(const GemmProblem &p) {
                    : !red ? LD_XC_GATHER
                    : p.row_quads ? LD_RC_GATHER_VEC
                                  : LD_RC_GATHER;
-    if (gather && !best) return fail("gemm: a gathered B needs a shape the tiled kernel takes (M, J >= 64, R >= 16)");
+    if (gather && !best) return fail("gemm: a gathered B needs a shape the tiled kernel takes (R >= 16)");
     if (p.C2 && !best) return fail("gemm: a second copy of the result needs a shape the tiled kernel takes");
     if (p.j_store > 0 && (!best || g.nsplit < 2))
         return fail("gemm: scratch columns need a tiled kernel and a split reduction");

@@ -48,8 +48,9 @@
 //     edge is shifted back so that it lies inside the matrix and stores only the
 //     rows/columns no other tile owns; a reduction step that would run past R is
 //     shifted back to end at R and the part the previous step already covered
-//     is zeroed on its way to LDS.  Needs M >= BM, J >= BN, R >= 16; smaller
-//     problems take the bounds-checked generic kernel.
+//     is zeroed on its way to LDS.  Needs R >= 16 and, on sides longer than GEMM_SHORT_TILE, M >= BM and J >= BN.  A matrix
+//     with fewer rows (columns) than a short side of the tile loads its last one in place of the missing ones and stores
+//     only its own.
 //   * The split is made once per element and workgroup, on the way from registers to LDS.  LDS holds the parts of both
 //     operand tiles as [part][octet][x] units of eight bf16 (x the free index, octet = r/8): lane (x, h) of a wavefront
 //     fetches its MFMA operand, r = 8h .. 8h+7 of row x, with one 128-bit read, consecutive lanes from
@@ -154,6 +155,9 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     constexpr bool GATHER = LB == LD_XC_GATHER || RG;
     static_assert(!RG || (RED && NT == 256), "lanes along the reduction: reduction batching only");
     static_assert(!RED || (LA == LD_RC_VEC && (LB == LD_RC_VEC || RG)), "reduction batching needs operands loaded along r");
+    constexpr bool SHORT_M = BM <= GEMM_SHORT_TILE, SHORT_J = BN <= GEMM_SHORT_TILE;
+    static_assert(!SHORT_M || NT / 4 >= BM, "one round of loads along r covers the rows of a short tile");
+    static_assert(!SHORT_J || NT / 4 >= BN, "and its columns");
 
     using TileA = PartTile<BM>;
     using TileB = PartTile<BN>;
@@ -171,8 +175,13 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     g.divTilesM.divmod(pid, rest, ti);
     g.divTilesJ.divmod(rest, split, tj);
     const int own_i0 = (int)ti * BM, own_j0 = (int)tj * BN;
-    const int i0 = own_i0 + BM <= g.M ? own_i0 : g.M - BM;  // shifted back at the edge
-    const int j0 = own_j0 + BN <= g.J ? own_j0 : g.J - BN;
+    int i0 = own_i0 + BM <= g.M ? own_i0 : g.M - BM;  // shifted back at the edge
+    int j0 = own_j0 + BN <= g.J ? own_j0 : g.J - BN;
+    // A matrix with fewer rows or columns than the tile: its last row or column is loaded in place of the missing ones.
+    if (SHORT_M && g.M < BM) i0 = 0;
+    if (SHORT_J && g.J < BN) j0 = 0;
+    auto row_at = [&](int i) { return SHORT_M && i >= g.M ? g.M - 1 : i; };
+    auto col_at = [&](int j) { return SHORT_J && j >= g.J ? g.J - 1 : j; };
 
     int step = (int)split * g.steps_per_split;
     int step_end = step + g.steps_per_split;
@@ -205,12 +214,12 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     } else if (LA == LD_XC_SCALAR) {
         a_x = tid % BM;
         a_r = (tid / BM) * NA;
-        voffA = (unsigned)(((long)a_r * g.sA + a_x) * 4);
+        voffA = (unsigned)(((long)a_r * g.sA + (row_at(i0 + a_x) - i0)) * 4);
         tileA = reinterpret_cast<const char *>(g.A + i0);
     } else {
         a_x = tid >> 2;
         a_r = (tid & 3) * 4;
-        voffA = (unsigned)(((long)a_x * g.sA + a_r) * 4);
+        voffA = (unsigned)(((long)(row_at(i0 + a_x) - i0) * g.sA + a_r) * 4);
         tileA = reinterpret_cast<const char *>(g.A + (long)i0 * g.sA);
     }
     // Lanes along r: the column offsets in bytes of the thread's column of every 64.
@@ -220,14 +229,14 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         b_r = (tid & 3) * 4;
         voffB = 0;
 #pragma unroll
-        for (int q = 0; q < (RG ? NB / 4 : 1); ++q) coffB[q] = (unsigned)g.coltab[j0 + b_x + q * (NT / 4)] * 4u;
+        for (int q = 0; q < (RG ? NB / 4 : 1); ++q) coffB[q] = (unsigned)g.coltab[col_at(j0 + b_x + q * (NT / 4))] * 4u;
         tileB = reinterpret_cast<const char *>(g.B);
     } else if (LB == LD_XC_GATHER) {
         b_x = tid % BN;
         b_r = (wave * 64 / BN) * NB;  // = (tid / BN) * NB, kept uniform: the row offsets are scalar loads
         unsigned img0, n0, img, n;
         g.divN.divmod((unsigned)j0, img0, n0);
-        g.divN.divmod((unsigned)(j0 + b_x), img, n);
+        g.divN.divmod((unsigned)col_at(j0 + b_x), img, n);
         voffB = (unsigned)(((long)(img - img0) * g.bsB + g.coltab[n]) * 4);
         tileB = reinterpret_cast<const char *>(g.B + (long)img0 * g.bsB);
     } else if (LB == LD_XC_SCALAR) {
@@ -235,13 +244,13 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         b_r = (tid / BN) * NB;
         unsigned img0, n0, img, n;
         g.divN.divmod((unsigned)j0, img0, n0);
-        g.divN.divmod((unsigned)(j0 + b_x), img, n);
+        g.divN.divmod((unsigned)col_at(j0 + b_x), img, n);
         voffB = (unsigned)(((long)b_r * g.sB + (long)(img - img0) * g.bsB + n) * 4);
         tileB = reinterpret_cast<const char *>(g.B + (long)img0 * g.bsB);
     } else {
         b_x = tid >> 2;
         b_r = (tid & 3) * 4;
-        voffB = (unsigned)(((long)b_x * g.sB + b_r) * 4);
+        voffB = (unsigned)(((long)(col_at(j0 + b_x) - j0) * g.sB + b_r) * 4);
         tileB = reinterpret_cast<const char *>(g.B + (long)j0 * g.sB);
     }
     constexpr int UA = LA == LD_RC_VEC ? NA / 4 : NA;  // load instructions per step and operand
@@ -603,12 +612,12 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         const float *arow[TM], *bcol[TN];
 #pragma unroll
         for (int a = 0; a < TM; ++a) {
-            const long i = i0 + wm * (TM * 32) + a * 32 + l32;
+            const long i = row_at(i0 + wm * (TM * 32) + a * 32 + l32);
             arow[a] = g.A + (LA == LD_XC_SCALAR ? i : i * g.sA);
         }
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
-            const unsigned j = (unsigned)(j0 + wn * (TN * 32) + b * 32 + l32);
+            const unsigned j = (unsigned)col_at(j0 + wn * (TN * 32) + b * 32 + l32);
             unsigned im = 0, n = j;
             if (!RED && LB != LD_RC_VEC) g.divN.divmod(j, im, n);
             bcol[b] = g.B + (GATHER               ? (long)im * g.bsB + g.coltab[n]
@@ -680,7 +689,8 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     // A store address is a wave-uniform row base plus a constant per-lane byte
     // offset (column, image and the lane half's four rows), as for the loads.
     // MODE 0: partial sums to the workspace; 1: alpha*acc (+bias); 2: also + beta*C.
-    const bool edge_tile = i0 != own_i0 || j0 != own_j0;  // an edge tile: some rows or columns belong to its neighbour
+    // An edge tile: some rows or columns belong to its neighbour, or lie outside the matrix.
+    const bool edge_tile = i0 != own_i0 || j0 != own_j0 || (SHORT_M && g.M < BM) || (SHORT_J && g.J < BN);
     auto write_out = [&](auto mode_tag, auto check_tag) {
         constexpr int MODE = decltype(mode_tag)::value;
         constexpr bool CHECK = decltype(check_tag)::value;
@@ -708,8 +718,9 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         float col_bias[TN];
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
-            const int jg = j0 + wn * (TN * 32) + b * 32 + l32;
-            own[b] = jg >= own_j0;  // else the neighbouring tile stores it
+            const int jt = j0 + wn * (TN * 32) + b * 32 + l32;
+            own[b] = jt >= own_j0 && (!SHORT_J || jt < g.J);  // else the neighbouring tile stores it, or there is no such column
+            const int jg = CHECK ? col_at(jt) : jt;
             col_bias[b] = MODE != 0 && g.bias_col ? g.bias_col[jg] : 0.0f;
             long col = jg - j0, mcol = jg - j0, tcol = 0;
             if (per_image) {
@@ -734,8 +745,10 @@ __global__ __launch_bounds__(WGM *WGN * 64)
             if (MODE != 0 && g.bias) {
 #pragma unroll
                 for (int v = 0; v < 16; ++v)
-                    bias_v[v] = *reinterpret_cast<const float *>(
-                        reinterpret_cast<const char *>(g.bias + iu + 8 * (v / 4) + (v % 4)) + 16 * half);
+                    bias_v[v] = CHECK && SHORT_M
+                                    ? g.bias[row_at(iu + 8 * (v / 4) + (v % 4) + 4 * half)]
+                                    : *reinterpret_cast<const float *>(
+                                          reinterpret_cast<const char *>(g.bias + iu + 8 * (v / 4) + (v % 4)) + 16 * half);
             } else {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) bias_v[v] = 0.0f;
@@ -754,11 +767,13 @@ __global__ __launch_bounds__(WGM *WGN * 64)
 #pragma unroll
                         for (int b = 0; b < TN; ++b)
                             held[MODE == 2 ? q : 0][MODE == 2 ? b : 0] =
-                                *reinterpret_cast<const float *>(out + (long)ir * row_bytes + voff[b]);
+                                !(CHECK && SHORT_M) || ir + 4 * half < g.M
+                                    ? *reinterpret_cast<const float *>(out + (long)ir * row_bytes + voff[b])
+                                    : 0.0f;
                     }
                 }
                 const int ir = iu + 8 * (v / 4) + (v % 4);  // uniform; the lane's row is ir + 4*half
-                if (CHECK && ir + 4 * half < own_i0) continue;
+                if (CHECK && (ir + 4 * half < own_i0 || (SHORT_M && ir + 4 * half >= g.M))) continue;
 #pragma unroll
                 for (int b = 0; b < TN; ++b) {
                     if (CHECK && !own[b]) continue;
@@ -785,8 +800,9 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         bool own[TN];
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
-            const int jg = j0 + wn * (TN * 32) + b * 32 + l32;
-            own[b] = jg >= own_j0;
+            const int jt = j0 + wn * (TN * 32) + b * 32 + l32;
+            own[b] = jt >= own_j0 && (!SHORT_J || jt < g.J);
+            const int jg = col_at(jt);
             unsigned im, n, y, x;
             g.divN.divmod((unsigned)jg, im, n);
             g.divCW.divmod(n, y, x);
@@ -827,7 +843,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                 float total = bsum[q] + __shfl_xor(bsum[q], 1);  // four lanes hold the quarters of a row
                 total += __shfl_xor(total, 2);
                 const int row = i0 + a_x + q * (NT / 4);
-                if (a_r == 0 && a_x + q * (NT / 4) < BM && row >= own_i0) dst[row * slots] = total;
+                if (a_r == 0 && a_x + q * (NT / 4) < BM && row >= own_i0 && (!SHORT_M || row < g.M)) dst[row * slots] = total;
             }
         }
     }

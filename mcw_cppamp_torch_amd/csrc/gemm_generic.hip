@@ -1,7 +1,8 @@
 // Bounds-checked fp32 MFMA GEMM for gfx950 (see gemm_mfma.h for the problem
-// statement): the fallback for problems with fewer rows or columns than the
-// smallest tile of the fast kernel (gemm_fast.h).  Every global access is
-// predicated, so any M, J, R work.
+// statement): the fallback for reductions shorter than a step of the fast kernel
+// (gemm_fast.h), for operands its 32-bit offsets do not reach and for forced
+// tiles that do not take a problem.  Every global access is predicated, so any
+// M, J, R work.
 //
 // Tiling: 2 x 2 wavefronts own a 64 x 64 tile of C, one v_mfma_f32_32x32x2_f32
 // accumulator per wavefront.  Both operand tiles are staged in LDS in

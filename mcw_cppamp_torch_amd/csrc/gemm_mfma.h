@@ -106,10 +106,14 @@ int gemm_launch(const GemmProblem &p);
 // within the kernels' 32-bit addressing, a tile the tuning switches allow): the test a gathered second
 // operand, which has no generic kernel, must pass before it is launched.
 bool gemm_tiled_fits(const GemmProblem &p);
+// The planner's estimate of the launch (and of the reduction of its partial sums), in microseconds: for choosing between
+// two ways to the same result.
+double gemm_estimate_us(const GemmProblem &p);
 
 // ---- shared between the kernel translation units ------------------------------
 
 constexpr int GEMM_BK = 16;  // reduction step of every kernel
+constexpr int GEMM_SHORT_TILE = 64;  // a tile side up to this length also takes a matrix that is shorter (gemm_fast.h)
 
 struct GemmArgs {
     const float *A;
@@ -182,8 +186,9 @@ int gemm_fast_256x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s
 int gemm_fast_64x64(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x256(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
+int gemm_fast_32x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);  // first operand along r only
 int gemm_fast_96x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);  // first operand along r only
-// The bounds-checked kernel for shapes smaller than a tile (gemm_generic.hip).
+// The bounds-checked kernel for reductions shorter than a step and operands beyond 32-bit offsets (gemm_generic.hip).
 int gemm_generic_64x64(const GemmArgs &g, bool a_rc, bool b_rc, bool red, hipStream_t s);
 
 }  // namespace thgpu

@@ -9,13 +9,13 @@ namespace thgpu {
 // The kernel bank as the first operand of a gradInput product, one element per lane:
 //   unit stride:  wt[c][m][kh][kw] = w[m][c][kH-1-kh][kW-1-kw]
 //   strided:      wt[(c, ph, pw)][(m, a', b')] = w[m][c][ph + sH*(A-1-a')][pw + sW*(Bk-1-b')], zero where that tap lies
-//                 outside the kernel and in the rows beyond C*sH*sW (the product's rows are padded to a whole tile).
+//                 outside the kernel.
 struct WeightJob {
     const float *w;
     float *wt;
     int M, C, kH, kW;
-    int sH, sW, A, Bk, rows, rows_pad;  // strided form only (sH = 0: unit stride)
-    unsigned count;                     // elements of wt; 0: no job
+    int sH, sW, A, Bk, rows;  // strided form only (sH = 0: unit stride)
+    unsigned count;           // elements of wt; 0: no job
 };
 
 __device__ __forceinline__ void reorder_weight(const WeightJob &j, unsigned idx) {
@@ -31,12 +31,10 @@ __device__ __forceinline__ void reorder_weight(const WeightJob &j, unsigned idx)
     const unsigned R = (unsigned)(j.M * j.A * j.Bk);
     const unsigned row = idx / R, r = idx % R;
     float v = 0.0f;
-    if (row < (unsigned)j.rows) {
-        const unsigned pw = row % j.sW, ph = (row / j.sW) % j.sH, c = row / (j.sW * j.sH);
-        const unsigned bb = r % j.Bk, aa = (r / j.Bk) % j.A, m = r / (j.Bk * j.A);
-        const unsigned kh = ph + j.sH * (j.A - 1 - aa), kw = pw + j.sW * (j.Bk - 1 - bb);
-        if (kh < (unsigned)j.kH && kw < (unsigned)j.kW) v = j.w[(((long)m * j.C + c) * j.kH + kh) * j.kW + kw];
-    }
+    const unsigned pw = row % j.sW, ph = (row / j.sW) % j.sH, c = row / (j.sW * j.sH);
+    const unsigned bb = r % j.Bk, aa = (r / j.Bk) % j.A, m = r / (j.Bk * j.A);
+    const unsigned kh = ph + j.sH * (j.A - 1 - aa), kw = pw + j.sW * (j.Bk - 1 - bb);
+    if (kh < (unsigned)j.kH && kw < (unsigned)j.kW) v = j.w[(((long)m * j.C + c) * j.kH + kh) * j.kW + kw];
     j.wt[idx] = v;
 }
 
