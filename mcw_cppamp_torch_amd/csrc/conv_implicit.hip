@@ -464,9 +464,17 @@ bool conv_use_gathered_gradinput(long B, int C, int H, int W, int M, int kH, int
     // product is also rounded less than the taps' sums that col2im adds up (2 x 64 planes 9x9: 1.39e-7 from 64 bits, columns
     // 1.59e-7), so it stays for single images too, where the columns are up to 30 % faster.
     const long Ho = H + 2L * pH - kH + 1, Wo = W + 2L * pW - kW + 1;
-    if (!strided && (C + 63L) / 64 * 64 * 8 <= C * 9L && ((long)H * W - Ho * Wo) * M <= 110 * Ho * Wo) return true;
+    if (!strided && C >= 64 && (C + 63L) / 64 * 64 * 8 <= C * 9L && ((long)H * W - Ho * Wo) * M <= 110 * Ho * Wo) return true;
+    // A strided layer whose residue classes take less than twice its work and fill the GPU keeps the one product until the
+    // columns are a third faster by estimate: their col2im is the part that the estimate knows least (3 -> 96 planes 11x11
+    // stride 4, 24 to 128 images: columns 1.15 to 1.3 times the gathered time, and a fused stack saves the padded copy as well).
+    double margin = 1.0;
+    if (strided) {
+        const PhaseGeom q = phase_geom(C, H, W, kH, kW, pH, pW, sH, sW);
+        if ((q.rows < 64 ? 64.0 : q.rows) * q.A * q.Bk <= 2.0 * C * kH * kW && B * q.Yn * (long)q.Xn >= 16384) margin = 1.35;
+    }
     return gathered_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW) <=
-           column_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
+           margin * column_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
 }
 
 long conv_implicit_gradinput_scratch(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH,

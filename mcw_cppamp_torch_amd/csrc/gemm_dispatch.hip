@@ -130,6 +130,8 @@ struct TileCfg {
     int below_rows;
     // The tile has no loader for a first operand contiguous along its rows.
     bool a_rc_only;
+    // Groups of wavefronts that share a workgroup's reduction (gemm_fast.h, finish_groups).
+    int groups = 1;
 };
 
 // Rate kept with k workgroups on a CU, by tile: measured on 3x3 forward products of 2304 reduction indices and exactly
@@ -138,6 +140,7 @@ const double kOcc2[5] = {0.0, 0.77, 1.0};
 const double kOcc3[5] = {0.0, 0.60, 0.91, 1.0};
 const double kOcc4[5] = {0.0, 0.57, 0.81, 0.95, 1.0};
 const double kOccSmall[5] = {0.0, 0.43, 0.75, 0.91, 1.0};
+const double kOcc1[2] = {0.0, 1.0};
 
 const TileCfg kCfgs[] = {
     {"128x128", 128, 128, 3, {0.38, 0.38, 0.38, 0.38, 0.39, 0.38}, gemm_fast_128x128, kOcc3, 0, false},
@@ -149,6 +152,7 @@ const TileCfg kCfgs[] = {
     {"64x128", 64, 128, 4, {0.33, 0.33, 0.33, 0.33, 0.34, 0.33}, gemm_fast_64x128, kOcc4, 128, false},
     {"96x128", 96, 128, 3, {0.35, 0, 0.35, 0, 0.37, 0.35}, gemm_fast_96x128, kOcc3, 128, true},
     {"32x128", 32, 128, 4, {0.22, 0, 0.22, 0, 0.22, 0.25}, gemm_fast_32x128, kOcc4, 33, true},
+    {"64x64k4", 64, 64, 1, {0.29, 0.29, 0.29, 0.29, 0.30, 0.25}, gemm_fast_64x64k4, kOcc1, 0, false, 4},
 };
 
 inline long cdiv(long a, long b) { return (a + b - 1) / b; }
@@ -165,11 +169,13 @@ double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_tot
     const double *kOcc = c.occ;
     const long tiles = cdiv(M, c.bm) * cdiv(J, c.bn);
     const long wgs = tiles * nsplit;
-    const long steps = cdiv(steps_total, nsplit);
+    const long steps = cdiv(cdiv(steps_total, nsplit), c.groups) * c.groups;
     const double per_step = 2.0 * c.bm * c.bn * GEMM_BK / kFlopsPerCycle / c.eff[layout];
-    const double ovh = 3000.0 + 6.0 * c.bm * c.bn / 64.0;
     const long slots = (long)cus * c.resident;
     const long full = wgs / slots, rest = wgs - full * slots;
+    // (A workgroup of groups has its CU to itself: where more than one follows another, nothing runs under its first loads and
+    // its stores: 395 x 3740 over 648, 413 tiles: 45.4 us, 37.3 with 64 x 64 tiles.)
+    const double ovh = 3000.0 + 6.0 * c.bm * c.bn / 64.0 + (c.groups > 1 && wgs > slots ? 6000.0 : 0.0);
     // A CU stores an output in half a cycle (4.8 TB/s over the chip); where a reduction is too short to hide that, a round
     // takes what its tiles' stores take and, at its start, one tile's more (20 indices, 225 x 161772: 64 us with two 128 x 256
     // tiles to a CU, 42 us with four of 64 x 128; an accumulating store also reads).
@@ -188,6 +194,7 @@ double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_tot
         if (full > 0) last = 0.5 * (last + round * rest / slots);
         t += last;
     }
+    if (c.groups > 1) t += 1000.0;  // the groups' sums through LDS
     if (nsplit > 1) t += 5000.0 + (double)(nsplit + 2) * M * J * 4.0 / (4.5e12 / 2.4e9);  // launch, bytes / (bytes per cycle)
     return t;
 }

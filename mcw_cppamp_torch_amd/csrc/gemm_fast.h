@@ -128,10 +128,105 @@ constexpr int gemm_min_waves() {
     return (BM / WGM) * (BN / WGN) / 64 >= 96 || by_lds < 3 ? 2 : 3;
 }
 
-template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED>
-__global__ __launch_bounds__(WGM *WGN * 64)
-    __attribute__((amdgpu_waves_per_eu(gemm_min_waves<BM, BN, WGM, WGN>()))) void gemm_fast_kernel(const GemmArgs g) {
-    constexpr int NT = WGM * WGN * 64;
+// The end of a workgroup of KG groups, each of which holds the sum of its own steps for the whole 64 x 64 tile: the groups'
+// sums meet in LDS and are added in the order of the groups, a thread taking the four outputs of one register quad of one
+// wavefront's block (and `rowsum`, the row sums of the first operand, likewise).
+//
+// What it is for: a step of the 64 x 64 tile has a latency of 0.4 to 0.6 us (its six products in a row, the split, LDS and
+// a barrier), which a CU with one or two workgroups does not hide.  Four steps at once take as long, in the same LDS
+// and registers that four workgroups of a quarter of the reduction would have, but without the partial sums, or with a
+// quarter of them: 3x3 layers of one and three 13x13 images 18.0 -> 17.4 and 23.3 -> 21.4 us with their split reductions
+// (27 -> 18 and 8 -> 5 parts), 50 images of 32 -> 64 planes 16x16 18.5 -> 16.0, their gradWeight 22.5 -> 19.0.
+// Finishing a reduction that is split over workgroups here as well, in the one that arrives last, was tried and taken back:
+// stores completed past the XCD's cache, a count and loads past it took the 4 us of the launch they replaced (256 x 169 over
+// 3456: 13.7 + 4, 18 to 20 us), and twice that with agent-scope fences.
+template <int BM, int BN, int WGN, bool RED, int KG>
+__device__ __forceinline__ void finish_groups(const GemmArgs &g, char *lds_a, char *lds_b, const floatx16 &acc, float rowsum,
+                                              bool rs_on, int group, int wave, int lane, unsigned tj, unsigned split, int i0, int j0, int own_i0,
+                                              int own_j0) {
+    static_assert(BM == 64 && BN == 64 && WGN == 2 && KG == 4, "sixteen wavefronts, sixteen quads of registers");
+    const int thread = threadIdx.x, half = lane >> 5, l32 = lane & 31;
+    // three groups' sums over the first operand's tiles, the last one's and the row sums over the second's
+    auto frag = [&](int k) { return reinterpret_cast<floatx4 *>(k < KG - 1 ? lds_a + k * (BM * BN * 4) : lds_b); };
+    float *const rows = reinterpret_cast<float *>(lds_b + BM * BN * 4);
+    static_assert((KG - 1) * BM * BN * 4 <= KG * 2 * PartTile<BM>::kBytes, "LDS of the first operand");
+    static_assert(BM * BN * 4 + KG * BM * 4 <= KG * 2 * PartTile<BN>::kBytes, "LDS of the second operand");
+    __syncthreads();  // the flags of lost bits have been read
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        frag(group)[(wave * 4 + q) * 64 + lane] = (floatx4){acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+    if (RED && rs_on) {
+        float total = rowsum + __shfl_xor(rowsum, 1);  // four lanes hold the quarters of a row
+        total += __shfl_xor(total, 2);
+        if ((lane & 3) == 0) rows[group * BM + wave * 16 + (lane >> 2)] = total;
+    }
+    __syncthreads();
+    const int of = thread >> 8, quad = (thread >> 6) & 3;  // whose outputs the thread takes over
+    floatx4 sum = frag(0)[(of * 4 + quad) * 64 + lane];
+#pragma unroll
+    for (int k = 1; k < KG; ++k) sum += frag(k)[(of * 4 + quad) * 64 + lane];
+    if (RED && rs_on && thread < BM) {
+        const int i = i0 + thread;
+        if (i >= own_i0 && i < g.M)
+            g.rowsum_ws[(long)i * g.nsplit * g.tilesJ + (long)split * g.tilesJ + tj] =
+                ((rows[thread] + rows[BM + thread]) + rows[2 * BM + thread]) + rows[3 * BM + thread];
+    }
+
+    // Four rows of one column.
+    const int j = j0 + (of % WGN) * 32 + l32, i_first = i0 + (of / WGN) * 32 + 8 * quad + 4 * half;
+    if (j < own_j0 || j >= g.J) return;
+    const float sign = l32 & 1 ? -1.0f : 1.0f;  // odd columns hold the negated sum
+    if (g.nsplit > 1) {
+        float *const ws = g.ws + (long)split * g.M * g.J + j;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (i_first + e >= own_i0 && i_first + e < g.M) ws[(long)(i_first + e) * g.J] = sum[e] * sign;
+        return;
+    }
+    const float alpha = sign * g.alpha;
+    unsigned im, n, y, x;
+    g.divN.divmod((unsigned)j, im, n);
+    g.divCW.divmod(n, y, x);
+    if (g.scatter) {
+        const int hy = (int)y * g.scat_sH - g.scat_pH, wx = (int)x * g.scat_sW - g.scat_pW;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = i_first + e;
+            unsigned c, rem, ph, pw;
+            g.divScatS.divmod((unsigned)i, c, rem);
+            g.divScatW.divmod(rem, ph, pw);
+            const int h = hy + (int)ph, w = wx + (int)pw;
+            if (i < own_i0 || i >= g.scat_rows || h < 0 || h >= g.scat_H || w < 0 || w >= g.scat_W) continue;
+            const long off = (long)im * g.bsC + ((long)c * g.scat_H + h) * g.scat_W + w;
+            float val = sum[e] * alpha + 0.0f;
+            if (g.mask) val = g.mask[off] > g.mask_threshold ? val : 0.0f;
+            g.C[off] = val;
+        }
+        return;
+    }
+    const bool per_image = !RED && (g.N != g.J || g.c_pitch != 0 || g.mask_pitch != 0 || g.C2 != nullptr);
+    const long col = !per_image ? (long)j : (long)im * g.bsC + (g.c_pitch ? (long)y * g.c_pitch + x : (long)n);
+    const long mcol = !per_image ? (long)j : (long)im * g.mask_bsC + (g.mask_pitch ? (long)y * g.mask_pitch + x : (long)n);
+    const long tcol = (long)im * g.c2_bsC + (long)y * g.c2_pitch + x;
+    const float col_bias = g.bias_col ? g.bias_col[j] : 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int i = i_first + e;
+        if (i < own_i0 || i >= g.M) continue;
+        float *const c = g.C + (long)i * g.sC + col;
+        float val = sum[e] * alpha + ((g.bias ? g.bias[i] : 0.0f) + col_bias);
+        if (g.beta != 0.0f) val += g.beta * *c;
+        if (g.act) val = val > g.act_threshold ? val : g.act_value;
+        if (g.mask) val = g.mask[(long)i * g.mask_sC + mcol] > g.mask_threshold ? val : 0.0f;
+        *c = val;
+        if (!RED && g.C2) g.C2[(long)i * g.c2_sC + tcol] = val;
+    }
+}
+
+template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG>
+__global__ __launch_bounds__(WGM *WGN * 64 * KG)
+    __attribute__((amdgpu_waves_per_eu(KG > 1 ? KG : gemm_min_waves<BM, BN, WGM, WGN>()))) void gemm_fast_kernel(const GemmArgs g) {
+    constexpr int NT = WGM * WGN * 64;  // threads of a group: the whole workgroup unless KG > 1
     constexpr int BK = GEMM_BK;
     constexpr int TM = BM / WGM / 32, TN = BN / WGN / 32;
     // A first operand along r whose 128-bit loads the threads do not divide (96 rows: 384 loads, 256 threads): the
@@ -161,10 +256,11 @@ __global__ __launch_bounds__(WGM *WGN * 64)
 
     using TileA = PartTile<BM>;
     using TileB = PartTile<BN>;
-    __shared__ __attribute__((aligned(16))) char As[2][TileA::kBytes];
-    __shared__ __attribute__((aligned(16))) char Bs[2][TileB::kBytes];
+    __shared__ __attribute__((aligned(16))) char As[KG][2][TileA::kBytes];
+    __shared__ __attribute__((aligned(16))) char Bs[KG][2][TileB::kBytes];
 
-    const int tid = threadIdx.x;
+    const int group = KG > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT) : 0;
+    const int tid = KG > 1 ? threadIdx.x % NT : threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: row bases stay uniform
     const int wm = wave / WGN, wn = wave % WGN;
     const int half = lane >> 5, l32 = lane & 31;
@@ -186,6 +282,13 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     int step = (int)split * g.steps_per_split;
     int step_end = step + g.steps_per_split;
     if (step_end > g.steps_total) step_end = g.steps_total;
+    int rounds = 0;  // loop iterations of the longest group
+    if constexpr (KG > 1) {
+        rounds = (step_end - step + KG - 1) / KG;
+        step += group * rounds;
+        if (step_end > step + rounds) step_end = step + rounds;
+        if (step_end < step) step_end = step;
+    }
     const int nsteps = step_end - step;
     int ld_img = 0, ld_r0 = step * BK;
     if (RED) {
@@ -393,8 +496,8 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     // where the loader gives a thread whole octets, otherwise four.
     constexpr int GA = (KA == LD_XC_SCALAR && NA % 8 == 0) ? 8 : 4;
     constexpr int GB = ((LB == LD_XC_SCALAR || LB == LD_XC_GATHER) && NB % 8 == 0) ? 8 : 4;
-    char *const a_dst = &As[0][0] + (a_r >> 3) * TileA::kOctet + a_x * 16 + (a_r & 7) * 2;
-    char *const b_dst = &Bs[0][0] + (b_r >> 3) * TileB::kOctet + b_x * 16 + (b_r & 7) * 2;
+    char *const a_dst = &As[group][0][0] + (a_r >> 3) * TileA::kOctet + a_x * 16 + (a_r & 7) * 2;
+    char *const b_dst = &Bs[group][0][0] + (b_r >> 3) * TileB::kOctet + b_x * 16 + (b_r & 7) * 2;
     unsigned lost = 0;  // see split_pair
     const unsigned odd_column = (unsigned)(b_x & 1) << 31;  // the sign of a thread's elements of the second operand
     auto stash_group = [&](auto kind_tag, auto group_tag, auto tile_tag, char *dst, const float *src, int q, auto sign) {
@@ -482,8 +585,8 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     // ---- main loop ----------------------------------------------------------------------
     // Step s multiplies from LDS buffer s&1, block by block; between the MFMAs the groups of
     // step s+1 are split and written to the other buffer and their registers refilled for step s+2.
-    const char *const a_src = &As[0][0] + half * TileA::kOctet + (wm * (TM * 32) + l32) * 16;
-    const char *const b_src = &Bs[0][0] + half * TileB::kOctet + (wn * (TN * 32) + l32) * 16;
+    const char *const a_src = &As[group][0][0] + half * TileA::kOctet + (wm * (TM * 32) + l32) * 16;
+    const char *const b_src = &Bs[group][0][0] + half * TileB::kOctet + (wn * (TN * 32) + l32) * 16;
     // Two sums in turn, so that the additions of one block run under the MFMAs of the next, where the registers hold both
     // (1 to 2 % on the 8-block tiles), and the parts of the longer side one block row ahead likewise.
     constexpr bool PING = !(TM == 2 && TN == 2 && WGN == 2) && !(TM * TN == 8 && LB == LD_RC_GATHER);
@@ -580,22 +683,31 @@ __global__ __launch_bounds__(WGM *WGN * 64)
         for_each_index(block_of, std::make_integer_sequence<int, BLOCKS>{});
         if (more) advance();
         else shift = 0;
-        __syncthreads();
+        if (KG == 1) __syncthreads();
     };
-    for (int s = 0; s < nsteps; s += 2) {
-        one_step(std::integral_constant<int, 0>{}, s);
-        if (s + 1 < nsteps) one_step(std::integral_constant<int, 1>{}, s + 1);
+    if constexpr (KG == 1) {
+        for (int s = 0; s < nsteps; s += 2) {
+            one_step(std::integral_constant<int, 0>{}, s);
+            if (s + 1 < nsteps) one_step(std::integral_constant<int, 1>{}, s + 1);
+        }
+    } else {
+        for (int s = 0; s < rounds; s += 2) {  // the last groups may have fewer steps, the barriers are everybody's
+            if (s < nsteps) one_step(std::integral_constant<int, 0>{}, s);
+            __syncthreads();
+            if (s + 1 < nsteps) one_step(std::integral_constant<int, 1>{}, s + 1);
+            __syncthreads();
+        }
     }
 
     // ---- what the split could not hold -----------------------------------------------------
     // Did any thread's element lose bits?  (The operand tiles in LDS have been read: the loop ends with a barrier.)
-    unsigned *const lost_of = reinterpret_cast<unsigned *>(&As[0][0]);
+    unsigned *const lost_of = reinterpret_cast<unsigned *>(&As[0][0][0]);
     const bool lost_here = __builtin_amdgcn_ballot_w64((lost & 0xffffu) != 0) != 0;
-    if (lane == 0) lost_of[wave] = lost_here ? 1u : 0u;
+    if (lane == 0) lost_of[group * (NT / 64) + wave] = lost_here ? 1u : 0u;
     __syncthreads();
     unsigned lost_any = 0;
 #pragma unroll
-    for (int w = 0; w < NT / 64; ++w) lost_any |= lost_of[w];
+    for (int w = 0; w < KG * NT / 64; ++w) lost_any |= lost_of[w];
     // The wavefront's outputs in fp32, straight from the operands: eight reduction indices at a time, four to a lane half,
     // whose loads are in flight together.  (A step that would run past R is moved back as in the main loop.)
     const float column_sign = l32 & 1 ? -1.0f : 1.0f;  // of the accumulators
@@ -684,6 +796,12 @@ __global__ __launch_bounds__(WGM *WGN * 64)
             for (int v = 0; v < 16; ++v) odd |= __builtin_amdgcn_classf(acc[a][b][v], 0x297);  // NaN, infinite, denormal
     if (__builtin_amdgcn_ballot_w64(odd)) recompute();
 
+    // ---- groups ------------------------------------------------------------------------
+    if constexpr (KG > 1) {
+        finish_groups<BM, BN, WGN, RED, KG>(g, &As[0][0][0], &Bs[0][0][0], acc[0][0], bsum[0], rs_on, group, wave, lane, tj, split, i0, j0, own_i0, own_j0);
+        return;
+    }
+
     // ---- epilogue ----------------------------------------------------------------------
     // Accumulator register v of lane l holds D[8*(v/4) + 4*(l/32) + v%4][l%32].
     // A store address is a wave-uniform row base plus a constant per-lane byte
@@ -735,6 +853,11 @@ __global__ __launch_bounds__(WGM *WGN * 64)
             mvoff[b] = (unsigned)(mcol * 4 + 4 * half * mask_row_bytes);
             tvoff[b] = (unsigned)(tcol * 4 + 4 * half * twin_row_bytes);
         }
+        // Whether the lane's row ir + 4*half belongs to the tile above or lies below the matrix, of which an edge tile has only
+        // one kind: a single comparison.
+        const bool few_rows = SHORT_M && g.M < BM;
+        const int edge_lane = few_rows ? -4 * half : 4 * half;
+        auto not_ours = [&](int ir) { return edge_lane < (few_rows ? ir - g.M + 1 : own_i0 - ir); };
         // Rows outermost, the wavefront's column blocks innermost: the stores of one output row follow each other
         // directly, so a cache line that two neighbouring 128-byte segments share (rows are rarely 128-byte aligned)
         // is completed while it is still in L2 instead of going out to memory twice.
@@ -773,7 +896,7 @@ __global__ __launch_bounds__(WGM *WGN * 64)
                     }
                 }
                 const int ir = iu + 8 * (v / 4) + (v % 4);  // uniform; the lane's row is ir + 4*half
-                if (CHECK && (ir + 4 * half < own_i0 || (SHORT_M && ir + 4 * half >= g.M))) continue;
+                if (CHECK && not_ours(ir)) continue;
 #pragma unroll
                 for (int b = 0; b < TN; ++b) {
                     if (CHECK && !own[b]) continue;
@@ -866,14 +989,14 @@ __global__ __launch_bounds__(WGM *WGN * 64)
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED>
+template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG = 1>
 int gemm_fast_go(const GemmArgs &g, hipStream_t s) {
-    hipLaunchKernelGGL((gemm_fast_kernel<BM, BN, WGM, WGN, LA, LB, RED>), dim3(g.total), dim3(WGM * WGN * 64), 0, s, g);
+    hipLaunchKernelGGL((gemm_fast_kernel<BM, BN, WGM, WGN, LA, LB, RED, KG>), dim3(g.total), dim3(WGM * WGN * 64 * KG), 0, s, g);
     return 0;
 }
 
 // Dispatch over the loader kinds for one tile configuration.
-template <int BM, int BN, int WGM, int WGN>
+template <int BM, int BN, int WGM, int WGN, int KG = 1>
 int gemm_fast_dispatch(const GemmArgs &g, int la, int lb, bool red, hipStream_t s) {
 #define THGPU_CASE(LA_, LB_)                                                           \
     if (la == LA_ && lb == LB_) {                                                      \
@@ -884,14 +1007,14 @@ int gemm_fast_dispatch(const GemmArgs &g, int la, int lb, bool red, hipStream_t 
         } else {                                                                       \
             if (red) {                                                                 \
                 if constexpr (LA_ == LD_RC_VEC && LB_ != LD_XC_SCALAR && LB_ != LD_XC_GATHER) \
-                    return gemm_fast_go<BM, BN, WGM, WGN, LA_, LB_, true>(g, s);       \
+                    return gemm_fast_go<BM, BN, WGM, WGN, LA_, LB_, true, KG>(g, s);     \
                 else                                                                   \
                     return fail("gemm: reduction batching needs operands loaded along r"); \
             }                                                                          \
             if constexpr (LB_ == LD_RC_GATHER || LB_ == LD_RC_GATHER_VEC)              \
                 return fail("gemm: a gather along r needs reduction batching");        \
             else                                                                       \
-                return gemm_fast_go<BM, BN, WGM, WGN, LA_, LB_, false>(g, s);          \
+                return gemm_fast_go<BM, BN, WGM, WGN, LA_, LB_, false, KG>(g, s);        \
         }                                                                              \
     }
     THGPU_CASE(LD_RC_VEC, LD_RC_VEC)

@@ -183,6 +183,7 @@ int gemm_fast_128x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s
 int gemm_fast_192x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_128x256(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_256x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
+int gemm_fast_64x64k4(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x64(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x256(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);

@@ -45,7 +45,7 @@ def test_blas_product_of_an_empty_sum(gt, n):
 
 
 # tile -> (rows, columns); the BLAS entry point is column-major, so C's columns n are the kernels' rows
-TILES = {"32x128": (32, 128), "64x64": (64, 64), "64x128": (64, 128), "64x256": (64, 256)}
+TILES = {"32x128": (32, 128), "64x64": (64, 64), "64x64k4": (64, 64), "64x128": (64, 128), "64x256": (64, 256)}
 ROWS = [1, 31, 32, 33, 63, 64, 65]
 COLS = [1, 63, 64, 65, 127, 128, 300]
 
