@@ -502,6 +502,16 @@ int thgpu_SpatialConvolutionMM_updateGradInputTwin(THGPUTensor *input, THGPUTens
                                                    THGPUTensor *gradInput, int kW, int kH, int dW, int dH, int padW,
                                                    int padH, int flags, float threshold, THGPUTensor *twin,
                                                    int *wrote_twin);
+/* updateGradInput followed by accGradParameters of the same module, input and gradOutput (nn.Module.backward,
+ * mcw_nn/Module.lua:24-33), with fewer launches where both gather from padded images: the input is padded by the launch that
+ * pads gradOutput, and split reductions and small products of the two share launches.  Results are those of the two calls.
+ * flags: THGPU_FUSE_INPUT_MASK with `threshold` and THGPU_GRADOUTPUT_IN_TWIN as in updateGradInputTwin,
+ * THGPU_INPUT_IN_PADDED_BUFFER as in accGradParametersFused; `twin` and `wrote_twin` may be NULL. */
+int thgpu_SpatialConvolutionMM_backward(THGPUTensor *input, THGPUTensor *gradOutput, THGPUTensor *weight,
+                                        THGPUTensor *gradWeight, THGPUTensor *gradBias, THGPUTensor *finput,
+                                        THGPUTensor *fgradInput, THGPUTensor *gradInput, int kW, int kH, int dW, int dH,
+                                        int padW, int padH, float scale, int flags, float threshold, THGPUTensor *twin,
+                                        int *wrote_twin);
 /* 1 when updateOutput / accGradParameters of a layer with these sizes would gather from the padded image in the
  * current mode (and so profit from an input that already lies in a padded buffer), 0 otherwise. */
 int thgpu_conv_gathers(long B, int C, int H, int W, int M, int kW, int kH, int dW, int dH, int padW, int padH);

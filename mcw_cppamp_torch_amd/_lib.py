@@ -206,6 +206,8 @@ _SIGNATURES = {
     "thgpu_SpatialConvolutionMM_updateOutputFused": (c_int, [TensorP] * 6 + [c_int] * 7 + [c_float] * 2),
     "thgpu_SpatialConvolutionMM_updateGradInputFused": (c_int, [TensorP] * 6 + [c_int] * 7 + [c_float]),
     "thgpu_SpatialConvolutionMM_accGradParametersFused": (c_int, [TensorP] * 6 + [c_int] * 6 + [c_float, c_int]),
+    "thgpu_SpatialConvolutionMM_backward": (c_int, [TensorP] * 8 + [c_int] * 6 + [c_float, c_int, c_float, TensorP,
+                                                    ctypes.POINTER(c_int)]),
     "thgpu_conv_gathers": (c_int, [c_long] + [c_int] * 10),
     "thgpu_SpatialConvolutionMM_gradOutputTwin": (c_int, [TensorP] * 4 + [c_int] * 6 + [ctypes.POINTER(c_int)]),
     "thgpu_SpatialConvolutionMM_updateGradInputTwin": (c_int, [TensorP] * 6 + [c_int] * 7 + [c_float, TensorP,

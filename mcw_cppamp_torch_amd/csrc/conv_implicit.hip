@@ -77,11 +77,13 @@ __device__ __forceinline__ void pad_four(const PadJob &j, unsigned block) {
 __global__ __launch_bounds__(256) void pad_planes_kernel(const PadJob j) { pad_four(j, blockIdx.x); }
 
 // Both preparations of a gradInput product in one launch (they are independent, and the kernel bank alone is a
-// launch of a few microseconds of work): the first pad_blocks workgroups pad gradOutput, the rest re-order the bank.
-__global__ __launch_bounds__(256) void pad_planes_and_weights_kernel(const PadJob pad, unsigned pad_blocks,
-                                                                      const WeightJob wj) {
+// launch of a few microseconds of work): the first pad_blocks workgroups pad gradOutput, the next weight_blocks re-order the
+// bank, and the rest pad the input for the gradWeight product of the same layer.
+__global__ __launch_bounds__(256) void pad_planes_and_weights_kernel(const PadJob pad, unsigned pad_blocks, const WeightJob wj,
+                                                                      unsigned weight_blocks, const PadJob input) {
     if (blockIdx.x < pad_blocks) pad_four(pad, blockIdx.x);
-    else reorder_weight(wj, (blockIdx.x - pad_blocks) * 256u + threadIdx.x);
+    else if (blockIdx.x < pad_blocks + weight_blocks) reorder_weight(wj, (blockIdx.x - pad_blocks) * 256u + threadIdx.x);
+    else pad_four(input, blockIdx.x - pad_blocks - weight_blocks);
 }
 
 // t[(c, kh, kw)] = c*plane + kh*pitch + kw
@@ -486,39 +488,55 @@ long conv_implicit_gradinput_scratch(long B, int C, int H, int W, int M, int kH,
     return B * M * (H + kH - 1L) * (W + kW - 1L) + (long)C * M * kH * kW;
 }
 
-// out[plane][y][x] = in[plane][y - top][x - left], zero outside the H x W source; out planes are Hp x Wp.  With a
-// weight job the same launch also re-orders the kernel bank.
-static int pad_planes_into(const float *in, long planes, int H, int W, int top, int left, long Hp, long Wp, float *out,
-                           const WeightJob *wj = nullptr) {
+// out[plane][y][x] = in[plane][y - top][x - left], zero outside the H x W source; out planes are Hp x Wp.
+struct PadSpec {
+    const float *in = nullptr;
+    long planes = 0;  // 0: nothing to pad
+    int H = 0, W = 0, top = 0, left = 0;
+    long Hp = 0, Wp = 0;
+    float *out = nullptr;
+    long total() const { return planes * Hp * Wp; }
+};
+
+static PadJob pad_job(const PadSpec &p) {
+    PadJob j;
+    j.in = p.in;
+    j.out = p.out;
+    j.total = (unsigned)p.total();
+    j.H = p.H;
+    j.W = p.W;
+    j.pH = p.top;
+    j.pW = p.left;
+    j.Hp = (int)p.Hp;
+    j.Wp = (int)p.Wp;
+    j.divWp = FastDiv((uint32_t)(p.Wp > 0 ? p.Wp : 1));
+    j.divHp = FastDiv((uint32_t)(p.Hp > 0 ? p.Hp : 1));
+    j.aligned = (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
+    return j;
+}
+
+// Pads; with a weight job the same launch also re-orders the kernel bank, and with `input` it pads a second buffer.
+static int pad_planes_into(const PadSpec &pad, const WeightJob *wj = nullptr, const PadSpec *input = nullptr) {
     hipStream_t s = stream();
     if (!s) return 1;
-    const long total = planes * Hp * Wp;
-    if (total <= 0 && !wj) return 0;
-    if (total >= (1L << 31)) return fail("pad: %ld elements exceed 32-bit indexing", total);
+    const long total = pad.total(), second = input ? input->total() : 0;
+    if (total <= 0 && !wj && second <= 0) return 0;
+    if (total >= (1L << 31) || second >= (1L << 31))
+        return fail("pad: %ld elements exceed 32-bit indexing", total > second ? total : second);
     {
-        const char *label = planes == 0 ? "kernel_bank_reorder"
-                            : prof_enabled() ? prof_label("pad_planes planes=%ld %dx%d p=%dx%d", planes, H, W, top, left)
+        const char *label = pad.planes == 0 && second == 0 ? "kernel_bank_reorder"
+                            : prof_enabled() ? prof_label("pad_planes planes=%ld %dx%d p=%dx%d", pad.planes, pad.H, pad.W, pad.top, pad.left)
                                              : "pad_planes";
         const double wbytes = wj ? 4.0 * (wj->count + (double)wj->M * wj->C * wj->kH * wj->kW) : 0.0;
-        LaunchScope scope(label, 0.0, 4.0 * (total + planes * H * W) + wbytes);
-        PadJob pj;
-        pj.in = in;
-        pj.out = out;
-        pj.total = (unsigned)total;
-        pj.H = H;
-        pj.W = W;
-        pj.pH = top;
-        pj.pW = left;
-        pj.Hp = (int)Hp;
-        pj.Wp = (int)Wp;
-        pj.divWp = FastDiv((uint32_t)Wp);
-        pj.divHp = FastDiv((uint32_t)Hp);
-        pj.aligned = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+        const double second_bytes = second > 0 ? 4.0 * (second + input->planes * input->H * input->W) : 0.0;
+        LaunchScope scope(label, 0.0, 4.0 * (total + pad.planes * pad.H * pad.W) + wbytes + second_bytes);
+        const PadJob pj = pad_job(pad);
         const unsigned pad_blocks = (unsigned)((total + 1023) / 1024);
-        if (wj) {
-            const unsigned wblocks = (wj->count + 255u) / 256u;
-            hipLaunchKernelGGL(pad_planes_and_weights_kernel, dim3(pad_blocks + wblocks), dim3(256), 0, s, pj, pad_blocks,
-                               *wj);
+        if (wj || second > 0) {
+            WeightJob none = {};
+            const unsigned wblocks = wj ? (wj->count + 255u) / 256u : 0;
+            hipLaunchKernelGGL(pad_planes_and_weights_kernel, dim3(pad_blocks + wblocks + (unsigned)((second + 1023) / 1024)),
+                               dim3(256), 0, s, pj, pad_blocks, wj ? *wj : none, wblocks, input ? pad_job(*input) : pj);
         } else {
             hipLaunchKernelGGL(pad_planes_kernel, dim3(pad_blocks), dim3(256), 0, s, pj);
         }
@@ -542,8 +560,22 @@ void conv_implicit_q_layout(int C, int H, int W, int kH, int kW, int pH, int pW,
     *Wq = W + kW - 1;
 }
 
+static PadSpec input_pad(const float *in, long planes, int H, int W, int pH, int pW, float *out) {
+    PadSpec p;
+    p.in = in;
+    p.planes = planes;
+    p.H = H;
+    p.W = W;
+    p.top = pH;
+    p.left = pW;
+    p.Hp = H + 2L * pH;
+    p.Wp = W + 2L * pW;
+    p.out = out;
+    return p;
+}
+
 int pad_planes_launch(const float *in, long planes, int H, int W, int pH, int pW, float *out) {
-    return pad_planes_into(in, planes, H, W, pH, pW, H + 2L * pH, W + 2L * pW, out);
+    return pad_planes_into(input_pad(in, planes, H, W, pH, pW, out));
 }
 
 int conv_implicit_forward(const float *padded, const float *weight, const float *bias, float *output, long B, int C,
@@ -577,6 +609,24 @@ int conv_implicit_forward(const float *padded, const float *weight, const float 
     return gemm_launch(p);
 }
 
+static int gradweight_operands(GemmProblem &p, const float *padded, const float *gradOutput, float *gradWeight, long B, int C,
+                               int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW, float scale,
+                               float *gradBias, bool *bias_done) {
+    const int Hp = H + 2 * pH, Wp = W + 2 * pW;
+    const int Ho = (Hp - kH) / sH + 1, Wo = (Wp - kW) / sW + 1;
+    p = gradweight_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
+    p.A = gradOutput;
+    p.B = padded;
+    p.rowtab = pixel_table(Ho, Wo, sH * Wp, sW);
+    p.coltab = p.j_store > 0 ? tap_table_padded(C, kH, kW, Hp * Wp, Wp, p.J) : tap_table(C, kH, kW, Hp * Wp, Wp);
+    if (!p.rowtab || !p.coltab) return 1;
+    p.C = gradWeight;
+    p.alpha = scale;
+    p.rowsum = gradBias;  // gradBias[m] += scale * sum of gradOutput[.][m][.]: the row sums of this product's A
+    p.rowsum_done = bias_done;
+    return 0;
+}
+
 int conv_implicit_gradweight(const float *padded, const float *gradOutput, float *gradWeight, long B, int C, int H,
                              int W, int M, int kH, int kW, int pH, int pW, int sH, int sW, float scale, float *gradBias,
                              bool *bias_done) {
@@ -590,83 +640,65 @@ int conv_implicit_gradweight(const float *padded, const float *gradOutput, float
         return conv_narrow_gradweight(padded, (long)C * Hp * Wp, gradOutput, gradWeight, gradBias, B, M, C * kH * kW, Ho,
                                       Wo, sH * Wp, taps, scale);
     }
-    GemmProblem p = gradweight_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
-    p.A = gradOutput;
-    p.B = padded;
-    p.rowtab = pixel_table(Ho, Wo, sH * Wp, sW);
-    p.coltab = p.j_store > 0 ? tap_table_padded(C, kH, kW, Hp * Wp, Wp, p.J) : tap_table(C, kH, kW, Hp * Wp, Wp);
-    if (!p.rowtab || !p.coltab) return 1;
-    p.C = gradWeight;
-    p.alpha = scale;
-    p.rowsum = gradBias;  // gradBias[m] += scale * sum of gradOutput[.][m][.]: the row sums of this product's A
-    p.rowsum_done = bias_done;
+    GemmProblem p;
+    if (gradweight_operands(p, padded, gradOutput, gradWeight, B, C, H, W, M, kH, kW, pH, pW, sH, sW, scale, gradBias, bias_done)) return 1;
     return gemm_launch(p);
 }
 
-// gradInput of a strided layer as one product over the residue classes of the pixel coordinates.
-static int conv_implicit_gradinput_strided(const float *gradOutput, const float *weight, float *scratch,
-                                           float *gradInput, long B, int C, int H, int W, int M, int kH, int kW, int pH,
-                                           int pW, int sH, int sW, InputMask mask, bool q_ready) {
-    hipStream_t s = stream();
-    if (!s) return 1;
-    if (mask.in && (mask.pitch > 0 || (mask.plane > 0 && mask.plane != (long)H * W)))
+// The gradInput product: what has to be padded and re-ordered before it, and its operands.
+struct GradInputPlan {
+    PadSpec pad;           // gradOutput into the product's padded layout (no planes: it is there)
+    WeightJob bank;
+    bool prepared = false; // neither is left to do
+    GemmProblem p;
+};
+
+// q_ready, twin: see conv_implicit_gradinput.  A launch that came before may have re-ordered the bank already.
+static int plan_gradinput(GradInputPlan &plan, const float *gradOutput, const float *weight, float *scratch, float *gradInput, long B,
+                          int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW, InputMask mask, bool q_ready,
+                          TwinOutput twin, bool *wrote_twin) {
+    const bool strided = sH != 1 || sW != 1;
+    if (strided && mask.in && (mask.pitch > 0 || (mask.plane > 0 && mask.plane != (long)H * W)))
         return fail("SpatialConvolutionMM: the strided gradInput product takes a densely packed mask only");
-    const PhaseGeom q = phase_geom(C, H, W, kH, kW, pH, pW, sH, sW);
     const int Ho = (H + 2 * pH - kH) / sH + 1, Wo = (W + 2 * pW - kW) / sW + 1;
+    int top, left, Hq, Wq;
+    conv_implicit_q_layout(C, H, W, kH, kW, pH, pW, sH, sW, &top, &left, &Hq, &Wq);
+    GemmProblem &p = plan.p;
+    p = strided ? gradinput_strided_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW)
+                : gradinput_problem(B, C, H, W, M, kH, kW, pH, pW);
     float *Q = scratch;
-    float *Wt = scratch + B * M * (long)q.Hq * q.Wq;
-    const long nw = (long)q.rows * M * q.A * q.Bk;
-    if (nw >= (1L << 31)) return fail("SpatialConvolutionMM: kernel bank too large for the strided gradInput product");
-    const WeightJob wj = bank_job(weight, Wt, C, H, W, M, kH, kW, pH, pW, sH, sW);
+    float *Wt = scratch + B * M * (long)Hq * Wq;
+    if ((long)p.M * p.R >= (1L << 31)) return fail("SpatialConvolutionMM: kernel bank too large for the gradInput product");
+    plan.bank = bank_job(weight, Wt, C, H, W, M, kH, kW, pH, pW, sH, sW);
     // With gradOutput already in place only the kernel bank is re-ordered (zero planes to pad), unless a launch before
     // this one has carried that job along.
     const bool bank_done = bank_job_done(Wt);
-    if (!(q_ready && bank_done) &&
-        pad_planes_into(gradOutput, q_ready ? 0 : B * M, Ho, Wo, q.A - 1, q.Bk - 1, q.Hq, q.Wq, Q, &wj))
-        return 1;
+    plan.prepared = q_ready && bank_done;
+    plan.pad.in = gradOutput;
+    plan.pad.planes = q_ready ? 0 : B * M;
+    plan.pad.H = Ho;
+    plan.pad.W = Wo;
+    plan.pad.top = top;
+    plan.pad.left = left;
+    plan.pad.Hp = Hq;
+    plan.pad.Wp = Wq;
+    plan.pad.out = Q;
     if (trim_tables()) return 1;
-    GemmProblem p = gradinput_strided_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
     p.A = Wt;
     p.B = Q;
-    p.rowtab = tap_table(M, q.A, q.Bk, q.Hq * q.Wq, q.Wq);
-    p.coltab = pixel_table(q.Yn, q.Xn, q.Wq, 1);
+    if (strided) {
+        const PhaseGeom q = phase_geom(C, H, W, kH, kW, pH, pW, sH, sW);
+        p.rowtab = tap_table(M, q.A, q.Bk, Hq * Wq, Wq);
+        p.coltab = pixel_table(q.Yn, q.Xn, Wq, 1);
+    } else {
+        p.rowtab = tap_table(M, kH, kW, Hq * Wq, Wq);
+        p.coltab = pixel_table(H, W, Wq, 1);
+    }
     if (!p.rowtab || !p.coltab) return 1;
     p.C = gradInput;
     p.mask = mask.in;
     p.mask_threshold = mask.threshold;
-    return gemm_launch(p);
-}
-
-int conv_implicit_gradinput(const float *gradOutput, const float *weight, float *scratch, float *gradInput, long B,
-                            int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW, InputMask mask,
-                            bool q_ready, TwinOutput twin, bool *wrote_twin) {
-    if (wrote_twin) *wrote_twin = false;
-    if (sH != 1 || sW != 1)  // (the scattered store keeps no second copy)
-        return conv_implicit_gradinput_strided(gradOutput, weight, scratch, gradInput, B, C, H, W, M, kH, kW, pH, pW, sH,
-                                               sW, mask, q_ready);
-    hipStream_t s = stream();
-    if (!s) return 1;
-    const int Ho = H + 2 * pH - kH + 1, Wo = W + 2 * pW - kW + 1;
-    const int qH = kH - 1 - pH, qW = kW - 1 - pW;
-    const int Hq = Ho + 2 * qH, Wq = Wo + 2 * qW;  // = H + kH - 1, W + kW - 1
-    float *Q = scratch;
-    float *Wt = scratch + B * M * (long)Hq * Wq;
-    const long nw = (long)M * C * kH * kW;
-    if (nw >= (1L << 31)) return fail("SpatialConvolutionMM: kernel bank too large for the gradInput product");
-    const WeightJob wj = bank_job(weight, Wt, C, H, W, M, kH, kW, pH, pW, sH, sW);
-    const bool bank_done = bank_job_done(Wt);
-    if (!(q_ready && bank_done) && pad_planes_into(gradOutput, q_ready ? 0 : B * M, Ho, Wo, qH, qW, Hq, Wq, Q, &wj))
-        return 1;
-    if (trim_tables()) return 1;
-    GemmProblem p = gradinput_problem(B, C, H, W, M, kH, kW, pH, pW);
-    p.A = Wt;
-    p.B = Q;
-    p.rowtab = tap_table(M, kH, kW, Hq * Wq, Wq);
-    p.coltab = pixel_table(H, W, Wq, 1);
-    if (!p.rowtab || !p.coltab) return 1;
-    p.C = gradInput;
-    p.mask = mask.in;
-    p.mask_threshold = mask.threshold;
+    if (strided) return 0;  // (the scattered store keeps no second copy)
     if (mask.in && mask.plane > 0) {
         p.mask_sC = mask.plane;
         p.mask_bsC = (long)C * mask.plane;
@@ -684,7 +716,47 @@ int conv_implicit_gradinput(const float *gradOutput, const float *weight, float 
         if (!gemm_tiled_fits(p)) p.C2 = nullptr;  // the copy's offsets exceed the kernels' addressing: do without
         if (wrote_twin) *wrote_twin = p.C2 != nullptr;
     }
-    return gemm_launch(p);
+    return 0;
+}
+
+int conv_implicit_gradinput(const float *gradOutput, const float *weight, float *scratch, float *gradInput, long B,
+                            int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW, InputMask mask,
+                            bool q_ready, TwinOutput twin, bool *wrote_twin) {
+    if (wrote_twin) *wrote_twin = false;
+    GradInputPlan plan;
+    if (plan_gradinput(plan, gradOutput, weight, scratch, gradInput, B, C, H, W, M, kH, kW, pH, pW, sH, sW, mask, q_ready, twin,
+                       wrote_twin))
+        return 1;
+    if (!plan.prepared && pad_planes_into(plan.pad, &plan.bank)) return 1;
+    return gemm_launch(plan.p);
+}
+
+// updateGradInput and accGradParameters of a layer whose products both gather, from one preparing launch.
+int conv_implicit_backward(const float *input, const float *padded, float *pad_into, const float *gradOutput, const float *weight,
+                           float *scratch, float *gradInput, float *gradWeight, float *gradBias, long B, int C, int H, int W,
+                           int M, int kH, int kW, int pH, int pW, int sH, int sW, InputMask mask, bool q_ready, TwinOutput twin,
+                           bool *wrote_twin, float scale, bool *bias_done) {
+    if (wrote_twin) *wrote_twin = false;
+    GradInputPlan plan;
+    if (plan_gradinput(plan, gradOutput, weight, scratch, gradInput, B, C, H, W, M, kH, kW, pH, pW, sH, sW, mask, q_ready, twin,
+                       wrote_twin))
+        return 1;
+    const PadSpec second = pad_into ? input_pad(input, B * C, H, W, pH, pW, pad_into) : PadSpec();
+    const bool narrow = conv_narrow_gradweight_fits(B, M, (long)C * kH * kW, (W + 2 * pW - kW) / sW + 1,
+                                                    (long)((H + 2 * pH - kH) / sH + 1) * ((W + 2 * pW - kW) / sW + 1), sW);
+    GemmProblem gw;
+    // (the tables of both products, before either is enqueued: a look-up that starts the cache over would free the other's)
+    if (!narrow && gradweight_operands(gw, pad_into ? pad_into : padded, gradOutput, gradWeight, B, C, H, W, M, kH, kW, pH, pW, sH, sW,
+                                       scale, gradBias, bias_done))
+        return 1;
+    if ((!plan.prepared || pad_into) &&
+        pad_planes_into(plan.prepared ? PadSpec() : plan.pad, plan.prepared ? nullptr : &plan.bank, pad_into ? &second : nullptr))
+        return 1;
+    if (!narrow) return gemm_launch_pair(plan.p, gw);
+    return gemm_launch(plan.p) || conv_implicit_gradweight(pad_into ? pad_into : padded, gradOutput, gradWeight, B, C, H, W, M, kH,
+                                                           kW, pH, pW, sH, sW, scale, gradBias, bias_done)
+               ? 1
+               : 0;
 }
 
 }  // namespace thgpu

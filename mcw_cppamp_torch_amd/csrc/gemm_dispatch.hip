@@ -39,41 +39,57 @@ __device__ __forceinline__ void rowsum_reduce(const RowSumJob &j, unsigned block
     if (lane == 0) j.out[row] += j.alpha * sum;
 }
 
+// The reduction of one product's partial sums and whatever rides with it.
+struct ReduceJob {
+    RowSumJob rs;
+    const float *ws;
+    float *C;
+    const float *bias, *bias_col;
+    int M, J, N;
+    long sC, bsC;
+    FastDiv divJ, divN, divCW;
+    int nsplit;
+    float alpha, beta;
+    int act;
+    float act_threshold, act_value;
+    const float *mask;
+    float mask_threshold;
+    int c_pitch, mask_pitch;
+    long mask_sC, mask_bsC;
+    float *C2;
+    long c2_sC, c2_bsC;
+    int c2_pitch;
+    unsigned j_store;
+    unsigned side_first_block;  // workgroups from this one on carry a job of the next layer's (side_jobs.h)
+    WeightJob side;
+    unsigned blocks;
+    bool quarters;
+};
+
 template <bool quarters>
-__global__ __launch_bounds__(256) void split_reduce_kernel(const RowSumJob rs, const float *__restrict__ ws, float *__restrict__ C,
-                                                           const float *__restrict__ bias, int M, int J, int N,
-                                                           long sC, long bsC, FastDiv divJ, FastDiv divN, int nsplit,
-                                                           float alpha, float beta, int act, float act_threshold,
-                                                           float act_value, const float *__restrict__ mask,
-                                                           float mask_threshold, int c_pitch, int mask_pitch,
-                                                           long mask_sC, long mask_bsC, FastDiv divCW,
-                                                           float *__restrict__ C2, long c2_sC, long c2_bsC, int c2_pitch,
-                                                           const unsigned side_first_block, const WeightJob side,
-                                                           const unsigned j_store,
-                                                           const float *__restrict__ bias_col) {
-    // workgroups behind the reduction's carry a job of the next layer's (side_jobs.h)
-    if (blockIdx.x >= side_first_block) {
-        reorder_weight(side, (blockIdx.x - side_first_block) * 256u + threadIdx.x);
+__device__ __forceinline__ void split_reduce(const ReduceJob &j, unsigned block) {
+    if (block >= j.side_first_block) {
+        reorder_weight(j.side, (block - j.side_first_block) * 256u + threadIdx.x);
         return;
     }
-    if (rs.out && blockIdx.x >= rs.first_block) {
-        rowsum_reduce(rs, blockIdx.x - rs.first_block);
+    if (j.rs.out && block >= j.rs.first_block) {
+        rowsum_reduce(j.rs, block - j.rs.first_block);
         return;
     }
     // With `quarters` the four wavefronts of a workgroup share 64 outputs, each adding a contiguous quarter of the
     // partial sums (for few outputs and many splits: one lane per output would leave the GPU idle behind a long
     // chain of loads); the quarters are then added in order.  Either way the order of the adds is fixed.
-    const unsigned total = (unsigned)M * (unsigned)J;
+    const unsigned total = (unsigned)j.M * (unsigned)j.J;
     const unsigned wave = threadIdx.x >> 6;
-    unsigned idx = quarters ? blockIdx.x * 64u + (threadIdx.x & 63u) : blockIdx.x * blockDim.x + threadIdx.x;
+    unsigned idx = quarters ? block * 64u + (threadIdx.x & 63u) : block * 256u + threadIdx.x;
     const bool valid = idx < total;
     if (!quarters && !valid) return;
-    const int per = quarters ? (nsplit + 3) / 4 : nsplit;
+    const int per = quarters ? (j.nsplit + 3) / 4 : j.nsplit;
     const int s_begin = quarters ? (int)wave * per : 0;
-    const int s_end = s_begin + per < nsplit ? s_begin + per : nsplit;
+    const int s_end = s_begin + per < j.nsplit ? s_begin + per : j.nsplit;
     // Eight partials are requested before the first is added; the adds stay in split order.
     float sum = 0.0f;
-    const float *src = ws + (valid ? idx : 0);
+    const float *src = j.ws + (valid ? idx : 0);
     for (int s0 = s_begin; s0 < s_end; s0 += 8) {
         float v[8];
 #pragma unroll
@@ -89,27 +105,43 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const RowSumJob rs, c
         if (wave != 0 || !valid) return;
         sum = ((part[0][threadIdx.x] + part[1][threadIdx.x]) + part[2][threadIdx.x]) + part[3][threadIdx.x];
     }
-    unsigned i, j;
-    divJ.divmod(idx, i, j);
-    if (j >= j_store) return;  // a scratch column of a product run wider than its result (GemmProblem::j_store)
-    long coff = j, moff = j, toff = 0;
-    if (N != J || c_pitch || mask_pitch || C2) {
+    unsigned row, col;
+    j.divJ.divmod(idx, row, col);
+    if (col >= j.j_store) return;  // a scratch column of a product run wider than its result (GemmProblem::j_store)
+    long coff = col, moff = col, toff = 0;
+    if (j.N != j.J || j.c_pitch || j.mask_pitch || j.C2) {
         unsigned im, n, y, x;
-        divN.divmod(j, im, n);
-        divCW.divmod(n, y, x);
-        coff = (long)im * bsC + (c_pitch ? (long)y * c_pitch + x : (long)n);
-        moff = (long)im * mask_bsC + (mask_pitch ? (long)y * mask_pitch + x : (long)n);
-        toff = (long)im * c2_bsC + (long)y * c2_pitch + x;
+        j.divN.divmod(col, im, n);
+        j.divCW.divmod(n, y, x);
+        coff = (long)im * j.bsC + (j.c_pitch ? (long)y * j.c_pitch + x : (long)n);
+        moff = (long)im * j.mask_bsC + (j.mask_pitch ? (long)y * j.mask_pitch + x : (long)n);
+        toff = (long)im * j.c2_bsC + (long)y * j.c2_pitch + x;
     }
-    float *c = C + (long)i * sC + coff;
-    float val = alpha * sum;
-    if (bias) val += bias[i];
-    if (bias_col) val += bias_col[j];
-    if (beta != 0.0f) val += beta * *c;
-    if (act) val = val > act_threshold ? val : act_value;
-    if (mask) val = mask[(long)i * mask_sC + moff] > mask_threshold ? val : 0.0f;
+    float *c = j.C + (long)row * j.sC + coff;
+    float val = j.alpha * sum;
+    if (j.bias) val += j.bias[row];
+    if (j.bias_col) val += j.bias_col[col];
+    if (j.beta != 0.0f) val += j.beta * *c;
+    if (j.act) val = val > j.act_threshold ? val : j.act_value;
+    if (j.mask) val = j.mask[(long)row * j.mask_sC + moff] > j.mask_threshold ? val : 0.0f;
     *c = val;
-    if (C2) C2[(long)i * c2_sC + toff] = val;  // the second copy (GemmProblem::C2)
+    if (j.C2) j.C2[(long)row * j.c2_sC + toff] = val;  // the second copy (GemmProblem::C2)
+}
+
+template <bool quarters>
+__global__ __launch_bounds__(256) void split_reduce_kernel(const ReduceJob j) {
+    split_reduce<quarters>(j, blockIdx.x);
+}
+
+// Two products' reductions in one launch.
+__global__ __launch_bounds__(256) void split_reduce_pair_kernel(const ReduceJob a, const ReduceJob b) {
+    if (blockIdx.x < a.blocks) {
+        if (a.quarters) split_reduce<true>(a, blockIdx.x);
+        else split_reduce<false>(a, blockIdx.x);
+    } else {
+        if (b.quarters) split_reduce<true>(b, blockIdx.x - a.blocks);
+        else split_reduce<false>(b, blockIdx.x - a.blocks);
+    }
 }
 
 struct TileCfg {
@@ -152,7 +184,7 @@ const TileCfg kCfgs[] = {
     {"64x128", 64, 128, 4, {0.33, 0.33, 0.33, 0.33, 0.34, 0.33}, gemm_fast_64x128, kOcc4, 128, false},
     {"96x128", 96, 128, 3, {0.35, 0, 0.35, 0, 0.37, 0.35}, gemm_fast_96x128, kOcc3, 128, true},
     {"32x128", 32, 128, 4, {0.22, 0, 0.22, 0, 0.22, 0.25}, gemm_fast_32x128, kOcc4, 33, true},
-    {"64x64k4", 64, 64, 1, {0.29, 0.29, 0.29, 0.29, 0.30, 0.25}, gemm_fast_64x64k4, kOcc1, 0, false, 4},
+    {"64x64k4", 64, 64, 1, {0.25, 0.25, 0.25, 0.25, 0.26, 0.27}, gemm_fast_64x64k4, kOcc1, 0, false, 4},
 };
 
 inline long cdiv(long a, long b) { return (a + b - 1) / b; }
@@ -324,10 +356,19 @@ double gemm_estimate_us(const GemmProblem &p) {
     return 4.0 + (compute > store ? compute : store);
 }
 
-int gemm_launch(const GemmProblem &p) {
-    hipStream_t s = stream();
-    if (!s) return 1;
-    if (p.M <= 0 || p.J <= 0) return 0;
+namespace {
+
+// A product on its way: what its launches need besides the workspace.
+struct Prepared {
+    const GemmProblem *p;
+    GemmArgs g;
+    const TileCfg *best;  // nullptr: the generic kernel
+    int la, lb;
+    bool red, rowsum;
+    size_t ws_floats, rowsum_floats;  // of partial sums and partial row sums together, of the latter
+};
+
+int gemm_prepare(const GemmProblem &p, Prepared &out) {
     if ((long)p.M * p.J >= (1L << 31)) return fail("gemm: output of %d x %d exceeds 32-bit tile indexing", p.M, p.J);
 
     // (one image's gradWeight runs as a reduction batch of one where it wants the row sums of A)
@@ -336,7 +377,7 @@ int gemm_launch(const GemmProblem &p) {
     if (gather && (!p.coltab || p.b_rc || !p.a_rc)) return fail("gemm: a gathered B needs both tables and an r-contiguous A");
     if (red && !(p.a_rc && (p.b_rc || gather))) return fail("gemm: reduction batching needs r-contiguous operands");
 
-    GemmArgs g;
+    GemmArgs &g = out.g;
     std::memset(&g, 0, sizeof(g));
     g.A = p.A;
     g.B = p.B;
@@ -440,23 +481,14 @@ int gemm_launch(const GemmProblem &p) {
     // (An unsplit product of few rows leaves them to their own launch, which reads as little and needs no scratch.)
     const bool rowsum = p.rowsum && best && red && !p.ws_fixed && (g.nsplit > 1 || p.M >= 64);
     if (p.rowsum_done) *p.rowsum_done = rowsum;
-    const size_t rowsum_floats = rowsum ? (size_t)g.nsplit * g.tilesJ * p.M : 0;
-    if (g.nsplit > 1 || rowsum) {
-        const size_t need = (g.nsplit > 1 ? (size_t)g.nsplit * p.M * p.J : 0) + rowsum_floats;
-        if (p.ws_fixed) {
-            if ((long)need > p.ws_fixed_floats)
-                return fail("gemm: %zu floats of partial sums exceed the fixed workspace of %ld", need, p.ws_fixed_floats);
-            g.ws = p.ws_fixed;
-        } else {
-            g.ws = workspace(sizeof(float) * need);
-        }
-        if (!g.ws) return 1;
-        if (rowsum) g.rowsum_ws = g.ws + (need - rowsum_floats);
-    }
+    out.rowsum_floats = rowsum ? (size_t)g.nsplit * g.tilesJ * p.M : 0;
+    out.ws_floats = (g.nsplit > 1 ? (size_t)g.nsplit * p.M * p.J : 0) + out.rowsum_floats;
+    if (p.ws_fixed && (long)out.ws_floats > p.ws_fixed_floats)
+        return fail("gemm: %zu floats of partial sums exceed the fixed workspace of %ld", out.ws_floats, p.ws_fixed_floats);
 
     // ---- loaders: r-contiguous operands use 128-bit loads (4-byte alignment suffices) --------
-    const int la = p.a_rc ? LD_RC_VEC : LD_XC_SCALAR;
-    const int lb = p.b_rc ? LD_RC_VEC
+    out.la = p.a_rc ? LD_RC_VEC : LD_XC_SCALAR;
+    out.lb = p.b_rc ? LD_RC_VEC
                    : !gather ? LD_XC_SCALAR
                    : !red ? LD_XC_GATHER
                    : p.row_quads ? LD_RC_GATHER_VEC
@@ -466,57 +498,158 @@ int gemm_launch(const GemmProblem &p) {
     if (p.j_store > 0 && (!best || g.nsplit < 2))
         return fail("gemm: scratch columns need a tiled kernel and a split reduction");
 
+    out.p = &p;
+    out.best = best;
+    out.red = red;
+    out.rowsum = rowsum;
+    return 0;
+}
+
+void use_workspace(Prepared &q, float *ws) {
+    q.g.ws = ws;
+    if (q.rowsum) q.g.rowsum_ws = ws + (q.ws_floats - q.rowsum_floats);
+}
+
+const char *product_label(const Prepared &q) {
+    const GemmProblem &p = *q.p;
+    return !prof_enabled() ? p.tag
+                           : prof_label("%s M=%d J=%d R=%ld tile=%s split=%d", p.tag, p.M, p.J,
+                                        (long)p.R * (q.red ? p.nb : 1), q.best ? q.best->name : "generic", q.g.nsplit);
+}
+
+int run_product(const Prepared &q, hipStream_t s) {
+    const GemmProblem &p = *q.p;
     int rc;
     {
-        const char *label = p.tag;
-        if (prof_enabled())
-            label = prof_label("%s M=%d J=%d R=%ld tile=%s split=%d", p.tag, p.M, p.J, (long)p.R * (red ? p.nb : 1),
-                               best ? best->name : "generic", g.nsplit);
-        LaunchScope scope(label, p.flops > 0 ? p.flops : 2.0 * p.M * p.J * (double)p.R * (red ? p.nb : 1), 0.0);
-        rc = best ? best->launch(g, la, lb, red, s) : gemm_generic_64x64(g, p.a_rc, p.b_rc, red, s);
+        LaunchScope scope(product_label(q), p.flops > 0 ? p.flops : 2.0 * p.M * p.J * (double)p.R * (q.red ? p.nb : 1), 0.0);
+        rc = q.best ? q.best->launch(q.g, q.la, q.lb, q.red, s) : gemm_generic_64x64(q.g, p.a_rc, p.b_rc, q.red, s);
     }
-    if (rc) return rc;
-    if (check_launch(p.tag)) return 1;
-    if (g.nsplit > 1 || rowsum) {
-        const long n = g.nsplit > 1 ? (long)p.M * p.J : 0;  // an unsplit product has stored its own result
-        RowSumJob rs;
-        std::memset(&rs, 0, sizeof(rs));
-        // few outputs, many splits: four wavefronts per 64 outputs.  From 4 K to 123 K outputs the launch alone takes the same
-        // either way up to 16 splits, 0.2 us less at 24, 0.5 at 32 and 2.4 at 64; behind its product (256 x 169 outputs in 27
-        // parts and two more like it, 3x3 layers of one 13x13 image) 12 as the line gave 53.1 -> 50.8 us a pass against 32.
-        const int quarters = (n > 0 && n < 128 * 1024 && g.nsplit >= 12) ? 1 : 0;
-        unsigned blocks = (unsigned)cdiv(n, quarters ? 64 : 256);
-        if (rowsum) {
-            rs.ws = g.rowsum_ws;
-            rs.out = p.rowsum;
-            rs.M = p.M;
-            rs.slots = (int)(g.nsplit * g.tilesJ);
-            rs.alpha = p.alpha;
-            rs.first_block = blocks;
-            blocks += (unsigned)cdiv(p.M, 4);
-        }
-        // A product that stores a second copy of its result for the next layer's gradInput product also carries that
-        // layer's pending kernel-bank job, if there is one.
-        WeightJob side = {};
-        const unsigned side_first = blocks;
-        double side_bytes = 0.0;
-        if (g.C2 && n > 0 && take_bank_job(side)) {
-            blocks += (side.count + 255u) / 256u;
-            side_bytes = 4.0 * (side.count + (double)side.M * side.C * side.kH * side.kW);
-        }
-        {
-            LaunchScope scope("gemm_split_reduce", 0.0,
-                              4.0 * n * (g.nsplit + 2 + (g.C2 ? 1 : 0)) + 4.0 * rowsum_floats + side_bytes);
-            auto kernel = quarters ? split_reduce_kernel<true> : split_reduce_kernel<false>;
-            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, rs, g.ws, p.C, p.bias,
-                               p.M, p.J, g.N, p.sC, p.bsC, FastDiv((uint32_t)p.J), g.divN, g.nsplit, p.alpha,
-                               p.beta, g.act, g.act_threshold, g.act_value, g.mask, g.mask_threshold, g.c_pitch,
-                               g.mask_pitch, g.mask_sC, g.mask_bsC, g.divCW, g.C2, g.c2_sC, g.c2_bsC, g.c2_pitch,
-                               side_first, side, (unsigned)(p.j_store > 0 ? p.j_store : p.J), p.bias_col);
-        }
-        if (check_launch("gemm_split_reduce")) return 1;
+    return rc ? rc : check_launch(p.tag);
+}
+
+// The reduction behind a product that was split or sums rows on the side; returns its bytes for the timing.
+double reduce_job(const Prepared &q, ReduceJob &job) {
+    const GemmProblem &p = *q.p;
+    const GemmArgs &g = q.g;
+    std::memset(static_cast<void *>(&job), 0, sizeof(job));
+    const long n = g.nsplit > 1 ? (long)p.M * p.J : 0;  // an unsplit product has stored its own result
+    // few outputs, many splits: four wavefronts per 64 outputs.  From 4 K to 123 K outputs the launch alone takes the same
+    // either way up to 16 splits, 0.2 us less at 24, 0.5 at 32 and 2.4 at 64; behind its product (256 x 169 outputs in 27
+    // parts and two more like it, 3x3 layers of one 13x13 image) 12 as the line gave 53.1 -> 50.8 us a pass against 32.
+    job.quarters = n > 0 && n < 128 * 1024 && g.nsplit >= 12;
+    job.blocks = (unsigned)cdiv(n, job.quarters ? 64 : 256);
+    if (q.rowsum) {
+        job.rs.ws = g.rowsum_ws;
+        job.rs.out = p.rowsum;
+        job.rs.M = p.M;
+        job.rs.slots = (int)(g.nsplit * g.tilesJ);
+        job.rs.alpha = p.alpha;
+        job.rs.first_block = job.blocks;
+        job.blocks += (unsigned)cdiv(p.M, 4);
     }
-    return 0;
+    // A product that stores a second copy of its result for the next layer's gradInput product also carries that
+    // layer's pending kernel-bank job, if there is one.
+    job.side_first_block = job.blocks;
+    double side_bytes = 0.0;
+    if (g.C2 && n > 0 && take_bank_job(job.side)) {
+        job.blocks += (job.side.count + 255u) / 256u;
+        side_bytes = 4.0 * (job.side.count + (double)job.side.M * job.side.C * job.side.kH * job.side.kW);
+    }
+    job.ws = g.ws;
+    job.C = p.C;
+    job.bias = p.bias;
+    job.bias_col = p.bias_col;
+    job.M = p.M;
+    job.J = p.J;
+    job.N = g.N;
+    job.sC = p.sC;
+    job.bsC = p.bsC;
+    job.divJ = FastDiv((uint32_t)p.J);
+    job.divN = g.divN;
+    job.divCW = g.divCW;
+    job.nsplit = g.nsplit;
+    job.alpha = p.alpha;
+    job.beta = p.beta;
+    job.act = g.act;
+    job.act_threshold = g.act_threshold;
+    job.act_value = g.act_value;
+    job.mask = g.mask;
+    job.mask_threshold = g.mask_threshold;
+    job.c_pitch = g.c_pitch;
+    job.mask_pitch = g.mask_pitch;
+    job.mask_sC = g.mask_sC;
+    job.mask_bsC = g.mask_bsC;
+    job.C2 = g.C2;
+    job.c2_sC = g.c2_sC;
+    job.c2_bsC = g.c2_bsC;
+    job.c2_pitch = g.c2_pitch;
+    job.j_store = (unsigned)(p.j_store > 0 ? p.j_store : p.J);
+    return 4.0 * n * (g.nsplit + 2 + (g.C2 ? 1 : 0)) + 4.0 * q.rowsum_floats + side_bytes;
+}
+
+int run_reduce(const ReduceJob &job, double bytes, hipStream_t s) {
+    {
+        LaunchScope scope("gemm_split_reduce", 0.0, bytes);
+        auto kernel = job.quarters ? split_reduce_kernel<true> : split_reduce_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3(job.blocks), dim3(256), 0, s, job);
+    }
+    return check_launch("gemm_split_reduce");
+}
+
+}  // namespace
+
+int gemm_launch(const GemmProblem &p) {
+    hipStream_t s = stream();
+    if (!s) return 1;
+    if (p.M <= 0 || p.J <= 0) return 0;
+    Prepared q;
+    if (gemm_prepare(p, q)) return 1;
+    if (q.ws_floats > 0) {
+        float *ws = p.ws_fixed ? p.ws_fixed : workspace(sizeof(float) * q.ws_floats);
+        if (!ws) return 1;
+        use_workspace(q, ws);
+    }
+    if (run_product(q, s)) return 1;
+    if (q.ws_floats == 0) return 0;
+    ReduceJob job;
+    const double bytes = reduce_job(q, job);
+    return run_reduce(job, bytes, s);
+}
+
+// Two products of which neither reads what the other writes.  Their split reductions share a launch, and where both are
+// small enough for the tile of four groups, so do they themselves (unless every launch is being timed, to keep a record of
+// each): a launch is 3 us to enqueue and 3 to 5 for the GPU to run and change over, as long as such a product takes.
+int gemm_launch_pair(const GemmProblem &a, const GemmProblem &b) {
+    hipStream_t s = stream();
+    if (!s) return 1;
+    if (a.M <= 0 || a.J <= 0 || b.M <= 0 || b.J <= 0 || a.ws_fixed || b.ws_fixed) return gemm_launch(a) || gemm_launch(b) ? 1 : 0;
+    Prepared qa, qb;
+    if (gemm_prepare(a, qa) || gemm_prepare(b, qb)) return 1;
+    const size_t first = (qa.ws_floats + 63) / 64 * 64;
+    if (first + qb.ws_floats > 0) {
+        float *ws = workspace(sizeof(float) * (first + qb.ws_floats));
+        if (!ws) return 1;
+        if (qa.ws_floats > 0) use_workspace(qa, ws);
+        if (qb.ws_floats > 0) use_workspace(qb, ws + first);
+    }
+    if (!prof_enabled() && qa.best && qb.best && qa.best->groups > 1 && qb.best->groups > 1 &&
+        gemm_fast_64x64k4_pair(qa.g, qa.la, qa.lb, qa.red, qb.g, qb.la, qb.lb, qb.red, s) == 0) {
+        if (check_launch(a.tag)) return 1;
+    } else if (run_product(qa, s) || run_product(qb, s)) {
+        return 1;
+    }
+    if (qa.ws_floats == 0 && qb.ws_floats == 0) return 0;
+    ReduceJob ja, jb;
+    double bytes = 0;
+    if (qa.ws_floats > 0) bytes += reduce_job(qa, ja);
+    if (qb.ws_floats > 0) bytes += reduce_job(qb, jb);
+    if (qb.ws_floats == 0) return run_reduce(ja, bytes, s);
+    if (qa.ws_floats == 0) return run_reduce(jb, bytes, s);
+    {
+        LaunchScope scope("gemm_split_reduce", 0.0, bytes);
+        hipLaunchKernelGGL(split_reduce_pair_kernel, dim3(ja.blocks + jb.blocks), dim3(256), 0, s, ja, jb);
+    }
+    return check_launch("gemm_split_reduce");
 }
 
 }  // namespace thgpu

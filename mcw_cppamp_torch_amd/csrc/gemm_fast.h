@@ -223,9 +223,9 @@ __device__ __forceinline__ void finish_groups(const GemmArgs &g, char *lds_a, ch
     }
 }
 
+// One workgroup of a product; As and Bs hold KG pairs of operand tiles.
 template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG>
-__global__ __launch_bounds__(WGM *WGN * 64 * KG)
-    __attribute__((amdgpu_waves_per_eu(KG > 1 ? KG : gemm_min_waves<BM, BN, WGM, WGN>()))) void gemm_fast_kernel(const GemmArgs g) {
+__device__ __forceinline__ void gemm_fast_tile(const GemmArgs &g, const unsigned block, char *const As, char *const Bs) {
     constexpr int NT = WGM * WGN * 64;  // threads of a group: the whole workgroup unless KG > 1
     constexpr int BK = GEMM_BK;
     constexpr int TM = BM / WGM / 32, TN = BN / WGN / 32;
@@ -256,9 +256,6 @@ __global__ __launch_bounds__(WGM *WGN * 64 * KG)
 
     using TileA = PartTile<BM>;
     using TileB = PartTile<BN>;
-    __shared__ __attribute__((aligned(16))) char As[KG][2][TileA::kBytes];
-    __shared__ __attribute__((aligned(16))) char Bs[KG][2][TileB::kBytes];
-
     const int group = KG > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT) : 0;
     const int tid = KG > 1 ? threadIdx.x % NT : threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: row bases stay uniform
@@ -266,7 +263,7 @@ __global__ __launch_bounds__(WGM *WGN * 64 * KG)
     const int half = lane >> 5, l32 = lane & 31;
 
     // ---- which tile, which part of the reduction --------------------------------
-    unsigned pid = xcd_remap(blockIdx.x, g.total);
+    unsigned pid = xcd_remap(block, g.total);
     unsigned ti, tj, split, rest;
     g.divTilesM.divmod(pid, rest, ti);
     g.divTilesJ.divmod(rest, split, tj);
@@ -496,8 +493,8 @@ __global__ __launch_bounds__(WGM *WGN * 64 * KG)
     // where the loader gives a thread whole octets, otherwise four.
     constexpr int GA = (KA == LD_XC_SCALAR && NA % 8 == 0) ? 8 : 4;
     constexpr int GB = ((LB == LD_XC_SCALAR || LB == LD_XC_GATHER) && NB % 8 == 0) ? 8 : 4;
-    char *const a_dst = &As[group][0][0] + (a_r >> 3) * TileA::kOctet + a_x * 16 + (a_r & 7) * 2;
-    char *const b_dst = &Bs[group][0][0] + (b_r >> 3) * TileB::kOctet + b_x * 16 + (b_r & 7) * 2;
+    char *const a_dst = As + group * (2 * TileA::kBytes) + (a_r >> 3) * TileA::kOctet + a_x * 16 + (a_r & 7) * 2;
+    char *const b_dst = Bs + group * (2 * TileB::kBytes) + (b_r >> 3) * TileB::kOctet + b_x * 16 + (b_r & 7) * 2;
     unsigned lost = 0;  // see split_pair
     const unsigned odd_column = (unsigned)(b_x & 1) << 31;  // the sign of a thread's elements of the second operand
     auto stash_group = [&](auto kind_tag, auto group_tag, auto tile_tag, char *dst, const float *src, int q, auto sign) {
@@ -585,8 +582,8 @@ __global__ __launch_bounds__(WGM *WGN * 64 * KG)
     // ---- main loop ----------------------------------------------------------------------
     // Step s multiplies from LDS buffer s&1, block by block; between the MFMAs the groups of
     // step s+1 are split and written to the other buffer and their registers refilled for step s+2.
-    const char *const a_src = &As[group][0][0] + half * TileA::kOctet + (wm * (TM * 32) + l32) * 16;
-    const char *const b_src = &Bs[group][0][0] + half * TileB::kOctet + (wn * (TN * 32) + l32) * 16;
+    const char *const a_src = As + group * (2 * TileA::kBytes) + half * TileA::kOctet + (wm * (TM * 32) + l32) * 16;
+    const char *const b_src = Bs + group * (2 * TileB::kBytes) + half * TileB::kOctet + (wn * (TN * 32) + l32) * 16;
     // Two sums in turn, so that the additions of one block run under the MFMAs of the next, where the registers hold both
     // (1 to 2 % on the 8-block tiles), and the parts of the longer side one block row ahead likewise.
     constexpr bool PING = !(TM == 2 && TN == 2 && WGN == 2) && !(TM * TN == 8 && LB == LD_RC_GATHER);
@@ -701,7 +698,7 @@ __global__ __launch_bounds__(WGM *WGN * 64 * KG)
 
     // ---- what the split could not hold -----------------------------------------------------
     // Did any thread's element lose bits?  (The operand tiles in LDS have been read: the loop ends with a barrier.)
-    unsigned *const lost_of = reinterpret_cast<unsigned *>(&As[0][0][0]);
+    unsigned *const lost_of = reinterpret_cast<unsigned *>(As);
     const bool lost_here = __builtin_amdgcn_ballot_w64((lost & 0xffffu) != 0) != 0;
     if (lane == 0) lost_of[group * (NT / 64) + wave] = lost_here ? 1u : 0u;
     __syncthreads();
@@ -798,7 +795,7 @@ __global__ __launch_bounds__(WGM *WGN * 64 * KG)
 
     // ---- groups ------------------------------------------------------------------------
     if constexpr (KG > 1) {
-        finish_groups<BM, BN, WGN, RED, KG>(g, &As[0][0][0], &Bs[0][0][0], acc[0][0], bsum[0], rs_on, group, wave, lane, tj, split, i0, j0, own_i0, own_j0);
+        finish_groups<BM, BN, WGN, RED, KG>(g, As, Bs, acc[0][0], bsum[0], rs_on, group, wave, lane, tj, split, i0, j0, own_i0, own_j0);
         return;
     }
 
@@ -987,6 +984,23 @@ __global__ __launch_bounds__(WGM *WGN * 64 * KG)
         if (edge_tile) write_out(integral_constant<int, 2>{}, integral_constant<bool, true>{});
         else write_out(integral_constant<int, 2>{}, integral_constant<bool, false>{});
     }
+}
+
+template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG>
+__global__ __launch_bounds__(WGM *WGN * 64 * KG)
+    __attribute__((amdgpu_waves_per_eu(KG > 1 ? KG : gemm_min_waves<BM, BN, WGM, WGN>()))) void gemm_fast_kernel(const GemmArgs g) {
+    __shared__ __attribute__((aligned(16))) char As[KG * 2 * PartTile<BM>::kBytes];
+    __shared__ __attribute__((aligned(16))) char Bs[KG * 2 * PartTile<BN>::kBytes];
+    gemm_fast_tile<BM, BN, WGM, WGN, LA, LB, RED, KG>(g, blockIdx.x, As, Bs);
+}
+
+// The workgroups of two products on the 64 x 64 tile of four groups, one after the other's.
+template <int LA, int LB, bool RED, int LA2, int LB2, bool RED2>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void gemm_pair_kernel(const GemmArgs a, const GemmArgs b) {
+    __shared__ __attribute__((aligned(16))) char As[4 * 2 * PartTile<64>::kBytes];
+    __shared__ __attribute__((aligned(16))) char Bs[4 * 2 * PartTile<64>::kBytes];
+    if (blockIdx.x < a.total) gemm_fast_tile<64, 64, 2, 2, LA, LB, RED, 4>(a, blockIdx.x, As, Bs);
+    else gemm_fast_tile<64, 64, 2, 2, LA2, LB2, RED2, 4>(b, blockIdx.x - a.total, As, Bs);
 }
 
 template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG = 1>

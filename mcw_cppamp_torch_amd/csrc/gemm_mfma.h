@@ -102,6 +102,8 @@ struct GemmProblem {
 
 // Enqueues the GEMM on the library stream.  Returns 0 or a recorded error.
 int gemm_launch(const GemmProblem &p);
+// Two products, neither of which reads what the other writes, in fewer launches.
+int gemm_launch_pair(const GemmProblem &a, const GemmProblem &b);
 // Whether one of the tiled kernels takes the problem (shape at least a tile, operand and output offsets
 // within the kernels' 32-bit addressing, a tile the tuning switches allow): the test a gathered second
 // operand, which has no generic kernel, must pass before it is launched.
@@ -184,6 +186,10 @@ int gemm_fast_192x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s
 int gemm_fast_128x256(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_256x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x64k4(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
+// A convolution's gradInput product (a) and its gradWeight product (b) in one launch; non-zero, and nothing launched, for
+// other loaders.
+int gemm_fast_64x64k4_pair(const GemmArgs &a, int la, int lb, bool red, const GemmArgs &b, int la2, int lb2, bool red2,
+                           hipStream_t s);
 int gemm_fast_64x64(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x256(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);

@@ -97,6 +97,13 @@ int conv_implicit_gradinput(const float *gradOutput, const float *weight, float 
                             int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW,
                             InputMask mask = InputMask(), bool q_ready = false, TwinOutput twin = TwinOutput(),
                             bool *wrote_twin = nullptr);
+// Both backward passes of a layer whose gradInput and gradWeight products gather, in fewer launches than one after the other.
+// `padded` is the input's padded image, or null and pad_into the buffer that it is to be made in.  No written buffer may be
+// one of the others.
+int conv_implicit_backward(const float *input, const float *padded, float *pad_into, const float *gradOutput, const float *weight,
+                           float *scratch, float *gradInput, float *gradWeight, float *gradBias, long B, int C, int H, int W,
+                           int M, int kH, int kW, int pH, int pW, int sH, int sW, InputMask mask, bool q_ready, TwinOutput twin,
+                           bool *wrote_twin, float scale, bool *bias_done);
 // Where gradOutput [B, M, Ho, Wo] lies inside the padded buffer the gathered gradInput product reads (the head of its
 // scratch): planes of Hq x Wq, the dense plane at row `top`, column `left`, zeros around it.
 void conv_implicit_q_layout(int C, int H, int W, int kH, int kW, int pH, int pW, int sH, int sW, int *top, int *left,

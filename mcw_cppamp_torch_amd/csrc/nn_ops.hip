@@ -476,6 +476,83 @@ int conv_acc_grad_parameters(THGPUTensor *input, THGPUTensor *gradOutput, THGPUT
     return bias_done ? 0 : gradbias_launch(dptr(go), dptr(gradBias), s.B, s.M, s.N, scale);
 }
 
+// updateGradInput and then accGradParameters.  Where both gather, every tensor is dense (input: or lies in its padded buffer)
+// and no buffer that one writes is one that the other reads, their preparations, split reductions and, if small, products
+// share launches; everything else, errors included, is one pass after the other.
+int conv_backward(THGPUTensor *input, THGPUTensor *gradOutput, THGPUTensor *weight, THGPUTensor *gradWeight,
+                  THGPUTensor *gradBias, THGPUTensor *finput, THGPUTensor *fgradInput, THGPUTensor *gradInput, int kW, int kH,
+                  int dW, int dH, int padW, int padH, float scale, bool mask_on, float mask_threshold,
+                  bool input_in_padded_buffer, bool twin_ready, THGPUTensor *twin, int *wrote_twin) {
+    auto one_by_one = [&]() {
+        return conv_update_grad_input(input, gradOutput, weight, finput, fgradInput, gradInput, kW, kH, dW, dH, padW, padH, mask_on,
+                                      mask_threshold, twin_ready, twin, wrote_twin) ||
+                       conv_acc_grad_parameters(input, gradOutput, gradWeight, gradBias, finput, fgradInput, kW, kH, dW, dH, padW,
+                                                padH, scale, input_in_padded_buffer)
+                   ? 1
+                   : 0;
+    };
+    if (wrote_twin) *wrote_twin = 0;
+    ConvShape s;
+    if (!gradOutput || !gradWeight || !gradBias || !finput || !fgradInput || !gradInput ||
+        conv_shape(s, input, weight, kW, kH, dW, dH, padW, padH))
+        return one_by_one();
+    PlaneLayout in_layout;
+    const bool direct = input_in_padded_buffer && interior_of_padded(input, s, padH, padW, in_layout);
+    auto owned = [](const THGPUTensor *t) { return (const void *)t->storage; };
+    const bool dense = (direct || tensor_ready(input, s.B * (long)s.C * s.H * s.W)) && !check_grad_output(s, gradOutput) &&
+                       tensor_ready(gradOutput, s.B * s.M * s.N) && tensor_ready(weight, (long)s.M * s.K) &&
+                       tensor_ready(gradWeight, (long)s.M * s.K) && gradWeight->nDimension == 2 && gradWeight->size[1] == s.K &&
+                       tensor_ready(gradBias, s.M) && direct == input_in_padded_buffer;
+    // the first five are written, all but gradWeight and gradBias are read
+    const THGPUTensor *const roles[] = {gradInput, finput, fgradInput, gradWeight, gradBias, input, gradOutput};
+    bool apart = true;  // (a tensor without a storage is about to get one of its own)
+    for (int w = 0; w < 5; ++w)
+        for (int r = 0; r < 7; ++r)
+            if (r != w && r != 3 && r != 4 &&
+                (roles[r] == roles[w] || (owned(roles[w]) && owned(roles[w]) == owned(roles[r]))))
+                apart = false;
+    if (twin && owned(twin) && (owned(twin) == owned(input) || owned(twin) == owned(finput) || owned(twin) == owned(fgradInput) ||
+                                owned(twin) == owned(gradWeight) || owned(twin) == owned(gradBias)))
+        apart = false;
+    if (!dense || !apart || g_finput_reuse || owned(weight) == owned(gradWeight) || owned(weight) == owned(gradBias) ||
+        !conv_use_gathered(s.B, s.C, s.H, s.W, s.M, kH, kW, padH, padW, dH, dW) ||
+        !conv_use_gathered_gradinput(s.B, s.C, s.H, s.W, s.M, kH, kW, padH, padW, dH, dW))
+        return one_by_one();
+
+    InputMask mask;
+    if (mask_on) {
+        PlaneLayout mask_layout;
+        if (!plane_layout(input, mask_layout) || !((dH == 1 && dW == 1) || mask_layout.dense)) return one_by_one();
+        mask.in = dptr(input);
+        mask.threshold = mask_threshold;
+        mask.plane = mask_layout.plane;
+        mask.pitch = mask_layout.dense ? 0 : (int)mask_layout.pitch;
+    }
+    const long need = conv_implicit_gradinput_scratch(s.B, s.C, s.H, s.W, s.M, kH, kW, padH, padW, dH, dW);
+    const TwinGeom tg = twin_geom(s, kH, kW, padH, padW, dH, dW);
+    const bool q_ready = twin_ready && tensor_ready(fgradInput, need) && zero_bordered(dptr(fgradInput), tg);
+    if (s.batched)
+        THGPUTensor_resize4d(gradInput, s.B, s.C, s.H, s.W);
+    else
+        THGPUTensor_resize3d(gradInput, s.C, s.H, s.W);
+    THGPUTensor_resize1d(fgradInput, need);
+    if (!tensor_ready(fgradInput, need) || !tensor_ready(gradInput, s.B * (long)s.C * s.H * s.W))
+        return fail("SpatialConvolutionMM: could not size gradInput/fgradInput");
+    if (!direct && size_padded(finput, s, padH, padW)) return 1;
+    TwinOutput second;
+    if (twin && !twin_output(twin, gradInput, second)) second = TwinOutput();
+    bool wrote = false, bias_done = false;
+    const float *padded = direct ? dptr(input) - ((long)padH * in_layout.pitch + padW) : nullptr;
+    if (conv_implicit_backward(dptr(input), padded, direct ? nullptr : dptr(finput), dptr(gradOutput), dptr(weight),
+                               dptr(fgradInput), dptr(gradInput), dptr(gradWeight),
+                               tuning().gradbias_separate ? nullptr : dptr(gradBias), s.B, s.C, s.H, s.W, s.M, kH, kW, padH, padW,
+                               dH, dW, mask, q_ready, second, &wrote, scale, &bias_done))
+        return 1;
+    g_zero_bordered[dptr(fgradInput)] = tg;  // the padded region now holds this gradOutput between zero borders
+    if (wrote_twin) *wrote_twin = wrote ? 1 : 0;
+    return bias_done ? 0 : gradbias_launch(dptr(gradOutput), dptr(gradBias), s.B, s.M, s.N, scale);
+}
+
 }  // namespace
 
 namespace thgpu {
@@ -582,6 +659,18 @@ int thgpu_SpatialConvolutionMM_accGradParametersFused(THGPUTensor *input, THGPUT
     if (flags & ~THGPU_INPUT_IN_PADDED_BUFFER) return fail("SpatialConvolutionMM: unknown flags");
     return conv_acc_grad_parameters(input, gradOutput, gradWeight, gradBias, finput, fgradInput, kW, kH, dW, dH, padW,
                                     padH, scale, (flags & THGPU_INPUT_IN_PADDED_BUFFER) != 0);
+}
+
+int thgpu_SpatialConvolutionMM_backward(THGPUTensor *input, THGPUTensor *gradOutput, THGPUTensor *weight,
+                                        THGPUTensor *gradWeight, THGPUTensor *gradBias, THGPUTensor *finput,
+                                        THGPUTensor *fgradInput, THGPUTensor *gradInput, int kW, int kH, int dW, int dH,
+                                        int padW, int padH, float scale, int flags, float threshold, THGPUTensor *twin,
+                                        int *wrote_twin) {
+    if (flags & ~(THGPU_FUSE_INPUT_MASK | THGPU_INPUT_IN_PADDED_BUFFER | THGPU_GRADOUTPUT_IN_TWIN))
+        return fail("SpatialConvolutionMM: unknown flags");
+    return conv_backward(input, gradOutput, weight, gradWeight, gradBias, finput, fgradInput, gradInput, kW, kH, dW, dH, padW,
+                         padH, scale, (flags & THGPU_FUSE_INPUT_MASK) != 0, threshold,
+                         (flags & THGPU_INPUT_IN_PADDED_BUFFER) != 0, (flags & THGPU_GRADOUTPUT_IN_TWIN) != 0, twin, wrote_twin);
 }
 
 int thgpu_conv_gathers(long B, int C, int H, int W, int M, int kW, int kH, int dW, int dH, int padW, int padH) {

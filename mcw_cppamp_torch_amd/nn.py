@@ -506,6 +506,17 @@ class SpatialConvolutionMM(Module):
         self._wrote_twin = bool(wrote.value)
         return self.gradInput
 
+    def backward(self, input, gradOutput, scale=1):
+        # updateGradInput, then accGradParameters: in one call of the library where both are this class's own
+        if self.gradInput is None or not _own_passes(self):
+            return Module.backward(self, input, gradOutput, scale)
+        _require_gpu(input, gradOutput, self.weight, self.gradWeight, self.gradBias, self.finput, self.fgradInput, self.gradInput)
+        flags = (1 if self.inputThreshold is not None else 0) | (2 if _in_padded_buffer(input, self.padH, self.padW) else 0)
+        _lib.check_status(lib.thgpu_SpatialConvolutionMM_backward(
+            input._p, gradOutput._p, self.weight._p, self.gradWeight._p, self.gradBias._p, self.finput._p, self.fgradInput._p,
+            self.gradInput._p, *(self._geom() + (float(scale), flags, float(self.inputThreshold or 0.0), None, None))))
+        return self.gradInput
+
     def accGradParameters(self, input, gradOutput, scale=1):
         _require_gpu(input, gradOutput, self.gradWeight, self.gradBias, self.finput, self.fgradInput)
         if _in_padded_buffer(input, self.padH, self.padW):
@@ -516,6 +527,13 @@ class SpatialConvolutionMM(Module):
         _lib.check_status(lib.thgpu_SpatialConvolutionMM_accGradParameters(
             input._p, gradOutput._p, self.gradWeight._p, self.gradBias._p, self.finput._p, self.fgradInput._p,
             *(self._geom() + (float(scale),))))
+
+
+def _own_passes(conv):
+    """Whether updateGradInput and accGradParameters of a convolution are SpatialConvolutionMM's: neither overridden by its
+    class nor set on it."""
+    return all(getattr(getattr(conv, m), "__func__", None) is getattr(SpatialConvolutionMM, m)
+               for m in ("updateGradInput", "accGradParameters"))
 
 
 class Linear(Module):

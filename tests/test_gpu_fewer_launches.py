@@ -3,7 +3,7 @@ its product and its bias gradient as one sum, the one-launch bias gradient of sm
 import numpy as np
 import pytest
 
-from helpers import rng_for
+from helpers import rng_for, uniform
 
 pytestmark = pytest.mark.gpu
 
@@ -162,3 +162,88 @@ print("allocations", lib.thgpu_device_alloc_calls() - before)
     out = subprocess.run([sys.executable, "-c", code], cwd=root, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
                          timeout=100)
     assert out.stdout.splitlines()[-1:] == ["allocations 0"], out.stdout
+
+
+BACKWARD = {  # B, C, H, W, M, kH, kW, pH, pW, sH, sW
+    "one_image": (1, 96, 13, 13, 70, 3, 3, 1, 1, 1, 1),       # both products on the tile of four groups, both split
+    "quads": (2, 64, 8, 12, 64, 3, 3, 1, 1, 1, 1),
+    "few_rows": (3, 64, 10, 9, 20, 3, 3, 1, 1, 1, 1),
+    "no_padding": (2, 64, 9, 9, 64, 3, 3, 0, 0, 1, 1),
+    "strided": (2, 20, 17, 19, 66, 5, 5, 2, 2, 2, 2),
+    "wide": (16, 64, 28, 28, 192, 3, 3, 1, 1, 1, 1),
+    "columns": (2, 3, 12, 12, 64, 5, 5, 1, 1, 1, 1),          # gradInput of three planes goes through columns
+}
+
+
+@pytest.mark.parametrize("threshold", [None, 0.25])
+@pytest.mark.parametrize("name", sorted(BACKWARD))
+def test_backward_gives_what_its_two_passes_give(gt, name, threshold):
+    """One call of the library for both passes against one after the other, bit for bit, twice (buffers new and kept)."""
+    B, C, H, W, M, kH, kW, pH, pW, sH, sW = BACKWARD[name]
+    rng = rng_for(405)
+    made = []
+    for _ in range(2):
+        m = gt.nn.SpatialConvolutionMM(C, M, kW, kH, sW, sH, 0, padW=pW, padH=pH, rng=rng_for(406))
+        m.gradWeight[...] = 0.5
+        m.gradBias[...] = -0.5
+        m.inputThreshold = threshold
+        made.append(m.gpu())
+    for _ in range(2):
+        x = dev(gt, uniform(rng, (B, C, H, W)))
+        outs = []
+        for i, m in enumerate(made):
+            o = m.forward(x)
+            if i == 0:
+                go = dev(gt, uniform(rng, o.size()))
+                gi = m.backward(x, go, 0.75)
+            else:
+                gi = m.updateGradInput(x, go)
+                m.accGradParameters(x, go, 0.75)
+            outs.append([t.float() for t in (gi, m.gradWeight, m.gradBias)])
+        for a, b in zip(*outs):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+def test_backward_with_shared_or_strided_tensors(gt):
+    """What the shared launches cannot take runs one pass after the other: a transposed gradOutput, a gradInput in the memory
+    of the input, one buffer for finput and fgradInput, a class with its own updateGradInput."""
+    B, C, H, W, M = 1, 64, 10, 10, 64
+    rng = rng_for(407)
+    x, go = uniform(rng, (B, C, H, W)), uniform(rng, (B, M, H, W))
+
+    def module(cls=gt.nn.SpatialConvolutionMM):
+        m = cls(C, M, 3, 3, 1, 1, 1, rng=rng_for(408))
+        m.gradWeight[...] = 0
+        m.gradBias[...] = 0
+        return m.gpu()
+
+    def results(m, dx, dgo, call):
+        m.forward(dx)
+        call(m, dx, dgo)
+        return [t.float() for t in (m.gradInput, m.gradWeight, m.gradBias)]
+
+    def passes(m, dx, dgo):
+        m.updateGradInput(dx, dgo)
+        m.accGradParameters(dx, dgo, 1)
+
+    merged = lambda m, dx, dgo: m.backward(dx, dgo)
+    ref = results(module(), dev(gt, x), dev(gt, go), passes)
+    swapped = dev(gt, np.ascontiguousarray(go.transpose(0, 1, 3, 2))).transpose(2, 3)
+    assert not swapped.isContiguous()
+    assert all(np.array_equal(a, b) for a, b in zip(results(module(), dev(gt, x), swapped, merged), ref))
+    one = module()
+    one.fgradInput = one.finput
+    assert all(np.array_equal(a, b) for a, b in zip(results(one, dev(gt, x), dev(gt, go), merged), ref))
+    pair = []
+    for call in (passes, merged):  # gradInput over the input: accGradParameters sees the gradient, as it did
+        m, dx = module(), dev(gt, x)
+        m.gradInput = dx
+        pair.append(results(m, dx, dev(gt, go), call))
+    assert all(np.array_equal(a, b) for a, b in zip(*pair))
+
+    class Halved(gt.nn.SpatialConvolutionMM):
+        def updateGradInput(self, input, gradOutput):
+            return gt.nn.SpatialConvolutionMM.updateGradInput(self, input, gradOutput).mul(0.5)
+
+    got = results(module(Halved), dev(gt, x), dev(gt, go), merged)
+    assert np.array_equal(got[0], 0.5 * ref[0]) and np.array_equal(got[1], ref[1])
