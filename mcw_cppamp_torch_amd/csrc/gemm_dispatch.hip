@@ -24,7 +24,6 @@ struct RowSumJob {
     float *out;
     int M, slots;
     float alpha;
-    unsigned first_block;  // workgroups from this one on work on the row sums, four rows each
 };
 
 __device__ __forceinline__ void rowsum_reduce(const RowSumJob &j, unsigned block) {
@@ -40,30 +39,31 @@ __device__ __forceinline__ void rowsum_reduce(const RowSumJob &j, unsigned block
 }
 
 // The reduction of one product's partial sums and whatever rides with it.
+//
+// In the order in which a wavefront needs it: it lives for 2 us, of which a second round of scalar loads before the partial
+// sums can be asked for is a tenth (14 reductions of a VGG-A step: 607 us, 643 with the row sums' job in front).
 struct ReduceJob {
-    RowSumJob rs;
+    unsigned rowsum_first_block, side_first_block;  // workgroups from these on do the jobs at the end
+    unsigned total;                                 // outputs: M*J
+    int nsplit;
     const float *ws;
     float *C;
-    const float *bias, *bias_col;
-    int M, J, N;
+    FastDiv divJ;
+    unsigned j_store;
+    int J, N;
     long sC, bsC;
-    FastDiv divJ, divN, divCW;
-    int nsplit;
+    const float *bias, *bias_col, *mask;
+    float *C2;
     float alpha, beta;
     int act;
-    float act_threshold, act_value;
-    const float *mask;
-    float mask_threshold;
-    int c_pitch, mask_pitch;
-    long mask_sC, mask_bsC;
-    float *C2;
-    long c2_sC, c2_bsC;
-    int c2_pitch;
-    unsigned j_store;
-    unsigned side_first_block;  // workgroups from this one on carry a job of the next layer's (side_jobs.h)
-    WeightJob side;
+    float act_threshold, act_value, mask_threshold;
+    int c_pitch, mask_pitch, c2_pitch;
+    FastDiv divN, divCW;
+    long mask_sC, mask_bsC, c2_sC, c2_bsC;
     unsigned blocks;
     bool quarters;
+    RowSumJob rs;
+    WeightJob side;  // a job of the next layer's (side_jobs.h)
 };
 
 template <bool quarters>
@@ -72,14 +72,14 @@ __device__ __forceinline__ void split_reduce(const ReduceJob &j, unsigned block)
         reorder_weight(j.side, (block - j.side_first_block) * 256u + threadIdx.x);
         return;
     }
-    if (j.rs.out && block >= j.rs.first_block) {
-        rowsum_reduce(j.rs, block - j.rs.first_block);
+    if (block >= j.rowsum_first_block) {
+        rowsum_reduce(j.rs, block - j.rowsum_first_block);
         return;
     }
     // With `quarters` the four wavefronts of a workgroup share 64 outputs, each adding a contiguous quarter of the
     // partial sums (for few outputs and many splits: one lane per output would leave the GPU idle behind a long
     // chain of loads); the quarters are then added in order.  Either way the order of the adds is fixed.
-    const unsigned total = (unsigned)j.M * (unsigned)j.J;
+    const unsigned total = j.total;
     const unsigned wave = threadIdx.x >> 6;
     unsigned idx = quarters ? block * 64u + (threadIdx.x & 63u) : block * 256u + threadIdx.x;
     const bool valid = idx < total;
@@ -538,13 +538,13 @@ double reduce_job(const Prepared &q, ReduceJob &job) {
     // parts and two more like it, 3x3 layers of one 13x13 image) 12 as the line gave 53.1 -> 50.8 us a pass against 32.
     job.quarters = n > 0 && n < 128 * 1024 && g.nsplit >= 12;
     job.blocks = (unsigned)cdiv(n, job.quarters ? 64 : 256);
+    job.rowsum_first_block = job.blocks;  // four rows to a workgroup
     if (q.rowsum) {
         job.rs.ws = g.rowsum_ws;
         job.rs.out = p.rowsum;
         job.rs.M = p.M;
         job.rs.slots = (int)(g.nsplit * g.tilesJ);
         job.rs.alpha = p.alpha;
-        job.rs.first_block = job.blocks;
         job.blocks += (unsigned)cdiv(p.M, 4);
     }
     // A product that stores a second copy of its result for the next layer's gradInput product also carries that
@@ -559,7 +559,7 @@ double reduce_job(const Prepared &q, ReduceJob &job) {
     job.C = p.C;
     job.bias = p.bias;
     job.bias_col = p.bias_col;
-    job.M = p.M;
+    job.total = (unsigned)p.M * (unsigned)p.J;
     job.J = p.J;
     job.N = g.N;
     job.sC = p.sC;
@@ -617,8 +617,8 @@ int gemm_launch(const GemmProblem &p) {
 }
 
 // Two products of which neither reads what the other writes.  Their split reductions share a launch, and where both are
-// small enough for the tile of four groups, so do they themselves (unless every launch is being timed, to keep a record of
-// each): a launch is 3 us to enqueue and 3 to 5 for the GPU to run and change over, as long as such a product takes.
+// small enough for the tile of four groups, so do they themselves: a launch is 3 us to enqueue and 3 to 5 for the GPU to
+// run and change over, as long as such a product takes.
 int gemm_launch_pair(const GemmProblem &a, const GemmProblem &b) {
     hipStream_t s = stream();
     if (!s) return 1;
@@ -632,7 +632,7 @@ int gemm_launch_pair(const GemmProblem &a, const GemmProblem &b) {
         if (qa.ws_floats > 0) use_workspace(qa, ws);
         if (qb.ws_floats > 0) use_workspace(qb, ws + first);
     }
-    if (!prof_enabled() && qa.best && qb.best && qa.best->groups > 1 && qb.best->groups > 1 &&
+    if (qa.best && qb.best && qa.best->groups > 1 && qb.best->groups > 1 &&
         gemm_fast_64x64k4_pair(qa.g, qa.la, qa.lb, qa.red, qb.g, qb.la, qb.lb, qb.red, s) == 0) {
         if (check_launch(a.tag)) return 1;
     } else if (run_product(qa, s) || run_product(qb, s)) {

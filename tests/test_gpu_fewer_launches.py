@@ -247,3 +247,48 @@ def test_backward_with_shared_or_strided_tensors(gt):
 
     got = results(module(Halved), dev(gt, x), dev(gt, go), merged)
     assert np.array_equal(got[0], 0.5 * ref[0]) and np.array_equal(got[1], ref[1])
+
+
+@pytest.mark.parametrize("case", ["fused", "plain", "derived module"])
+def test_container_backward_gives_what_its_two_passes_give(gt, case):
+    """Module by module against updateGradInput and then accGradParameters of the whole container, bit for bit."""
+    nn = gt.nn
+
+    class Noted(nn.ReLU):  # of another file: the container walks back in the plain order
+        def accGradParameters(self, input, gradOutput, scale=1):
+            seen.append("accGradParameters")
+
+        def updateGradInput(self, input, gradOutput):
+            seen.append("updateGradInput")
+            return nn.ReLU.updateGradInput(self, input, gradOutput)
+
+    seen = []
+
+    def stack():
+        rng = rng_for(409)
+        mods = [nn.SpatialConvolutionMM(3, 64, 5, 5, 2, 2, 2, rng=rng), nn.ReLU(), nn.SpatialMaxPooling(3, 3, 2, 2),
+                nn.SpatialConvolutionMM(64, 96, 3, 3, 1, 1, 1, rng=rng), Noted() if case == "derived module" else nn.ReLU(),
+                nn.SpatialConvolutionMM(96, 64, 3, 3, 1, 1, 1, rng=rng), nn.ReLU(),
+                nn.SpatialMaxPooling(2, 2), nn.View(64 * 7 * 7), nn.Linear(64 * 7 * 7, 20, rng=rng), nn.LogSoftMax()]
+        net = nn.Sequential()
+        for m in mods:
+            net.add(m)
+        net.gpu()
+        return net.fuse() if case == "fused" else net
+
+    rng = rng_for(410)
+    nets = [stack(), stack()]
+    for _ in range(2):
+        x, go = dev(gt, uniform(rng, (2, 3, 57, 57))), dev(gt, uniform(rng, (2, 20)))
+        got = []
+        for i, net in enumerate(nets):
+            net.zeroGradParameters()
+            net.forward(x)
+            if i == 0:
+                net.backward(x, go, 0.5)
+            else:
+                net.updateGradInput(x, go)
+                net.accGradParameters(x, go, 0.5)
+            got.append([net.gradInput.float()] + [g.float() for g in net.parameters()[1]])
+        assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(*got))
+    assert seen == (["updateGradInput", "accGradParameters"] * 4 if case == "derived module" else [])
