@@ -610,6 +610,8 @@ int thgpu_ClassNLLCriterion_updateOutput(THGPUTensor *input, THGPUTensor *target
                                          int sizeAverage);
 int thgpu_ClassNLLCriterion_updateGradInput(THGPUTensor *input, THGPUTensor *target, THGPUTensor *gradInput,
                                             int sizeAverage);
+/* The same with the resizing and the zeroing done too, in the one launch. */
+int thgpu_ClassNLLCriterion_gradInput(THGPUTensor *input, THGPUTensor *target, THGPUTensor *gradInput, int sizeAverage);
 
 #ifdef __cplusplus
 }

@@ -228,6 +228,7 @@ _SIGNATURES = {
     "thgpu_LogSoftMax_updateGradInput": (c_int, [TensorP] * 3),
     "thgpu_ClassNLLCriterion_updateOutput": (c_int, [TensorP] * 3 + [c_int]),
     "thgpu_ClassNLLCriterion_updateGradInput": (c_int, [TensorP] * 3 + [c_int]),
+    "thgpu_ClassNLLCriterion_gradInput": (c_int, [TensorP] * 3 + [c_int]),
 }
 for _k in HOST_TYPES:
     _SIGNATURES["THGPUStorage_copy%s" % _k] = (None, [StorageP, ctypes.POINTER(HostStorage[_k])])

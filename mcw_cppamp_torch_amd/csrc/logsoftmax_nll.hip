@@ -105,6 +105,22 @@ __global__ __launch_bounds__(256) void nll_bwd_kernel(const float *__restrict__ 
     }
 }
 
+// The whole gradient, zeros and all: one lane an element, which asks its frame's targets.  Zeroing and then writing the
+// targets were two launches (9 us of a step's 330 for 50 x 10 elements, whose enqueueing is what such a step waits for).
+__global__ __launch_bounds__(256) void nll_gradient_kernel(const float *__restrict__ target, float *__restrict__ gin,
+                                                           unsigned total, FastDiv divDim, long ndim, long ntarget, float grad) {
+    const unsigned idx = blockIdx.x * 256u + threadIdx.x;
+    if (idx >= total) return;
+    unsigned i, k;
+    divDim.divmod(idx, i, k);
+    float v = 0.0f;
+    for (long j = 0; j < ntarget; ++j) {
+        const long t = (long)target[i * ntarget + j] - 1;
+        if (t == (long)k && t < ndim) v = grad;
+    }
+    gin[idx] = v;
+}
+
 // nframe x dim of a vector or matrix; 0 on success.
 int frames(const THGPUTensor *t, long &nframe, long &dim) {
     if (t->nDimension == 1) {
@@ -210,11 +226,11 @@ int thgpu_ClassNLLCriterion_updateOutput(THGPUTensor *input, THGPUTensor *target
     return rc;
 }
 
-int thgpu_ClassNLLCriterion_updateGradInput(THGPUTensor *input, THGPUTensor *target, THGPUTensor *gradInput,
-                                            int sizeAverage) {
+static int nll_gradient(THGPUTensor *input, THGPUTensor *target, THGPUTensor *gradInput, int sizeAverage, bool whole) {
     if (!input || !target || !gradInput) return fail("ClassNLLCriterion: null tensor");
     long nframe, ndim;
     if (frames(input, nframe, ndim)) return 1;
+    if (whole) THGPUTensor_resizeAs(gradInput, input);
     const long ntarget = target->nDimension > 1 ? target->size[1] : 1;
     if (input->nDimension == 1 && ntarget > 1) return fail("multi-target not implemented");
     if (THGPUTensor_nElement(target) != nframe * ntarget) return fail("ClassNLLCriterion: one target per frame expected");
@@ -227,7 +243,15 @@ int thgpu_ClassNLLCriterion_updateGradInput(THGPUTensor *input, THGPUTensor *tar
     if (!tg) return 1;
     float grad = -1.0f;
     if (input->nDimension == 2 && sizeAverage) grad /= (float)nframe;
-    {
+    if (whole && nframe * ndim < (1L << 31)) {
+        LaunchScope scope("nll_bwd", 0.0, 4.0 * nframe * (ndim + ntarget));
+        hipLaunchKernelGGL(nll_gradient_kernel, dim3((unsigned)((nframe * ndim + 255) / 256)), dim3(256), 0, st, dptr(tg),
+                           dptr(gradInput), (unsigned)(nframe * ndim), FastDiv((uint32_t)ndim), ndim, ntarget, grad);
+    } else {
+        if (whole && fill_device(dptr(gradInput), nframe * ndim, 0.0f)) {
+            THGPUTensor_free(tg);
+            return 1;
+        }
         LaunchScope scope("nll_bwd", 0.0, 8.0 * nframe * ntarget);
         hipLaunchKernelGGL(nll_bwd_kernel, dim3((unsigned)((nframe + 255) / 256)), dim3(256), 0, st, dptr(tg),
                            dptr(gradInput), nframe, ndim, ntarget, grad);
@@ -235,6 +259,15 @@ int thgpu_ClassNLLCriterion_updateGradInput(THGPUTensor *input, THGPUTensor *tar
     const int rc = check_launch("nll_bwd");
     THGPUTensor_free(tg);
     return rc;
+}
+
+int thgpu_ClassNLLCriterion_updateGradInput(THGPUTensor *input, THGPUTensor *target, THGPUTensor *gradInput,
+                                            int sizeAverage) {
+    return nll_gradient(input, target, gradInput, sizeAverage, false);
+}
+
+int thgpu_ClassNLLCriterion_gradInput(THGPUTensor *input, THGPUTensor *target, THGPUTensor *gradInput, int sizeAverage) {
+    return nll_gradient(input, target, gradInput, sizeAverage, true);
 }
 
 }  // extern "C"

@@ -134,9 +134,18 @@ __global__ __launch_bounds__(256) void subsample_accgrad_final_kernel(const floa
     const int k = blockIdx.x * 256 + threadIdx.x;
     if (k >= C) return;
     float gb = gradBias[k], gw = gradWeight[k];
-    for (int b = 0; b < B; ++b) {
-        gb = __fadd_rn(gb, __fmul_rn(scale, partial[2 * ((long)b * C + k)]));
-        gw = __fadd_rn(gw, __fmul_rn(scale, partial[2 * ((long)b * C + k) + 1]));
+    const float2 *__restrict__ sums = reinterpret_cast<const float2 *>(partial) + k;
+    // Eight images are asked for before the first is added: one at a time, 50 images took 9 us.
+    for (int b0 = 0; b0 < B; b0 += 8) {
+        float2 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = b0 + u < B ? sums[(long)(b0 + u) * C] : make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if (b0 + u >= B) break;
+            gb = __fadd_rn(gb, __fmul_rn(scale, v[u].x));
+            gw = __fadd_rn(gw, __fmul_rn(scale, v[u].y));
+        }
     }
     gradBias[k] = gb;
     gradWeight[k] = gw;

@@ -940,8 +940,6 @@ class ClassNLLCriterion(Criterion):
 
     def updateGradInput(self, input, target):
         _require_gpu(input, target, self.gradInput)
-        self.gradInput.resizeAs(input)
-        self.gradInput.zero()
-        _lib.check_status(lib.thgpu_ClassNLLCriterion_updateGradInput(input._p, target._p, self.gradInput._p,
-                                                                      1 if self.sizeAverage else 0))
+        _lib.check_status(lib.thgpu_ClassNLLCriterion_gradInput(input._p, target._p, self.gradInput._p,
+                                                                1 if self.sizeAverage else 0))
         return self.gradInput

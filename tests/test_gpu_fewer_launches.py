@@ -292,3 +292,18 @@ def test_container_backward_gives_what_its_two_passes_give(gt, case):
             got.append([net.gradInput.float()] + [g.float() for g in net.parameters()[1]])
         assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(*got))
     assert seen == (["updateGradInput", "accGradParameters"] * 4 if case == "derived module" else [])
+
+
+@pytest.mark.parametrize("shape,targets", [((1,), [1]), ((7,), [7]), ((3, 5), [0, 5, 6]), ((130, 3), None), ((2, 1000), [1000, 1])])
+def test_criterion_gradient_of_one_launch(gt, shape, targets):
+    """Every element, whatever gradInput held; targets outside 1..n are skipped."""
+    frames, n = (shape if len(shape) == 2 else (1,) + shape)
+    t = np.array(targets if targets is not None else rng_for(411).integers(1, n + 1, size=frames), np.float32)
+    c = gt.nn.ClassNLLCriterion().gpu()
+    c.gradInput = gt.GPUTensor(frames + 1, n).fill(np.nan)
+    got = c.backward(gt.GPUTensor(*shape).fill(0), dev(gt, t)).float()
+    ref = np.zeros((frames, n), np.float32)
+    for i, k in enumerate(t.astype(int)):
+        if 1 <= k <= n:
+            ref[i, k - 1] = -1.0 / frames if len(shape) == 2 else -1.0
+    assert np.array_equal(got, ref.reshape(shape))
