@@ -216,7 +216,7 @@ def ref_benchmark(args, pkg):
         "layers": rows}))
 
 
-PLAN_TILES = ["128x128", "192x128", "64x256", "128x256", "256x128", "64x64", "64x128", "96x128"]
+PLAN_TILES = ["128x128", "192x128", "64x256", "128x256", "256x128", "64x64", "64x128", "96x128", "32x128", "64x64k4"]
 PLAN_SPLITS = [1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 59, 64, 96, 128, 170, 256]
 
 

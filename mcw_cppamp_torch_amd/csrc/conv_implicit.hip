@@ -319,10 +319,9 @@ WeightJob bank_job(const float *weight, float *wt, int C, int H, int W, int M, i
         wj.sW = sW;
         wj.A = q.A;
         wj.Bk = q.Bk;
-        wj.rows = q.rows;
         wj.count = (unsigned)((long)q.rows * M * q.A * q.Bk);
     } else {
-        wj.sH = wj.sW = wj.A = wj.Bk = wj.rows = 0;
+        wj.sH = wj.sW = wj.A = wj.Bk = 0;
         wj.count = (unsigned)((long)M * C * kH * kW);
     }
     return wj;
@@ -419,19 +418,23 @@ bool conv_use_gathered(long B, int C, int H, int W, int M, int kH, int kW, int p
     if (mode == 0 || !forward_fits(B, C, H, W, M, kH, kW, pH, pW, sH, sW)) return false;
     // Fewer planes than a 64-row tile: the columns and the bias gradient's pass over gradOutput go all the same (450 -> 18 planes
     // 11x11, 19 images: 1656 -> 900 us a pass).  Padded layers of fewer than 256 positions take as long either way (0.91 to
-    // 1.07 on ten layers of 64 and 128 positions; 1.5 without padding, where there is no copy to make).  Mode 2 keeps the
-    // columns of all of them, for callers that read them from finput.
-    const long Ho = (H + 2L * pH - kH) / sH + 1, Wo = (W + 2L * pW - kW) / sW + 1;
-    return M >= 64 || (mode == 1 && (B * Ho * Wo >= 256 || (pH == 0 && pW == 0)));
+    // 1.07 on ten layers of 64 and 128 positions; 1.5 without padding, where there is no copy to make), and columns of less
+    // than 512 KiB cost little more than the padded copy (3 -> 8 ... 48 planes 5x5 stride 2, three 38x38 images: 1.02 to
+    // 1.12; from 576 KiB on 64 -> 16 ... 60 planes 3x3 1.24 to 1.37, layers of 3 planes 0.95 to 1.04): those keep finput as
+    // it was.  Mode 2 keeps the columns of all of them, for callers that read them from finput.
+    const long Ho = (H + 2L * pH - kH) / sH + 1, Wo = (W + 2L * pW - kW) / sW + 1, positions = B * Ho * Wo;
+    return M >= 64 ||
+           (mode == 1 && ((positions >= 256 && positions >= 131072.0 / ((double)C * kH * kW)) || (pH == 0 && pW == 0)));
 }
 
 // What gradInput takes on either route, in microseconds: the planner's estimate of its product and the traffic around it, at
 // 4.5 TB/s and for the re-ordering of the kernel bank at 3.  The gathered product has one row per input plane (and residue
 // class) in tiles of 32 or 64 and one column per input pixel; the product on columns is often bound by writing them, of which
 // the estimate sees a part.  Over 329 layers (1 to 128 images, 3 to 1024 input planes, kernels of 3 to 11, strides of 1, 2 and 4),
-// both sides measured, the choice costs 0.6 % over the better one each time, at most 21 %; the rules before it (64-row
-// tiles, an excess of work below two) cost 10 times the time where a strided layer has few pixels and a long reduction,
-// which its unsplit product walks in a handful of workgroups (384 planes 7x7, 28x28 images: 21 us on columns, 192).
+// both sides measured, the smaller estimate costs 0.6 % over the better side, at most 21 % (1.2 % with the two exceptions in
+// conv_use_gathered_gradinput).  A rule on the excess of work stood here, which cost up to 10 times the time where a
+// strided layer has few pixels and a long reduction: its product cannot be split, and a handful of workgroups walked it
+// (16 -> 384 planes 7x7 stride 2, two 16x20 images: 17 us on columns, 198).
 static double gathered_gradinput_us(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
     const long N = ((H + 2L * pH - kH) / sH + 1) * ((W + 2L * pW - kW) / sW + 1);
     int top, left, Hq, Wq;

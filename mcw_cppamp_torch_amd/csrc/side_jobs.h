@@ -14,8 +14,8 @@ struct WeightJob {
     const float *w;
     float *wt;
     int M, C, kH, kW;
-    int sH, sW, A, Bk, rows;  // strided form only (sH = 0: unit stride)
-    unsigned count;           // elements of wt; 0: no job
+    int sH, sW, A, Bk;  // strided form only (sH = 0: unit stride)
+    unsigned count;     // elements of wt; 0: no job
 };
 
 __device__ __forceinline__ void reorder_weight(const WeightJob &j, unsigned idx) {

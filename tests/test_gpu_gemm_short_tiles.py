@@ -80,12 +80,13 @@ def test_blas_products_shorter_than_a_tile(gt, tile, ta, tb, split, switches):
 
 LAYERS = {  # B, C, H, W, M, kH, kW, pH, pW, sH, sW
     "rows_37_strided": (5, 3, 101, 77, 37, 5, 5, 0, 0, 3, 3),
-    "rows_1": (3, 5, 20, 23, 1, 3, 3, 1, 1, 1, 1),
-    "rows_31_quads": (2, 7, 16, 20, 31, 3, 3, 1, 1, 1, 1),     # image rows of whole quads
-    "rows_32_taps_25": (4, 1, 24, 24, 32, 5, 5, 2, 2, 1, 1),
-    "rows_33_one_image": (1, 40, 19, 17, 33, 3, 3, 1, 1, 1, 1),
+    "rows_1": (7, 5, 20, 23, 1, 3, 3, 1, 1, 1, 1),
+    "rows_31_quads": (7, 7, 16, 20, 31, 3, 3, 1, 1, 1, 1),     # image rows of whole quads
+    "rows_32_taps_25": (10, 1, 24, 24, 32, 5, 5, 2, 2, 1, 1),
+    "rows_33_one_image": (1, 48, 19, 17, 33, 3, 3, 1, 1, 1, 1),
     "rows_63_long": (6, 40, 12, 12, 63, 5, 5, 0, 0, 1, 1),
     "few_positions": (1, 64, 7, 7, 20, 4, 4, 0, 0, 1, 1),      # 16 positions
+    "small_columns": (2, 7, 16, 20, 31, 3, 3, 1, 1, 1, 1),     # 158 KB of columns: they stay
     "strided_few_classes": (2, 3, 30, 41, 70, 5, 3, 1, 0, 2, 1),
 }
 
@@ -120,5 +121,30 @@ def test_layers_of_few_planes_without_columns(gt, name, tile, switches):
     labels = labels_of(gt, lambda: m.accGradParameters(dx, dgo, 2.0), ("gemm_conv", "im2col"))
     assert np.array_equal(guard_w.float(), np.vstack([gw, np.full((1, K), 9, np.float32)]))
     assert np.array_equal(guard_b.float(), np.append(gb, np.float32(9)))
-    if tile is None and not name == "few_positions":
-        assert not any("generic" in l or l.startswith("im2col") for l in labels), labels
+    if tile is None:       # (a forced tile that gradWeight does not fit leaves the whole layer on columns)
+        assert any(l.startswith("im2col") for l in labels) == (name == "small_columns"), labels
+    if tile is None and name != "few_positions":
+        assert not any("generic" in l for l in labels), labels
+
+
+@pytest.mark.parametrize("at", [5, 150, 251, 398])  # a step of each of the four groups
+@pytest.mark.parametrize("tile", ["32x128", "64x64k4"])
+def test_values_that_bf16_parts_do_not_hold(gt, tile, at, switches):
+    """A 24-bit number below 2^-110 against a large partner, an infinity and a NaN: multiplied in fp32, as on the other tiles
+    (one product a result, so exact), wherever in the reduction they stand."""
+    switches("gemm_tile", tile)
+    switches("gemm_split", "1")
+    m, n, k = 200, 40, 399
+    a, b = np.zeros((k, m), np.float32), np.ones((n, k), np.float32)
+    a[at, 3] = np.float32(2.0 ** -118 * (1 + 2.0 ** -23))
+    a[at, 70], a[at, 71] = np.inf, np.nan
+    b[:, at] = 2.0 ** 100
+    b[7, at] = -(2.0 ** 100)
+    c = gt.GPUTensor(n * m).fill(0)
+    da, db = dev(gt, a.ravel()), dev(gt, b.ravel())
+    labels = labels_of(gt, lambda: gt.gputorch.gemm("n", "n", m, n, k, 1.0, da, m, db, k, 0.0, c, m), "gemm_blas")
+    assert "tile=%s " % tile in labels[0]
+    got = c.float().reshape(n, m)
+    ref = b[:, at:at + 1] * a[at]
+    ref[:, 70], ref[:, 71] = np.copysign(np.inf, b[:, at]), np.nan
+    assert np.array_equal(got, ref, equal_nan=True)
