@@ -164,6 +164,7 @@ struct TileCfg {
     bool a_rc_only;
     // Groups of wavefronts that share a workgroup's reduction (gemm_fast.h, finish_groups).
     int groups = 1;
+    bool folds = false;  // sums in two levels (gemm_fold_steps)
 };
 
 // Rate kept with k workgroups on a CU, by tile: measured on 3x3 forward products of 2304 reduction indices and exactly
@@ -184,6 +185,7 @@ const TileCfg kCfgs[] = {
     {"64x128", 64, 128, 4, {0.33, 0.33, 0.33, 0.33, 0.34, 0.33}, gemm_fast_64x128, kOcc4, 128, false},
     {"96x128", 96, 128, 3, {0.35, 0, 0.35, 0, 0.37, 0.35}, gemm_fast_96x128, kOcc3, 128, true},
     {"32x128", 32, 128, 4, {0.22, 0, 0.22, 0, 0.22, 0.25}, gemm_fast_32x128, kOcc4, 33, true},
+    {"64x64f", 64, 64, 4, {0, 0, 0, 0, 0.29, 0}, gemm_fast_64x64f, kOccSmall, 0, true, 1, true},
     {"64x64k4", 64, 64, 1, {0.25, 0.25, 0.25, 0.25, 0.26, 0.27}, gemm_fast_64x64k4, kOcc1, 0, false, 4},
 };
 
@@ -231,6 +233,21 @@ double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_tot
     return t;
 }
 
+// Few outputs and many splits: four wavefronts share 64 outputs of the split reduction (reduce_job).
+inline bool reduced_in_quarters(long outputs, int nsplit) { return outputs > 0 && outputs < 128 * 1024 && nsplit >= 12; }
+
+// Additions in a row on the way to one output, level by level: a wavefront's steps, its workgroup's groups, the parts.  n
+// roundings of a sum that grows evenly to its full size come to n / 2 times the mean square of one of the full sum, and levels
+// add up, so this is what an order of summation is judged by.
+double plan_chain(const TileCfg &c, long outputs, int steps_total, int nsplit) {
+    const int steps = (int)cdiv(cdiv(steps_total, nsplit), c.groups);
+    double n = steps;
+    if (c.folds && gemm_fold_steps(steps) < steps) n = gemm_fold_steps(steps) + (double)steps / gemm_fold_steps(steps);
+    if (c.groups > 1) n += c.groups;
+    if (nsplit > 1) n += reduced_in_quarters(outputs, nsplit) ? (double)cdiv(nsplit, 4) + 4.0 : nsplit;
+    return n;
+}
+
 // The tile configuration and reduction split for a problem; cfg == nullptr when no tiled kernel takes it.
 struct GemmPlan {
     const TileCfg *cfg = nullptr;
@@ -271,6 +288,8 @@ GemmPlan rank_plans(const GemmProblem &p, int steps_total, bool any) {
         if (force && std::strcmp(force, c.name) != 0) continue;
         if (!force && c.below_rows > 0 && p.M >= c.below_rows) continue;
         if (c.a_rc_only && !p.a_rc) continue;
+        if (c.folds && (layout != 4 || (!force && p.max_chain <= 0.0))) continue;
+        const double best_chain = plan.cfg ? plan_chain(*plan.cfg, (long)p.M * p.J, steps_total, plan.nsplit) : 0.0;  // so far
         const long tiles = cdiv(p.M, c.bm) * cdiv(p.J, c.bn);
         // (a product run wider than its result has one narrow tile per row block: it may split further to fill the GPU)
         const int split_cap = p.j_store > 0 ? 1024 : 256;
@@ -285,6 +304,13 @@ GemmPlan rank_plans(const GemmProblem &p, int steps_total, bool any) {
             if (ns > 1 && p.ws_fixed && (long)ns * p.M * p.J > p.ws_fixed_floats) break;  // partial sums must fit
             const int sps = (int)cdiv(steps_total, ns);
             if (sps > 0 && (int)cdiv(steps_total, sps) != ns) continue;  // would leave an empty split
+            if (!force && fsplit <= 0) {
+                const double chain = plan_chain(c, (long)p.M * p.J, steps_total, ns);
+                if (p.max_chain > 0.0 && chain > p.max_chain) continue;
+                // (the tile of groups, the last one, does with fewer parts what the others split further: not at the price of
+                // longer sums, 282 x 294 over 2272 steps in 85 parts 1.41e-7 from 64 bits, in 10 of four groups 1.61e-7)
+                if (c.groups > 1 && plan.cfg && chain > best_chain) continue;
+            }
             if (any) {
                 plan.cfg = &c;
                 plan.nsplit = ns;
@@ -304,7 +330,7 @@ GemmPlan rank_plans(const GemmProblem &p, int steps_total, bool any) {
 
 // What the planner's answer depends on.
 struct PlanKey {
-    long v[21];
+    long v[22];
     bool operator<(const PlanKey &o) const { return std::memcmp(v, o.v, sizeof(v)) < 0; }
 };
 
@@ -320,7 +346,8 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
     const PlanKey key = {{p.M, p.J, p.R, p.N, steps_total, p.nb > 1 || p.rowsum,
                           (p.a_rc ? 1 : 0) + (p.b_rc ? 2 : 0) + (p.rowtab ? 4 : 0) + (p.scatter ? 8 : 0) + (p.C2 ? 16 : 0), p.j_store,
                           p.sA, p.sB, p.sC, p.bsB, p.bsC, p.b_extent, p.C2 ? p.c2_sC : 0, p.C2 ? p.c2_bsC : 0,
-                          p.C2 ? p.c2_pitch : 0, p.C2 ? p.c_w : 0, p.ws_fixed ? 1 : 0, p.ws_fixed ? p.ws_fixed_floats : 0, p.beta != 0.0f}};
+                          p.C2 ? p.c2_pitch : 0, p.C2 ? p.c_w : 0, p.ws_fixed ? 1 : 0, p.ws_fixed ? p.ws_fixed_floats : 0, p.beta != 0.0f,
+                          (long)(16.0 * p.max_chain)}};
     {
         std::lock_guard<std::mutex> lock(mutex);
         const auto it = plans.find(key);
@@ -344,7 +371,8 @@ inline int steps_of(const GemmProblem &p) {
 
 bool gemm_tiled_fits(const GemmProblem &p) {
     if (p.M <= 0 || p.J <= 0 || (long)p.M * p.J >= (1L << 31)) return false;
-    return rank_plans(p, steps_of(p), true).cfg != nullptr;
+    // (where the first tile and split will not do, the answer is the planner's, which keeps it)
+    return (p.max_chain > 0.0 ? plan_gemm(p, steps_of(p)) : rank_plans(p, steps_of(p), true)).cfg != nullptr;
 }
 
 double gemm_estimate_us(const GemmProblem &p) {
@@ -469,6 +497,7 @@ int gemm_prepare(const GemmProblem &p, Prepared &out) {
         g.nsplit = (int)cdiv(g.steps_total, sps);
     }
     g.steps_per_split = (int)cdiv(g.steps_total, g.nsplit);
+    g.fold_steps = gemm_fold_steps(g.steps_per_split);
     g.tilesM = (unsigned)cdiv(p.M, bm);
     g.tilesJ = (unsigned)cdiv(p.J, bn);
     g.divTilesM = FastDiv(g.tilesM);
@@ -536,7 +565,7 @@ double reduce_job(const Prepared &q, ReduceJob &job) {
     // few outputs, many splits: four wavefronts per 64 outputs.  From 4 K to 123 K outputs the launch alone takes the same
     // either way up to 16 splits, 0.2 us less at 24, 0.5 at 32 and 2.4 at 64; behind its product (256 x 169 outputs in 27
     // parts and two more like it, 3x3 layers of one 13x13 image) 12 as the line gave 53.1 -> 50.8 us a pass against 32.
-    job.quarters = n > 0 && n < 128 * 1024 && g.nsplit >= 12;
+    job.quarters = reduced_in_quarters(n, g.nsplit);
     job.blocks = (unsigned)cdiv(n, job.quarters ? 64 : 256);
     job.rowsum_first_block = job.blocks;  // four rows to a workgroup
     if (q.rowsum) {

@@ -223,8 +223,9 @@ __device__ __forceinline__ void finish_groups(const GemmArgs &g, char *lds_a, ch
     }
 }
 
-// One workgroup of a product; As and Bs hold KG pairs of operand tiles.
-template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG>
+// One workgroup of a product; As and Bs hold KG pairs of operand tiles.  FOLD: every g.fold_steps steps (an even number) a
+// wavefront's sum goes to a second one and starts over (gemm_chain).
+template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG, bool FOLD = false>
 __device__ __forceinline__ void gemm_fast_tile(const GemmArgs &g, const unsigned block, char *const As, char *const Bs) {
     constexpr int NT = WGM * WGN * 64;  // threads of a group: the whole workgroup unless KG > 1
     constexpr int BK = GEMM_BK;
@@ -682,7 +683,21 @@ __device__ __forceinline__ void gemm_fast_tile(const GemmArgs &g, const unsigned
         else shift = 0;
         if (KG == 1) __syncthreads();
     };
-    if constexpr (KG == 1) {
+    if constexpr (FOLD) {
+        static_assert(KG == 1 && TM * TN == 1, "one more block of sums in the registers");
+        floatx16 folded = {};
+        for (int s = 0; s < nsteps;) {
+            const int until = nsteps - s > g.fold_steps ? s + g.fold_steps : nsteps;
+            do {
+                one_step(std::integral_constant<int, 0>{}, s);
+                if (s + 1 < nsteps) one_step(std::integral_constant<int, 1>{}, s + 1);
+                s += 2;
+            } while (s < until);
+            folded += acc[0][0];
+            acc[0][0] = (floatx16){};
+        }
+        acc[0][0] = folded;
+    } else if constexpr (KG == 1) {
         for (int s = 0; s < nsteps; s += 2) {
             one_step(std::integral_constant<int, 0>{}, s);
             if (s + 1 < nsteps) one_step(std::integral_constant<int, 1>{}, s + 1);
@@ -986,12 +1001,12 @@ __device__ __forceinline__ void gemm_fast_tile(const GemmArgs &g, const unsigned
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG>
+template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG, bool FOLD = false>
 __global__ __launch_bounds__(WGM *WGN * 64 * KG)
     __attribute__((amdgpu_waves_per_eu(KG > 1 ? KG : gemm_min_waves<BM, BN, WGM, WGN>()))) void gemm_fast_kernel(const GemmArgs g) {
     __shared__ __attribute__((aligned(16))) char As[KG * 2 * PartTile<BM>::kBytes];
     __shared__ __attribute__((aligned(16))) char Bs[KG * 2 * PartTile<BN>::kBytes];
-    gemm_fast_tile<BM, BN, WGM, WGN, LA, LB, RED, KG>(g, blockIdx.x, As, Bs);
+    gemm_fast_tile<BM, BN, WGM, WGN, LA, LB, RED, KG, FOLD>(g, blockIdx.x, As, Bs);
 }
 
 // The workgroups of two products on the 64 x 64 tile of four groups, one after the other's.
@@ -1003,9 +1018,9 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
     else gemm_fast_tile<64, 64, 2, 2, LA2, LB2, RED2, 4>(b, blockIdx.x - a.total, As, Bs);
 }
 
-template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG = 1>
+template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG = 1, bool FOLD = false>
 int gemm_fast_go(const GemmArgs &g, hipStream_t s) {
-    hipLaunchKernelGGL((gemm_fast_kernel<BM, BN, WGM, WGN, LA, LB, RED, KG>), dim3(g.total), dim3(WGM * WGN * 64 * KG), 0, s, g);
+    hipLaunchKernelGGL((gemm_fast_kernel<BM, BN, WGM, WGN, LA, LB, RED, KG, FOLD>), dim3(g.total), dim3(WGM * WGN * 64 * KG), 0, s, g);
     return 0;
 }
 

@@ -88,6 +88,9 @@ struct GemmProblem {
     // the narrowest tile runs on the tiled kernels: its column table is padded with entries that repeat a valid one.
     // The reduction is always split (the partial sums are J wide, the final pass stores j_store).  0: all J columns.
     int j_store = 0;
+    // Only tiles and splits with no more than so many additions in a row on the way to a result (plan_chain in
+    // gemm_dispatch.hip) are considered, unless a tile or split is forced.  0: all, but the tile that sums in two levels.
+    double max_chain = 0.0;
     const char *tag = "gemm";     // name used by per-kernel timing
     // Flops the per-kernel timing credits the launch with; 0 means the product's own 2*M*J*R*nb.  A
     // convolution pass sets its algorithmic 2*M*N*K*B here, which a gathered gradInput product (one
@@ -117,6 +120,14 @@ double gemm_estimate_us(const GemmProblem &p);
 constexpr int GEMM_BK = 16;  // reduction step of every kernel
 constexpr int GEMM_SHORT_TILE = 64;  // a tile side up to this length also takes a matrix that is shorter (gemm_fast.h)
 
+// The tile that sums in two levels (gemm_fast_64x64f) moves its sum to the second one after an even number of steps (they come
+// in pairs) near the root of those that it walks.
+inline int gemm_fold_steps(int steps) {
+    int f = 4;
+    while (f * f < steps) f += 2;
+    return f;
+}
+
 struct GemmArgs {
     const float *A;
     const float *B;
@@ -131,6 +142,7 @@ struct GemmArgs {
     int steps_per_split;  // reduction steps one workgroup walks
     int steps_total;      // nb * steps_per_img
     int nsplit;
+    int fold_steps;       // on the tile that sums in two levels: see gemm_fold_steps
     unsigned tilesM, tilesJ, total;
     FastDiv divN, divTilesM, divTilesJ, divSpi;
     float alpha, beta;
@@ -191,6 +203,8 @@ int gemm_fast_64x64k4(const GemmArgs &g, int la, int lb, bool red, hipStream_t s
 int gemm_fast_64x64k4_pair(const GemmArgs &a, int la, int lb, bool red, const GemmArgs &b, int la2, int lb2, bool red2,
                            hipStream_t s);
 int gemm_fast_64x64(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
+// The same tile, summing in two levels: gathering products without reduction batching.
+int gemm_fast_64x64f(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x256(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_32x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);  // first operand along r only

@@ -802,3 +802,69 @@ def test_random_layers_with_a_handful_of_taps_integer_exact(gt, gathered_route, 
     oracle.conv_accGradParameters(go, finput_ref, gw, gb, 3.0)
     m.accGradParameters(dx, dev(gt, go), 3.0)
     assert np.array_equal(m.gradWeight.float(), gw) and np.array_equal(m.gradBias.float(), gb)
+
+
+def taps(a, kh, kw, Ho, Wo, sH, sW):
+    return a[:, :, kh:kh + (Ho - 1) * sH + 1:sH, kw:kw + (Wo - 1) * sW + 1:sW]
+
+
+def relative_error(got, ref):
+    return float(np.linalg.norm((got.astype(np.float64) - ref).ravel()) / np.linalg.norm(ref.ravel()))
+
+
+@pytest.mark.parametrize("layer", [(16, 44, 54, 58, 58, 5, 5, 2, 2, 1, 1), (8, 151, 42, 42, 48, 3, 3, 1, 1, 1, 1),
+                                   (57, 134, 19, 19, 55, 3, 3, 0, 0, 1, 1), (64, 96, 27, 27, 256, 5, 5, 2, 2, 1, 1),
+                                   (37, 57, 20, 20, 51, 3, 3, 0, 0, 1, 1), (4, 40, 33, 35, 24, 5, 5, 2, 2, 4, 4)])
+def test_gradinput_is_as_near_to_64_bits_as_on_columns(gt, layer):
+    """Layers whose planes do not fill 64-row tiles, on whichever route the library takes.  Both sides round the same products
+    of the same parts and differ in the order of the additions, which the planner holds to no more in a row than columns
+    have; the error of 60 thousand results and more is known to half a percent, the count of additions is good to a few."""
+    B, C, H, W, M, kH, kW, pH, pW, sH, sW = layer
+    rng = rng_for(49)
+    Ho, Wo = (H + 2 * pH - kH) // sH + 1, (W + 2 * pW - kW) // sW + 1
+    go, w = uniform(rng, (B, M, Ho, Wo)), uniform(rng, (M, C * kH * kW))
+    ref = np.zeros((B, C, H + 2 * pH, W + 2 * pW))
+    g64, w64 = go.astype(np.float64).reshape(B, M, Ho * Wo), w.astype(np.float64).reshape(M, C, kH, kW)
+    for kh in range(kH):
+        for kw in range(kW):
+            taps(ref, kh, kw, Ho, Wo, sH, sW)[...] += (w64[:, :, kh, kw].T @ g64).reshape(B, C, Ho, Wo)
+    ref = ref[:, :, pH:pH + H, pW:pW + W]
+    m = gt.nn.SpatialConvolutionMM(C, M, kW, kH, sW, sH, 0, padW=pW, padH=pH)
+    m._assign("weight", w)
+    m.gpu()
+    lib, errors = gt._lib.lib, {}
+    x, dgo = gt.GPUTensor(B, C, H, W).fill(0), dev(gt, go)
+    before = lib.thgpu_conv_get_mode()
+    try:
+        for mode in (0, 1):
+            assert lib.thgpu_conv_set_mode(mode) == 0
+            errors[mode] = relative_error(m.updateGradInput(x, dgo).float(), ref)
+    finally:
+        assert lib.thgpu_conv_set_mode(before) == 0
+    print(layer, errors)
+    assert errors[1] <= 1.05 * errors[0]
+
+
+def test_gradweight_of_groups_is_as_near_to_64_bits_as_of_parts(gt, switches):
+    """A long reduction over a small result: the tile of four groups does with fewer parts, but not with longer sums than the
+    tile that splits it further."""
+    B, C, H, W, M, k, p = 5, 6, 79, 92, 282, 7, 3
+    rng = rng_for(50)
+    x, go = uniform(rng, (B, C, H, W)), uniform(rng, (B, M, H, W))
+    xp, ref = padded(x, p, p).astype(np.float64), np.zeros((M, C, k, k))
+    for b in range(B):
+        g = go[b].astype(np.float64).reshape(M, H * W)
+        for kh in range(k):
+            for kw in range(k):
+                ref[:, :, kh, kw] += g @ taps(xp[b:b + 1], kh, kw, H, W, 1, 1).reshape(C, H * W).T
+    errors = []
+    for tile in (None, "192x128"):
+        switches("gemm_tile", tile)
+        m = gt.nn.SpatialConvolutionMM(C, M, k, k, 1, 1, p)
+        m.gradWeight[...] = 0
+        m.gradBias[...] = 0
+        m.gpu()
+        m.accGradParameters(dev(gt, x), dev(gt, go), 1)
+        errors.append(relative_error(m.gradWeight.float(), ref.reshape(M, -1)))
+    print(errors)
+    assert errors[0] <= 1.05 * errors[1]
