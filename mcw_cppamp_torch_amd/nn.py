@@ -194,22 +194,7 @@ class Sequential(Module):
         self.output = cur
         return cur
 
-    def backward(self, input, gradOutput, scale=1):
-        # updateGradInput and accGradParameters module by module, where nothing tells the two orders apart: accGradParameters
-        # of this file's modules reads their input and gradOutput, which no module in front writes.  A convolution's two
-        # passes then share launches.  A container with passes of its own, a module of a derived class or with a pass set
-        # on it, or one that is there twice, keeps the plain order.
-        mods = self.modules
-        if (not mods or not _own_passes(self, Sequential) or len(set(id(m) for m in mods)) != len(mods) or
-                not all(type(m).__module__ == __name__ and _own_passes(m, type(m)) for m in mods)):
-            return Module.backward(self, input, gradOutput, scale)
-        return self._walk_back(input, gradOutput, scale)
-
     def updateGradInput(self, input, gradOutput):
-        return self._walk_back(input, gradOutput, None)
-
-    def _walk_back(self, input, gradOutput, scale):
-        # (scale None: updateGradInput alone)
         # mcw_nn/Sequential.lua:45-57.  After fuse(), a module whose gradInput is the gradOutput of a convolution in
         # front of it (_grad_consumer) also stores it in the padded layout that convolution's gradInput product
         # gathers from, and the convolution is told so -- only here, where nothing can touch either copy in between;
@@ -224,21 +209,13 @@ class Sequential(Module):
             if link is not None:
                 consumer, ci = link
                 twin = consumer._gradOutputTwin(self.modules[ci - 1].output if ci > 0 else input)
-            go = cur
-            ready = ready_for is m and ready_for is not None
-            if scale is not None and isinstance(m, SpatialConvolutionMM) and m.gradInput is not None and _own_passes(m):
-                cur = m._backwardTwin(inp, go, twin, ready, scale)
-                ready_for = link[0] if (twin is not None and m._wrote_twin) else None
-                continue
-            if twin is not None or ready:
-                cur = m._updateGradInputTwin(inp, go, twin, ready)
+            if twin is not None or (ready_for is m and ready_for is not None):
+                cur = m._updateGradInputTwin(inp, cur, twin, ready_for is m)
                 ready_for = link[0] if (twin is not None and m._wrote_twin) else None
             else:
-                cur = m.updateGradInput(inp, go)
+                cur = m.updateGradInput(inp, cur)
                 if not (isinstance(m, Threshold) and m.fusedBackward):   # that one hands its gradOutput on untouched
                     ready_for = None
-            if scale is not None:
-                m.accGradParameters(inp, go, scale)
         self.gradInput = cur
         return cur
 
@@ -530,22 +507,16 @@ class SpatialConvolutionMM(Module):
         return self.gradInput
 
     def backward(self, input, gradOutput, scale=1):
-        # updateGradInput, then accGradParameters: in one call of the library where both are this class's own
+        # updateGradInput, then accGradParameters: in one call of the library where both are this class's own.  (A container's
+        # backward keeps the order of mcw_nn/Module.lua:24-33, gradInput of all its modules first: a module that fails there
+        # leaves no gradient accumulated behind it.)
         if self.gradInput is None or not _own_passes(self):
             return Module.backward(self, input, gradOutput, scale)
-        return self._backwardTwin(input, gradOutput, None, False, scale)
-
-    def _backwardTwin(self, input, gradOutput, twin, ready, scale):
-        """_updateGradInputTwin and accGradParameters."""
         _require_gpu(input, gradOutput, self.weight, self.gradWeight, self.gradBias, self.finput, self.fgradInput, self.gradInput)
-        flags = ((1 if self.inputThreshold is not None else 0) | (2 if _in_padded_buffer(input, self.padH, self.padW) else 0) |
-                 (8 if ready else 0))
-        wrote = ctypes.c_int(0)
+        flags = (1 if self.inputThreshold is not None else 0) | (2 if _in_padded_buffer(input, self.padH, self.padW) else 0)
         _lib.check_status(lib.thgpu_SpatialConvolutionMM_backward(
             input._p, gradOutput._p, self.weight._p, self.gradWeight._p, self.gradBias._p, self.finput._p, self.fgradInput._p,
-            self.gradInput._p, *(self._geom() + (float(scale), flags, float(self.inputThreshold or 0.0),
-                                                 twin._p if twin is not None else None, ctypes.byref(wrote)))))
-        self._wrote_twin = bool(wrote.value)
+            self.gradInput._p, *(self._geom() + (float(scale), flags, float(self.inputThreshold or 0.0), None, None))))
         return self.gradInput
 
     def accGradParameters(self, input, gradOutput, scale=1):
@@ -560,10 +531,10 @@ class SpatialConvolutionMM(Module):
             *(self._geom() + (float(scale),))))
 
 
-def _own_passes(module, cls=SpatialConvolutionMM):
-    """Whether updateGradInput and accGradParameters of a module are those of `cls`: neither overridden by a derived class nor
-    set on the module."""
-    return all(getattr(getattr(module, m), "__func__", None) is getattr(cls, m)
+def _own_passes(module):
+    """Whether updateGradInput and accGradParameters of a module are SpatialConvolutionMM's: neither overridden by a derived
+    class nor set on the module."""
+    return all(getattr(getattr(module, m), "__func__", None) is getattr(SpatialConvolutionMM, m)
                for m in ("updateGradInput", "accGradParameters"))
 
 

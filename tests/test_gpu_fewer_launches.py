@@ -1,5 +1,7 @@
 """Operators that stand for several launches: parameter updates of many tensors at once, nn.Linear's bias in the store of
 its product and its bias gradient as one sum, the one-launch bias gradient of small convolution layers."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -251,10 +253,10 @@ def test_backward_with_shared_or_strided_tensors(gt):
 
 @pytest.mark.parametrize("case", ["fused", "plain", "derived module"])
 def test_container_backward_gives_what_its_two_passes_give(gt, case):
-    """Module by module against updateGradInput and then accGradParameters of the whole container, bit for bit."""
+    """Against updateGradInput and then accGradParameters of the whole container, bit for bit."""
     nn = gt.nn
 
-    class Noted(nn.ReLU):  # of another file: the container walks back in the plain order
+    class Noted(nn.ReLU):  # of another file
         def accGradParameters(self, input, gradOutput, scale=1):
             seen.append("accGradParameters")
 
@@ -292,6 +294,90 @@ def test_container_backward_gives_what_its_two_passes_give(gt, case):
             got.append([net.gradInput.float()] + [g.float() for g in net.parameters()[1]])
         assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(*got))
     assert seen == (["updateGradInput", "accGradParameters"] * 4 if case == "derived module" else [])
+
+
+@pytest.mark.parametrize("where", ["outer", "nested"])
+def test_container_backward_keeps_the_order_of_its_passes(gt, where):
+    """gradInput of every module before the first accGradParameters, nested containers included: a module that changes its
+    gradInput while it accumulates does not change what the modules in front of it receive."""
+    nn = gt.nn
+
+    class Cleared(nn.ReLU):
+        def accGradParameters(self, input, gradOutput, scale=1):
+            self.gradInput.zero()
+
+    def stack(cls):
+        rng = rng_for(412)
+        net = nn.Sequential().add(nn.SpatialConvolutionMM(3, 64, 3, 3, 1, 1, 1, rng=rng))
+        tail = [cls(), nn.View(64 * 36), nn.Linear(64 * 36, 5, rng=rng)]
+        if where == "nested":
+            inner = nn.Sequential()
+            for m in tail:
+                inner.add(m)
+            net.add(inner)
+        else:
+            for m in tail:
+                net.add(m)
+        return net.gpu()
+
+    rng = rng_for(413)
+    x, go = dev(gt, uniform(rng, (2, 3, 6, 6))), dev(gt, uniform(rng, (2, 5)))
+    got = []
+    for cls in (Cleared, nn.ReLU):
+        net = stack(cls)
+        net.zeroGradParameters()
+        net.forward(x)
+        got.append(net.backward(x, go).float())
+    assert np.any(got[1] != 0) and np.array_equal(got[0], got[1])
+
+
+def test_container_backward_that_fails_accumulates_nothing(gt):
+    """The first module meets an input of another size when every module behind it has its gradInput."""
+    nn = gt.nn
+    net = nn.Sequential().add(nn.SpatialConvolutionMM(3, 64, 3, 3, 1, 1, 1)).add(nn.ReLU())
+    net.add(nn.SpatialConvolutionMM(64, 64, 3, 3, 1, 1, 1)).gpu()
+    rng = rng_for(414)
+    x, go = dev(gt, uniform(rng, (2, 3, 9, 9))), dev(gt, uniform(rng, (2, 64, 9, 9)))
+    net.zeroGradParameters()
+    net.forward(x)
+    with pytest.raises(gt._lib.THGPUError):
+        net.backward(dev(gt, uniform(rng, (2, 3, 8, 9))), go)
+    assert all(np.all(g.float() == 0) for g in net.parameters()[1])
+    net.backward(x, go)
+    assert all(np.any(g.float() != 0) for g in net.parameters()[1])
+
+
+def test_backward_with_a_second_copy_of_gradinput(gt):
+    """thgpu_SpatialConvolutionMM_backward between two convolutions, as a caller that walks back module by module has it: gradOutput
+    already in the layer's padded buffer, gradInput stored in the next one's too, against the two calls, bit for bit."""
+    lib, nn = gt._lib.lib, gt.nn
+    rng = rng_for(415)
+    x, go = dev(gt, uniform(rng, (2, 64, 9, 9))), dev(gt, uniform(rng, (2, 64, 9, 9)))
+    got = []
+    for merged in (True, False):
+        front = nn.SpatialConvolutionMM(64, 64, 3, 3, 1, 1, 1, rng=rng_for(416)).gpu()
+        behind = nn.SpatialConvolutionMM(64, 64, 3, 3, 1, 1, 1, rng=rng_for(417)).gpu()
+        for _ in range(2):
+            behind.zeroGradParameters()
+            mid = front.forward(x)
+            behind.forward(mid)
+            twin = front._gradOutputTwin(x)
+            if merged:
+                wrote = ctypes.c_int(-1)
+                gt._lib.check_status(lib.thgpu_SpatialConvolutionMM_backward(
+                    mid._p, go._p, behind.weight._p, behind.gradWeight._p, behind.gradBias._p, behind.finput._p,
+                    behind.fgradInput._p, behind.gradInput._p, *(behind._geom() + (1.0, 0, 0.0, twin._p if twin is not None else None,
+                                                                                  ctypes.byref(wrote)))))
+                stored = wrote.value
+            else:
+                behind._updateGradInputTwin(mid, go, twin, False)
+                stored = int(behind._wrote_twin)
+                behind.accGradParameters(mid, go, 1)
+            gi = front._updateGradInputTwin(x, behind.gradInput, None, stored == 1)
+            got.append([stored] + [t.float() for t in (gi, behind.gradInput, behind.gradWeight, behind.gradBias)])
+    for a, b in ((got[0], got[2]), (got[1], got[3])):
+        assert a[0] == b[0] and all(np.array_equal(u.view(np.uint32), v.view(np.uint32)) for u, v in zip(a[1:], b[1:]))
+    assert got[1][0] == 1
 
 
 @pytest.mark.parametrize("shape,targets", [((1,), [1]), ((7,), [7]), ((3, 5), [0, 5, 6]), ((130, 3), None), ((2, 1000), [1000, 1])])
