@@ -531,11 +531,13 @@ class SpatialConvolutionMM(Module):
             *(self._geom() + (float(scale),))))
 
 
+_CONV_PASSES = tuple((m, getattr(SpatialConvolutionMM, m)) for m in ("updateGradInput", "accGradParameters"))
+
+
 def _own_passes(module):
-    """Whether updateGradInput and accGradParameters of a module are SpatialConvolutionMM's: neither overridden by a derived
-    class nor set on the module."""
-    return all(getattr(getattr(module, m), "__func__", None) is getattr(SpatialConvolutionMM, m)
-               for m in ("updateGradInput", "accGradParameters"))
+    """Whether updateGradInput and accGradParameters of a module are the two above: neither overridden by a derived class, nor set
+    on the module, nor replaced on the class since."""
+    return all(getattr(getattr(module, m), "__func__", None) is own for m, own in _CONV_PASSES)
 
 
 class Linear(Module):

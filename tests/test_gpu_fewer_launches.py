@@ -251,6 +251,17 @@ def test_backward_with_shared_or_strided_tensors(gt):
     assert np.array_equal(got[0], 0.5 * ref[0]) and np.array_equal(got[1], ref[1])
 
 
+def test_backward_calls_a_pass_that_replaces_the_class_own(gt, monkeypatch):
+    conv, seen = gt.nn.SpatialConvolutionMM, []
+    for name in ("updateGradInput", "accGradParameters"):
+        own = getattr(conv, name)
+        monkeypatch.setattr(conv, name, lambda self, *args, own=own, name=name: (seen.append(name), own(self, *args))[1])
+        m = conv(3, 64, 3, 3, 1, 1, 1).gpu()
+        x = gt.GPUTensor(1, 3, 9, 9).fill(1)
+        m.backward(x, m.forward(x))
+        assert seen == (["updateGradInput"] if name == "updateGradInput" else ["updateGradInput", "updateGradInput", name])
+
+
 @pytest.mark.parametrize("case", ["fused", "plain", "derived module"])
 def test_container_backward_gives_what_its_two_passes_give(gt, case):
     """Against updateGradInput and then accGradParameters of the whole container, bit for bit."""
