@@ -121,6 +121,18 @@ __global__ __launch_bounds__(256) void nll_gradient_kernel(const float *__restri
     gin[idx] = v;
 }
 
+// Whether nll_gradient_kernel beats zeroing and a lane per frame.  It reads every target for every element of the frame, where
+// the two launches cost 3 us more and a quarter of a microsecond per target, and its single stores stream at half the rate:
+//   elements x targets per frame    one launch         two
+//     128 K x 1, 16, 100, 1000      3.4, 4, 15, 135    6.8, 7.3, 30, 250 us
+//     640 K x 100                   31                 25
+//     1 M x 8, 16                   6.6, 10.2          6.8, 8.1
+//     2 M x 2, 4                    5.7, 7.6           6.8, 6.8
+//     4 M x 1, 8                    7.5, 19            6.8, 8.4
+inline bool nll_in_one_launch(long elements, long targets) {
+    return elements <= (3L << 20) && (elements - (1L << 19)) * targets <= (1L << 22);
+}
+
 // nframe x dim of a vector or matrix; 0 on success.
 int frames(const THGPUTensor *t, long &nframe, long &dim) {
     if (t->nDimension == 1) {
@@ -243,7 +255,7 @@ static int nll_gradient(THGPUTensor *input, THGPUTensor *target, THGPUTensor *gr
     if (!tg) return 1;
     float grad = -1.0f;
     if (input->nDimension == 2 && sizeAverage) grad /= (float)nframe;
-    if (whole && nframe * ndim < (1L << 31)) {
+    if (whole && nll_in_one_launch(nframe * ndim, ntarget)) {
         LaunchScope scope("nll_bwd", 0.0, 4.0 * nframe * (ndim + ntarget));
         hipLaunchKernelGGL(nll_gradient_kernel, dim3((unsigned)((nframe * ndim + 255) / 256)), dim3(256), 0, st, dptr(tg),
                            dptr(gradInput), (unsigned)(nframe * ndim), FastDiv((uint32_t)ndim), ndim, ntarget, grad);

@@ -404,3 +404,27 @@ def test_criterion_gradient_of_one_launch(gt, shape, targets):
         if 1 <= k <= n:
             ref[i, k - 1] = -1.0 / frames if len(shape) == 2 else -1.0
     assert np.array_equal(got, ref.reshape(shape))
+
+
+# elements and targets a frame on either side of the lines between one launch and two
+@pytest.mark.parametrize("frames,n,targets,launches", [(50, 10, 1, 1), (128, 1000, 100, 1), (64, 10000, 100, 2), (768, 4096, 1, 1),
+                                                       (769, 4096, 1, 2), (1024, 2000, 4, 2), (4096, 1000, 8, 2)])
+def test_criterion_gradient_takes_one_launch_where_that_is_less_work(gt, frames, n, targets, launches):
+    rng = rng_for(418)
+    t = rng.integers(0, n + 2, size=(frames, targets)).astype(np.float32)
+    c, x, dt = gt.nn.ClassNLLCriterion().gpu(), gt.GPUTensor(frames, n).fill(0), dev(gt, t)
+    c.gradInput = gt.GPUTensor(frames, n).fill(np.nan)
+    gt.gputorch.synchronize()
+    gt.gputorch.prof_reset()
+    gt.gputorch.prof_enable(True)
+    try:
+        got = c.backward(x, dt)
+        gt.gputorch.synchronize()
+        report = gt.gputorch.prof_report()
+    finally:
+        gt.gputorch.prof_enable(False)
+        gt.gputorch.prof_reset()
+    ref = np.zeros((frames, n + 2), np.float32)
+    np.put_along_axis(ref, t.astype(np.int64), np.float32(-1.0 / frames), 1)
+    assert np.array_equal(got.float(), ref[:, 1:-1])
+    assert sum(r["calls"] for r in report.values()) == launches, report
