@@ -234,14 +234,14 @@ GemmProblem gradweight_problem(long B, int C, int H, int W, int M, int kH, int k
     return p;
 }
 
-// gradInput's sum on columns, in additions in a row: over the output planes in the product, over the taps that meet a pixel in
-// col2im.  The gathered product has one sum over both instead, M*kH*kW/16 additions on a tile that does not sum in two levels,
-// and its results were up to 1.7 times as far from 64 bits for it (44 -> 58 planes 5x5, 73 images 54x58: 1.78e-7, on columns
-// 1.07e-7; 96 -> 256 planes 5x5, 64 images 27x27 in four parts: 1.90e-7, 1.24e-7).  Where columns are an alternative, the
-// gathered product takes a tile and split that add up no more than they do (GemmProblem::max_chain), or is not taken: these
-// two layers 1.04e-7 and 1.26e-7, 291 -> 331 and 390 -> 444 us (columns 666 and 505).
-double column_chain(int M, int kH, int kW, double positions_per_pixel) {
-    return (M + GEMM_BK - 1) / GEMM_BK + kH * kW * positions_per_pixel;
+// What gradInput is rounded on columns: over the output planes in the product, over the taps that meet a pixel in col2im.  The
+// gathered product has one sum over both instead, M*kH*kW/16 steps on a tile that does not sum in two levels, and its results
+// were up to 1.7 times as far from 64 bits for it (44 -> 58 planes 5x5, 73 images 54x58: 1.78e-7, on columns 1.07e-7; 96 -> 256
+// planes 5x5, 64 images 27x27 in four parts: 1.90e-7, 1.24e-7).  Where columns are an alternative, the gathered product takes a
+// tile and split that round no more than they do (GemmProblem::max_roundings), or is not taken: these two layers 1.04e-7 and
+// 1.26e-7, 291 -> 331 and 390 -> 444 us (columns 666 and 505).
+double column_roundings(int M, int kH, int kW, double positions_per_pixel) {
+    return gemm_roundings((M + GEMM_BK - 1) / GEMM_BK) + gemm_roundings(kH * kW * positions_per_pixel);
 }
 
 // Unit stride only: one column per input pixel, one reduction index per (output plane, tap).
@@ -265,7 +265,7 @@ GemmProblem gradinput_problem(long B, int C, int H, int W, int M, int kH, int kW
     // Planes that fill 64-row tiles to eight ninths, little work on pixels that no position covers: gathered by every tile
     // (conv_use_gathered_gradinput).
     const bool fills = C >= 64 && (C + 63L) / 64 * 64 * 8 <= C * 9L && ((long)H * W - Ho * Wo) * M <= 110L * Ho * Wo;
-    if (!fills && conv_mode() == 1) p.max_chain = column_chain(M, kH, kW, (double)Ho * Wo / ((double)H * W));
+    if (!fills && conv_mode() == 1) p.max_roundings = column_roundings(M, kH, kW, (double)Ho * Wo / ((double)H * W));
     return p;
 }
 
@@ -317,7 +317,7 @@ GemmProblem gradinput_strided_problem(long B, int C, int H, int W, int M, int kH
     p.tag = "gemm_conv_gradinput";
     // (residue classes that fill 64-row tiles with less than twice the layer's work: gathered by every tile)
     const bool fills = (q.rows < 64 ? 64.0 : q.rows) * q.A * q.Bk <= 2.0 * C * kH * kW;
-    if (!fills && conv_mode() == 1) p.max_chain = column_chain(M, kH, kW, (double)Ho * Wo / ((double)H * W));
+    if (!fills && conv_mode() == 1) p.max_roundings = column_roundings(M, kH, kW, (double)Ho * Wo / ((double)H * W));
     return p;
 }
 
@@ -484,14 +484,14 @@ bool conv_use_gathered_gradinput(long B, int C, int H, int W, int M, int kH, int
     if (mode == 2) return strided || C >= 64;
     // Unit stride, planes that fill 64-row tiles, little work on pixels that no position covers: gathered, on any tile (for single
     // images too, where the columns are up to 30 % faster).
-    if (!strided && gradinput_problem(B, C, H, W, M, kH, kW, pH, pW).max_chain == 0.0) return true;
+    if (!strided && gradinput_problem(B, C, H, W, M, kH, kW, pH, pW).max_roundings < 0.0) return true;
     // A strided layer whose residue classes take less than twice its work and fill the GPU keeps the one product until the
     // columns are a third faster by estimate: their col2im is the part that the estimate knows least (3 -> 96 planes 11x11
     // stride 4, 24 to 128 images: columns 1.15 to 1.3 times the gathered time, and a fused stack saves the padded copy as well).
     double margin = 1.0;
     if (strided) {
         const GemmProblem p = gradinput_strided_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
-        if (p.max_chain == 0.0 && p.J >= 16384) margin = 1.35;
+        if (p.max_roundings < 0.0 && p.J >= 16384) margin = 1.35;
     }
     return gathered_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW) <=
            margin * column_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW);

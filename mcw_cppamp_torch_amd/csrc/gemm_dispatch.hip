@@ -236,15 +236,14 @@ double model_cycles(const TileCfg &c, int layout, long M, long J, long steps_tot
 // Few outputs and many splits: four wavefronts share 64 outputs of the split reduction (reduce_job).
 inline bool reduced_in_quarters(long outputs, int nsplit) { return outputs > 0 && outputs < 128 * 1024 && nsplit >= 12; }
 
-// Additions in a row on the way to one output, level by level: a wavefront's steps, its workgroup's groups, the parts.  n
-// roundings of a sum that grows evenly to its full size come to n / 2 times the mean square of one of the full sum, and levels
-// add up, so this is what an order of summation is judged by.
-double plan_chain(const TileCfg &c, long outputs, int steps_total, int nsplit) {
-    const int steps = (int)cdiv(cdiv(steps_total, nsplit), c.groups);
-    double n = steps;
-    if (c.folds && gemm_fold_steps(steps) < steps) n = gemm_fold_steps(steps) + (double)steps / gemm_fold_steps(steps);
-    if (c.groups > 1) n += c.groups;
-    if (nsplit > 1) n += reduced_in_quarters(outputs, nsplit) ? (double)cdiv(nsplit, 4) + 4.0 : nsplit;
+// What one output of a plan is rounded, level by level (gemm_roundings): a wavefront's steps, its workgroup's groups, the parts.
+double plan_roundings(const TileCfg &c, long outputs, int steps_total, int nsplit) {
+    const long part = cdiv(steps_total, nsplit), walk = cdiv(part, c.groups);
+    const int f = gemm_fold_steps((int)walk);
+    double n = c.folds && f < walk ? gemm_roundings(f) + gemm_roundings((double)walk / f) : gemm_roundings((double)walk);
+    if (c.groups > 1 && walk > 0) n += gemm_roundings((double)cdiv(part, walk));
+    if (nsplit > 1)
+        n += reduced_in_quarters(outputs, nsplit) ? gemm_roundings((double)cdiv(nsplit, 4)) + gemm_roundings(4) : gemm_roundings(nsplit);
     return n;
 }
 
@@ -288,8 +287,8 @@ GemmPlan rank_plans(const GemmProblem &p, int steps_total, bool any) {
         if (force && std::strcmp(force, c.name) != 0) continue;
         if (!force && c.below_rows > 0 && p.M >= c.below_rows) continue;
         if (c.a_rc_only && !p.a_rc) continue;
-        if (c.folds && (layout != 4 || (!force && p.max_chain <= 0.0))) continue;
-        const double best_chain = plan.cfg ? plan_chain(*plan.cfg, (long)p.M * p.J, steps_total, plan.nsplit) : 0.0;  // so far
+        if (c.folds && (layout != 4 || (!force && p.max_roundings < 0.0))) continue;
+        const double best_roundings = plan.cfg ? plan_roundings(*plan.cfg, (long)p.M * p.J, steps_total, plan.nsplit) : 0.0;
         const long tiles = cdiv(p.M, c.bm) * cdiv(p.J, c.bn);
         // (a product run wider than its result has one narrow tile per row block: it may split further to fill the GPU)
         const int split_cap = p.j_store > 0 ? 1024 : 256;
@@ -305,11 +304,11 @@ GemmPlan rank_plans(const GemmProblem &p, int steps_total, bool any) {
             const int sps = (int)cdiv(steps_total, ns);
             if (sps > 0 && (int)cdiv(steps_total, sps) != ns) continue;  // would leave an empty split
             if (!force && fsplit <= 0) {
-                const double chain = plan_chain(c, (long)p.M * p.J, steps_total, ns);
-                if (p.max_chain > 0.0 && chain > p.max_chain) continue;
+                const double roundings = plan_roundings(c, (long)p.M * p.J, steps_total, ns);
+                if (p.max_roundings >= 0.0 && roundings > p.max_roundings) continue;
                 // (the tile of groups, the last one, does with fewer parts what the others split further: not at the price of
                 // longer sums, 282 x 294 over 2272 steps in 85 parts 1.41e-7 from 64 bits, in 10 of four groups 1.61e-7)
-                if (c.groups > 1 && plan.cfg && chain > best_chain) continue;
+                if (c.groups > 1 && plan.cfg && roundings > best_roundings) continue;
             }
             if (any) {
                 plan.cfg = &c;
@@ -347,7 +346,7 @@ GemmPlan plan_gemm(const GemmProblem &p, int steps_total) {
                           (p.a_rc ? 1 : 0) + (p.b_rc ? 2 : 0) + (p.rowtab ? 4 : 0) + (p.scatter ? 8 : 0) + (p.C2 ? 16 : 0), p.j_store,
                           p.sA, p.sB, p.sC, p.bsB, p.bsC, p.b_extent, p.C2 ? p.c2_sC : 0, p.C2 ? p.c2_bsC : 0,
                           p.C2 ? p.c2_pitch : 0, p.C2 ? p.c_w : 0, p.ws_fixed ? 1 : 0, p.ws_fixed ? p.ws_fixed_floats : 0, p.beta != 0.0f,
-                          (long)(16.0 * p.max_chain)}};
+                          (long)(4096.0 * p.max_roundings)}};
     {
         std::lock_guard<std::mutex> lock(mutex);
         const auto it = plans.find(key);
@@ -372,7 +371,7 @@ inline int steps_of(const GemmProblem &p) {
 bool gemm_tiled_fits(const GemmProblem &p) {
     if (p.M <= 0 || p.J <= 0 || (long)p.M * p.J >= (1L << 31)) return false;
     // (where the first tile and split will not do, the answer is the planner's, which keeps it)
-    return (p.max_chain > 0.0 ? plan_gemm(p, steps_of(p)) : rank_plans(p, steps_of(p), true)).cfg != nullptr;
+    return (p.max_roundings >= 0.0 ? plan_gemm(p, steps_of(p)) : rank_plans(p, steps_of(p), true)).cfg != nullptr;
 }
 
 double gemm_estimate_us(const GemmProblem &p) {

@@ -224,7 +224,7 @@ __device__ __forceinline__ void finish_groups(const GemmArgs &g, char *lds_a, ch
 }
 
 // One workgroup of a product; As and Bs hold KG pairs of operand tiles.  FOLD: every g.fold_steps steps (an even number) a
-// wavefront's sum goes to a second one and starts over (gemm_chain).
+// wavefront's sum goes to a second one and starts over (gemm_roundings).
 template <int BM, int BN, int WGM, int WGN, int LA, int LB, bool RED, int KG, bool FOLD = false>
 __device__ __forceinline__ void gemm_fast_tile(const GemmArgs &g, const unsigned block, char *const As, char *const Bs) {
     constexpr int NT = WGM * WGN * 64;  // threads of a group: the whole workgroup unless KG > 1

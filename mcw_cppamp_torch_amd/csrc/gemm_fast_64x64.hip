@@ -10,7 +10,7 @@ int gemm_fast_64x64(const GemmArgs &g, int la, int lb, bool red, hipStream_t s) 
 }
 
 // Summing in two levels, for gathered gradInput products whose single long sum would be rounded more than the short ones that
-// col2im adds up (GemmProblem::max_chain).  A kernel of its own: with one more block of sums (93 -> 117 registers) four workgroups run on
+// col2im adds up (GemmProblem::max_roundings).  A kernel of its own: with one more block of sums (93 -> 117 registers) four workgroups run on
 // a CU where five did, which costs the other products of this tile 1 to 3 %.  134 planes from 495 indices (3x3, 57 images 19x19): 1.10e-7 -> 7.7e-8
 // from 64 bits (columns 7.7e-8), 49.6 -> 50.1 us.
 int gemm_fast_64x64f(const GemmArgs &g, int la, int lb, bool red, hipStream_t s) {

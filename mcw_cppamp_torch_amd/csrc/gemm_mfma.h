@@ -88,9 +88,9 @@ struct GemmProblem {
     // the narrowest tile runs on the tiled kernels: its column table is padded with entries that repeat a valid one.
     // The reduction is always split (the partial sums are J wide, the final pass stores j_store).  0: all J columns.
     int j_store = 0;
-    // Only tiles and splits with no more than so many additions in a row on the way to a result (plan_chain in
-    // gemm_dispatch.hip) are considered, unless a tile or split is forced.  0: all, but the tile that sums in two levels.
-    double max_chain = 0.0;
+    // Only tiles and splits whose results are rounded no more than so often (gemm_roundings) are considered, unless a tile or
+    // split is forced.  Negative: all, but the tile that sums in two levels.
+    double max_roundings = -1.0;
     const char *tag = "gemm";     // name used by per-kernel timing
     // Flops the per-kernel timing credits the launch with; 0 means the product's own 2*M*J*R*nb.  A
     // convolution pass sets its algorithmic 2*M*N*K*B here, which a gathered gradInput product (one
@@ -119,6 +119,10 @@ double gemm_estimate_us(const GemmProblem &p);
 
 constexpr int GEMM_BK = 16;  // reduction step of every kernel
 constexpr int GEMM_SHORT_TILE = 64;  // a tile side up to this length also takes a matrix that is shorter (gemm_fast.h)
+
+// A sum of n terms of one size added up one after the other, in roundings of the full sum: the first is exact, and the square of
+// the error of adding the k-th goes with k / n.  Sums of sums add up.
+inline double gemm_roundings(double n) { return n > 1.0 ? (n + 1.0) / 2.0 - 1.0 / n : 0.0; }
 
 // The tile that sums in two levels (gemm_fast_64x64f) moves its sum to the second one after an even number of steps (they come
 // in pairs) near the root of those that it walks.
