@@ -408,7 +408,7 @@ def _short(name):
     return re.sub(r"\(.*", "", name)
 
 
-FAMILIES = [("gemm_fast", "gemm"), ("gemm_generic", "gemm"), ("im2col", "im2col"), ("col2im", "col2im"),
+FAMILIES = [("gemm_fast", "gemm"), ("gemm_generic", "gemm"), ("gemm_pair", "gemm"), ("im2col", "im2col"), ("col2im", "col2im"),
             ("maxpool_bwd", "maxpool_bwd"), ("maxpool_fwd", "maxpool_fwd"), ("threshold_fwd", "threshold_fwd"),
             ("threshold_bwd", "threshold_bwd"), ("split_reduce", "gemm_split_reduce"),
             ("gradbias_partial", "gradbias"), ("gradbias_final", "gradbias_final"), ("fill_kernel", "fill"),

@@ -545,11 +545,16 @@ const char *product_label(const Prepared &q) {
                                         (long)p.R * (q.red ? p.nb : 1), q.best ? q.best->name : "generic", q.g.nsplit);
 }
 
+double product_flops(const Prepared &q) {
+    const GemmProblem &p = *q.p;
+    return p.flops > 0 ? p.flops : 2.0 * p.M * p.J * (double)p.R * (q.red ? p.nb : 1);
+}
+
 int run_product(const Prepared &q, hipStream_t s) {
     const GemmProblem &p = *q.p;
     int rc;
     {
-        LaunchScope scope(product_label(q), p.flops > 0 ? p.flops : 2.0 * p.M * p.J * (double)p.R * (q.red ? p.nb : 1), 0.0);
+        LaunchScope scope(product_label(q), product_flops(q), 0.0);
         rc = q.best ? q.best->launch(q.g, q.la, q.lb, q.red, s) : gemm_generic_64x64(q.g, p.a_rc, p.b_rc, q.red, s);
     }
     return rc ? rc : check_launch(p.tag);
@@ -661,7 +666,15 @@ int gemm_launch_pair(const GemmProblem &a, const GemmProblem &b) {
         if (qb.ws_floats > 0) use_workspace(qb, ws + first);
     }
     if (qa.best && qb.best && qa.best->groups > 1 && qb.best->groups > 1 &&
-        gemm_fast_64x64k4_pair(qa.g, qa.la, qa.lb, qa.red, qb.g, qb.la, qb.lb, qb.red, s) == 0) {
+        gemm_fast_64x64k4_pairs(qa.la, qa.lb, qa.red, qb.la, qb.lb, qb.red)) {
+        const char *label = "gemm_conv_backward";
+        if (prof_enabled())
+            label = prof_label("%s M=%d+%d J=%d+%d R=%d+%ld tile=%s split=%d+%d", label, a.M, b.M, a.J, b.J, a.R,
+                               (long)b.R * b.nb, qa.best->name, qa.g.nsplit, qb.g.nsplit);
+        {
+            LaunchScope scope(label, product_flops(qa) + product_flops(qb), 0.0);
+            if (gemm_fast_64x64k4_pair(qa.g, qb.g, qb.lb, s)) return 1;
+        }
         if (check_launch(a.tag)) return 1;
     } else if (run_product(qa, s) || run_product(qb, s)) {
         return 1;

@@ -202,10 +202,9 @@ int gemm_fast_192x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s
 int gemm_fast_128x256(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_256x128(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 int gemm_fast_64x64k4(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
-// A convolution's gradInput product (a) and its gradWeight product (b) in one launch; non-zero, and nothing launched, for
-// other loaders.
-int gemm_fast_64x64k4_pair(const GemmArgs &a, int la, int lb, bool red, const GemmArgs &b, int la2, int lb2, bool red2,
-                           hipStream_t s);
+// A convolution's gradInput product (a) and its gradWeight product (b) in one launch, and whether the loaders are theirs.
+bool gemm_fast_64x64k4_pairs(int la, int lb, bool red, int la2, int lb2, bool red2);
+int gemm_fast_64x64k4_pair(const GemmArgs &a, const GemmArgs &b, int lb2, hipStream_t s);
 int gemm_fast_64x64(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);
 // The same tile, summing in two levels: gathering products without reduction batching.
 int gemm_fast_64x64f(const GemmArgs &g, int la, int lb, bool red, hipStream_t s);

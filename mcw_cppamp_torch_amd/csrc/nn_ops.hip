@@ -493,8 +493,7 @@ int conv_backward(THGPUTensor *input, THGPUTensor *gradOutput, THGPUTensor *weig
     };
     if (wrote_twin) *wrote_twin = 0;
     ConvShape s;
-    // (with per-kernel timing on every launch is a record of its own, so none is shared)
-    if (prof_enabled() || !gradOutput || !gradWeight || !gradBias || !finput || !fgradInput || !gradInput ||
+    if (!gradOutput || !gradWeight || !gradBias || !finput || !fgradInput || !gradInput ||
         conv_shape(s, input, weight, kW, kH, dW, dH, padW, padH))
         return one_by_one();
     PlaneLayout in_layout;

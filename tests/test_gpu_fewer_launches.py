@@ -167,7 +167,8 @@ print("allocations", lib.thgpu_device_alloc_calls() - before)
 
 
 BACKWARD = {  # B, C, H, W, M, kH, kW, pH, pW, sH, sW
-    "one_image": (1, 96, 13, 13, 70, 3, 3, 1, 1, 1, 1),       # both products on the tile of four groups, both split
+    "one_image": (1, 96, 13, 13, 70, 3, 3, 1, 1, 1, 1),       # 96 planes do not fill 64-row tiles: gradInput on columns
+    "groups": (1, 128, 13, 13, 70, 3, 3, 1, 1, 1, 1),         # both products on the tile of four groups, both split
     "quads": (2, 64, 8, 12, 64, 3, 3, 1, 1, 1, 1),
     "few_rows": (3, 64, 10, 9, 20, 3, 3, 1, 1, 1, 1),
     "no_padding": (2, 64, 9, 9, 64, 3, 3, 0, 0, 1, 1),
@@ -204,6 +205,55 @@ def test_backward_gives_what_its_two_passes_give(gt, name, threshold):
             outs.append([t.float() for t in (gi, m.gradWeight, m.gradBias)])
         for a, b in zip(*outs):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+def launches(gt, call):
+    """{label's family: calls} of what a call enqueues."""
+    gt.gputorch.synchronize()
+    gt.gputorch.prof_reset()
+    gt.gputorch.prof_enable(True)
+    try:
+        call()
+        gt.gputorch.synchronize()
+        found = {}
+        for label, r in gt.gputorch.prof_report().items():
+            family = label.split(" ")[0]
+            found[family] = found.get(family, 0) + r["calls"]
+        return found
+    finally:
+        gt.gputorch.prof_enable(False)
+        gt.gputorch.prof_reset()
+
+
+# name -> what one call enqueues and what the two passes do
+_TWO = {"gemm_conv_gradinput": 1, "gemm_conv_gradweight": 1}
+SHARED = {
+    "groups": ({"pad_planes": 1, "gemm_conv_backward": 1, "gemm_split_reduce": 1}, {"pad_planes": 2, "gemm_split_reduce": 2, **_TWO}),
+    "quads": ({"pad_planes": 1, "gemm_conv_backward": 1, "gemm_split_reduce": 1}, {"pad_planes": 2, "gemm_split_reduce": 2, **_TWO}),
+    "no_padding": ({"pad_planes": 1, "gemm_conv_backward": 1, "gemm_split_reduce": 1}, {"pad_planes": 1, "gemm_split_reduce": 2, **_TWO}),
+    "wide": ({"pad_planes": 1, "gemm_split_reduce": 1, **_TWO}, {"pad_planes": 2, "gemm_split_reduce": 2, **_TWO}),
+    "columns": (None, None),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SHARED))
+def test_backward_shares_launches(gt, name):
+    """What per-kernel timing sees is what runs without it, and where both products gather it is fewer launches than two passes
+    make; a layer with columns in one of them makes the same."""
+    B, C, H, W, M, kH, kW, pH, pW, sH, sW = BACKWARD[name]
+    rng = rng_for(419)
+    m = gt.nn.SpatialConvolutionMM(C, M, kW, kH, sW, sH, 0, padW=pW, padH=pH, rng=rng_for(420)).gpu()
+    x = dev(gt, uniform(rng, (B, C, H, W)))
+    go = dev(gt, uniform(rng, m.forward(x).size()))
+    for _ in range(2):
+        shared = launches(gt, lambda: m.backward(x, go))
+        apart = launches(gt, lambda: (m.updateGradInput(x, go), m.accGradParameters(x, go)))
+    print(name, shared, apart)
+    want = SHARED[name]
+    if want[0] is None:
+        assert shared == apart and "col2im" in shared
+    else:
+        assert (shared, apart) == want
 
 
 def test_backward_with_shared_or_strided_tensors(gt):
