@@ -503,19 +503,17 @@ int conv_backward(THGPUTensor *input, THGPUTensor *gradOutput, THGPUTensor *weig
                        tensor_ready(gradOutput, s.B * s.M * s.N) && tensor_ready(weight, (long)s.M * s.K) &&
                        tensor_ready(gradWeight, (long)s.M * s.K) && gradWeight->nDimension == 2 && gradWeight->size[1] == s.K &&
                        tensor_ready(gradBias, s.M) && direct == input_in_padded_buffer;
-    // the first five are written, all but gradWeight and gradBias are read
-    const THGPUTensor *const roles[] = {gradInput, finput, fgradInput, gradWeight, gradBias, input, gradOutput};
+    // the first five and the twin are written, all but gradWeight, gradBias and the twin are read (a weight in finput's memory is
+    // read by the pass before the one that pads the input over it)
+    const THGPUTensor *const roles[] = {gradInput, finput, fgradInput, gradWeight, gradBias, input, gradOutput, weight};
+    auto same = [&](const THGPUTensor *a, const THGPUTensor *b) { return a == b || (owned(a) && owned(a) == owned(b)); };
     bool apart = true;  // (a tensor without a storage is about to get one of its own)
     for (int w = 0; w < 5; ++w)
-        for (int r = 0; r < 7; ++r)
-            if (r != w && r != 3 && r != 4 &&
-                (roles[r] == roles[w] || (owned(roles[w]) && owned(roles[w]) == owned(roles[r]))))
-                apart = false;
-    if (twin && owned(twin) && (owned(twin) == owned(input) || owned(twin) == owned(finput) || owned(twin) == owned(fgradInput) ||
-                                owned(twin) == owned(gradWeight) || owned(twin) == owned(gradBias)))
-        apart = false;
-    if (!dense || !apart || g_finput_reuse || owned(weight) == owned(gradWeight) || owned(weight) == owned(gradBias) ||
-        !conv_use_gathered(s.B, s.C, s.H, s.W, s.M, kH, kW, padH, padW, dH, dW) ||
+        for (int r = 0; r < 8; ++r)
+            if (r != w && r != 3 && r != 4 && same(roles[r], roles[w])) apart = false;
+    for (const THGPUTensor *role : roles)
+        if (twin && same(twin, role)) apart = false;
+    if (!dense || !apart || g_finput_reuse || !conv_use_gathered(s.B, s.C, s.H, s.W, s.M, kH, kW, padH, padW, dH, dW) ||
         !conv_use_gathered_gradinput(s.B, s.C, s.H, s.W, s.M, kH, kW, padH, padW, dH, dW))
         return one_by_one();
 

@@ -301,6 +301,33 @@ def test_backward_with_shared_or_strided_tensors(gt):
     assert np.array_equal(got[0], 0.5 * ref[0]) and np.array_equal(got[1], ref[1])
 
 
+@pytest.mark.parametrize("shared", ["finput in the weight's memory", "second copy in gradOutput's memory"])
+def test_backward_with_a_buffer_that_the_other_pass_reads(gt, shared):
+    """Where one pass writes what the other reads, the two run in their order: gradInput is of the weight as it was, gradWeight
+    of the gradOutput that the store of gradInput left."""
+    lib, rng = gt._lib.lib, rng_for(421)
+    x, go = uniform(rng, (1, 64, 10, 10)), uniform(rng, (1, 64, 10, 10))
+    got = []
+    for merged in (True, False):
+        m = gt.nn.SpatialConvolutionMM(64, 64, 3, 3, 1, 1, 1, rng=rng_for(422)).gpu()
+        m.zeroGradParameters()
+        dx, dgo, twin = dev(gt, x), dev(gt, go), None
+        m.forward(dx)
+        if shared.startswith("finput"):
+            m.finput = gt.GPUTensor().set(m.weight)
+        else:
+            twin = gt.GPUTensor().set(dgo)
+        if merged:
+            gt._lib.check_status(lib.thgpu_SpatialConvolutionMM_backward(
+                dx._p, dgo._p, m.weight._p, m.gradWeight._p, m.gradBias._p, m.finput._p, m.fgradInput._p, m.gradInput._p,
+                *(m._geom() + (1.0, 0, 0.0, twin._p if twin is not None else None, None))))
+        else:
+            m._updateGradInputTwin(dx, dgo, twin, False)
+            m.accGradParameters(dx, dgo, 1)
+        got.append([t.float() for t in (m.gradInput, m.gradWeight, m.gradBias)])
+    assert all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(*got))
+
+
 def test_backward_calls_a_pass_that_replaces_the_class_own(gt, monkeypatch):
     conv, seen = gt.nn.SpatialConvolutionMM, []
     for name in ("updateGradInput", "accGradParameters"):
