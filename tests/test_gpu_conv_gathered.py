@@ -210,7 +210,8 @@ def test_gathered_conv_random_geometry(gt, gathered_route, cfg):
 
 
 @pytest.mark.parametrize("split", [1, 3])
-@pytest.mark.parametrize("tile", ["128x128", "192x128", "64x256", "128x256", "256x128", "64x64", "64x128", "96x128"])
+@pytest.mark.parametrize("tile", ["128x128", "192x128", "64x256", "128x256", "256x128", "64x64", "64x128", "96x128",
+                                  "32x128", "64x64k4"])
 def test_gathered_conv_every_tile_configuration(gt, gathered_route, tile, split, switches):
     """Every tile of the GEMM has its own gathering kernels (plain and reduction-batched); the library's choice
     would leave most of them to the large benchmark shapes, so each is forced here on a shape all of them fit."""
@@ -233,8 +234,8 @@ def test_gathered_conv_every_tile_configuration(gt, gathered_route, tile, split,
 
 
 def test_mode_1_gathers_where_a_tiled_kernel_takes_the_product(gt):
-    """The library's own choice: narrow and wide layers alike compute without columns; a layer too small for the
-    tiled kernels (fewer than 64 output planes) stays on the column route."""
+    """The library's own choice: narrow and wide layers alike compute without columns; a layer of fewer than 64 output planes
+    with little to gather (fewer than 256 positions here) keeps them."""
     lib = gt._lib.lib
     before = lib.thgpu_conv_get_mode()
     assert lib.thgpu_conv_set_mode(1) == 0
@@ -483,11 +484,11 @@ SHORT_ROWS = [
 ]
 
 
-@pytest.mark.parametrize("tile", ["64x128", "64x256"])
+@pytest.mark.parametrize("tile", ["64x128", "64x256", "32x128", "64x64f", "64x64k4"])
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("cfg", SHORT_ROWS)
 def test_strided_gradinput_short_row_kernel_integer_exact(gt, gathered_route, switches, cfg, masked, tile):
-    """A scattered product of fewer than 64 rows runs on a 64-row tile and drops the rows behind its own.  Small integers
+    """A scattered product of fewer rows than its tile drops the rows behind its own.  Small integers
     make every sum exact, so the result must equal the oracle's bit for bit, with and without the fused nn.Threshold
     mask, and nothing outside gradInput may be written."""
     B, C, H, W, kH, kW, pH, pW, sH, sW = cfg
@@ -802,6 +803,66 @@ def test_random_layers_with_a_handful_of_taps_integer_exact(gt, gathered_route, 
     oracle.conv_accGradParameters(go, finput_ref, gw, gb, 3.0)
     m.accGradParameters(dx, dev(gt, go), 3.0)
     assert np.array_equal(m.gradWeight.float(), gw) and np.array_equal(m.gradBias.float(), gb)
+
+
+TWO_LEVELS = [
+    # B, C, H, W, M, kH, kW, pH, pW: the steps of the reduction
+    (2, 64, 9, 7, 2, 3, 3, 1, 1),        # 2, the second partial
+    (3, 70, 11, 13, 24, 3, 3, 1, 1),     # 14, an edge tile in either direction
+    (1, 131, 17, 15, 58, 5, 5, 2, 2),    # 91 and a part
+    (2, 64, 8, 8, 455, 3, 3, 0, 0),      # 256
+]
+
+
+@pytest.mark.parametrize("split", [1, 3])
+@pytest.mark.parametrize("cfg", TWO_LEVELS)
+def test_gradinput_on_the_tile_that_sums_in_two_levels_integer_exact(gt, gathered_route, switches, cfg, split):
+    """Bit for bit on small integers, unsplit and in parts; and with an infinity, a NaN and a number whose bits the bf16 parts do
+    not hold in gradOutput, which wherever they stand reach the pixels that read them and no other."""
+    B, C, H, W, M, kH, kW, pH, pW = cfg
+    geo = (kH, kW, pH, pW, 1, 1)
+    rng = rng_for(54)
+    ints = lambda lo, hi, shape: rng.integers(lo, hi + 1, size=shape).astype(np.float32)
+    x, w = ints(-2, 2, (B, C, H, W)), ints(1, 2, (M, C * kH * kW))
+    go = ints(-2, 2, (B, M, H + 2 * pH - kH + 1, W + 2 * pW - kW + 1))
+    m = gt.nn.SpatialConvolutionMM(C, M, kW, kH, 1, 1, 0, padW=pW, padH=pH)
+    m._assign("weight", w)
+    m.gpu()
+    switches("gemm_tile", "64x64f")
+    switches("gemm_split", split)
+    for value in (None, np.inf, np.nan, np.float32(2.0 ** -120 * (1 + 2.0 ** -23))):
+        if value is not None:
+            go[:] = 0
+            go[B - 1, M - 1, 1, 2] = value
+        with np.errstate(invalid="ignore"):
+            ref, _ = oracle.conv_updateGradInput(go, w, x.shape, *geo)
+        gt.gputorch.synchronize()
+        gt.gputorch.prof_reset()
+        gt.gputorch.prof_enable(True)
+        try:
+            got = m.updateGradInput(dev(gt, x), dev(gt, go)).float()
+            gt.gputorch.synchronize()
+            labels = [k for k in gt.gputorch.prof_report() if k.startswith("gemm_conv_gradinput")]
+        finally:
+            gt.gputorch.prof_enable(False)
+            gt.gputorch.prof_reset()
+        steps = (M * kH * kW + 15) // 16
+        assert len(labels) == 1 and "tile=64x64f split=%d" % min(split, max(1, steps // 8)) in labels[0], labels
+        assert np.array_equal(got, ref, equal_nan=True) if value is None or np.isfinite(value) else \
+            np.array_equal(np.isfinite(got), touched(go, x.shape, geo)), value
+
+
+def touched(go, shape, geo):
+    """Where gradInput stays finite: no tap meets the pixel from a position that is not.  (The products of such a position with
+    the zeros around it are NaN on columns and on the gathered route alike.)"""
+    kH, kW, pH, pW, _, _ = geo
+    B, C, H, W = shape
+    bad = ~np.isfinite(go).all(axis=1)
+    out = np.zeros((B, H + 2 * pH, W + 2 * pW), bool)
+    for kh in range(kH):
+        for kw in range(kW):
+            out[:, kh:kh + bad.shape[1], kw:kw + bad.shape[2]] |= bad
+    return np.broadcast_to(~out[:, None, pH:pH + H, pW:pW + W], shape)
 
 
 def taps(a, kh, kw, Ho, Wo, sH, sW):

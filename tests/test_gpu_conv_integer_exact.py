@@ -21,7 +21,8 @@ pytestmark = pytest.mark.gpu
 import oracle  # noqa: E402
 
 TILES = {"128x128": (128, 128), "192x128": (192, 128), "64x256": (64, 256), "128x256": (128, 256),
-         "256x128": (256, 128), "64x64": (64, 64), "64x128": (64, 128), "96x128": (96, 128)}
+         "256x128": (256, 128), "64x64": (64, 64), "64x128": (64, 128), "96x128": (96, 128),
+         "32x128": (32, 128), "64x64k4": (64, 64)}
 
 SHAPES = {
     # name: B, C, H, W, M, kH, kW, pH, pW, sH, sW
@@ -141,7 +142,7 @@ def test_integer_conv_exact_every_tile_and_split(gt, name, mode, tile, split, sw
     B, C, H, W, M, kH, kW, pH, pW, sH, sW = SHAPES[name]
     K = C * kH * kW
     bm, bn = TILES[tile]
-    if M < bm or K < bn:
+    if (M < bm and bm > 64) or (K < bn and bn > 64):  # (sides of 64 and less take shorter matrices)
         pytest.skip("the gradWeight product (%d x %d) is smaller than the tile" % (M, K))
     switches("gemm_tile", tile)
     switches("gemm_split", split)

@@ -128,6 +128,14 @@ CASES = [
     ({"gemm_tile": "64x64"}, ("conv", 8, 64, 4, 2, 1), 2),   # ... with its rows padded to a tile
     ({"gemm_tile": "96x128"}, ("conv", 96, 100, 3, 1, 1), 2),  # the 96-row tile: thresholded output, masked gradInput
     ({"gemm_tile": "64x128"}, ("conv", 12, 64, 4, 2, 1), 2),   # a masked scattered store of 48 of a tile's 64 rows
+    # the store behind the groups' sums: bias, threshold, mask; in the split reduction instead; masked and scattered
+    ({"gemm_tile": "64x64k4", "gemm_split": "1"}, ("conv", 64, 64, 3, 1, 1), 2),
+    ({"gemm_tile": "64x64k4", "gemm_split": "2"}, ("conv", 70, 100, 3, 1, 1), 2),
+    ({"gemm_tile": "64x64k4"}, ("conv", 12, 64, 4, 2, 1), 2),
+    ({"gemm_tile": "64x64k4", "gemm_split": "1"}, ("conv", 8, 16, 3, 1, 1), 0),
+    ({"gemm_tile": "64x64f"}, ("conv", 64, 64, 3, 1, 1), 2),   # the tile that sums in two levels (gradInput alone)
+    ({"gemm_tile": "64x64f", "gemm_split": "3"}, ("conv", 64, 64, 3, 1, 1), 2),
+    ({"gemm_tile": "32x128"}, ("conv", 12, 64, 4, 2, 1), 2),
 ]
 
 
@@ -242,9 +250,10 @@ TWIN_SPEC = [("conv", 3, 64, 5, 2, 2), ("relu",), ("pool", 3, 2), ("conv", 64, 1
              ("conv", 128, 64, 3, 1, 1), ("relu",), ("pool", 2, 2), ("conv", 64, 64, 5, 1, 2), ("relu",), ("pool", 3, 2)]
 
 
-@pytest.mark.parametrize("forced", [{}, {"gemm_split": "3"}, {"gemm_split": "1"}, {"pool_bwd_tile": "1"},
+@pytest.mark.parametrize("forced", [{}, {"gemm_split": "3"}, {"gemm_split": "1"}, {"gemm_tile": "64x64k4", "gemm_split": "1"},
+                                    {"gemm_tile": "64x64k4", "gemm_split": "3"}, {"pool_bwd_tile": "1"},
                                     {"pool_bwd_cell": "1"}, {"pool_bwd_pixels": "4096"}, {"pool_bwd_pixels": "500"}],
-                         ids=["auto", "split", "unsplit", "pool_tile", "pool_cell", "pool_staged", "pool_staged_strips"])
+                         ids=["auto", "split", "unsplit", "groups", "groups_split", "pool_tile", "pool_cell", "pool_staged", "pool_staged_strips"])
 def test_gradients_written_into_the_next_products_padded_buffer(gt, forced, switches):
     """In a fused Sequential on the gathered route every producer of a convolution's gradOutput (max-pooling backward,
     a unit-stride convolution's gradInput product through its epilogue or its split reduction) also stores it in that

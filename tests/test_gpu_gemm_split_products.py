@@ -102,8 +102,9 @@ def test_results_below_the_normal_range(gt):
 
 
 TILES = {"128x128": (128, 128), "192x128": (192, 128), "64x256": (64, 256), "128x256": (128, 256),
-         "256x128": (256, 128), "64x64": (64, 64), "64x128": (64, 128), "96x128": (96, 128)}
-LAYOUTS = [(tile, ta, tb) for tile in TILES for ta in "nt" for tb in "nt" if not (tile == "96x128" and ta == "t")]
+         "256x128": (256, 128), "64x64": (64, 64), "64x128": (64, 128), "96x128": (96, 128),
+         "32x128": (32, 128), "64x64k4": (64, 64)}
+LAYOUTS = [(tile, ta, tb) for tile in TILES for ta in "nt" for tb in "nt" if not (tile in ("96x128", "32x128") and ta == "t")]
 
 
 def blas(gt, ta, tb, A, B):

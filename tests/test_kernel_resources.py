@@ -9,7 +9,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 BUILD = os.path.join(ROOT, "mcw_cppamp_torch_amd", "build")
 LLVM = "/opt/rocm/llvm/bin"
-TILES = ["128x128", "192x128", "64x256", "128x256", "256x128", "64x64", "64x128", "96x128"]
+TILES = ["128x128", "192x128", "64x256", "128x256", "256x128", "64x64", "64x128", "96x128", "32x128", "64x64k4"]
 
 
 def kernels(obj, tmp_path):
@@ -38,6 +38,7 @@ def test_tiled_gemm_kernels_keep_their_registers(tile, tmp_path):
     if not os.path.exists(LLVM + "/clang-offload-bundler"):
         pytest.skip("no ROCm LLVM tools")
     found = kernels(obj, tmp_path)
-    assert len(found) >= 6 and all("gemm_fast_kernel" in name for name in found)
+    assert len(found) >= 6 and all("gemm_fast_kernel" in name or "gemm_pair_kernel" in name for name in found)
+    assert any("gemm_pair_kernel" in name for name in found) == (tile == "64x64k4")
     spilled = {name: k["vgpr_spill_count"] for name, k in found.items() if k["vgpr_spill_count"] > 2}
     assert not spilled, spilled
