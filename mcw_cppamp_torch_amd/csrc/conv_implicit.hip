@@ -234,14 +234,34 @@ GemmProblem gradweight_problem(long B, int C, int H, int W, int M, int kH, int k
     return p;
 }
 
+// gradInput's product where it goes through columns: one row per (input plane, tap), one column per output position.
+GemmProblem column_gradinput_problem(long B, int C, int M, int kH, int kW, int Ho, int Wo) {
+    const long N = (long)Ho * Wo, K = (long)C * kH * kW;
+    GemmProblem p;
+    p.a_rc = false;
+    p.sA = K;
+    p.sB = N;
+    p.bsB = (long)M * N;
+    p.sC = N;
+    p.bsC = K * N;
+    p.M = (int)K;
+    p.J = (int)(B * N);
+    p.N = (int)N;
+    p.R = M;
+    return p;
+}
+
 // What gradInput is rounded on columns: over the output planes in the product, over the taps that meet a pixel in col2im.  The
 // gathered product has one sum over both instead, M*kH*kW/16 steps on a tile that does not sum in two levels, and its results
 // were up to 1.7 times as far from 64 bits for it (44 -> 58 planes 5x5, 73 images 54x58: 1.78e-7, on columns 1.07e-7; 96 -> 256
 // planes 5x5, 64 images 27x27 in four parts: 1.90e-7, 1.24e-7).  Where columns are an alternative, the gathered product takes a
 // tile and split that round no more than they do (GemmProblem::max_roundings), or is not taken: these two layers 1.04e-7 and
 // 1.26e-7, 291 -> 331 and 390 -> 444 us (columns 666 and 505).
-double column_roundings(int M, int kH, int kW, double positions_per_pixel) {
-    return gemm_roundings((M + GEMM_BK - 1) / GEMM_BK) + gemm_roundings(kH * kW * positions_per_pixel);
+// (With few images the product on columns is itself on the tile of groups or split, whose sums are shorter than one over M/16
+// steps: its own plan is asked.)
+double column_roundings(long B, int C, int H, int W, int M, int kH, int kW, int Ho, int Wo) {
+    return gemm_plan_roundings(column_gradinput_problem(B, C, M, kH, kW, Ho, Wo)) +
+           gemm_roundings(kH * kW * ((double)Ho * Wo / ((double)H * W)));
 }
 
 // Unit stride only: one column per input pixel, one reduction index per (output plane, tap).
@@ -265,7 +285,7 @@ GemmProblem gradinput_problem(long B, int C, int H, int W, int M, int kH, int kW
     // Planes that fill 64-row tiles to eight ninths, little work on pixels that no position covers: gathered by every tile
     // (conv_use_gathered_gradinput).
     const bool fills = C >= 64 && (C + 63L) / 64 * 64 * 8 <= C * 9L && ((long)H * W - Ho * Wo) * M <= 110L * Ho * Wo;
-    if (!fills && conv_mode() == 1) p.max_roundings = column_roundings(M, kH, kW, (double)Ho * Wo / ((double)H * W));
+    if (!fills && conv_mode() == 1) p.max_roundings = column_roundings(B, C, H, W, M, kH, kW, Ho, Wo);
     return p;
 }
 
@@ -317,7 +337,7 @@ GemmProblem gradinput_strided_problem(long B, int C, int H, int W, int M, int kH
     p.tag = "gemm_conv_gradinput";
     // (residue classes that fill 64-row tiles with less than twice the layer's work: gathered by every tile)
     const bool fills = (q.rows < 64 ? 64.0 : q.rows) * q.A * q.Bk <= 2.0 * C * kH * kW;
-    if (!fills && conv_mode() == 1) p.max_roundings = column_roundings(M, kH, kW, (double)Ho * Wo / ((double)H * W));
+    if (!fills && conv_mode() == 1) p.max_roundings = column_roundings(B, C, H, W, M, kH, kW, Ho, Wo);
     return p;
 }
 
@@ -428,8 +448,8 @@ static bool gradinput_fits(long B, int C, int H, int W, int M, int kH, int kW, i
     return gemm_tiled_fits(gradinput_problem(B, C, H, W, M, kH, kW, pH, pW));
 }
 
-// Forward and gradWeight gather wherever a tiled kernel takes the product: the gathered products run at the rate of those on
-// columns, and the columns' trip through memory is saved.
+// Forward and gradWeight of 64 output planes and more gather wherever a tiled kernel takes the product: the gathered products
+// run at the rate of those on columns, and the columns' trip through memory is saved.
 bool conv_use_gathered(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
     const int mode = conv_mode();
     if (mode == 0 || !forward_fits(B, C, H, W, M, kH, kW, pH, pW, sH, sW)) return false;
@@ -462,19 +482,9 @@ static double gathered_gradinput_us(long B, int C, int H, int W, int M, int kH, 
 }
 
 static double column_gradinput_us(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
-    const long N = ((H + 2L * pH - kH) / sH + 1) * ((W + 2L * pW - kW) / sW + 1), K = (long)C * kH * kW;
-    GemmProblem p;
-    p.a_rc = false;
-    p.sA = K;
-    p.sB = N;
-    p.bsB = (long)M * N;
-    p.sC = N;
-    p.bsC = K * N;
-    p.M = (int)K;
-    p.J = (int)(B * N);
-    p.N = (int)N;
-    p.R = M;
-    return gemm_estimate_us(p) + 4.0 * B * (1.7 * K * N + (double)C * H * W) / 4.5e6;
+    const int Ho = (H + 2 * pH - kH) / sH + 1, Wo = (W + 2 * pW - kW) / sW + 1;
+    const long N = (long)Ho * Wo, K = (long)C * kH * kW;
+    return gemm_estimate_us(column_gradinput_problem(B, C, M, kH, kW, Ho, Wo)) + 4.0 * B * (1.7 * K * N + (double)C * H * W) / 4.5e6;
 }
 
 bool conv_use_gathered_gradinput(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
@@ -489,12 +499,24 @@ bool conv_use_gathered_gradinput(long B, int C, int H, int W, int M, int kH, int
     // columns are a third faster by estimate: their col2im is the part that the estimate knows least (3 -> 96 planes 11x11
     // stride 4, 24 to 128 images: columns 1.15 to 1.3 times the gathered time, and a fused stack saves the padded copy as well).
     double margin = 1.0;
+    GemmProblem p;
     if (strided) {
-        const GemmProblem p = gradinput_strided_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
+        p = gradinput_strided_problem(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
         if (p.max_roundings < 0.0 && p.J >= 16384) margin = 1.35;
     }
-    return gathered_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW) <=
-           margin * column_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
+    const double gathered = gathered_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
+    const double columns = column_gradinput_us(B, C, H, W, M, kH, kW, pH, pW, sH, sW);
+    if (gathered <= margin * columns) return true;
+    // A workgroup of the strided col2im walks sH*sW residue pairs one after the other, 0.7 us each where too few images hide it
+    // (one to sixteen 112x112 images: stride 2 1.5 us over the launch, 3 5, 4 11, 5 18).  On 1911 layers of few images whose
+    // classes fill the tiles, that explains 100 of the 105 that were gathered before there was an estimate and took longer on
+    // columns.  They gather again where the product is rounded no more than on columns: 38 layers, 1.58 times as fast (1.00
+    // to 2.25), 0.99 times as far from 64 bits.
+    if (!strided || !col2im_walks_classes(W, kH, kW, sH, sW)) return false;
+    const int Ho = (H + 2 * pH - kH) / sH + 1, Wo = (W + 2 * pW - kW) / sW + 1;
+    const double stream = 4.0 * B * C * ((double)kH * kW * Ho * Wo + (double)H * W) / 4.5e6, walk = 0.7 * sH * sW;
+    return walk > stream && gathered <= columns + (walk - stream) &&
+           gemm_plan_roundings(p) <= column_roundings(B, C, H, W, M, kH, kW, Ho, Wo);
 }
 
 long conv_implicit_gradinput_scratch(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH,

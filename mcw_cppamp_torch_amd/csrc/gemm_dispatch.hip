@@ -374,6 +374,12 @@ bool gemm_tiled_fits(const GemmProblem &p) {
     return (p.max_roundings >= 0.0 ? plan_gemm(p, steps_of(p)) : rank_plans(p, steps_of(p), true)).cfg != nullptr;
 }
 
+double gemm_plan_roundings(const GemmProblem &p) {
+    const GemmPlan plan = plan_gemm(p, steps_of(p));
+    // (the generic kernel takes reductions of less than a step, which count as one term)
+    return plan.cfg ? plan_roundings(*plan.cfg, (long)p.M * p.J, steps_of(p), plan.nsplit) : gemm_roundings(steps_of(p));
+}
+
 double gemm_estimate_us(const GemmProblem &p) {
     const GemmPlan plan = plan_gemm(p, steps_of(p));
     if (plan.cfg) return plan.cycles / 2400.0;

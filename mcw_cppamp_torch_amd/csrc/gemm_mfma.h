@@ -107,13 +107,15 @@ struct GemmProblem {
 int gemm_launch(const GemmProblem &p);
 // Two products, neither of which reads what the other writes, in fewer launches.
 int gemm_launch_pair(const GemmProblem &a, const GemmProblem &b);
-// Whether one of the tiled kernels takes the problem (shape at least a tile, operand and output offsets
-// within the kernels' 32-bit addressing, a tile the tuning switches allow): the test a gathered second
+// Whether one of the tiled kernels takes the problem (a reduction of at least a step, operand and output offsets
+// within the kernels' 32-bit addressing, a tile the tuning switches and max_roundings allow): the test a gathered second
 // operand, which has no generic kernel, must pass before it is launched.
 bool gemm_tiled_fits(const GemmProblem &p);
 // The planner's estimate of the launch (and of the reduction of its partial sums), in microseconds: for choosing between
 // two ways to the same result.
 double gemm_estimate_us(const GemmProblem &p);
+// How often the results of the planner's tile and split are rounded (gemm_roundings).
+double gemm_plan_roundings(const GemmProblem &p);
 
 // ---- shared between the kernel translation units ------------------------------
 

@@ -715,6 +715,11 @@ long im2col_plan_selftest() {
     return bad;
 }
 
+// Whether the kernel that walks the residue pairs of the pixel coordinates takes a layer.
+bool col2im_walks_classes(int W, int kH, int kW, int sH, int sW) {
+    return !tuning().col2im_generic && (sW > 1 || sH > 1) && W >= 64 && (kH + sH - 1) / sH <= 3 && (kW + sW - 1) / sW <= 3;
+}
+
 int col2im_launch(const float *col, long B, int C, int H, int W, int kH, int kW, int pH, int pW, int sH, int sW,
                   float *im, InputMask mask) {
     ConvGeom g;
@@ -744,7 +749,7 @@ int col2im_launch(const float *col, long B, int C, int H, int W, int kH, int kW,
     }
     const int th = (kH + sH - 1) / sH, tw = (kW + sW - 1) / sW;
     const int Qh = (H - 1 + pH) / sH + 1, Qw = (W - 1 + pW) / sW + 1;  // quotient ranges of (h+pH)/sH, (w+pW)/sW
-    if (!tuning().col2im_generic && (sW > 1 || sH > 1) && W >= 64 && th <= 3 && tw <= 3) {
+    if (col2im_walks_classes(W, kH, kW, sH, sW)) {
         // R quotient rows per workgroup: about 256 (qh, qw) pairs, image rows within the LDS budget
         int R = 256 / Qw;
         if (R < 1) R = 1;

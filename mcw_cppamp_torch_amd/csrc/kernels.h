@@ -38,6 +38,7 @@ int im2col_launch(const float *im, long B, int C, int H, int W, int kH, int kW, 
                   float *col);
 int col2im_launch(const float *col, long B, int C, int H, int W, int kH, int kW, int pH, int pW, int sH, int sW,
                   float *im, InputMask mask = InputMask());
+bool col2im_walks_classes(int W, int kH, int kW, int sH, int sW);
 // out_plane / out_pitch: floats between the output's planes and rows when it is not densely packed (0: dense).
 int maxpool_fwd_launch(const float *in, long planes, int H, int W, int kH, int kW, int dH, int dW, float *out,
                        float *indices, long out_plane = 0, int out_pitch = 0);

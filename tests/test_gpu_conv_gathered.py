@@ -875,7 +875,8 @@ def relative_error(got, ref):
 
 @pytest.mark.parametrize("layer", [(16, 44, 54, 58, 58, 5, 5, 2, 2, 1, 1), (8, 151, 42, 42, 48, 3, 3, 1, 1, 1, 1),
                                    (57, 134, 19, 19, 55, 3, 3, 0, 0, 1, 1), (64, 96, 27, 27, 256, 5, 5, 2, 2, 1, 1),
-                                   (37, 57, 20, 20, 51, 3, 3, 0, 0, 1, 1), (4, 40, 33, 35, 24, 5, 5, 2, 2, 4, 4)])
+                                   (37, 57, 20, 20, 51, 3, 3, 0, 0, 1, 1), (4, 40, 33, 35, 24, 5, 5, 2, 2, 4, 4),
+                                   (2, 3, 112, 112, 16, 11, 11, 2, 2, 4, 4), (8, 4, 112, 112, 96, 8, 8, 2, 2, 4, 4)])
 def test_gradinput_is_as_near_to_64_bits_as_on_columns(gt, layer):
     """Layers whose planes do not fill 64-row tiles, on whichever route the library takes.  Both sides round the same products
     of the same parts and differ in the order of the additions, which the planner holds to no more in a row than columns
@@ -904,6 +905,36 @@ def test_gradinput_is_as_near_to_64_bits_as_on_columns(gt, layer):
         assert lib.thgpu_conv_set_mode(before) == 0
     print(layer, errors)
     assert errors[1] <= 1.05 * errors[0]
+
+
+@pytest.mark.parametrize("layer,gathers", [((2, 3, 112, 112, 16, 11, 11, 2, 2, 4, 4), True), ((8, 4, 112, 112, 96, 8, 8, 2, 2, 4, 4), True),
+                                           ((2, 3, 82, 97, 181, 3, 3, 1, 1, 3, 3), True),
+                                           ((8, 3, 112, 112, 64, 11, 11, 2, 2, 4, 4), False),   # rounded more often than columns
+                                           ((1, 8, 56, 56, 48, 9, 9, 4, 4, 4, 4), False)])      # another col2im, no long walk
+def test_strided_layers_of_few_images_gather_where_col2im_is_a_long_walk(gt, layer, gathers):
+    """The library's own choice, bit for bit on small integers."""
+    B, C, H, W, M, kH, kW, pH, pW, sH, sW = layer
+    rng = rng_for(55)
+    Ho, Wo = (H + 2 * pH - kH) // sH + 1, (W + 2 * pW - kW) // sW + 1
+    go = rng.integers(-2, 3, size=(B, M, Ho, Wo)).astype(np.float32)
+    w = rng.integers(-2, 3, size=(M, C * kH * kW)).astype(np.float32)
+    m = gt.nn.SpatialConvolutionMM(C, M, kW, kH, sW, sH, 0, padW=pW, padH=pH)
+    m._assign("weight", w)
+    m.gpu()
+    lib = gt._lib.lib
+    before = lib.thgpu_conv_get_mode()
+    assert lib.thgpu_conv_set_mode(1) == 0
+    gt.gputorch.prof_reset()
+    gt.gputorch.prof_enable(True)
+    try:
+        got = m.updateGradInput(gt.GPUTensor(B, C, H, W).fill(0), dev(gt, go)).float()
+        labels = list(gt.gputorch.prof_report())
+    finally:
+        gt.gputorch.prof_enable(False)
+        gt.gputorch.prof_reset()
+        assert lib.thgpu_conv_set_mode(before) == 0
+    assert any(l.startswith("col2im") for l in labels) != gathers, labels
+    assert np.array_equal(got, oracle.conv_updateGradInput(go, w, (B, C, H, W), kH, kW, pH, pW, sH, sW)[0])
 
 
 def test_gradweight_of_groups_is_as_near_to_64_bits_as_of_parts(gt, switches):
