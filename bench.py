@@ -508,13 +508,13 @@ def summarise(args):
             key = (_short(r["Kernel_Name"]), r["Grid_Size"])
             agg.setdefault(key, collections.defaultdict(float))[r["Counter_Name"]] += float(r["Counter_Value"])
             agg[key]["_n_" + r["Counter_Name"]] += 1
-        out.append("%-58s %9s %9s %9s %9s %9s" % ("kernel (grid)", "launches", "mfma_busy", "wait_any", "wait_lds", "lds_confl"))
+        out.append("%-66s %9s %9s %9s %9s %9s" % ("kernel (grid)", "launches", "mfma_busy", "wait_any", "wait_lds", "lds_confl"))
         for (name, grid), c in agg.items():
             n = c["_n_SQ_BUSY_CU_CYCLES"] or 1
             busy = c["SQ_VALU_MFMA_BUSY_CYCLES"] / max(c["SQ_BUSY_CU_CYCLES"], 1) / 4   # per SIMD of a busy CU
             wave = max(c["SQ_WAVE_CYCLES"], 1)
-            out.append("%-58s %9d %8.1f%% %8.1f%% %8.1f%% %8.2f%%" % (
-                ("%s (%s)" % (name, grid))[:58], n, 100 * busy, 100 * c["SQ_WAIT_INST_ANY"] / wave,
+            out.append("%-66s %9d %8.1f%% %8.1f%% %8.1f%% %8.2f%%" % (
+                ("%s (%s)" % (name, grid))[:66], n, 100 * busy, 100 * c["SQ_WAIT_INST_ANY"] / wave,
                 100 * c["SQ_WAIT_INST_LDS"] / wave, 100 * c["SQ_LDS_BANK_CONFLICT"] / max(c["SQ_ACTIVE_INST_LDS"], 1)))
         out.append("mfma_busy = SQ_VALU_MFMA_BUSY_CYCLES / (4 * SQ_BUSY_CU_CYCLES); wait_* = SQ_WAIT_INST_* / SQ_WAVE_CYCLES; "
                    "lds_confl = SQ_LDS_BANK_CONFLICT / SQ_ACTIVE_INST_LDS.")
