@@ -521,8 +521,11 @@ int thgpu_conv_gathers(long B, int C, int H, int W, int M, int kW, int kH, int d
  *   mode 0: that route; finput and fgradInput hold the K x N columns as in the reference.
  *   mode 1 (initial): per layer and pass, the GEMM gathers its second operand from a zero-padded copy
  *           of the image and no columns exist, where the shape allows it and it is the faster route
- *           (forward and gradWeight: wherever a tiled kernel takes the product; gradInput: by the time that either
- *           route is estimated to take); the column route otherwise.
+ *           (forward and gradWeight: wherever a tiled kernel takes the product, with fewer than 64 output planes only
+ *           unpadded or from 256 output positions and 512 KiB of columns on; gradInput: unit-stride layers whose input planes
+ *           fill 64-row tiles, others by the time that either route is estimated to take; layers that do not fill such
+ *           tiles, and strided ones that few images alone make faster, only where the gathered product's results are
+ *           rounded no more often); the column route otherwise.
  *   mode 2: gathered wherever the shape allows it and fills 64-row tiles (64 output planes; 64 input planes for the
  *           gradInput of a unit-stride layer).
  * On the gathered route finput holds the padded input ([B,] C, H+2padH, W+2padW) and fgradInput the

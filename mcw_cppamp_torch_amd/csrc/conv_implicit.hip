@@ -468,10 +468,10 @@ bool conv_use_gathered(long B, int C, int H, int W, int M, int kH, int kW, int p
 // 4.5 TB/s and for the re-ordering of the kernel bank at 3.  The gathered product has one row per input plane (and residue
 // class) in tiles of 32 or 64 and one column per input pixel; the product on columns is often bound by writing them, of which
 // the estimate sees a part.  Over 329 layers (1 to 128 images, 3 to 1024 input planes, kernels of 3 to 11, strides of 1, 2 and 4),
-// both sides measured, the smaller estimate costs 0.6 % over the better side, at most 21 % (1.2 % with the two exceptions in
-// conv_use_gathered_gradinput).  A rule on the excess of work stood here, which cost up to 10 times the time where a
-// strided layer has few pixels and a long reduction: its product cannot be split, and a handful of workgroups walked it
-// (16 -> 384 planes 7x7 stride 2, two 16x20 images: 17 us on columns, 198).
+// both sides measured, the smaller estimate costs 0.6 % over the better side, at most 21 % (1.2 % with the exceptions in
+// conv_use_gathered_gradinput), before the limit on roundings.  A rule on the excess of work stood here, which cost up to 10
+// times the time where a strided layer has few pixels and a long reduction: its product cannot be split, and a handful of
+// workgroups walked it (16 -> 384 planes 7x7 stride 2, two 16x20 images: 17 us on columns, 198).
 static double gathered_gradinput_us(long B, int C, int H, int W, int M, int kH, int kW, int pH, int pW, int sH, int sW) {
     const long N = ((H + 2L * pH - kH) / sH + 1) * ((W + 2L * pW - kW) / sW + 1);
     int top, left, Hq, Wq;
@@ -492,12 +492,14 @@ bool conv_use_gathered_gradinput(long B, int C, int H, int W, int M, int kH, int
     if (mode == 0 || !gradinput_fits(B, C, H, W, M, kH, kW, pH, pW, sH, sW)) return false;
     const bool strided = sH != 1 || sW != 1;
     if (mode == 2) return strided || C >= 64;
-    // Unit stride, planes that fill 64-row tiles, little work on pixels that no position covers: gathered, on any tile (for single
-    // images too, where the columns are up to 30 % faster).
+    // Unit stride, planes that fill 64-row tiles, little work on pixels that no position covers: gathered, on any tile.  Over 400
+    // such layers of one to six images that takes 1.01 times as long as columns (1.10 at one image, at most 1.78) and is 0.86
+    // times as far from 64 bits (at most 1.16); where it is slower, 0.91 times.
     if (!strided && gradinput_problem(B, C, H, W, M, kH, kW, pH, pW).max_roundings < 0.0) return true;
     // A strided layer whose residue classes take less than twice its work and fill the GPU keeps the one product until the
-    // columns are a third faster by estimate: their col2im is the part that the estimate knows least (3 -> 96 planes 11x11
-    // stride 4, 24 to 128 images: columns 1.15 to 1.3 times the gathered time, and a fused stack saves the padded copy as well).
+    // columns are a third faster by estimate.  Between the two lines neither route is faster (21 of 132 layers with kernels of 2 to
+    // 11, strides of 2 to 4 and 32 to 192 planes: columns 0.83 to 1.19 times the gathered time, 1.00 in the mean), and a fused
+    // stack saves the padded copy as well; twice the estimate would cost 2 % over the better side.
     double margin = 1.0;
     GemmProblem p;
     if (strided) {
